@@ -63,6 +63,9 @@ SIGNATURES: dict[str, list] = {
     "hsn_gather_concat_bwd": [P, P, P, P, P, P, I, I, I, I, I, I, P],
     "hsn_grouped_unit_mlp_fwd": [P, P, P, P, P, P, P, P, I, I, I, I, I, P],
     "hsn_grouped_unit_mlp_bwd": [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, P],
+    "hsn_grouped_unit_mlp_workspace": [I, I, I, I, I, I, P],
+    "hsn_grouped_unit_mlp_fwd_ws": [P, P, I, P, P, P, P, P, P, I, I, I, I, I, P, L, P],
+    "hsn_grouped_unit_mlp_bwd_ws": [P, P, I, P, P, P, P, P, P, P, P, P, I, I, I, I, I, P, L, P],
     "hsn_csr_messages": [P, P, P, P, P, P, P, I, I, I, I, I, I, P],
     "hsn_csr_messages_bwd": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P],
     "hsn_gated_delta_update": [P, P, P, P, P, P, P, P, I, I, I, I, I, P],

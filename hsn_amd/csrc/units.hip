@@ -20,6 +20,7 @@
 
 #include "../../include/hsn_ops.h"
 #include "abi_util.h"
+#include "unit_math.cuh"
 
 namespace hsn {
 // Raise a kernel's dynamic-LDS limit to 160 KiB once per (kernel, device) (runtime.cpp).
@@ -31,16 +32,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ v4f mfma(float a, float b, v4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-constexpr float kRsqrt2 = 0.70710678118654752f;
-constexpr float kRsqrt2Pi = 0.39894228040143268f;
-
-// The exact GELU x/2 (1 + erf(x / sqrt 2)) and its derivative Phi(x) + x phi(x)
-// (kernels/include/hsn_ops.h:104-113), from the device library's erff / expf.
-__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erff(x * kRsqrt2)); }
-__device__ __forceinline__ float gelu_grad(float x) {
-    return 0.5f * (1.0f + erff(x * kRsqrt2)) + x * expf(-0.5f * x * x) * kRsqrt2Pi;
 }
 
 // The next (up to) 16 pairs p >= cur of unit j, in order: lane i < n holds the i-th, `cur`

@@ -24,6 +24,8 @@ raises.
 
 from __future__ import annotations
 
+import ctypes
+import functools
 from typing import Any, Optional
 
 import torch
@@ -307,12 +309,44 @@ state_update_op.register_autograd(_update_grad, setup_context=_update_setup)
 # --------------------------------------------------------------------------------------------
 
 
+@functools.lru_cache(maxsize=1024)
+def _mlp_workspace_bytes(P: int, M: int, d: int, H: int, code: int, backward: int) -> int:
+    """The workspace of the products over the pairs in unit order; 0 for a shape they do not take
+    (host arithmetic)."""
+    out = ctypes.c_int64(0)
+    call("hsn_grouped_unit_mlp_workspace", P, M, d, H, code, backward, ctypes.byref(out))
+    return int(out.value)
+
+
+def _mlp_space(P: int, M: int, d: int, H: int, backward: int, idx: Tensor, v: Tensor,
+               *operands: Tensor) -> Optional[tuple[Tensor, int, Tensor, int]]:
+    """``(idx, its bits, workspace, bytes)`` of a call of the products in unit order, or ``None``
+    where the kernels without a workspace take it: another shape, operands off four-element
+    alignment (a view into a buffer), or indices neither int32 nor int64."""
+    if idx.dtype not in (torch.int32, torch.int64):
+        return None
+    nbytes = _mlp_workspace_bytes(P, M, d, H, _code(v), backward)
+    step = 4 * v.element_size()
+    if nbytes == 0 or any(t.data_ptr() % step for t in (v, *operands)):
+        return None
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=v.device)
+    return idx.contiguous(), 64 if idx.dtype == torch.int64 else 32, ws, nbytes
+
+
 def _mlp_body(v: Tensor, idx: Tensor, w1: Tensor, b1: Tensor, w2: Tensor,
               b2: Tensor) -> tuple[Tensor, Tensor]:
     P, M, d, H = v.shape[0], w1.shape[0], w2.shape[2], w1.shape[2]
-    v, idx, w1, b1, w2, b2 = (v.contiguous(), _i32(idx), w1.contiguous(), b1.contiguous(),
-                              w2.contiguous(), b2.contiguous())
+    v, w1, b1, w2, b2 = (v.contiguous(), w1.contiguous(), b1.contiguous(), w2.contiguous(),
+                         b2.contiguous())
     out, hidden = v.new_empty((P, d)), v.new_empty((P, H))
+    space = _mlp_space(P, M, d, H, 0, idx, v, w1, w2)
+    if space is not None:
+        idx, bits, ws, nbytes = space
+        call("hsn_grouped_unit_mlp_fwd_ws", ptr(v), ptr(idx), bits, ptr(w1), ptr(b1), ptr(w2),
+             ptr(b2), ptr(hidden), ptr(out), P, M, d, H, _code(v), ptr(ws), nbytes,
+             stream_of(v.device))
+        return out, hidden
+    idx = _i32(idx)
     call("hsn_grouped_unit_mlp_fwd", ptr(v), ptr(idx), ptr(w1), ptr(b1), ptr(w2), ptr(b2),
          ptr(hidden), ptr(out), P, M, d, H, _code(v), stream_of(v.device))
     return out, hidden
@@ -334,10 +368,18 @@ def _mlp_fake(v, idx, w1, b1, w2, b2):
 def _mlp_bwd_body(v: Tensor, idx: Tensor, w1: Tensor, w2: Tensor, hidden: Tensor,
                   dout: Tensor) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
     P, M, d, H = v.shape[0], w1.shape[0], w2.shape[2], w1.shape[2]
-    v, idx, w1, w2, hidden, dout = (v.contiguous(), _i32(idx), w1.contiguous(), w2.contiguous(),
-                                    hidden.contiguous(), dout.contiguous())
+    v, w1, w2, hidden, dout = (v.contiguous(), w1.contiguous(), w2.contiguous(),
+                               hidden.contiguous(), dout.contiguous())
     dv, dw1, dw2 = torch.empty_like(v), torch.empty_like(w1), torch.empty_like(w2)
     db1, db2 = w1.new_empty((M, H)), w2.new_empty((M, d))
+    space = _mlp_space(P, M, d, H, 1, idx, v, w1, w2, dout)
+    if space is not None:
+        idx, bits, ws, nbytes = space
+        call("hsn_grouped_unit_mlp_bwd_ws", ptr(v), ptr(idx), bits, ptr(w1), ptr(w2), ptr(hidden),
+             ptr(dout), ptr(dv), ptr(dw1), ptr(db1), ptr(dw2), ptr(db2), P, M, d, H, _code(v),
+             ptr(ws), nbytes, stream_of(v.device))
+        return dv, dw1, db1, dw2, db2
+    idx = _i32(idx)
     call("hsn_grouped_unit_mlp_bwd", ptr(v), ptr(idx), ptr(w1), ptr(w2), ptr(hidden), ptr(dout),
          ptr(dv), ptr(dw1), ptr(db1), ptr(dw2), ptr(db2), P, M, d, H, _code(v), 1,
          stream_of(v.device))

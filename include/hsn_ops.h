@@ -81,6 +81,31 @@ int hsn_grouped_unit_mlp_bwd(const void* v, const int32_t* unit_idx, const void*
                              int deterministic, void* stream);
 
 /*
+ * The grouped unit MLP and its backward on a workspace: the same contract and results as
+ * hsn_grouped_unit_mlp_{fwd,bwd} up to the order of the fp32 sums, as matrix products over the
+ * pairs in unit order (64-column tiles, each unit's weights read once a tile of 32 or 64 pairs).
+ * unit_idx [P] is int32_t or int64_t (`index_bits`); a pair whose unit lies outside [0,M) takes
+ * part in nothing and gets no output. hsn_grouped_unit_mlp_workspace gives the bytes (`backward`
+ * 0 or 1), or 0 for a shape these do not take: M <= 1024, d a multiple of 4 up to 256, H a
+ * multiple of 4. The operands must be aligned to four elements, the workspace to 256 bytes. The
+ * workspace's contents before the call do not matter, and nothing is kept in it after it. Every
+ * sum has a fixed order.
+ */
+int hsn_grouped_unit_mlp_workspace(int P, int M, int d, int H, int dtype, int backward,
+                                   int64_t* bytes);
+int hsn_grouped_unit_mlp_fwd_ws(const void* v, const void* unit_idx, int index_bits,
+                                const void* W1, const void* b1, const void* W2, const void* b2,
+                                void* hidden_saved, void* out, int P, int M, int d, int H,
+                                int dtype, void* workspace, int64_t workspace_bytes,
+                                void* stream);
+int hsn_grouped_unit_mlp_bwd_ws(const void* v, const void* unit_idx, int index_bits,
+                                const void* W1, const void* W2, const void* hidden_saved,
+                                const void* grad_out, void* grad_v, void* grad_W1, void* grad_b1,
+                                void* grad_W2, void* grad_b2, int P, int M, int d, int H,
+                                int dtype, void* workspace, int64_t workspace_bytes,
+                                void* stream);
+
+/*
  * The CSR neighbour messages (reference hsn_ops.h:132-143): i = cell_idx[r,k],
  *   m[r,k,:] = sum_{e in [indptr[i], indptr[i+1])} a[e] (V h[r, indices[e], :]),
  * V [d,d] as [d_out, d_in]. h [B,N,d]; indptr [N+1]; indices, a [E]; cell_idx [B,K] (repeats

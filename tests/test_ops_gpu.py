@@ -413,3 +413,63 @@ def test_unit_mlp_forward_paths_match_oracle(ops, cuda_device, P, M, d, H):
         bar = 1e-5 * (max(1.0, (P / M / 64) ** 0.5) if name[1] in "Wb" else 1.0)
         err = (got.double().cpu() - want).abs() / want.abs().clamp(min=1.0)
         assert float(err.max()) <= bar, f"{name}: worst {float(err.max()):.3e} (bar {bar:.1e})"
+
+
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("counts,d,H", [
+    ([1], 4, 4),                   # the smallest: one pair
+    ([31, 0, 32, 33], 16, 68),     # around the 32-row tile, a unit without pairs, a hidden tail of 4
+    ([5, 700, 64], 36, 100),       # 4d = 144 and d off the 64-column tiles, a unit of two blocks
+    ([1500], 64, 128),             # one unit of several blocks
+    ([3] * 70, 8, 64),             # more units than a wavefront's lanes
+])
+def test_unit_mlp_in_unit_order_matches_oracle(ops, cuda_device, counts, d, H, dtype, index):
+    """The products over the pairs in unit order at the edges of their tiles, blocks and units,
+    with pairs whose unit lies outside the bank: those take part in nothing (their rows of
+    ``hidden``, ``out`` and ``grad_v`` are not written). Against the float64 oracle on the same
+    rounded inputs; the weight gradients' bar grows with the square root of a unit's pairs."""
+    from oracle import hsn_oracle as O
+
+    g = torch.Generator().manual_seed(len(counts) * 1000 + d)
+    M = len(counts)
+    idx = torch.repeat_interleave(torch.arange(M), torch.tensor(counts))
+    idx = idx[torch.randperm(idx.numel(), generator=g)]
+    outside = torch.tensor([-1, M, 2**31 - 1])
+    all_idx = torch.cat([idx[:1], outside, idx[1:]]) if idx.numel() > 1 else idx
+    kept = (all_idx >= 0) & (all_idx < M)
+    P = all_idx.numel()
+    rnd = lambda *s, scale=0.5: (torch.randn(*s, generator=g) * scale).to(dtype)  # noqa: E731
+    v, W1, b1 = rnd(P, 4 * d), rnd(M, 4 * d, H, scale=(4 * d) ** -0.5), rnd(M, H)
+    W2, b2, dout = rnd(M, H, d, scale=H ** -0.5), rnd(M, d), rnd(P, d)
+    dev = cuda_device
+    D = [t.to(dev) for t in (v, all_idx.to(index), W1, b1, W2, b2)]
+    out, hidden = ops.mlp_op(*D)
+    got = ops.mlp_backward(D[0], D[1], D[2], D[4], hidden, dout.to(dev))
+    f64 = [t.double() for t in (v[kept], W1, b1, W2, b2, dout[kept])]
+    want_out, want_h = O.grouped_unit_mlp(f64[0], idx, *f64[1:5])
+    _close(hidden.cpu()[kept], want_h, dtype, "hidden")
+    _close(out.cpu()[kept], want_out, dtype, "out")
+    want = O.grouped_unit_mlp_bwd(f64[0], idx, f64[1], f64[3], hidden.cpu()[kept].double(), f64[5])
+    _close(got[0].cpu()[kept], want[0], dtype, "grad_v")
+    bar = TOL[dtype] * max(1.0, (max(counts) / 64) ** 0.5)
+    for name, g_, w_ in zip(("dW1", "db1", "dW2", "db2"), got[1:], want[1:]):
+        err = (g_.double().cpu() - w_).abs() / w_.abs().clamp(min=1.0)
+        assert float(err.max()) <= bar, f"{name}: worst {float(err.max()):.3e} (bar {bar:.1e})"
+    again = ops.mlp_backward(D[0], D[1], D[2], D[4], hidden, dout.to(dev))
+    for a, b in zip(got[1:], again[1:]):
+        assert torch.equal(a, b)  # every sum has a fixed order
+
+
+def test_unit_mlp_takes_operands_off_the_four_element_alignment(ops, cuda_device):
+    """A view into a buffer, one element in: the kernels without a workspace take it, with the
+    same results up to the order of the fp32 sums."""
+    g = torch.Generator().manual_seed(5)
+    P, M, d, H = 40, 3, 16, 64
+    dev = cuda_device
+    rnd = lambda *s: (torch.randn(*s, generator=g) * 0.3).to(dev)  # noqa: E731
+    v, W1, b1, W2, b2 = rnd(P, 4 * d), rnd(M, 4 * d, H), rnd(M, H), rnd(M, H, d), rnd(M, d)
+    idx = torch.randint(0, M, (P,), generator=g).to(dev)
+    shifted = torch.empty(v.numel() + 1, device=dev)[1:].view(P, 4 * d).copy_(v)
+    for a, b in zip(ops.mlp_op(v, idx, W1, b1, W2, b2), ops.mlp_op(shifted, idx, W1, b1, W2, b2)):
+        torch.testing.assert_close(a, b, atol=1e-5, rtol=1e-5)
