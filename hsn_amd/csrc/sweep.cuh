@@ -1383,69 +1383,10 @@ __global__ __launch_bounds__(kWave* kMaxChunks) void bwd_chunk(BwdArgs a) {
     if (w == 0 && dq0 && kslot == 0) dq0[int64_t(b) * d + col] = static_cast<float>(R_out);
 }
 
-// ------------------------------------------------------------------------------------------
-// The RMS candidate: a prologue normalises the candidate input once (the only cross-column
-// quantity of the round, computed from inputs only), an epilogue applies the norm's VJP.
-// ------------------------------------------------------------------------------------------
-
 // The RMS workspace: [slots, d] of the storage type, then [slots] fp32 of 1/rms at a 16-byte
 // aligned offset.
 inline size_t rms_inv_offset(int64_t slots, int d, size_t elem) {
     return (size_t(slots) * size_t(d) * elem + 15) & ~size_t(15);
-}
-
-// ynorm[s, x] = y[s, x] * inv[s] * w[x],  inv[s] = rsqrt(mean_x y^2 + eps): a wavefront per slot
-template <typename IN>
-__global__ __launch_bounds__(256) void rms_prologue(const IN* y, const float* w, IN* ynorm,
-                                                    float* inv, int64_t slots, int d, float eps) {
-    const int64_t s = int64_t(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave;
-    if (s >= slots) return;
-    const int lane = lane_id();
-    float sum = 0.0f;
-    for (int x = lane; x < d; x += kWave) {
-        const float v = to_f32(y[s * d + x]);
-        sum += v * v;
-    }
-    for (int m = 1; m < kWave; m <<= 1) sum += __shfl_xor(sum, m, kWave);
-    const float r = rsqrtf(sum / static_cast<float>(d) + eps);
-    if (lane == 0) inv[s] = r;
-    for (int x = lane; x < d; x += kWave) store_f32(ynorm, s * d + x, to_f32(y[s * d + x]) * r * w[x]);
-}
-
-// dL/dw[x] = sum over slots of dpre[x] y[x] inv (one workgroup per column, fixed-shape tree)
-template <typename IN>
-__global__ __launch_bounds__(256) void rms_weight_grad(const IN* y, const IN* dpre, const float* inv,
-                                                       float* dw, int64_t slots, int d) {
-    __shared__ float part[256];
-    const int x = blockIdx.x;
-    float acc = 0.0f;
-    for (int64_t s = threadIdx.x; s < slots; s += blockDim.x)
-        acc += to_f32(dpre[s * d + x]) * to_f32(y[s * d + x]) * inv[s];
-    part[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) dw[x] = part[0];
-}
-
-// dy[x] = inv w[x] dpre[x] - inv^3 y[x] / d * sum_x' dpre[x'] w[x'] y[x'], in place over dpre
-template <typename IN>
-__global__ __launch_bounds__(256) void rms_input_grad(const IN* y, IN* dy, const float* inv,
-                                                      const float* w, int64_t slots, int d) {
-    const int64_t s = int64_t(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave;
-    if (s >= slots) return;
-    const int lane = lane_id();
-    const float r = inv[s];
-    float dot = 0.0f;
-    for (int x = lane; x < d; x += kWave) dot += to_f32(dy[s * d + x]) * w[x] * to_f32(y[s * d + x]);
-    for (int m = 1; m < kWave; m <<= 1) dot += __shfl_xor(dot, m, kWave);
-    const float k3 = r * r * r * dot / static_cast<float>(d);
-    for (int x = lane; x < d; x += kWave) {
-        const float v = r * w[x] * to_f32(dy[s * d + x]) - k3 * to_f32(y[s * d + x]);
-        store_f32(dy, s * d + x, v);
-    }
 }
 
 namespace {

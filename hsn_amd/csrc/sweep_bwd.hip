@@ -6,6 +6,7 @@
 #include "sweep.cuh"
 #include "abi_util.h"
 #include "chain_host.h"
+#include "rms.cuh"
 
 using namespace hsn;
 
@@ -92,16 +93,12 @@ extern "C" int hsn_win_backward(const void* y, const void* gate_pre, const void*
     if (cand_norm) {  // the normalised candidate input (the forward's, recomputed)
         void* rms_scratch = ws + L.rms;
         inv = reinterpret_cast<float*>(static_cast<char*>(rms_scratch) + rms_inv_offset(nslots, d, elem));
-        const int blocks = static_cast<int>((nslots + 3) / 4);
         if (io_dtype == HSN_DTYPE_F32)
-            hipLaunchKernelGGL((rms_prologue<float>), dim3(blocks), dim3(256), 0, st,
-                               static_cast<const float*>(y), cand_w,
-                               static_cast<float*>(rms_scratch), inv, nslots, d, cand_eps);
+            rms::launch_prologue(static_cast<const float*>(y), cand_w, static_cast<float*>(rms_scratch),
+                                 inv, nslots, d, cand_eps, st);
         else
-            hipLaunchKernelGGL((rms_prologue<bf16_t>), dim3(blocks), dim3(256), 0, st,
-                               static_cast<const bf16_t*>(y), cand_w,
-                               static_cast<bf16_t*>(rms_scratch), inv, nslots, d, cand_eps);
-        HSN_HIP(hipGetLastError());
+            rms::launch_prologue(static_cast<const bf16_t*>(y), cand_w, static_cast<bf16_t*>(rms_scratch),
+                                 inv, nslots, d, cand_eps, st);
         pre = rms_scratch;
     }
     if (L.evmap) {
@@ -125,25 +122,12 @@ extern "C" int hsn_win_backward(const void* y, const void* gate_pre, const void*
             HSN_HIP((launch_bwd<bf16_t, Packed32, true>(a, g.S, lds, st)));
     }
     if (cand_norm) {  // the norm's VJP: dy holds dL/dpre
-        const int blocks = static_cast<int>((nslots + 3) / 4);
-        if (io_dtype == HSN_DTYPE_F32) {
-            if (d_cand_w)
-                hipLaunchKernelGGL((rms_weight_grad<float>), dim3(d), dim3(256), 0, st,
-                                   static_cast<const float*>(y), static_cast<const float*>(dy), inv,
-                                   d_cand_w, nslots, d);
-            hipLaunchKernelGGL((rms_input_grad<float>), dim3(blocks), dim3(256), 0, st,
-                               static_cast<const float*>(y), static_cast<float*>(dy), inv, cand_w,
-                               nslots, d);
-        } else {
-            if (d_cand_w)
-                hipLaunchKernelGGL((rms_weight_grad<bf16_t>), dim3(d), dim3(256), 0, st,
-                                   static_cast<const bf16_t*>(y), static_cast<const bf16_t*>(dy),
-                                   inv, d_cand_w, nslots, d);
-            hipLaunchKernelGGL((rms_input_grad<bf16_t>), dim3(blocks), dim3(256), 0, st,
-                               static_cast<const bf16_t*>(y), static_cast<bf16_t*>(dy), inv,
-                               cand_w, nslots, d);
-        }
-        HSN_HIP(hipGetLastError());
+        if (io_dtype == HSN_DTYPE_F32)
+            rms::launch_vjp(static_cast<const float*>(y), static_cast<float*>(dy), inv, cand_w, d_cand_w,
+                            reinterpret_cast<float*>(ws + L.rms), nslots, d, st);
+        else
+            rms::launch_vjp(static_cast<const bf16_t*>(y), static_cast<bf16_t*>(dy), inv, cand_w, d_cand_w,
+                            reinterpret_cast<bf16_t*>(ws + L.rms), nslots, d, st);
     }
     HSN_ABI_END
 }

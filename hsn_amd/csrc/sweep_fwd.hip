@@ -7,6 +7,7 @@
 #include "sweep.cuh"
 #include "abi_util.h"
 #include "chain_host.h"
+#include "rms.cuh"
 
 using namespace hsn;
 
@@ -16,17 +17,14 @@ namespace {
 // (layout: rms_inv_offset) and returns it.
 const void* rms_normalise(const void* y, int io_dtype, const float* cand_w, float cand_eps,
                           void* ws, int64_t slots, int d, hipStream_t st) {
-    const int blocks = static_cast<int>((slots + 3) / 4);
     const size_t elem = io_dtype == HSN_DTYPE_F32 ? 4 : 2;
     float* inv = reinterpret_cast<float*>(static_cast<char*>(ws) + rms_inv_offset(slots, d, elem));
     if (io_dtype == HSN_DTYPE_F32)
-        hipLaunchKernelGGL((rms_prologue<float>), dim3(blocks), dim3(256), 0, st,
-                           static_cast<const float*>(y), cand_w, static_cast<float*>(ws), inv,
-                           slots, d, cand_eps);
+        rms::launch_prologue(static_cast<const float*>(y), cand_w, static_cast<float*>(ws), inv, slots, d,
+                             cand_eps, st);
     else
-        hipLaunchKernelGGL((rms_prologue<bf16_t>), dim3(blocks), dim3(256), 0, st,
-                           static_cast<const bf16_t*>(y), cand_w, static_cast<bf16_t*>(ws),
-                           inv, slots, d, cand_eps);
+        rms::launch_prologue(static_cast<const bf16_t*>(y), cand_w, static_cast<bf16_t*>(ws), inv, slots,
+                             d, cand_eps, st);
     return ws;
 }
 

@@ -746,3 +746,48 @@ def test_backward_resets_at_chunk_edges_and_padded_nans(dev, path):
         assert not bool(torch.isnan(g_[0]).any()), name
         _close(g_[~nan], w_[~nan], F32_TOL, name)
     assert not bool(torch.isnan(dy[1, 127:]).any()) and not bool(torch.isnan(dg[1, 127:]).any())
+
+
+@pytest.mark.parametrize("io", ["f32", "bf16"])
+@pytest.mark.parametrize("B,T,K,d,shift", [
+    (1, 1, 2, 4, 0),      # two slots, one lane group's quarter used
+    (2, 9, 3, 24, 0),     # d off the lanes' power of two
+    (3, 50, 4, 64, 0),    # more slots than one workgroup of the norm's VJP
+    (1, 33, 5, 132, 0),   # 64 lanes a slot, half of them idle
+    (1, 7, 2, 256, 0),    # the widest
+    (2, 9, 3, 30, 0),     # d not a multiple of 4: a row a wavefront
+    (2, 9, 3, 24, 1),     # rows off the four-element alignment: a row a wavefront
+])
+def test_rms_candidate_at_the_edges_of_its_lanes(dev, B, T, K, d, shift, io):
+    """The RMS candidate's prologue and VJP over their layouts (four columns a lane, and a row a
+    wavefront) against the float64 oracle: h_sel, dy and the gain's gradient, whose bar grows with
+    the square root of its slots (the random walk of the fp32 roundings)."""
+    from hsn_amd import window
+
+    g = torch.Generator().manual_seed(1000 * d + B)
+    N, dt = max(4, K + 1), torch.float32 if io == "f32" else torch.bfloat16
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    y, gate, w = rnd(B, T, K, d).to(dt), rnd(B, T, K, d).to(dt), 1.0 + 0.2 * rnd(d)
+    logits, cost = rnd(B, T, N, 1), torch.full((1,), 0.5 / K)
+    reset = torch.zeros(B, T, dtype=torch.bool)
+    h0, q0 = 0.1 * rnd(B, N, d), rnd(B, d)
+    age0, pos0 = torch.zeros(B, N, dtype=torch.int64), torch.zeros(B, dtype=torch.int64)
+    dsel = rnd(B, T, K, d).to(dt)
+    kw = dict(cand_norm=True, cand_w=w)
+    want = O.window_forward(logits, y.double(), gate.double(), reset, h0.double(), q0.double(), age0,
+                            pos0, cost, k=K, cand_norm=True, cand_w=w.double())
+    yd = y.to(dev)
+    if shift:  # a contiguous view one element into a buffer
+        yd = torch.empty(y.numel() + shift, dtype=dt, device=dev)[shift:].view(y.shape).copy_(y)
+    got = window.window_forward(logits.to(dev), yd, gate.to(dev), reset.to(dev), h0.to(dev), q0.to(dev),
+                                age0.to(dev), pos0.to(dev), cost.to(dev), window.RouteConfig(k=K),
+                                cand_norm=True, cand_w=w.to(dev))
+    tol = F32_TOL if io == "f32" else BF16_TOL
+    _close(got["h_sel"], want["h_sel"].float(), tol, "h_sel")
+    ref = O.window_backward(y, gate, want["h_old"].to(dt), want["cells"], want["valid"], reset, N, None,
+                            None, dsel, None, None, **kw)
+    dy, _, _, _, d_w = window.backward(yd, gate.to(dev), want["h_old"].to(dt).to(dev), got["slots"],
+                                       reset.to(dev), N, None, None, dsel.to(dev), None, None,
+                                       cand_norm=True, cand_w=w.to(dev))
+    _close(dy, ref[0], tol, "dy")
+    _close(d_w, ref[4], tol * max(1.0, (B * T * K) ** 0.5 / 8), "d_cand_w")
