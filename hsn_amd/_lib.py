@@ -69,6 +69,7 @@ SIGNATURES: dict[str, list] = {
     "hsn_csr_messages": [P, P, P, P, P, P, P, I, I, I, I, I, I, P],
     "hsn_csr_messages_bwd": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, P],
     "hsn_gated_delta_update": [P, P, P, P, P, P, P, P, I, I, I, I, I, P],
+    "hsn_gated_delta_update_copy": [P, P, P, I, P, P, P, P, P, P, P, P, I, I, I, I, I, P],
     "hsn_gated_delta_update_bwd": [P, P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, P],
     "hsn_tr_adamw": [P, P, P, P, P, I, I, P, P],
     "hsn_tr_adamw_units": [P, P, P, P, P, I, I, I, P, F, F, P],

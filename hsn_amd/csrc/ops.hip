@@ -6,6 +6,7 @@
 // needs no atomics (valid slots name distinct cells) and every sum has a fixed order, so the
 // results are reproducible run to run whatever `deterministic` says.
 #include "common.cuh"
+#include "index.cuh"
 
 #include <type_traits>
 
@@ -13,11 +14,20 @@ namespace hsn {
 
 namespace {
 
-// grad_h = G (the copy the slot pass then overwrites), or zero when G is NULL.
+// grad_h = G (the copy the slot pass then overwrites), or zero when G is NULL: 16 bytes a thread
+// where both are aligned to them, and the elements past the last 16 bytes one a thread. HBM-bound;
+// 16.8 M fp32 elements: 27 us, zeroing 11.5 (one element a thread: 35 and 25).
 template <typename F>
-__global__ __launch_bounds__(256) void copy_or_zero(const F* src, F* dst, int64_t n) {
+__global__ __launch_bounds__(256) void copy_or_zero(const F* src, F* dst, int64_t n, int64_t n16) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = src ? src[i] : from_f32<F>(0.0f);
+    constexpr int64_t kPer = 16 / sizeof(F);
+    if (i < n16) {
+        reinterpret_cast<uint4*>(dst)[i] =
+            src ? reinterpret_cast<const uint4*>(src)[i] : make_uint4(0u, 0u, 0u, 0u);
+    } else {
+        const int64_t e = n16 * kPer + (i - n16);
+        if (e < n) dst[e] = src ? src[e] : from_f32<F>(0.0f);
+    }
 }
 
 // A thread per (row, column) walks the row's K slots in order, 8 at a time: the group's valid
@@ -26,8 +36,8 @@ __global__ __launch_bounds__(256) void copy_or_zero(const F* src, F* dst, int64_
 // (in-place order, as if each slot read h after the slots before it).
 template <typename F>
 __global__ __launch_bounds__(256) void gated_update_fwd(F* h, F* q, int32_t* age,
-                                                        const int32_t* cell_idx,
-                                                        const int32_t* valid, const F* c,
+                                                        Idx cell_idx,
+                                                        Flags valid, const F* c,
                                                         const F* bgate, F* h_old_saved, int B,
                                                         int N, int d, int K) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -42,7 +52,7 @@ __global__ __launch_bounds__(256) void gated_update_fwd(F* h, F* q, int32_t* age
 #pragma unroll
         for (int i = 0; i < G; ++i) {
             const int64_t s = int64_t(r) * K + k0 + i;
-            on[i] = k0 + i < K && valid[s] != 0;
+            on[i] = k0 + i < K && valid[s];
             cell[i] = on[i] ? cell_idx[s] : -1;
             cv[i] = on[i] ? to_f32(c[s * d + x]) : 0.0f;
             bv[i] = on[i] ? to_f32(bgate[s * d + x]) : 0.0f;
@@ -76,8 +86,8 @@ __global__ __launch_bounds__(256) void gated_update_fwd(F* h, F* q, int32_t* age
 }
 
 template <typename F>
-__global__ __launch_bounds__(256) void gated_update_bwd(const int32_t* cell_idx,
-                                                        const int32_t* valid, const F* c,
+__global__ __launch_bounds__(256) void gated_update_bwd(Idx cell_idx,
+                                                        Flags valid, const F* c,
                                                         const F* bgate, const F* h_old,
                                                         const F* G, const F* g, F* grad_h,
                                                         F* grad_q, F* grad_c, F* grad_b, int B,
@@ -96,7 +106,7 @@ __global__ __launch_bounds__(256) void gated_update_bwd(const int32_t* cell_idx,
 #pragma unroll
         for (int i = 0; i < S; ++i) {
             const int64_t s = int64_t(r) * K + k0 + i;
-            on[i] = k0 + i < K && valid[s] != 0;
+            on[i] = k0 + i < K && valid[s];
             hi[i] = on[i] ? (int64_t(r) * N + cell_idx[s]) * d + x : 0;
         }
 #pragma unroll
@@ -126,7 +136,7 @@ __global__ __launch_bounds__(256) void gated_update_bwd(const int32_t* cell_idx,
 
 template <typename F>
 __global__ __launch_bounds__(256) void gather_fwd(const F* u, const F* eps, const F* h, const F* m,
-                                                  const int32_t* cell_idx, F* v, int B, int N,
+                                                  Idx cell_idx, F* v, int B, int N,
                                                   int d, int K) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t w = 4 * int64_t(d);
@@ -144,7 +154,7 @@ __global__ __launch_bounds__(256) void gather_fwd(const F* u, const F* eps, cons
 }
 
 template <typename F>
-__global__ __launch_bounds__(256) void gather_bwd(const F* grad_v, const int32_t* cell_idx,
+__global__ __launch_bounds__(256) void gather_bwd(const F* grad_v, Idx cell_idx,
                                                   F* grad_u, F* grad_eps, F* grad_h, F* grad_m,
                                                   int B, int N, int d, int K) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -197,14 +207,14 @@ __global__ __launch_bounds__(256) void gather_bwd(const F* grad_v, const int32_t
 // each slot writes its cell's sum over the slots up to it (the same cells found by a scan of the
 // earlier slots), so the cell's last slot writes the whole sum.
 template <typename F>
-__global__ __launch_bounds__(256) void gather_bwd_narrow(const F* grad_v, const int32_t* cell_idx,
+__global__ __launch_bounds__(256) void gather_bwd_narrow(const F* grad_v, Idx cell_idx,
                                                          F* grad_u, F* grad_eps, F* grad_h,
                                                          F* grad_m, int B, int N, int d, int K) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (e >= int64_t(B) * d) return;
     const int r = static_cast<int>(e / d), x = static_cast<int>(e - int64_t(r) * d);
     const int64_t w = 4 * int64_t(d);
-    const int32_t* cells = cell_idx + int64_t(r) * K;
+    const int64_t s0 = int64_t(r) * K;
     const F* gv = grad_v + int64_t(r) * K * w;
     float su = 0.0f, se = 0.0f;
     for (int i = 0; i < K; ++i) {
@@ -212,16 +222,138 @@ __global__ __launch_bounds__(256) void gather_bwd_narrow(const F* grad_v, const 
         su += to_f32(g[x]);
         se += to_f32(g[d + x]);
         grad_m[(int64_t(r) * K + i) * d + x] = g[3 * d + x];
-        const int c = cells[i];
+        const int c = cell_idx[s0 + i];
         float sum = 0.0f;
         for (int j = 0; j <= i; ++j)
-            if (cells[j] == c) sum += to_f32(gv[j * w + 2 * d + x]);
+            if (cell_idx[s0 + j] == c) sum += to_f32(gv[j * w + 2 * d + x]);
         grad_h[(int64_t(r) * N + c) * d + x] = from_f32<F>(sum);
     }
     grad_u[int64_t(r) * d + x] = from_f32<F>(su);
     grad_eps[int64_t(r) * d + x] = from_f32<F>(se);
 }
 
+// The update into fresh tensors in two launches that write disjoint cells: workgroup (r, i) of the
+// copy takes row r's i-th kCopyCells cells that no valid slot names, with their ages, and zeroes
+// the named ones' ages; a workgroup a row of the other takes the slots as gated_update_fwd does
+// (the old values from h, or from h_new where an earlier batch of the row's slots wrote the cell).
+// Bound by the copy of h. At B 256, N 1024, d 64, K 16 in fp32: 38 + 14 us; as clones of h, q
+// and the ages, the in-place kernel and a masked fill of the ages 57, and as one launch 52 (the
+// slots' registers halve the copies' workgroups a CU).
+constexpr int kCopyCells = 64;
+
+template <typename F>
+__global__ __launch_bounds__(256) void update_copy_rest(const F* h, const void* age, int age_wide,
+                                                        Idx cell_idx, Flags valid, F* h_new,
+                                                        void* age_new, int N, int d, int K, int quads) {
+    const int r = blockIdx.x, tid = threadIdx.x;
+    const int64_t row = int64_t(r) * N, s0 = int64_t(r) * K;
+    __shared__ uint8_t named[kCopyCells];
+    const int n0 = int(blockIdx.y) * kCopyCells, nc = min(kCopyCells, N - n0);
+    const int64_t base = (row + n0) * d;
+    // four elements a thread and U cells in flight; the first go out before the flags are known
+    using Quad = std::conditional_t<sizeof(F) == 4, uint4, uint2>;
+    constexpr int U = 4;
+    const int dq = quads ? d / 4 : 1, per = 256 / dq;  // cells the workgroup copies at once
+    const int n1 = tid / dq, x = tid - n1 * dq;
+    const Quad* src = reinterpret_cast<const Quad*>(h + base) + x;
+    Quad* dst = reinterpret_cast<Quad*>(h_new + base) + x;
+    Quad q[U];  // (a cell past the range reads the range's last)
+    const int first = quads && n1 < per ? n1 : nc;
+    if (first < nc)
+#pragma unroll
+        for (int u = 0; u < U; ++u) q[u] = src[int64_t(min(first + u * per, nc - 1)) * dq];
+    if (tid < kCopyCells) named[tid] = 0;
+    __syncthreads();
+    for (int k = tid; k < K; k += 256) {
+        const int n = valid[s0 + k] ? cell_idx[s0 + k] - n0 : -1;
+        if (n >= 0 && n < nc) named[n] = 1;  // equal writes: any order
+    }
+    __syncthreads();
+    if (tid < nc) {
+        const int64_t a = row + n0 + tid;
+        if (age_wide)
+            static_cast<int64_t*>(age_new)[a] = named[tid] ? 0 : static_cast<const int64_t*>(age)[a];
+        else
+            static_cast<int32_t*>(age_new)[a] = named[tid] ? 0 : static_cast<const int32_t*>(age)[a];
+    }
+    for (int nb = first; nb < nc; nb += U * per) {
+        if (nb != first)
+#pragma unroll
+            for (int u = 0; u < U; ++u) q[u] = src[int64_t(min(nb + u * per, nc - 1)) * dq];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (nb + u * per < nc && !named[nb + u * per]) dst[int64_t(nb + u * per) * dq] = q[u];
+    }
+    if (!quads)
+        for (int e = tid; e < nc * d; e += 256)
+            if (!named[e / d]) h_new[base + e] = h[base + e];
+}
+
+template <typename F>
+__global__ __launch_bounds__(256) void update_copy_slots(const F* h, const F* q, Idx cell_idx,
+                                                         Flags valid, const F* c, const F* bgate,
+                                                         F* h_new, F* q_new, F* h_old_saved, int N,
+                                                         int d, int K) {
+    const int r = blockIdx.x, tid = threadIdx.x;
+    const int64_t row = int64_t(r) * N, s0 = int64_t(r) * K;
+    constexpr int kSlots = 1024;
+    __shared__ int slot[kSlots], repeats;  // whether two valid slots of the row may name one cell
+    if (tid == 0) repeats = K > kSlots;
+    for (int k = tid; k < min(K, kSlots); k += 256) slot[k] = valid[s0 + k] ? cell_idx[s0 + k] : -1;
+    __syncthreads();
+    for (int k = tid; k < min(K, kSlots); k += 256)
+        for (int t = 0; slot[k] >= 0 && t < k; ++t)
+            if (slot[t] == slot[k]) repeats = 1;
+    __syncthreads();
+    constexpr int G = 8;
+    for (int x = tid; x < d; x += 256) {
+        float delta = 0.0f;
+        for (int k0 = 0; k0 < K; k0 += G) {
+            bool on[G];
+            int cell[G];
+            float cv[G], bv[G], old[G], stored[G];
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                const int64_t s = s0 + k0 + i;
+                on[i] = k0 + i < K && valid[s];
+                cell[i] = on[i] ? cell_idx[s] : -1;
+                cv[i] = on[i] ? to_f32(c[s * d + x]) : 0.0f;
+                bv[i] = on[i] ? to_f32(bgate[s * d + x]) : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < G; ++i) old[i] = on[i] ? to_f32(h[(row + cell[i]) * d + x]) : 0.0f;
+            for (int t = 0; repeats && t < k0; ++t) {  // a cell an earlier batch wrote: its stored value
+                const int ct = valid[s0 + t] ? cell_idx[s0 + t] : -2;
+#pragma unroll
+                for (int i = 0; i < G; ++i)
+                    if (on[i] && cell[i] == ct) old[i] = to_f32(h_new[(row + ct) * d + x]);
+            }
+#pragma unroll
+            for (int i = 0; i < G; ++i) {
+                stored[i] = 0.0f;
+                if (k0 + i >= K) continue;
+                const int64_t o = (s0 + k0 + i) * d + x;
+                if (on[i]) {
+                    float prev = old[i];
+#pragma unroll
+                    for (int t = 0; t < i; ++t)
+                        if (on[t] && cell[t] == cell[i]) prev = stored[t];  // the latest earlier slot
+                    const F st = from_f32<F>((1.0f - bv[i]) * prev + bv[i] * cv[i]);
+                    stored[i] = to_f32(st);
+                    h_new[(row + cell[i]) * d + x] = st;
+                    h_old_saved[o] = from_f32<F>(prev);
+                    delta += stored[i] - prev;
+                } else {
+                    h_old_saved[o] = from_f32<F>(0.0f);
+                }
+            }
+        }
+        const int64_t qi = int64_t(r) * d + x;
+        q_new[qi] = from_f32<F>(to_f32(q[qi]) + delta / static_cast<float>(N));
+    }
+}
+
+inline bool aligned(const void* p, size_t to) { return reinterpret_cast<uintptr_t>(p) % to == 0; }
 inline int grid_of(int64_t n) { return static_cast<int>((n + 255) / 256); }
 
 }  // namespace
@@ -233,6 +365,8 @@ inline int grid_of(int64_t n) { return static_cast<int>((n + 255) / 256); }
 using namespace hsn;
 
 namespace {
+
+constexpr int kWidths = HSN_CELLS_I64 | HSN_VALID_U8;
 
 void check_dims(int B, int N, int d, int K, const char* who) {
     HSN_REQUIRE(B >= 1 && N >= 1 && d >= 1 && K >= 1, HSN_ERR_INVALID_ARGUMENT,
@@ -254,8 +388,36 @@ void by_dtype(int dtype, Args&&... args) {
 }
 
 template <typename F>
+void launch_copy_or_zero(const F* src, F* dst, int64_t n, hipStream_t st) {
+    constexpr int64_t kPer = 16 / sizeof(F);
+    const int64_t n16 = aligned(src, 16) && aligned(dst, 16) ? n / kPer : 0;
+    hipLaunchKernelGGL((copy_or_zero<F>), dim3(grid_of(n16 + (n - n16 * kPer))), dim3(256), 0, st, src,
+                       dst, n, n16);
+}
+
+// The width bits of a dtype code (HSN_CELLS_I64 and so on), taken off it.
+Idx cells_of(const void* p, int dtype) { return Idx{p, (dtype & HSN_CELLS_I64) != 0}; }
+Flags flags_of(const void* p, int dtype) { return Flags{p, (dtype & HSN_VALID_U8) != 0}; }
+
+template <typename F>
+struct RunUpdateCopy {
+    static void run(const void* h, const void* q, const void* age, int age_wide, Idx cell_idx,
+                    Flags valid, const void* c, const void* b, void* h_new, void* q_new,
+                    void* age_new, void* h_old_saved, int B, int N, int d, int K, hipStream_t st) {
+        const int quads = d % 4 == 0 && d <= 1024 && aligned(h, 4 * sizeof(F)) && aligned(h_new, 4 * sizeof(F));
+        hipLaunchKernelGGL((update_copy_rest<F>), dim3(B, (N + kCopyCells - 1) / kCopyCells), dim3(256),
+                           0, st, static_cast<const F*>(h), age, age_wide, cell_idx, valid,
+                           static_cast<F*>(h_new), age_new, N, d, K, quads);
+        hipLaunchKernelGGL((update_copy_slots<F>), dim3(B), dim3(256), 0, st, static_cast<const F*>(h),
+                           static_cast<const F*>(q), cell_idx, valid, static_cast<const F*>(c),
+                           static_cast<const F*>(b), static_cast<F*>(h_new), static_cast<F*>(q_new),
+                           static_cast<F*>(h_old_saved), N, d, K);
+    }
+};
+
+template <typename F>
 struct RunUpdate {
-    static void run(void* h, void* q, int32_t* age, const int32_t* cell_idx, const int32_t* valid,
+    static void run(void* h, void* q, int32_t* age, Idx cell_idx, Flags valid,
                     const void* c, const void* b, void* h_old_saved, int B, int N, int d, int K,
                     hipStream_t st) {
         hipLaunchKernelGGL((gated_update_fwd<F>), dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
@@ -267,12 +429,11 @@ struct RunUpdate {
 
 template <typename F>
 struct RunUpdateBwd {
-    static void run(const int32_t* cell_idx, const int32_t* valid, const void* c, const void* b,
+    static void run(Idx cell_idx, Flags valid, const void* c, const void* b,
                     const void* h_old, const void* G, const void* g, void* grad_h, void* grad_q,
                     void* grad_c, void* grad_b, int B, int N, int d, int K, hipStream_t st) {
         const int64_t n = int64_t(B) * N * d;
-        hipLaunchKernelGGL((copy_or_zero<F>), dim3(grid_of(n)), dim3(256), 0, st,
-                           static_cast<const F*>(G), static_cast<F*>(grad_h), n);
+        launch_copy_or_zero(static_cast<const F*>(G), static_cast<F*>(grad_h), n, st);
         hipLaunchKernelGGL((gated_update_bwd<F>), dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
                            cell_idx, valid, static_cast<const F*>(c), static_cast<const F*>(b),
                            static_cast<const F*>(h_old), static_cast<const F*>(G),
@@ -285,7 +446,7 @@ struct RunUpdateBwd {
 template <typename F>
 struct RunGather {
     static void run(const void* u, const void* eps, const void* h, const void* m,
-                    const int32_t* cell_idx, void* v, int B, int N, int d, int K, hipStream_t st) {
+                    Idx cell_idx, void* v, int B, int N, int d, int K, hipStream_t st) {
         hipLaunchKernelGGL((gather_fwd<F>), dim3(grid_of(int64_t(B) * K * 4 * d)), dim3(256), 0,
                            st, static_cast<const F*>(u), static_cast<const F*>(eps),
                            static_cast<const F*>(h), static_cast<const F*>(m), cell_idx,
@@ -295,11 +456,10 @@ struct RunGather {
 
 template <typename F>
 struct RunGatherBwd {
-    static void run(const void* grad_v, const int32_t* cell_idx, void* grad_u, void* grad_eps,
+    static void run(const void* grad_v, Idx cell_idx, void* grad_u, void* grad_eps,
                     void* grad_h, void* grad_m, int B, int N, int d, int K, hipStream_t st) {
         const int64_t n = int64_t(B) * N * d;
-        hipLaunchKernelGGL((copy_or_zero<F>), dim3(grid_of(n)), dim3(256), 0, st,
-                           static_cast<const F*>(nullptr), static_cast<F*>(grad_h), n);
+        launch_copy_or_zero(static_cast<const F*>(nullptr), static_cast<F*>(grad_h), n, st);
         // fp32 rows: repeats forwarded in registers in slot order (exact); 16-bit rows: each
         // cell's sum kept in fp32 and rounded once
         auto kernel = std::is_same<F, float>::value ? gather_bwd<F> : gather_bwd_narrow<F>;
@@ -317,10 +477,10 @@ extern "C" int hsn_gather_concat(const void* u, const void* eps, const void* h, 
                                  int dtype, void* stream) {
     HSN_ABI_BEGIN
     check_dims(B, N, d, K, "hsn_gather_concat");
-    check_dtype(dtype, "hsn_gather_concat");
+    check_dtype(dtype & ~kWidths, "hsn_gather_concat");
     HSN_REQUIRE(u && eps && h && m && cell_idx && v, HSN_ERR_INVALID_ARGUMENT,
                 "hsn_gather_concat: a pointer is NULL");
-    by_dtype<RunGather>(dtype, u, eps, h, m, cell_idx, v, B, N, d, K, as_stream(stream));
+    by_dtype<RunGather>(dtype & ~kWidths, u, eps, h, m, cells_of(cell_idx, dtype), v, B, N, d, K, as_stream(stream));
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }
@@ -330,12 +490,12 @@ extern "C" int hsn_gather_concat_bwd(const void* grad_v, const int32_t* cell_idx
                                      int d, int K, int dtype, int deterministic, void* stream) {
     HSN_ABI_BEGIN
     check_dims(B, N, d, K, "hsn_gather_concat_bwd");
-    check_dtype(dtype, "hsn_gather_concat_bwd");
+    check_dtype(dtype & ~kWidths, "hsn_gather_concat_bwd");
     HSN_REQUIRE(deterministic == 0 || deterministic == 1, HSN_ERR_INVALID_ARGUMENT,
                 "hsn_gather_concat_bwd: deterministic must be 0 or 1");
     HSN_REQUIRE(grad_v && cell_idx && grad_u && grad_eps && grad_h && grad_m,
                 HSN_ERR_INVALID_ARGUMENT, "hsn_gather_concat_bwd: a pointer is NULL");
-    by_dtype<RunGatherBwd>(dtype, grad_v, cell_idx, grad_u, grad_eps, grad_h, grad_m, B, N, d, K,
+    by_dtype<RunGatherBwd>(dtype & ~kWidths, grad_v, cells_of(cell_idx, dtype), grad_u, grad_eps, grad_h, grad_m, B, N, d, K,
                            as_stream(stream));
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
@@ -347,11 +507,33 @@ extern "C" int hsn_gated_delta_update(void* h, void* q, int32_t* age, const int3
                                       void* stream) {
     HSN_ABI_BEGIN
     check_dims(B, N, d, K, "hsn_gated_delta_update");
-    check_dtype(dtype, "hsn_gated_delta_update");
+    check_dtype(dtype & ~kWidths, "hsn_gated_delta_update");
     HSN_REQUIRE(h && q && age && cell_idx && valid && c && b && h_old_saved,
                 HSN_ERR_INVALID_ARGUMENT, "hsn_gated_delta_update: a pointer is NULL");
-    by_dtype<RunUpdate>(dtype, h, q, age, cell_idx, valid, c, b, h_old_saved, B, N, d, K,
+    by_dtype<RunUpdate>(dtype & ~kWidths, h, q, age, cells_of(cell_idx, dtype), flags_of(valid, dtype), c, b, h_old_saved, B, N, d, K,
                         as_stream(stream));
+    HSN_HIP(hipGetLastError());
+    HSN_ABI_END
+}
+
+extern "C" int hsn_gated_delta_update_copy(const void* h, const void* q, const void* age,
+                                           int age_bits, const int32_t* cell_idx,
+                                           const int32_t* valid, const void* c, const void* b,
+                                           void* h_new, void* q_new, void* age_new,
+                                           void* h_old_saved, int B, int N, int d, int K, int dtype,
+                                           void* stream) {
+    HSN_ABI_BEGIN
+    check_dims(B, N, d, K, "hsn_gated_delta_update_copy");
+    check_dtype(dtype & ~kWidths, "hsn_gated_delta_update_copy");
+    HSN_REQUIRE(h && q && age && cell_idx && valid && c && b && h_new && q_new && age_new && h_old_saved,
+                HSN_ERR_INVALID_ARGUMENT, "hsn_gated_delta_update_copy: a pointer is NULL");
+    HSN_REQUIRE(age_bits == 32 || age_bits == 64, HSN_ERR_INVALID_ARGUMENT,
+                "hsn_gated_delta_update_copy: age_bits must be 32 or 64");
+    HSN_REQUIRE(N <= 65534 * kCopyCells, HSN_ERR_INVALID_ARGUMENT,
+                "hsn_gated_delta_update_copy: N above 4194176");
+    by_dtype<RunUpdateCopy>(dtype & ~kWidths, h, q, age, age_bits == 64 ? 1 : 0, cells_of(cell_idx, dtype),
+                            flags_of(valid, dtype), c, b, h_new, q_new, age_new, h_old_saved, B, N, d, K,
+                            as_stream(stream));
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }
@@ -363,11 +545,11 @@ extern "C" int hsn_gated_delta_update_bwd(const int32_t* cell_idx, const int32_t
                                           int B, int N, int d, int K, int dtype, void* stream) {
     HSN_ABI_BEGIN
     check_dims(B, N, d, K, "hsn_gated_delta_update_bwd");
-    check_dtype(dtype, "hsn_gated_delta_update_bwd");
+    check_dtype(dtype & ~kWidths, "hsn_gated_delta_update_bwd");
     HSN_REQUIRE(cell_idx && valid && c && b && h_old_saved && grad_h_out && grad_q_out &&
                     grad_h && grad_q && grad_c && grad_b,
                 HSN_ERR_INVALID_ARGUMENT, "hsn_gated_delta_update_bwd: a pointer is NULL");
-    by_dtype<RunUpdateBwd>(dtype, cell_idx, valid, c, b, h_old_saved, grad_h_out, grad_q_out,
+    by_dtype<RunUpdateBwd>(dtype & ~kWidths, cells_of(cell_idx, dtype), flags_of(valid, dtype), c, b, h_old_saved, grad_h_out, grad_q_out,
                            grad_h, grad_q, grad_c, grad_b, B, N, d, K, as_stream(stream));
     HSN_HIP(hipGetLastError());
     HSN_ABI_END

@@ -17,6 +17,7 @@
 #include <algorithm>
 
 #include "common.cuh"
+#include "index.cuh"
 
 #include "../../include/hsn_ops.h"
 #include "abi_util.h"
@@ -1163,8 +1164,8 @@ __global__ __launch_bounds__(256) void mlp_dv_tiles(const int32_t* unit_idx, con
 // ------------------------------------------------------------------------------------------
 
 struct Csr {
-    const int32_t* indptr;   // [N + 1]
-    const int32_t* indices;  // [E]
+    Idx indptr;   // [N + 1]
+    Idx indices;  // [E]
     int N, E;
     // the edge range of row i, clamped into [0, E] (empty for a row outside [0, N))
     __device__ __forceinline__ void range(int i, int& e0, int& e1) const {
@@ -1181,7 +1182,7 @@ struct Csr {
 // into LDS (row stride `ld`); every thread of the workgroup takes (slot, column) pairs and walks
 // its slot's edges in order.
 template <typename T>
-__device__ __forceinline__ void gather_sums(const T* h, const T* a, const int32_t* cell_idx,
+__device__ __forceinline__ void gather_sums(const T* h, const T* a, Idx cell_idx,
                                             const Csr& g, int s0, int BK, int K, int d, int c0,
                                             int nc, float* S, int ld) {
     for (int x = threadIdx.x; x < 16 * nc; x += blockDim.x) {
@@ -1212,7 +1213,7 @@ constexpr int kListCap = 1024;
 constexpr size_t kListLds = (17 + 16 + 2 * size_t(kListCap)) * 4;
 template <typename T>
 __device__ __forceinline__ void gather_sums_listed(const T* h, const T* a,
-                                                   const int32_t* cell_idx, const Csr& g, int s0,
+                                                   Idx cell_idx, const Csr& g, int s0,
                                                    int BK, int K, int d, float* S) {
     __shared__ int lstart[17], le0[16], lsrc[kListCap];
     __shared__ float lw[kListCap];
@@ -1278,7 +1279,7 @@ __device__ __forceinline__ void gather_sums_listed(const T* h, const T* a,
 // (BK / 16, d / 64) workgroups: m[s][o] = sum_c V[o][c] S[s][c] for 16 slots (S in LDS).
 template <typename T>
 __global__ __launch_bounds__(256) void csr_fwd(const T* h, const Csr g, const T* a, const T* V,
-                                               const int32_t* cell_idx, T* m, int B, int K,
+                                               Idx cell_idx, T* m, int B, int K,
                                                int d) {
     extern __shared__ float S[];  // [16][d]
     const int lane = lane_id(), w = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
@@ -1308,7 +1309,7 @@ __global__ __launch_bounds__(256) void csr_fwd(const T* h, const Csr g, const T*
 constexpr int kDhCells = 128;
 template <typename T>
 __global__ __launch_bounds__(64) void csr_dh(const Csr g, const T* a, const T* V,
-                                             const int32_t* cell_idx, const T* grad_m, T* grad_h,
+                                             Idx cell_idx, const T* grad_m, T* grad_h,
                                              int K, int d) {
     __shared__ float acc[kDhCells][64];
     const int r = blockIdx.x, lane = lane_id(), c = blockIdx.y * 64 + lane;
@@ -1346,7 +1347,7 @@ __global__ __launch_bounds__(64) void csr_dh(const Csr g, const T* a, const T* V
 // selected row i, in order, of grad_m[r, k] . (V h[r, j]).
 template <typename T>
 __global__ __launch_bounds__(256) void csr_da(const T* h, const Csr g, const T* V,
-                                              const int32_t* cell_idx, const T* grad_m, T* grad_a,
+                                              Idx cell_idx, const T* grad_m, T* grad_a,
                                               int B, int K, int d) {
     const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = lane_id();
     if (e >= g.E) return;
@@ -1404,9 +1405,37 @@ __host__ __device__ inline DhLds dh_lds(int K) {
     return L;
 }
 
+// Entries [p0, p0 + cnt) of the row's edge list into LDS: an entry's source (-1 outside
+// [from, to)), weight and slot; every thread of the workgroup calls it.
 template <typename T>
+__device__ __forceinline__ void list_edges(const Csr& g, const T* a, const int* se0, const int* start,
+                                           int K, int p0, int cnt, int from, int to, int* lsrc,
+                                           float* lw, int* lslot) {
+    for (int x = threadIdx.x; x < cnt; x += 256) {
+        const int pos = p0 + x;
+        int klo = 0, khi = K;  // start[klo] <= pos < start[khi]
+        while (khi - klo > 1) {
+            const int mid = (klo + khi) >> 1;
+            if (start[mid] <= pos) klo = mid;
+            else khi = mid;
+        }
+        const int e = se0[klo] + pos - start[klo];
+        const int src = g.indices[e];
+        lsrc[x] = src >= from && src < to ? src : -1;
+        lw[x] = load_f32(a, e);
+        lslot[x] = klo;
+    }
+}
+
+// With TOUCHED (fp32; grad_h zeroed before) one workgroup takes a row's 64 columns of every cell:
+// its wavefronts share the list's entries, and the first entry of a source sums all of the
+// source's in list order, so a cell no entry names costs nothing but the zeroing. A list longer
+// than kDhList continues from the sums of the blocks before, exact in fp32 only: 16-bit storage
+// walks every cell. At B 256, N 1024, K 16, d 64 with 8 edges a cell: 31.5 + 11.8 us (the zeroing), 54
+// by cells (every wavefront walking the whole list, u computed once per 128 cells).
+template <typename T, bool TOUCHED>
 __global__ __launch_bounds__(256) void csr_dh_rows(const Csr g, const T* a, const T* V,
-                                                   const int32_t* cell_idx, const T* grad_m,
+                                                   Idx cell_idx, const T* grad_m,
                                                    T* grad_h, int K, int d) {
     extern __shared__ __align__(16) unsigned char lds[];
     const DhLds L = dh_lds(K);
@@ -1478,25 +1507,40 @@ __global__ __launch_bounds__(256) void csr_dh_rows(const Csr g, const T* a, cons
     }
     __syncthreads();
     const int total = start[K];
+    if constexpr (TOUCHED) {
+        const int c = c0 + lane;
+        T* gh = grad_h + int64_t(r) * g.N * d + c;
+        for (int p0 = 0; p0 < total; p0 += kDhList) {
+            const int cnt = min(kDhList, total - p0);
+            __syncthreads();  // the last block's list is read, its sums are stored
+            list_edges(g, a, se0, start, K, p0, cnt, 0, g.N, lsrc, lw, lslot);
+            __syncthreads();
+            for (int t = wave; t < cnt; t += 4) {  // uniform in the wavefront
+                const int src = uniform(lsrc[t]);
+                bool first = src >= 0;
+                for (int q = 0; first && q < t; q += 64)
+                    first = ballot(q + lane < t && lsrc[q + lane] == src) == 0ull;
+                if (!first) continue;
+                float sum = p0 > 0 && c < d ? to_f32(gh[int64_t(src) * d]) : 0.0f;
+                for (int q = t & ~63; q < cnt; q += 64) {
+                    uint64_t hits = ballot(q + lane >= t && q + lane < cnt && lsrc[q + lane] == src);
+                    while (hits) {  // uniform
+                        const int e = q + __builtin_ctzll(hits);
+                        hits &= hits - 1;
+                        sum += lw[e] * u[lslot[e] * 64 + lane];
+                    }
+                }
+                if (c < d) store_f32(gh, int64_t(src) * d, sum);
+            }
+        }
+        return;
+    }
     const int lo = n0 + 32 * wave, hi = min(lo + 32, g.N);
     for (int n = lo; n < hi; ++n) acc[(n - n0) * 64 + lane] = 0.0f;
     for (int p0 = 0; p0 < total; p0 += kDhList) {
         const int cnt = min(kDhList, total - p0);
         __syncthreads();  // the last block's walk is done
-        for (int x = tid; x < cnt; x += 256) {
-            const int pos = p0 + x;
-            int klo = 0, khi = K;  // start[klo] <= pos < start[khi]
-            while (khi - klo > 1) {
-                const int mid = (klo + khi) >> 1;
-                if (start[mid] <= pos) klo = mid;
-                else khi = mid;
-            }
-            const int e = se0[klo] + pos - start[klo];
-            const int src = g.indices[e];
-            lsrc[x] = src >= n0 && src < min(n0 + 128, g.N) ? src : -1;
-            lw[x] = load_f32(a, e);
-            lslot[x] = klo;
-        }
+        list_edges(g, a, se0, start, K, p0, cnt, n0, min(n0 + 128, g.N), lsrc, lw, lslot);
         __syncthreads();
         for (int i0 = 0; i0 < cnt; i0 += 64) {  // 64 entries a lane, broadcast in order
             const int m = min(64, cnt - i0);
@@ -1527,7 +1571,7 @@ __global__ __launch_bounds__(256) void csr_dh_rows(const Csr g, const T* a, cons
 // and csr_dV_sum adds the groups in order.
 template <typename T>
 __global__ __launch_bounds__(256) void csr_dV_groups(const T* h, const Csr g, const T* a,
-                                                     const int32_t* cell_idx, const T* grad_m,
+                                                     Idx cell_idx, const T* grad_m,
                                                      T* grad_V, float* part, int B, int K, int d,
                                                      int group_slots) {
     __shared__ float S[16 * 16];
@@ -1596,14 +1640,16 @@ __global__ __launch_bounds__(256) void csr_u(const T* V, const T* grad_m, float*
     }
 }
 
-// grad_a from U: a wavefront per edge e (target row i, source j) adds U[r, k] . h[r, j] over the
-// slots that selected row i, in order. The slots' cells and indptr are staged in LDS
-// ((B K + N + 1) ints within 64 KiB); the slots are found 64 at a time by a ballot and taken in
-// ascending order from its set bits.
+// grad_a from U: a wavefront takes eight consecutive edges (mostly one target row's), each with
+// target row i and source j, and adds U[r, k] . h[r, j] over the slots that selected row i, in
+// order. The slots' cells and indptr are staged in LDS ((B K + N + 1) ints within 64 KiB); the
+// slots of a row are found once for its edges, 64 at a time by a ballot, and taken in ascending
+// order from its set bits. At E 8192 and 4096 slots: 22.6 us (an edge a wavefront, every workgroup
+// of four staging and searching all slots: 27).
+constexpr int kDaEdges = 8;
 template <typename T>
 __global__ __launch_bounds__(256) void csr_da_u(const T* h, const Csr g, const float* U,
-                                                const int32_t* cell_idx, T* grad_a, int B, int K,
-                                                int d) {
+                                                Idx cell_idx, T* grad_a, int B, int K, int d) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int BK = B * K;
     int* cells = reinterpret_cast<int*>(lds);
@@ -1611,41 +1657,79 @@ __global__ __launch_bounds__(256) void csr_da_u(const T* h, const Csr g, const f
     for (int x = threadIdx.x; x < BK; x += 256) cells[x] = cell_idx[x];
     for (int x = threadIdx.x; x <= g.N; x += 256) ptr[x] = g.indptr[x];
     __syncthreads();
-    const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = lane_id();
-    if (e >= g.E) return;
-    int lo = 0, hi = g.N;  // the target row: the last i with indptr[i] <= e
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (ptr[mid] <= e) lo = mid;
-        else hi = mid;
+    const int lane = lane_id(), ebase = (blockIdx.x * 4 + (threadIdx.x >> 6)) * kDaEdges;
+    const int e = ebase + lane;
+    const bool mine = lane < kDaEdges && e < g.E;
+    int owner = -1, src = 0;
+    if (mine) {
+        int lo = 0, hi = g.N;  // the target row: the last i with indptr[i] <= e
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (ptr[mid] <= e) lo = mid;
+            else hi = mid;
+        }
+        const int e0 = min(max(ptr[lo], 0), g.E), e1 = min(max(ptr[lo + 1], e0), g.E);
+        src = g.indices[e];
+        if (e >= e0 && e < e1 && src >= 0 && src < g.N) owner = lo;
     }
-    const int e0 = min(max(ptr[lo], 0), g.E), e1 = min(max(ptr[lo + 1], e0), g.E);
-    const int src = g.indices[e];
-    float acc = 0.0f;
-    if (e >= e0 && e < e1 && src >= 0 && src < g.N) {
+    int srcs[kDaEdges];
+    float acc[kDaEdges];
+#pragma unroll
+    for (int i = 0; i < kDaEdges; ++i) srcs[i] = __builtin_amdgcn_readlane(src, i), acc[i] = 0.0f;
+    for (uint64_t left = ballot(owner >= 0); left;) {  // uniform
+        const int row = __builtin_amdgcn_readlane(owner, __builtin_ctzll(left));
+        const uint64_t same = ballot(owner == row);
+        left &= ~same;
         for (int f0 = 0; f0 < BK; f0 += 64) {
-            uint64_t hits = ballot(f0 + lane < BK && cells[f0 + lane] == lo);
+            uint64_t hits = ballot(f0 + lane < BK && cells[f0 + lane] == row);
             while (hits) {  // uniform
                 const int flat = f0 + __builtin_ctzll(hits);
                 hits &= hits - 1;
-                const T* hr = h + (int64_t(flat / K) * g.N + src) * d;
+                const T* hr = h + int64_t(flat / K) * g.N * d;
                 const float* u = U + int64_t(flat) * d;
-                for (int c = lane; c < d; c += 64) acc += u[c] * load_f32(hr, c);
+                for (int c = lane; c < d; c += 64) {
+                    const float uv = u[c];
+                    float hv[kDaEdges];
+#pragma unroll
+                    for (int i = 0; i < kDaEdges; ++i)
+                        hv[i] = (same >> i) & 1 ? load_f32(hr, int64_t(srcs[i]) * d + c) : 0.0f;
+#pragma unroll
+                    for (int i = 0; i < kDaEdges; ++i)
+                        if ((same >> i) & 1) acc[i] += uv * hv[i];
+                }
             }
         }
     }
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kWave);
-    if (lane == 0) store_f32(grad_a, e, acc);
+#pragma unroll
+    for (int i = 0; i < kDaEdges; ++i) {
+        for (int off = 32; off > 0; off >>= 1) acc[i] += __shfl_xor(acc[i], off, kWave);
+        if (lane == 0 && ebase + i < g.E) store_f32(grad_a, ebase + i, acc[i]);
+    }
 }
 
+// The groups' sums of 16 elements a workgroup: 16 runs of groups an element, added in run order.
 template <typename T>
 __global__ __launch_bounds__(256) void csr_dV_sum(const float* part, T* grad_V, int groups, int dd) {
-    const int x = blockIdx.x * 256 + threadIdx.x;
-    if (x >= dd) return;
-    float sum = 0.0f;  // the loads issued 8 at a time; the sum keeps the groups' order
+    __shared__ float red[16][17];
+    const int x = blockIdx.x * 16 + threadIdx.x % 16, run = threadIdx.x / 16;
+    float sum = 0.0f;
+    if (x < dd) {
 #pragma unroll 8
-    for (int i = 0; i < groups; ++i) sum += part[int64_t(i) * dd + x];
-    store_f32(grad_V, x, sum);
+        for (int i = run; i < groups; i += 16) sum += part[int64_t(i) * dd + x];
+    }
+    red[run][threadIdx.x % 16] = sum;
+    __syncthreads();
+    if (run == 0 && x < dd) {
+        float t = 0.0f;
+        for (int i = 0; i < 16; ++i) t += red[i][threadIdx.x];
+        store_f32(grad_V, x, t);
+    }
+}
+
+static __global__ __launch_bounds__(256) void zero_floats(float* p, int64_t n, int64_t n16) {
+    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n16) reinterpret_cast<float4*>(p)[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    else if (4 * n16 + (i - n16) < n) p[4 * n16 + (i - n16)] = 0.0f;
 }
 
 // grad_a with the slots' cells staged in LDS (B K <= 16384): a wavefront per edge e (target row
@@ -1653,7 +1737,7 @@ __global__ __launch_bounds__(256) void csr_dV_sum(const float* part, T* grad_V, 
 // (V^T grad_m[r, k]) . h[r, j] for each, lane c taking column c (then a wavefront sum).
 template <typename T>
 __global__ __launch_bounds__(256) void csr_da_rows(const T* h, const Csr g, const T* V,
-                                                   const int32_t* cell_idx, const T* grad_m,
+                                                   Idx cell_idx, const T* grad_m,
                                                    T* grad_a, int B, int K, int d) {
     extern __shared__ __align__(16) unsigned char lds[];
     int* cells = reinterpret_cast<int*>(lds);
@@ -1707,6 +1791,11 @@ void check_dtype(int dtype, const char* who) {
     HSN_REQUIRE(dtype == HSN_DTYPE_F32 || dtype == HSN_DTYPE_F16 || dtype == HSN_DTYPE_BF16,
                 HSN_ERR_UNSUPPORTED_DTYPE, std::string(who) + ": unknown dtype code");
 }
+
+// The width bits of the messages' dtype code, taken off it.
+constexpr int kWidths = HSN_CELLS_I64 | HSN_GRAPH_I64;
+Idx cells_of(const void* p, int dtype) { return Idx{p, (dtype & HSN_CELLS_I64) != 0}; }
+Idx graph_of(const void* p, int dtype) { return Idx{p, (dtype & HSN_GRAPH_I64) != 0}; }
 
 void check_units(int P, int M, int d, int H, const char* who) {
     HSN_REQUIRE(P >= 1 && M >= 1 && d >= 1 && H >= 1, HSN_ERR_INVALID_ARGUMENT,
@@ -1842,8 +1931,8 @@ struct RunMlpBwd {
 
 template <typename T>
 struct RunCsr {
-    static void run(const void* h, const int32_t* indptr, const int32_t* indices, const void* a,
-                    const void* V, const int32_t* idx, void* m, int B, int N, int d, int K, int E,
+    static void run(const void* h, Idx indptr, Idx indices, const void* a,
+                    const void* V, Idx idx, void* m, int B, int N, int d, int K, int E,
                     hipStream_t st) {
         const units::Csr g{indptr, indices, N, E};
         // S [16][d] in dynamic LDS beside the static edge list: above the default 64 KiB from
@@ -1860,8 +1949,8 @@ struct RunCsr {
 
 template <typename T>
 struct RunCsrBwd {
-    static void run(const void* h, const int32_t* indptr, const int32_t* indices, const void* a,
-                    const void* V, const int32_t* idx, const void* dm, void* dh, void* da,
+    static void run(const void* h, Idx indptr, Idx indices, const void* a,
+                    const void* V, Idx idx, const void* dm, void* dh, void* da,
                     void* dV, int B, int N, int d, int K, int E, hipStream_t st) {
         const units::Csr g{indptr, indices, N, E};
         // grad_V first: with more than one group of slots its fp32 partial sums live in grad_h's
@@ -1882,7 +1971,7 @@ struct RunCsrBwd {
                            static_cast<const T*>(a), idx, static_cast<const T*>(dm),
                            static_cast<T*>(dV), part, B, K, d, group_slots);
         if (part)
-            hipLaunchKernelGGL((units::csr_dV_sum<T>), dim3((d * d + 255) / 256), dim3(256), 0, st,
+            hipLaunchKernelGGL((units::csr_dV_sum<T>), dim3((d * d + 15) / 16), dim3(256), 0, st,
                                part, static_cast<T*>(dV), groups, d * d);
         // grad_a next, from U = grad_m V in grad_h's memory when it fits there
         const bool u_fits = reinterpret_cast<uintptr_t>(dh) % 4 == 0 &&
@@ -1891,7 +1980,8 @@ struct RunCsrBwd {
             float* U = static_cast<float*>(dh);
             hipLaunchKernelGGL((units::csr_u<T>), dim3(chunks, (d + 63) / 64), dim3(256), 0, st,
                                static_cast<const T*>(V), static_cast<const T*>(dm), U, BK, d);
-            hipLaunchKernelGGL((units::csr_da_u<T>), dim3((E + 3) / 4), dim3(256),
+            hipLaunchKernelGGL((units::csr_da_u<T>),
+                               dim3((E + 4 * units::kDaEdges - 1) / (4 * units::kDaEdges)), dim3(256),
                                size_t(4) * (BK + N + 1),
                                st, static_cast<const T*>(h), g, U, idx, static_cast<T*>(da), B,
                                K, d);
@@ -1905,8 +1995,17 @@ struct RunCsrBwd {
                                static_cast<const T*>(h), g, static_cast<const T*>(V), idx,
                                static_cast<const T*>(dm), static_cast<T*>(da), B, K, d);
         }
-        if (K <= 64)
-            hipLaunchKernelGGL((units::csr_dh_rows<T>), dim3(B, (d + 63) / 64, (N + 127) / 128),
+        if (K <= 64 && sizeof(T) == 4) {
+            const int64_t n = int64_t(B) * N * d;
+            const int64_t n16 = reinterpret_cast<uintptr_t>(dh) % 16 == 0 ? n / 4 : 0;
+            hipLaunchKernelGGL(units::zero_floats, dim3(static_cast<unsigned>((n - 3 * n16 + 255) / 256)),
+                               dim3(256), 0, st, static_cast<float*>(dh), n, n16);
+            hipLaunchKernelGGL((units::csr_dh_rows<T, true>), dim3(B, (d + 63) / 64), dim3(256),
+                               units::dh_lds(K).bytes, st, g, static_cast<const T*>(a),
+                               static_cast<const T*>(V), idx, static_cast<const T*>(dm),
+                               static_cast<T*>(dh), K, d);
+        } else if (K <= 64)
+            hipLaunchKernelGGL((units::csr_dh_rows<T, false>), dim3(B, (d + 63) / 64, (N + 127) / 128),
                                dim3(256), units::dh_lds(K).bytes, st, g, static_cast<const T*>(a),
                                static_cast<const T*>(V), idx, static_cast<const T*>(dm),
                                static_cast<T*>(dh), K, d);
@@ -1960,10 +2059,10 @@ extern "C" int hsn_csr_messages(const void* h, const int32_t* indptr, const int3
                                 int B, int N, int d, int K, int E, int dtype, void* stream) {
     HSN_ABI_BEGIN
     check_csr(B, N, d, K, E, "hsn_csr_messages");
-    check_dtype(dtype, "hsn_csr_messages");
+    check_dtype(dtype & ~kWidths, "hsn_csr_messages");
     HSN_REQUIRE(h && indptr && V && cell_idx && m && (E == 0 || (indices && a)),
                 HSN_ERR_INVALID_ARGUMENT, "hsn_csr_messages: a pointer is NULL");
-    by_dtype<RunCsr>(dtype, h, indptr, indices, a, V, cell_idx, m, B, N, d, K, E,
+    by_dtype<RunCsr>(dtype & ~kWidths, h, graph_of(indptr, dtype), graph_of(indices, dtype), a, V, cells_of(cell_idx, dtype), m, B, N, d, K, E,
                      as_stream(stream));
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
@@ -1976,13 +2075,13 @@ extern "C" int hsn_csr_messages_bwd(const void* h, const int32_t* indptr, const 
                                     int deterministic, void* stream) {
     HSN_ABI_BEGIN
     check_csr(B, N, d, K, E, "hsn_csr_messages_bwd");
-    check_dtype(dtype, "hsn_csr_messages_bwd");
+    check_dtype(dtype & ~kWidths, "hsn_csr_messages_bwd");
     HSN_REQUIRE(deterministic == 0 || deterministic == 1, HSN_ERR_INVALID_ARGUMENT,
                 "hsn_csr_messages_bwd: deterministic must be 0 or 1");
     HSN_REQUIRE(h && indptr && V && cell_idx && grad_m && grad_h && grad_V &&
                     (E == 0 || (indices && a && grad_a)),
                 HSN_ERR_INVALID_ARGUMENT, "hsn_csr_messages_bwd: a pointer is NULL");
-    by_dtype<RunCsrBwd>(dtype, h, indptr, indices, a, V, cell_idx, grad_m, grad_h, grad_a, grad_V,
+    by_dtype<RunCsrBwd>(dtype & ~kWidths, h, graph_of(indptr, dtype), graph_of(indices, dtype), a, V, cells_of(cell_idx, dtype), grad_m, grad_h, grad_a, grad_V,
                         B, N, d, K, E, as_stream(stream));
     HSN_HIP(hipGetLastError());
     HSN_ABI_END

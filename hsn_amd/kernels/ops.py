@@ -128,13 +128,45 @@ def _flags(t: Tensor) -> Tensor:
     return t.to(torch.int32).contiguous()
 
 
+def _index(t: Tensor) -> Tensor:
+    """An index tensor an op takes as it is (int32 or int64), contiguous."""
+    return t.contiguous() if t.dtype == torch.int64 else _i32(t)
+
+
+#: The dtype code's width bits (include/hsn_ops.h): the kernels read these arrays as they are.
+_CELLS_I64, _GRAPH_I64, _VALID_U8 = 0x100, 0x200, 0x400
+
+
+def _cells(t: Tensor) -> tuple[Tensor, int]:
+    """``cell_idx`` as the library reads it, with its width bit: int32, or int64 in place (the
+    kernels clamp each index into [-1, 2^31 - 1])."""
+    if t.dtype == torch.int64:
+        return t.contiguous(), _CELLS_I64
+    return _i32(t), 0
+
+
+def _graph(indptr: Tensor, indices: Tensor) -> tuple[Tensor, Tensor, int]:
+    """A CSR's two arrays with their width bit; of two widths both narrow."""
+    if indptr.dtype == torch.int64 and indices.dtype == torch.int64:
+        return indptr.contiguous(), indices.contiguous(), _GRAPH_I64
+    return _i32(indptr), _i32(indices), 0
+
+
+def _valid(t: Tensor) -> tuple[Tensor, int]:
+    """The slots' flags with their width bit: bool in place, integers as int32."""
+    if t.dtype == torch.bool:
+        return t.contiguous(), _VALID_U8
+    return _flags(t), 0
+
+
 def _gather_body(u: Tensor, eps: Tensor, h: Tensor, m: Tensor, idx: Tensor) -> Tensor:
     B, N, d = h.shape
     K = idx.shape[1]
-    u, eps, h, m, idx = u.contiguous(), eps.contiguous(), h.contiguous(), m.contiguous(), _i32(idx)
+    u, eps, h, m = u.contiguous(), eps.contiguous(), h.contiguous(), m.contiguous()
+    idx, wide = _cells(idx)
     v = h.new_empty((B, K, 4 * d))
     call("hsn_gather_concat", ptr(u), ptr(eps), ptr(h), ptr(m), ptr(idx), ptr(v), B, N, d, K,
-         _code(h), stream_of(h.device))
+         _code(h) | wide, stream_of(h.device))
     return v
 
 
@@ -152,11 +184,11 @@ def _gather_fake(u, eps, h, m, idx):
 def _gather_bwd_body(dv: Tensor, idx: Tensor, n: int) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     B, K, width = dv.shape
     d = width // 4
-    dv, idx = dv.contiguous(), _i32(idx)
+    dv, (idx, wide) = dv.contiguous(), _cells(idx)
     du, de = dv.new_empty((B, d)), dv.new_empty((B, d))
     dh, dm = dv.new_empty((B, n, d)), dv.new_empty((B, K, d))
     call("hsn_gather_concat_bwd", ptr(dv), ptr(idx), ptr(du), ptr(de), ptr(dh), ptr(dm), B, n, d,
-         K, _code(dv), 1, stream_of(dv.device))
+         K, _code(dv) | wide, 1, stream_of(dv.device))
     return du, de, dh, dm
 
 
@@ -193,9 +225,10 @@ def _update(h: Tensor, q: Tensor, age: Tensor, idx: Tensor, valid: Tensor, c: Te
     B, N, d = h.shape
     K = idx.shape[1]
     old = torch.empty_like(c, memory_format=torch.contiguous_format)
-    call("hsn_gated_delta_update", ptr(h), ptr(q), ptr(age), ptr(_i32(idx)), ptr(_flags(valid)),
-         ptr(c.contiguous()), ptr(b.contiguous()), ptr(old), B, N, d, K, _code(h),
-         stream_of(h.device))
+    (idx, wide), (valid, byte) = _cells(idx), _valid(valid)
+    c, b = c.contiguous(), b.contiguous()
+    call("hsn_gated_delta_update", ptr(h), ptr(q), ptr(age), ptr(idx), ptr(valid), ptr(c), ptr(b),
+         ptr(old), B, N, d, K, _code(h) | wide | byte, stream_of(h.device))
     return old
 
 
@@ -223,14 +256,26 @@ def _update_inplace_fake(h, q, age, idx, valid, c, b):
 
 
 def _functional(h, q, age, idx, valid, c, b):
+    B, N, d = h.shape
+    K = idx.shape[1]
+    if age.dtype not in (torch.int32, torch.int64) or N > 4194176:
+        return _functional_by_copies(h, q, age, idx, valid, c, b)
+    h, q, age, c, b = h.contiguous(), q.contiguous(), age.contiguous(), c.contiguous(), b.contiguous()
+    hn, qn, an, old = torch.empty_like(h), torch.empty_like(q), torch.empty_like(age), torch.empty_like(c)
+    (idx, wide), (valid, byte) = _cells(idx), _valid(valid)
+    call("hsn_gated_delta_update_copy", ptr(h), ptr(q), ptr(age), 64 if age.dtype == torch.int64 else 32,
+         ptr(idx), ptr(valid), ptr(c), ptr(b), ptr(hn), ptr(qn), ptr(an), ptr(old), B, N, d, K,
+         _code(h) | wide | byte, stream_of(h.device))
+    return hn, qn, an, old
+
+
+def _functional_by_copies(h, q, age, idx, valid, c, b):
+    """The functional update where its kernel does not take the ages' dtype or the cell count: the
+    in-place update of copies."""
     hn = h.clone(memory_format=torch.contiguous_format)
     qn = q.clone(memory_format=torch.contiguous_format)
-    if age.dtype == torch.int32:
-        an = age.clone(memory_format=torch.contiguous_format)
-        old = _update(hn, qn, an, idx, valid, c, b)
-        return hn, qn, an, old
-    # wider ages stay exact: the kernel zeroes the selected cells of an int32 mask of ones, and
-    # the same cells' ages are zeroed in the caller's dtype
+    # the kernel zeroes the selected cells of an int32 mask of ones, and the same cells' ages are
+    # zeroed in the caller's dtype
     keep = torch.ones(age.shape, dtype=torch.int32, device=age.device)
     old = _update(hn, qn, keep, idx, valid, c, b)
     return hn, qn, age.masked_fill(keep == 0, 0), old
@@ -269,8 +314,9 @@ def _update_bwd_body(idx: Tensor, valid: Tensor, c: Tensor, b: Tensor, old: Tens
     c, b, old, G, g = c.contiguous(), b.contiguous(), old.contiguous(), G.contiguous(), g.contiguous()
     dh, dq = torch.empty_like(G), torch.empty_like(g)
     dc, db = torch.empty_like(c), torch.empty_like(b)
-    call("hsn_gated_delta_update_bwd", ptr(_i32(idx)), ptr(_flags(valid)), ptr(c), ptr(b), ptr(old),
-         ptr(G), ptr(g), ptr(dh), ptr(dq), ptr(dc), ptr(db), B, N, d, K, _code(G),
+    (idx, wide), (valid, byte) = _cells(idx), _valid(valid)
+    call("hsn_gated_delta_update_bwd", ptr(idx), ptr(valid), ptr(c), ptr(b), ptr(old), ptr(G), ptr(g),
+         ptr(dh), ptr(dq), ptr(dc), ptr(db), B, N, d, K, _code(G) | wide | byte,
          stream_of(G.device))
     return dh, dq, dc, db
 
@@ -423,11 +469,11 @@ def _messages_body(h: Tensor, indptr: Tensor, indices: Tensor, a: Tensor, V: Ten
                    idx: Tensor) -> Tensor:
     B, N, d = h.shape
     K, E = idx.shape[1], a.numel()
-    h, indptr, indices, a, V, idx = (h.contiguous(), _i32(indptr), _i32(indices), a.contiguous(),
-                                     V.contiguous(), _i32(idx))
+    h, a, V = h.contiguous(), a.contiguous(), V.contiguous()
+    (indptr, indices, graph), (idx, wide) = _graph(indptr, indices), _cells(idx)
     m = h.new_empty((B, K, d))
     call("hsn_csr_messages", ptr(h), ptr(indptr), ptr(indices), ptr(a), ptr(V), ptr(idx), ptr(m),
-         B, N, d, K, E, _code(h), stream_of(h.device))
+         B, N, d, K, E, _code(h) | graph | wide, stream_of(h.device))
     return m
 
 
@@ -448,12 +494,12 @@ def _messages_bwd_body(h: Tensor, indptr: Tensor, indices: Tensor, a: Tensor, V:
                        idx: Tensor, dm: Tensor) -> tuple[Tensor, Tensor, Tensor]:
     B, N, d = h.shape
     K, E = idx.shape[1], a.numel()
-    h, indptr, indices, a, V, idx, dm = (h.contiguous(), _i32(indptr), _i32(indices),
-                                         a.contiguous(), V.contiguous(), _i32(idx),
-                                         dm.contiguous())
+    h, a, V, dm = h.contiguous(), a.contiguous(), V.contiguous(), dm.contiguous()
+    (indptr, indices, graph), (idx, wide) = _graph(indptr, indices), _cells(idx)
     dh, da, dV = torch.empty_like(h), torch.empty_like(a), torch.empty_like(V)
     call("hsn_csr_messages_bwd", ptr(h), ptr(indptr), ptr(indices), ptr(a), ptr(V), ptr(idx),
-         ptr(dm), ptr(dh), ptr(da), ptr(dV), B, N, d, K, E, _code(h), 1, stream_of(h.device))
+         ptr(dm), ptr(dh), ptr(da), ptr(dV), B, N, d, K, E, _code(h) | graph | wide, 1,
+         stream_of(h.device))
     return dh, da, dV
 
 
@@ -538,7 +584,7 @@ def gather_concat(u: Optional[Tensor], eps: Tensor, h: Tensor, m: Tensor, cell_i
     if u.dtype != h.dtype or eps.dtype != h.dtype:
         raise ValueError("u, eps and h must have the same state dtype")
     return _eager(gather_op, _gather_body, u.contiguous(), eps.contiguous(), h.contiguous(),
-                  m.to(h.dtype).contiguous(), _i32(cell_idx))
+                  m.to(h.dtype).contiguous(), _index(cell_idx))
 
 
 def grouped_unit_mlp(v: Tensor, unit_idx: Tensor, bank: Any, *, static: bool = False,
@@ -572,7 +618,7 @@ def grouped_unit_mlp(v: Tensor, unit_idx: Tensor, bank: Any, *, static: bool = F
     # reach the masters through the cast
     w1 = bank.W1 if w1_flat is None else \
         w1_flat.reshape(bank.in_dim, bank.n_units, bank.hidden).permute(1, 0, 2)
-    out, _ = _eager(mlp_op, _mlp_body, v.to(dtype).contiguous(), _i32(unit_idx),
+    out, _ = _eager(mlp_op, _mlp_body, v.to(dtype).contiguous(), _index(unit_idx),
                     w1.to(dtype).contiguous(), bank.b1.to(dtype).contiguous(),
                     bank.W2.to(dtype).contiguous(), bank.b2.to(dtype).contiguous())
     return out
@@ -596,9 +642,9 @@ def csr_messages(h: Tensor, graph: Any, V: Any, cell_idx: Tensor, *,
         raise ValueError("CSR messages need a projection without bias")
     a = graph.edge_weights() if weights is None else weights.reshape(-1)[graph._edge_pos]
     dtype = _dtype_for(h)
-    return _eager(messages_op, _messages_body, h.to(dtype).contiguous(), _i32(graph.indptr),
-                  _i32(graph.indices), a.to(dtype).contiguous(), V.weight.to(dtype).contiguous(),
-                  _i32(cell_idx))
+    return _eager(messages_op, _messages_body, h.to(dtype).contiguous(), _index(graph.indptr),
+                  _index(graph.indices), a.to(dtype).contiguous(), V.weight.to(dtype).contiguous(),
+                  _index(cell_idx))
 
 
 def _check_valid(valid: Any, shape: tuple, device: torch.device) -> None:
@@ -658,6 +704,6 @@ def gated_delta_update(state: Any, cell_idx: Tensor, c: Tensor, b: Tensor, valid
     if validate:
         _check_selection(cell_idx, valid, int(h.shape[1]))
     hn, qn, age, _ = _eager(state_update_op, _functional, h.contiguous(), state.q.contiguous(),
-                            state.age.contiguous(), _i32(cell_idx), _flags(valid), c.contiguous(),
+                            state.age.contiguous(), _index(cell_idx), valid.contiguous(), c.contiguous(),
                             b.contiguous())
     return _with_state(state, hn, qn, age, state.pos)

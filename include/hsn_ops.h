@@ -25,6 +25,15 @@ extern "C" {
 #define HSN_DTYPE_F16 1
 #define HSN_DTYPE_BF16 2
 
+/*
+ * Or'ed into the dtype code of the gather, the messages and the gated update: the widths of the
+ * call's index and flag arrays where they are not int32_t. cell_idx int64_t; indptr and indices
+ * int64_t; valid one byte a flag. An int64_t index is clamped into [-1, 2^31 - 1] as it is read.
+ */
+#define HSN_CELLS_I64 0x100
+#define HSN_GRAPH_I64 0x200
+#define HSN_VALID_U8 0x400
+
 #define HSN_OK 0
 #define HSN_ERR_INVALID_ARGUMENT 1
 #define HSN_ERR_UNSUPPORTED_DTYPE 2
@@ -139,6 +148,17 @@ int hsn_csr_messages_bwd(const void* h, const int32_t* indptr, const int32_t* in
 int hsn_gated_delta_update(void* h, void* q, int32_t* age, const int32_t* cell_idx,
                            const int32_t* valid, const void* c, const void* b, void* h_old_saved,
                            int B, int N, int d, int K, int dtype, void* stream);
+
+/*
+ * The gated delta update into fresh tensors (the same values as a copy updated in place): h_new
+ * [B,N,d], q_new [B,d], age_new [B,N] (the ages int32_t or int64_t: `age_bits`) and h_old_saved;
+ * h, q and age are only read. No output may overlap an input. N <= 4194176.
+ */
+int hsn_gated_delta_update_copy(const void* h, const void* q, const void* age, int age_bits,
+                                const int32_t* cell_idx, const int32_t* valid, const void* c,
+                                const void* b, void* h_new, void* q_new, void* age_new,
+                                void* h_old_saved, int B, int N, int d, int K, int dtype,
+                                void* stream);
 
 /*
  * Its backward (reference hsn_ops.h:173-187), from G = grad_h_out [B,N,d], g = grad_q_out [B,d]:

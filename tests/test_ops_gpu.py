@@ -473,3 +473,74 @@ def test_unit_mlp_takes_operands_off_the_four_element_alignment(ops, cuda_device
     shifted = torch.empty(v.numel() + 1, device=dev)[1:].view(P, 4 * d).copy_(v)
     for a, b in zip(ops.mlp_op(v, idx, W1, b1, W2, b2), ops.mlp_op(shifted, idx, W1, b1, W2, b2)):
         torch.testing.assert_close(a, b, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,N,K,d", [(1, 1, 1, 4), (3, 130, 19, 36), (2, 64, 8, 6), (2, 65, 9, 300)])
+def test_update_into_fresh_tensors_equals_the_update_in_place(ops, cuda_device, B, N, K, d, dtype):
+    """One launch that copies and updates gives the copies' in-place update bit for bit: a partial
+    last block of copied cells, d off the four-element copies and above the workgroup's threads,
+    padded slots, and cells repeated inside a batch of 8 slots and across batches."""
+    g = torch.Generator().manual_seed(B * 100 + N)
+    dev = cuda_device
+    rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)  # noqa: E731
+    h, q, c, b = rnd(B, N, d), rnd(B, d), rnd(B, K, d), rnd(B, K, d)
+    cells = torch.randint(0, N, (B, K), generator=g)
+    if K > 8:
+        cells[0, 5], cells[0, K - 1] = cells[0, 2], cells[0, 2]
+    valid = torch.rand(B, K, generator=g) > 0.2
+    age = torch.randint(0, 9, (B, N), generator=g)
+    h2, q2, age2 = h.clone(), q.clone(), age.to(torch.int32).to(dev)
+    old = ops.update_inplace(h2, q2, age2, cells.to(torch.int32).to(dev),
+                             valid.to(torch.int32).to(dev), c, b)
+    for dt in (torch.int32, torch.int64):
+        got = ops.update_op(h, q, age.to(dt).to(dev), cells.to(dev), valid.to(dev), c, b)
+        assert got[2].dtype == dt
+        for name, x, y in zip(("h", "q", "age", "old"), got, (h2, q2, age2.to(dt), old)):
+            assert torch.equal(x, y), name
+
+
+@pytest.mark.parametrize("E_extra", [0, 5])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_ops_read_either_index_width(ops, cuda_device, dtype, E_extra):
+    """int64 indices and bool flags read in place give the int32 arrays' results bit for bit, in
+    every op that takes them; the messages on uneven rows, more than one block of cells a
+    workgroup, and (``E_extra``) edges past the last row, whose grad_a is zero."""
+    from oracle import hsn_oracle as O
+
+    g = torch.Generator().manual_seed(77 + E_extra)
+    dev = cuda_device
+    B, N, K, d = 300, 270, 5, 20
+    rnd = lambda *s: (torch.randn(*s, generator=g) * 0.5).to(dtype)  # noqa: E731
+    cells = torch.randint(0, N, (B, K), generator=g)
+    valid = torch.rand(B, K, generator=g) > 0.2
+    deg = torch.randint(0, 6, (N,), generator=g)
+    indptr = torch.cat([torch.zeros(1, dtype=torch.int64), deg.cumsum(0)])
+    E = int(indptr[-1]) + E_extra
+    indices = torch.randint(0, N, (E,), generator=g)
+    h, V, a, dm = rnd(B, N, d), rnd(d, d), rnd(E), rnd(B, K, d)
+    u, eps, q, G, dv = rnd(B, d), rnd(B, d), rnd(B, d), rnd(B, N, d), rnd(B, K, 4 * d)
+    D = {k: t.to(dev) for k, t in dict(h=h, V=V, a=a, dm=dm, u=u, eps=eps, q=q, G=G, dv=dv).items()}
+
+    def run(i, f):
+        cell, ip, ix, ok = (cells.to(i).to(dev), indptr.to(i).to(dev), indices.to(i).to(dev),
+                            valid.to(f).to(dev))
+        out = [ops.messages_op(D["h"], ip, ix, D["a"], D["V"], cell),
+               *ops.messages_backward(D["h"], ip, ix, D["a"], D["V"], cell, D["dm"]),
+               ops.gather_op(D["u"], D["eps"], D["h"], D["dm"], cell),
+               *ops.gather_backward(D["dv"], cell, N),
+               *ops.update_backward(cell, ok, D["dm"], D["dm"], D["dm"], D["G"], D["q"])]
+        return out
+
+    wide, narrow = run(torch.int64, torch.bool), run(torch.int32, torch.int32)
+    for i, (x, y) in enumerate(zip(wide, narrow)):
+        assert torch.equal(x, y), i
+    want = O.csr_messages_bwd(h.double(), indptr, indices[:E - E_extra], a[:E - E_extra].double(),
+                              V.double(), cells, dm.double())
+    _close(wide[1], want[0], dtype, "grad_h")
+    _close(wide[2][:E - E_extra], want[1], dtype, "grad_a", scaled=True)
+    assert bool((wide[2][E - E_extra:] == 0).all())
+    _close(wide[3], want[2], dtype, "grad_V", scaled=True)
+    mixed = ops.messages_op(D["h"], indptr.to(dev), indices.to(torch.int32).to(dev), D["a"], D["V"],
+                            cells.to(dev))
+    assert torch.equal(mixed, wide[0])
