@@ -252,7 +252,10 @@ def _trainer_main(args) -> int:
     torch.cuda.synchronize()
     kernel_ms = sum(a.elapsed_time(b) for a, b in events) / args.steps
     achieved = elements * TRAINER_BYTES_PER_ELEMENT / (kernel_ms * 1e-3) / 1e9
-    launches = -(-len([n for n in sizes if n]) // 88)  # tensors a launch of the AdamW pass
+    # tensors a launch of the AdamW pass: 200 in a packed launch (lists of up to 65535 chunks of
+    # 1024 elements), else 88
+    per_launch = 200 if sum(-(-n // 1024) for n in sizes) <= 65535 else 88
+    launches = -(-len([n for n in sizes if n]) // per_launch)
     result = {
         "metric": f"trainer AdamW pass elements/sec ({args.trainer} parameter list, 1 GPU)",
         "value": elements / pass_secs,

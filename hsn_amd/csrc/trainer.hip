@@ -19,6 +19,7 @@
 // workgroup), a thread four elements 256 apart, so every load and store of a wavefront is one
 // coalesced run. The passes are HBM-bound: AdamW moves 28 bytes an element (four rows read, three
 // written).
+#include <algorithm>
 #include <string>
 #include <type_traits>
 
@@ -41,8 +42,8 @@ enum TrOp : int { kAdamW, kAdamWUnits, kLerp, kScale64, kCopy, kLimitSquares, kL
 
 // The by-value launch descriptor (under the 4 KiB of kernel arguments): T tensors a launch (a
 // longer list takes several), and with U the unit coefficients of the stacked-unit AdamW, whose
-// 1.5 KiB leave room for 48 tensors; the other passes take 88 (the model's 198 tensors in three
-// launches, not five).
+// 1.5 KiB leave room for 48 tensors; the other passes take 88 where the list does not pack
+// (TrPackT below).
 template <int T, bool U>
 struct TrArgsT {
     static constexpr int kTensors = T;
@@ -55,11 +56,43 @@ struct TrArgsT {
     float f[8];
     float u[U ? 6 : 1][U ? kTrUnits : 1];
     const double* coef;  // scale64: the coefficient, one f64 on the device
+    __device__ __forceinline__ float* row(int r, int j) const { return p[r][j]; }
+    __device__ __forceinline__ int64_t count(int j) const { return numel[j]; }
+    __device__ __forceinline__ int first(int j) const { return chunk0[j]; }
 };
 using TrArgsUnits = TrArgsT<48, true>;
 using TrArgs = TrArgsT<88, false>;
 static_assert(sizeof(TrArgsUnits) <= 4096 && sizeof(TrArgs) <= 4096,
               "kernel arguments take at most 4 KiB");
+// The same in 4 bytes an operand and 4 more a tensor: each row's lowest address and every tensor's
+// distance from it in elements (below 2^32: 16 GiB), the first chunks in 16 bits, and a tensor's
+// elements as its chunks and the last chunk's 1..1024. Up to 200 tensors of four operands, 333 of
+// two, 500 of one a launch, where they hold at most 65535 chunks (67 M elements): the model's 198
+// tensors in one launch a pass (three before: copy, scale, AdamW and lerp 60 -> 31.8 us of GPU time
+// a step). A longer list's launches are long enough without it.
+template <int ROWS>
+struct TrPackT {
+    static constexpr int kTensors = (4096 - 96) / (4 * ROWS + 4);
+    static constexpr int kRows = ROWS;
+    float* base[ROWS];
+    uint32_t off[ROWS][kTensors];
+    uint32_t span[kTensors];  // the first chunk << 16 | the last chunk's elements less one (read as
+                              // words: 16-bit kernel arguments are no scalar loads)
+    int32_t n, flag;
+    float f[8];
+    const double* coef;
+    __device__ __forceinline__ float* row(int r, int j) const { return r < ROWS ? base[r] + off[r][j] : nullptr; }
+    __device__ __forceinline__ int64_t count(int j) const {
+        const int end = j + 1 < n ? first(j + 1) : int(gridDim.x);
+        return int64_t(end - first(j) - 1) * kTrChunk + (span[j] & 0xffffu) + 1;
+    }
+    __device__ __forceinline__ int first(int j) const { return static_cast<int>(span[j] >> 16); }
+};
+static_assert(sizeof(TrPackT<1>) <= 4096 && sizeof(TrPackT<2>) <= 4096 && sizeof(TrPackT<4>) <= 4096,
+              "kernel arguments take at most 4 KiB");
+constexpr int kTrPackChunks = 65535;
+template <int OP>
+using TrPackOf = TrPackT<OP == kScale64 ? 1 : OP == kLerp || OP == kCopy ? 2 : 4>;
 template <int OP>
 using TrArgsOf = std::conditional_t<OP == kAdamWUnits, TrArgsUnits, TrArgs>;
 
@@ -166,19 +199,19 @@ __device__ __forceinline__ void tr_op(const A& a, const TrUniform& q, int64_t o,
 // Measured on an AdamW pass over 1 GiB rows: 5.77 TB/s, against 6.16 TB/s for a plain copy; 16-byte
 // accesses (runs of four elements a thread, loads issued together or per run) and sixteen elements
 // a thread measured 5.3-5.4 TB/s, a grid-stride loop 4.5 TB/s.
-template <int OP>
-__global__ __launch_bounds__(kTrThreads) void tr_pass(TrArgsOf<OP> a) {
+template <int OP, typename Args>
+__global__ __launch_bounds__(kTrThreads) void tr_pass(Args a) {
     constexpr int kRd = TrRows<OP>::rd;
     const int c = blockIdx.x;
     int lo = 0, hi = a.n - 1;  // the tensor holding chunk c: the last j with chunk0[j] <= c
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (a.chunk0[mid] <= c) lo = mid;
+        if (a.first(mid) <= c) lo = mid;
         else hi = mid - 1;
     }
     const int j = uniform(lo);
-    const int64_t base = int64_t(c - a.chunk0[j]) * kTrChunk;
-    const int64_t numel = a.numel[j];
+    const int64_t base = int64_t(c - a.first(j)) * kTrChunk;
+    const int64_t numel = a.count(j);
     TrUniform q{};
     if constexpr (OP == kAdamWUnits) {
         __shared__ float su[6][kTrUnits];
@@ -193,7 +226,7 @@ __global__ __launch_bounds__(kTrThreads) void tr_pass(TrArgsOf<OP> a) {
     }
     if constexpr (OP == kScale64) q.coef = *a.coef;
     if constexpr (OP == kLimitProject) {
-        const float* group = a.p[3][j];
+        const float* group = a.row(3, j);
         q.scale = group[0];
         q.clipped = group[1] != 0.0f;
     }
@@ -206,18 +239,68 @@ __global__ __launch_bounds__(kTrThreads) void tr_pass(TrArgsOf<OP> a) {
         if (o >= numel) break;
         float x[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) x[r] = (kRd >> r & 1) ? a.p[r][j][o] : 0.0f;
+        for (int r = 0; r < 4; ++r) x[r] = (kRd >> r & 1) ? a.row(r, j)[o] : 0.0f;
         tr_op<OP>(a, q, o, x);
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            if (wr >> r & 1) a.p[r][j][o] = x[r];
+            if (wr >> r & 1) a.row(r, j)[o] = x[r];
     }
 }
 
-// The list, in launches of at most TrArgsOf<OP>::kTensors tensors (empty tensors skipped).
+// The list in packed launches, where it holds at most kTrPackChunks chunks and every row's tensors
+// lie within 2^32 elements of its lowest address; false where they do not (nothing launched).
+template <int OP>
+bool tr_launch_packed(const TrArgsOf<OP>& w, float* const* const rows[kTrRows], const int64_t* numels,
+                      int n, hipStream_t st) {
+    using Pack = TrPackOf<OP>;
+    int64_t chunks = 0;
+    uintptr_t low[Pack::kRows];
+    for (int r = 0; r < Pack::kRows; ++r) low[r] = UINTPTR_MAX;
+    for (int j = 0; j < n; ++j) {
+        if (numels[j] == 0) continue;
+        if (numels[j] > int64_t(kTrPackChunks) * kTrChunk) return false;
+        chunks += (numels[j] + kTrChunk - 1) / kTrChunk;
+        if (chunks > kTrPackChunks) return false;
+        for (int r = 0; r < Pack::kRows; ++r)
+            low[r] = std::min(low[r], reinterpret_cast<uintptr_t>(rows[r][j]));
+    }
+    for (int j = 0; j < n; ++j) {
+        if (numels[j] == 0) continue;
+        for (int r = 0; r < Pack::kRows; ++r) {
+            const uintptr_t d = reinterpret_cast<uintptr_t>(rows[r][j]) - low[r];
+            if (d % 4 != 0 || d / 4 > UINT32_MAX) return false;
+        }
+    }
+    Pack a{};
+    a.flag = w.flag;
+    for (int k = 0; k < 8; ++k) a.f[k] = w.f[k];
+    a.coef = w.coef;
+    for (int r = 0; r < Pack::kRows; ++r) a.base[r] = reinterpret_cast<float*>(low[r]);
+    for (int j = 0; j < n;) {
+        int m = 0, at = 0;
+        for (; j < n && m < Pack::kTensors; ++j) {
+            if (numels[j] == 0) continue;
+            for (int r = 0; r < Pack::kRows; ++r)
+                a.off[r][m] = static_cast<uint32_t>((reinterpret_cast<uintptr_t>(rows[r][j]) - low[r]) / 4);
+            a.span[m] = uint32_t(at) << 16 | static_cast<uint32_t>((numels[j] - 1) % kTrChunk);
+            at += static_cast<int>((numels[j] + kTrChunk - 1) / kTrChunk);
+            ++m;
+        }
+        if (m == 0) break;
+        a.n = m;
+        hipLaunchKernelGGL((tr_pass<OP, Pack>), dim3(at), dim3(kTrThreads), 0, st, a);
+        HSN_HIP(hipGetLastError());
+    }
+    return true;
+}
+
+// The list, packed where it can be, else in launches of at most TrArgsOf<OP>::kTensors tensors
+// (empty tensors skipped).
 template <int OP>
 void tr_launch(TrArgsOf<OP>& a, float* const* const rows[kTrRows], const int64_t* numels, int n,
                hipStream_t st) {
+    if constexpr (OP != kAdamWUnits)
+        if (tr_launch_packed<OP>(a, rows, numels, n, st)) return;
     int j = 0;
     while (j < n) {
         int m = 0, chunks = 0;
@@ -235,7 +318,7 @@ void tr_launch(TrArgsOf<OP>& a, float* const* const rows[kTrRows], const int64_t
         if (m == 0) break;
         a.n = m;
         a.chunk0[m] = chunks;
-        hipLaunchKernelGGL(tr_pass<OP>, dim3(chunks), dim3(kTrThreads), 0, st, a);
+        hipLaunchKernelGGL((tr_pass<OP, TrArgsOf<OP>>), dim3(chunks), dim3(kTrThreads), 0, st, a);
         HSN_HIP(hipGetLastError());
     }
 }

@@ -397,3 +397,44 @@ def test_adamw_pass_replays_in_a_graph(dev):
             g.mul_(-0.5)
         for g in theirs[1]:
             g.mul_(-0.5)
+
+
+@pytest.mark.parametrize("n", [1, 199, 200, 201, 333, 334, 1001])
+def test_packed_launches_at_their_edges(dev, n):
+    """Lists around the packed launches' tensor counts (200 of four operands, 333 of two, 500 of
+    one), with tensors of 1, 1023, 1024 and 1025 elements and empty ones among them, each pass bit
+    for bit the multi-tensor operation."""
+    from hsn_amd import trainer
+
+    g = torch.Generator(device=dev).manual_seed(n)
+    sizes = [(1, 1023, 1024, 1025, 0, 7, 4096)[i % 7] for i in range(n)]
+    make = lambda: [torch.randn(k, device=dev, generator=g) for k in sizes]  # noqa: E731
+    a, b = make(), make()
+    want = [x.clone() for x in a]
+    torch._foreach_lerp_(want, b, 0.3)
+    assert trainer.lerp(a, b, 0.3)
+    assert all(torch.equal(x, y) for x, y in zip(a, want))
+    assert trainer.copy(a, b) and all(torch.equal(x, y) for x, y in zip(a, b))
+    c = torch.tensor([0.7], dtype=torch.float64, device=dev)
+    assert trainer.scale64(a, c)
+    assert all(torch.equal(x, (y.double() * c).float()) for x, y in zip(a, b))
+    p, m, v = make(), make(), [t.square() for t in make()]
+    P, M, V = ([t.clone() for t in x] for x in (p, m, v))
+    hyper = dict(lr=1e-3, beta1=0.9, beta2=0.999, eps=1e-8, weight_decay=0.01)
+    assert trainer.adamw(p, b, m, v, step=3, **hyper)
+    full = [i for i, k in enumerate(sizes) if k]
+    for i in range(0, len(full), 40):  # the same step in short lists
+        some = full[i:i + 40]
+        assert trainer.adamw(*([x[j] for j in some] for x in (P, b, M, V)), step=3, **hyper)
+    for x, y in ((p, P), (m, M), (v, V)):
+        assert all(torch.equal(s, t) for s, t in zip(x, y))
+
+
+def test_a_list_of_more_chunks_than_a_packed_launch_takes(dev):
+    """Above 65535 chunks of 1024 elements the wide descriptors take the list."""
+    from hsn_amd import trainer
+
+    srcs = [torch.arange(k, device=dev, dtype=torch.float32) for k in (40_000_003, 5, 28_000_000)]
+    dsts = [torch.empty_like(s) for s in srcs]
+    assert trainer.copy(dsts, srcs)
+    assert all(torch.equal(d, s) for d, s in zip(dsts, srcs))
