@@ -998,5 +998,730 @@ __global__ __launch_bounds__(kChainThreads) void chain_bwd(BwdArgs a) {
     }
 }
 
+// ------------------------------------------------------------------------------------------
+// The chains, several cells a wavefront (chain_fwd4, chain_bwd4)
+// ------------------------------------------------------------------------------------------
+//
+// For d a multiple of 4 up to 256 and rows aligned to four elements, a cell's columns lie in L
+// lanes, four a lane (16-byte accesses of fp32 rows, 8-byte ones of bf16), and a wavefront walks
+// 64 / L cells side by side, so one instruction serves an event of each. The cells are taken
+// heaviest first, so neighbours hold about as many events; a lane whose cell has no event left
+// masks its accesses. A cell of more than kHeavy events is walked by a wavefront alone, a column a
+// lane: side by side, the longest chain of a workgroup takes each event at the pace of four cells'
+// instructions (N 4096 with a Zipf bias, 1024 events in the heaviest cells: forward 2.18 ms, all
+// cells side by side, 1.64 with the heavy ones alone).
+//
+// What bounds it is a cell's chain of loads, with 64 / L cells' rows in flight a wavefront. Measured
+// (us, forward and backward; one cell a wavefront in brackets): B64 T512 N1024 d64 K16 bf16 97 and
+// 115 (120 and 128); B128 T128 N512 d128 K8 fp32 75 and 104 (80 and 123), 67 and 93 being their
+// bytes at a copy's 5.03 TB/s; B256 T1024 N4096 d64 K32 bf16 Zipf 1639 and 1695 (1734 and 1654). Eight
+// wavefronts a workgroup and about two workgroups a CU: four wavefronts 109 and 120 at the first
+// shape, 2048 workgroups 149 and 131. Batches of four events 97 and 116, all cells' 200 events side
+// by side (kHeavy 200) 111 and 122.
+//
+// The row maxima are marked per interval between a cell's events on three scales (positions, 16
+// and 256 of them), at most five LDS atomics an interval instead of one a position and wavefront;
+// cells without an event keep one maximum a wavefront.
+
+constexpr int kQuadWaves = 8;
+constexpr int kQuadThreads = 64 * kQuadWaves;
+constexpr int kHeavy = 64;
+constexpr int NB = 2;  // events of a cell in a batch, two batches in flight
+
+struct RawB { uint32_t v[2]; };  // four bf16
+struct RawF { uint32_t v[4]; };  // four fp32
+template <typename IO>
+using Raw = std::conditional_t<sizeof(IO) == 4, RawF, RawB>;
+
+__device__ __forceinline__ RawF load_raw(rsrc_t r, uint32_t vo, const float*) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, vo, 0u, 0);
+    return RawF{{v[0], v[1], v[2], v[3]}};
+}
+__device__ __forceinline__ RawB load_raw(rsrc_t r, uint32_t vo, const bf16_t*) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, vo, 0u, 0);
+    return RawB{{static_cast<uint32_t>(v[0]), static_cast<uint32_t>(v[1])}};
+}
+__device__ __forceinline__ float lane_of(const RawF& q, int i) { return __uint_as_float(q.v[i]); }
+__device__ __forceinline__ float lane_of(const RawB& q, int i) {
+    return __uint_as_float(i & 1 ? q.v[i / 2] & 0xffff0000u : q.v[i / 2] << 16);
+}
+__device__ __forceinline__ void store4(const float (&x)[4], rsrc_t r, uint32_t vo, const float*) {
+    decltype(__builtin_amdgcn_raw_buffer_load_b128(r, 0u, 0u, 0)) v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = __float_as_uint(x[i]);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, vo, 0u, 0);
+}
+__device__ __forceinline__ void store4(const float (&x)[4], rsrc_t r, uint32_t vo, const bf16_t*) {
+    decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0u, 0u, 0)) v;
+    v[0] = uint32_t(from_f32<bf16_t>(x[0]).bits) | uint32_t(from_f32<bf16_t>(x[1]).bits) << 16;
+    v[1] = uint32_t(from_f32<bf16_t>(x[2]).bits) | uint32_t(from_f32<bf16_t>(x[3]).bits) << 16;
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, vo, 0u, 0);
+}
+
+// LDS words of a quad workgroup: chain_words, and the maxima's two coarse scales.
+__host__ __device__ inline int coarse_words(int T) { return (T + 15) / 16 + (T + 255) / 256; }
+__host__ __device__ inline int quad_words(int T, int C, int stage) {
+    return chain_words(T, C, stage) + coarse_words(T);
+}
+
+// val into the maxima of positions [p0, p1), by the L lanes of a group.
+template <int L>
+__device__ __forceinline__ void mark_run(uint32_t* tab, int p0, int p1, uint32_t val, int l) {
+    for (int p = p0 + l; p < p1; p += L) atomicMax(&tab[p], val);
+}
+template <int L>
+__device__ __forceinline__ void mark(uint32_t* hm, uint32_t* hc, uint32_t* hs, int p0, int p1,
+                                     uint32_t val, int l) {
+    if (p0 >= p1 || val == 0u) return;
+    const int a = min(p1, (p0 + 15) & ~15);
+    mark_run<L>(hm, p0, a, val, l);
+    if (a >= p1) return;
+    const int b = p1 & ~15;  // [a, b) is whole blocks of 16
+    mark_run<L>(hm, b, p1, val, l);
+    const int c0 = a / 16, c1 = b / 16, ca = min(c1, (c0 + 15) & ~15);
+    mark_run<L>(hc, c0, ca, val, l);
+    if (ca >= c1) return;
+    const int cb = c1 & ~15;
+    mark_run<L>(hc, cb, c1, val, l);
+    mark_run<L>(hs, ca / 16, cb / 16, val, l);
+}
+
+// The cells of more than kHeavy events: the first of the order (heaviest first).
+__device__ __forceinline__ int heavy_cells(const int* cptr, const int* order, int nc) {
+    int lo = 0, hi = nc;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1, ci = order[mid];
+        if (cptr[ci + 1] - cptr[ci] > kHeavy) lo = mid + 1;
+        else hi = mid;
+    }
+    return uniform(lo);
+}
+
+template <typename IO, int L, bool DELTA, bool HMAX>
+__global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
+    extern __shared__ uint32_t lds_u[];
+    constexpr int Q = kWave / L;
+    int b, g;
+    group_coords(b, g);
+    const int tid = threadIdx.x, lane = lane_id(), l = lane % L, gq = lane / L;
+    const int T = a.T, N = a.N, d = a.d, K = a.K;
+    const int TW = (T + 31) / 32;
+    int* nr = reinterpret_cast<int*>(lds_u);                  // [T + 2]
+    uint32_t* rbits = lds_u + (T + 2);                        // [TW]
+    int* nx = reinterpret_cast<int*>(rbits + TW);             // [TW + 1]
+    uint32_t* hm = reinterpret_cast<uint32_t*>(nx + TW + 1);  // [T]
+    int* next = reinterpret_cast<int*>(hm + T);               // [1]
+    int* cptr = next + 1;                                     // [C + 1]
+    int* cev = cptr + a.C + 1;                                // [stage]
+    int* order = cev + a.stage;                               // [C]
+    uint32_t* hc = reinterpret_cast<uint32_t*>(order + a.C);  // [(T + 15) / 16]
+    uint32_t* hs = hc + (T + 15) / 16;                        // [(T + 255) / 256]
+    const int c_begin = g * a.C, c_end = min(N, c_begin + a.C);
+    const int nc = c_end - c_begin;
+    const int32_t* ptr = a.ptr + int64_t(b) * (N + 1);
+    const int32_t* ev = a.ev + int64_t(b) * T * K;
+    const int pc0 = ptr[c_begin];
+    const int nst = min(ptr[c_end] - pc0, a.stage);
+    const int pad_begin = ptr[N];
+    for (int i = tid; i <= nc; i += kQuadThreads) cptr[i] = ptr[c_begin + i];
+    for (int i = tid; i < nst; i += kQuadThreads) cev[i] = ev[pc0 + i];
+    if constexpr (HMAX) {
+        for (int p = tid; p < T; p += kQuadThreads) hm[p] = 0u;
+        for (int p = tid; p < coarse_words(T); p += kQuadThreads) hc[p] = 0u;
+    }
+    if (tid == 0) next[0] = 0;
+    const int lrT = reset_table(a.reset ? a.reset + int64_t(b) * T : nullptr, T, nr, rbits, nx,
+                                tid, kQuadThreads);
+    heavy_first(cptr, nc, order, tid, kQuadThreads);
+    const int64_t slot0 = int64_t(b) * T * K;
+    const uint32_t row_bytes = uint32_t(T) * K * d * sizeof(IO);
+    const IO* kind = nullptr;
+    const rsrc_t ry = make_rsrc(static_cast<const IO*>(a.y) + slot0 * d, row_bytes);
+    const rsrc_t rg = make_rsrc(static_cast<const IO*>(a.g) + slot0 * d, row_bytes);
+    const rsrc_t rho = make_rsrc(a.h_old ? static_cast<IO*>(a.h_old) + slot0 * d : nullptr,
+                                 a.h_old ? row_bytes : 0u);
+    const rsrc_t rhs = make_rsrc(a.h_sel ? static_cast<IO*>(a.h_sel) + slot0 * d : nullptr,
+                                 a.h_sel ? row_bytes : 0u);
+    const rsrc_t rdl = make_rsrc(a.delta ? a.delta + slot0 * d : nullptr,
+                                 a.delta ? uint32_t(T) * K * d * 4u : 0u);
+    const int n_slots = T * K;
+    const bool pads = pad_begin < n_slots;  // cell 0 then also writes the padded slots: by itself
+    const bool cin = 4 * l < d;
+    const uint32_t ocol = uint32_t(4 * l) * sizeof(IO), ocol4 = uint32_t(4 * l) * 4u;
+    const uint32_t srow = uint32_t(d) * sizeof(IO), srow4 = uint32_t(d) * 4u;
+    const rsrc_t rh0 = make_rsrc(a.h0 + int64_t(b) * N * d, uint32_t(N) * srow4);
+    const rsrc_t rhT = make_rsrc(a.h_T ? a.h_T + int64_t(b) * N * d : nullptr,
+                                 a.h_T ? uint32_t(N) * srow4 : 0u);
+    const int nr0 = nr[0];
+
+    auto end_age = [&](int c, int tprev) __attribute__((always_inline)) {
+        int64_t age;
+        if (tprev >= 0 && tprev >= lrT) age = (T - 1) - tprev;
+        else if (lrT >= 0) age = T - lrT;
+        else age = a.age0[int64_t(b) * N + c] + T;
+        a.age_T[int64_t(b) * N + c] = age;
+    };
+
+    // one cell by the whole wavefront, a column a lane and register (lane + 64 v): the cells of more
+    // than kHeavy events, whose chain a wavefront of several cells would walk more slowly, and cell
+    // 0 where the row has padded slots
+    constexpr int V = L <= 16 ? 1 : L / 16;
+    constexpr bool want_max = HMAX;
+    uint32_t voff[V], voff4[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const bool in = lane + 64 * v < d;
+        voff[v] = in ? uint32_t(lane + 64 * v) * sizeof(IO) : kOob;
+        voff4[v] = in ? uint32_t(lane + 64 * v) * 4u : kOob;
+    }
+    auto single = [&](auto pad_cell, int ci) __attribute__((always_inline)) {
+        constexpr bool kPadCell = decltype(pad_cell)::value;
+        const int c = c_begin + ci;
+        const int e_beg = uniform(cptr[ci]), e_end = uniform(cptr[ci + 1]);
+        float h[V];
+        const float* h0c = a.h0 + (int64_t(b) * N + c) * d;
+#pragma unroll
+        for (int v = 0; v < V; ++v) h[v] = lane + 64 * v < d ? h0c[lane + 64 * v] : 0.0f;
+        float hold_last[V];  // the state before the latest event (cell 0's padded slots)
+#pragma unroll
+        for (int v = 0; v < V; ++v) hold_last[v] = 0.0f;
+        uint32_t vprev = want_max ? cell_abs_max<V>(h, lane, d) : 0u;
+        int tprev = -1, s = 0;
+        int nrprev = nr[0];  // the first reset after the latest event
+        // cell 0's padded slots at positions below `limit`, in time order (a window of 64 of
+        // them in the lanes)
+        int pp = pad_begin, pwb = -1, pwv = 0;
+        auto flush = [&](int limit) __attribute__((always_inline)) {
+            while (pp < n_slots) {
+                if (pwb < 0 || pp >= pwb + kEvWin) {
+                    pwb = pp;
+                    pwv = lane < n_slots - pp ? ev[pp + lane] : 0x7fffffff;
+                }
+                const int off = pp - pwb;
+                const uint64_t below = ballot(lane >= off && (pwv >> 8) < limit);
+                const int n = __popcll(below);
+                for (int i = 0; i < n; ++i) {
+                    const int q = __builtin_amdgcn_readlane(pwv, off + i);
+                    const int t = q >> 8;
+                    const uint32_t so = uint32_t(t * K + (q & 255)) * srow;
+                    const bool same = t == tprev;
+                    const bool zero = nrprev <= t;
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        const float now = zero ? 0.0f : h[v];
+                        bstore_f32<IO>(same ? hold_last[v] : now, rho, voff[v], so);
+                        bstore_f32<IO>(same ? h[v] : now, rhs, voff[v], so);
+                    }
+                }
+                pp += n;
+                if (off + n < kEvWin) break;  // the next one is at or after `limit`
+            }
+        };
+        // one event: position t, its slot's byte offsets (so: storage rows, so4: fp32 rows) and
+        // the first reset after t
+        auto update = [&](auto pad_c, int t, uint32_t so, uint32_t so4, int nrq, const IO (&yv)[V],
+                          const IO (&gv)[V]) __attribute__((always_inline)) {
+            constexpr bool kPad = decltype(pad_c)::value;
+            const bool zero = nrprev <= t;  // a reset since the cell's last event
+            if constexpr (want_max) max_interval(hm, s, min(t, nrprev), vprev, lane);
+            if constexpr (kPad) flush(t);
+#pragma unroll
+            for (int v = 0; v < V; ++v) {
+                const float hold = zero ? 0.0f : h[v];
+                const float bg = fast_sigmoid(to_f32(gv[v]));
+                const float cand = fast_tanh(to_f32(yv[v]));
+                const float hn = (1.0f - bg) * hold + bg * cand;
+                bstore_f32<IO>(hold, rho, voff[v], so);
+                bstore_f32<IO>(hn, rhs, voff[v], so);
+                if constexpr (DELTA) bstore(hn - hold, rdl, voff4[v], so4);
+                if constexpr (kPad) hold_last[v] = hold;
+                h[v] = hn;
+            }
+            if constexpr (want_max) vprev = cell_abs_max<V>(h, lane, d);
+            s = t;
+            tprev = t;
+            nrprev = nrq;
+            if constexpr (kPad) flush(t + 1);
+        };
+        // windows of 64 events (one per lane), in batches of 4 with two batches in flight; a
+        // window's positions, slot offsets and next resets are computed for all its events at
+        // once (lane i: event i) and read per event with readlane
+        auto walk = [&](auto staged_c, auto pad_c) __attribute__((always_inline)) {
+            constexpr bool kStaged = decltype(staged_c)::value;
+            for (int w0 = e_beg; w0 < e_end; w0 += kEvWin) {
+                const int m = min(kEvWin, e_end - w0);
+                int evw;
+                if constexpr (kStaged) evw = lane < m ? cev[w0 - pc0 + lane] : 0;
+                else evw = lane < m ? ev[w0 + lane] : 0;
+                const int tw = evw >> 8;
+                const int slw = tw * K + (evw & 255);
+                const uint32_t sow = uint32_t(slw) * srow;
+                const uint32_t so4w = uint32_t(slw) * srow4;
+                const int nrw = lane < m ? nr[tw + 1] : T;
+                IO ya[4][V], ga[4][V], yb[4][V], gb[4][V];
+                auto fetch = [&](int j, IO (&yv)[4][V], IO (&gv)[4][V])
+                                 __attribute__((always_inline)) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t so = __builtin_amdgcn_readlane(sow, min(j + i, kEvWin - 1));
+                        fetch_rows<IO, V>(yv[i], gv[i], ry, rg, voff, so, j + i < m);
+                    }
+                };
+                auto step = [&](int j, const IO (&yv)[4][V], const IO (&gv)[4][V])
+                                __attribute__((always_inline)) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if (j + i < m) {
+                            const int idx = j + i;
+                            update(pad_c, __builtin_amdgcn_readlane(tw, idx),
+                                   __builtin_amdgcn_readlane(sow, idx),
+                                   DELTA ? __builtin_amdgcn_readlane(so4w, idx) : 0u,
+                                   __builtin_amdgcn_readlane(nrw, idx), yv[i], gv[i]);
+                        }
+                    }
+                };
+                fetch(0, ya, ga);
+                for (int j = 0; j < m; j += 2 * 4) {
+                    fetch(j + 4, yb, gb);
+                    step(j, ya, ga);
+                    if (j + 4 >= m) break;
+                    fetch(j + 2 * 4, ya, ga);
+                    step(j + 4, yb, gb);
+                }
+            }
+        };
+        if constexpr (kPadCell) walk(std::false_type{}, std::true_type{});
+        else if (e_end - pc0 <= nst) walk(std::true_type{}, std::false_type{});
+        else walk(std::false_type{}, std::false_type{});
+        if constexpr (kPadCell) flush(T);
+        if (want_max) max_interval(hm, s, min(T, nrprev), vprev, lane);
+        const bool cleared = nrprev < T;  // a reset after the cell's last event
+        if (a.h_T) {
+            float* hTc = a.h_T + (int64_t(b) * N + c) * d;
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+                if (lane + 64 * v < d) hTc[lane + 64 * v] = cleared ? 0.0f : h[v];
+        }
+        if (a.age_T && lane == 0) end_age(c, tprev);
+    };
+
+    const int heavy = heavy_cells(cptr, order, nc);
+    uint32_t idle = 0u;  // the largest |h| of the cells without an event (this lane's columns)
+    for (;;) {
+        int item = lane == 0 ? atomicAdd(next, 1) : 0;  // a heavy cell, or the next Q light ones
+        item = __builtin_amdgcn_readfirstlane(item);
+        if (item < heavy) {
+            const int ci = uniform(order[item]);
+            if (!(pads && c_begin + ci == 0)) single(std::false_type{}, ci);
+            continue;
+        }
+        const int slot = heavy + (item - heavy) * Q;
+        if (slot >= nc) break;
+        const int my = slot + gq;
+        const int ci = my < nc ? order[my] : 0;
+        const int c = c_begin + ci;
+        const bool has = my < nc && !(pads && c == 0);
+        const int e0 = has ? cptr[ci] : 0;
+        const int n = has ? cptr[ci + 1] - e0 : 0;
+        // heaviest first, so the first group's cell has the most events (the lone cell 0 aside)
+        int nmax = 0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) nmax = max(nmax, __builtin_amdgcn_readlane(n, q * L));
+        const uint32_t oh = has && cin ? uint32_t(c) * srow4 + ocol4 : kOob;
+        float h[4];
+        {
+            const RawF raw = load_raw(rh0, oh, static_cast<const float*>(nullptr));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) h[i] = lane_of(raw, i);
+        }
+        if (nmax == 0) {  // uniform: no cell of the wavefront has an event
+            if constexpr (HMAX)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) idle = umax(idle, abs_bits(h[i]));
+            const bool cleared = nr0 < T;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) h[i] = cleared ? 0.0f : h[i];
+            store4(h, rhT, oh, static_cast<const float*>(nullptr));
+            if (a.age_T && l == 0 && has) end_age(c, -1);
+            continue;
+        }
+        auto abs_max = [&]() __attribute__((always_inline)) {
+            uint32_t m = 0u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m = umax(m, abs_bits(h[i]));
+            return group_max<L>(m);
+        };
+        uint32_t vprev = 0u;
+        int tprev = -1, s = 0, nrprev = nr0;
+        struct Batch {
+            Raw<IO> y[NB], g[NB];
+            int t[NB], sl[NB], nr[NB];
+        };
+        auto walk = [&](auto staged_c) __attribute__((always_inline)) {
+            constexpr bool kStaged = decltype(staged_c)::value;
+            auto fetch = [&](int j, Batch& q) __attribute__((always_inline)) {
+                int e[NB];
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const int at = e0 + min(j + i, max(n - 1, 0));
+                    if constexpr (kStaged) e[i] = n > 0 ? cev[at - pc0] : 0;
+                    else e[i] = n > 0 ? ev[at] : 0;
+                }
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const bool in = j + i < n;
+                    q.t[i] = e[i] >> 8;
+                    q.sl[i] = q.t[i] * K + (e[i] & 255);
+                    q.nr[i] = nr[q.t[i] + 1];
+                    const uint32_t vo = in && cin ? uint32_t(q.sl[i]) * srow + ocol : kOob;
+                    q.y[i] = load_raw(ry, vo, kind);
+                    q.g[i] = load_raw(rg, vo, kind);
+                }
+            };
+            auto step = [&](int j, const Batch& q) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    if (j + i >= nmax) break;  // uniform
+                    const bool in = j + i < n;
+                    const int t = q.t[i];
+                    const bool zero = nrprev <= t;  // a reset since the cell's last event
+                    if constexpr (HMAX)
+                        if (in) mark<L>(hm, hc, hs, s, min(t, nrprev), vprev, l);
+                    const uint32_t vo = in && cin ? uint32_t(q.sl[i]) * srow + ocol : kOob;
+                    float hold[4], hn[4], dl[4];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        hold[x] = zero ? 0.0f : h[x];
+                        const float bg = fast_sigmoid(lane_of(q.g[i], x));
+                        const float cand = fast_tanh(lane_of(q.y[i], x));
+                        hn[x] = (1.0f - bg) * hold[x] + bg * cand;
+                        dl[x] = hn[x] - hold[x];
+                    }
+                    store4(hold, rho, vo, kind);
+                    store4(hn, rhs, vo, kind);
+                    if constexpr (DELTA)
+                        store4(dl, rdl, in && cin ? uint32_t(q.sl[i]) * srow4 + ocol4 : kOob,
+                               static_cast<const float*>(nullptr));
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) h[x] = in ? hn[x] : h[x];
+                    if constexpr (HMAX) {
+                        const uint32_t v = abs_max();
+                        vprev = in ? v : vprev;
+                    }
+                    s = in ? t : s;
+                    tprev = in ? t : tprev;
+                    nrprev = in ? q.nr[i] : nrprev;
+                }
+            };
+            Batch qa, qb;
+            fetch(0, qa);
+            if constexpr (HMAX) vprev = abs_max();  // the start state's, once its load is back
+            for (int j = 0; j < nmax; j += 2 * NB) {
+                fetch(j + NB, qb);
+                step(j, qa);
+                if (j + NB >= nmax) break;
+                fetch(j + 2 * NB, qa);
+                step(j + NB, qb);
+            }
+        };
+        if (ballot(has && e0 + n - pc0 > nst) == 0ull) walk(std::true_type{});
+        else walk(std::false_type{});
+        if constexpr (HMAX)
+            if (has) mark<L>(hm, hc, hs, s, min(T, nrprev), vprev, l);
+        const bool cleared = nrprev < T;  // a reset after the cell's last event
+#pragma unroll
+        for (int i = 0; i < 4; ++i) h[i] = cleared ? 0.0f : h[i];
+        store4(h, rhT, oh, static_cast<const float*>(nullptr));
+        if (a.age_T && l == 0 && has) end_age(c, tprev);
+    }
+    if constexpr (HMAX) {
+        const uint32_t v = wave_max_from_groups<1>(idle);
+        if (lane < L) mark<L>(hm, hc, hs, 0, min(T, nr0), v, l);
+    }
+    if (pads && g == 0 && tid < kWave) single(std::true_type{}, 0);
+    if (a.pos_T && g == 0 && tid == 0) a.pos_T[b] = lrT >= 0 ? int64_t(T - lrT) : a.pos0[b] + T;
+    if constexpr (HMAX) {  // the group's maxima, reduced over the groups by summary_delta
+        __syncthreads();
+        const int G = gridDim.y;
+        uint32_t* hg = a.hm_groups + int64_t(b) * T * G + g;
+        for (int p = tid; p < T; p += kQuadThreads)
+            hg[int64_t(p) * G] = umax(hm[p], umax(hc[p / 16], hs[p / 256]));
+    }
+}
+
+template <typename IO, int L>
+__global__ __launch_bounds__(kQuadThreads, sizeof(IO) == 4 ? 4 : 5) void chain_bwd4(BwdArgs a) {
+    extern __shared__ uint32_t lds_u[];
+    constexpr int Q = kWave / L;
+    int b, g;
+    group_coords(b, g);
+    const int tid = threadIdx.x, lane = lane_id(), l = lane % L, gq = lane / L;
+    const int T = a.T, N = a.N, d = a.d, K = a.K;
+    const int TW = (T + 31) / 32;
+    int* nr = reinterpret_cast<int*>(lds_u);
+    uint32_t* rbits = lds_u + (T + 2);
+    int* nx = reinterpret_cast<int*>(rbits + TW);
+    int* next = nx + TW + 1 + T;  // the layout of chain_fwd4 (no row maxima used)
+    int* cptr = next + 1;
+    int* cev = cptr + a.C + 1;
+    int* order = cev + a.stage;
+    const int c_begin = g * a.C, c_end = min(N, c_begin + a.C);
+    const int nc = c_end - c_begin;
+    const int32_t* ptr = a.ptr + int64_t(b) * (N + 1);
+    const int32_t* ev = a.ev + int64_t(b) * T * K;
+    const int pc0 = ptr[c_begin];
+    const int nst = min(ptr[c_end] - pc0, a.stage);
+    for (int i = tid; i <= nc; i += kQuadThreads) cptr[i] = ptr[c_begin + i];
+    for (int i = tid; i < nst; i += kQuadThreads) cev[i] = ev[pc0 + i];
+    if (tid == 0) next[0] = 0;
+    reset_table(a.reset ? a.reset + int64_t(b) * T : nullptr, T, nr, rbits, nx, tid, kQuadThreads);
+    heavy_first(cptr, nc, order, tid, kQuadThreads);
+    const int64_t slot0 = int64_t(b) * T * K;
+    const uint32_t row_bytes = uint32_t(T) * K * d * sizeof(IO);
+    const IO* kind = nullptr;
+    const float* f32 = nullptr;
+    const rsrc_t ry = make_rsrc(static_cast<const IO*>(a.y) + slot0 * d, row_bytes);
+    const rsrc_t rg = make_rsrc(static_cast<const IO*>(a.g) + slot0 * d, row_bytes);
+    const rsrc_t rho = make_rsrc(static_cast<const IO*>(a.h_old) + slot0 * d, row_bytes);
+    const rsrc_t rds = make_rsrc(a.dsel ? static_cast<const IO*>(a.dsel) + slot0 * d : nullptr,
+                                 a.dsel ? row_bytes : 0u);
+    const rsrc_t rdy = make_rsrc(static_cast<IO*>(a.dy) + slot0 * d, row_bytes);
+    const rsrc_t rdg = make_rsrc(static_cast<IO*>(a.dg) + slot0 * d, row_bytes);
+    const rsrc_t rsh = make_rsrc(a.share + int64_t(b) * T * d, uint32_t(T) * d * 4u);
+    const bool cin = 4 * l < d;
+    const uint32_t ocol = uint32_t(4 * l) * sizeof(IO), ocol4 = uint32_t(4 * l) * 4u;
+    const uint32_t srow = uint32_t(d) * sizeof(IO), srow4 = uint32_t(d) * 4u;
+    const rsrc_t rdhT = make_rsrc(a.dh_T ? a.dh_T + int64_t(b) * N * d : nullptr,
+                                  a.dh_T ? uint32_t(N) * srow4 : 0u);
+    const rsrc_t rdh0 = make_rsrc(a.dh0 ? a.dh0 + int64_t(b) * N * d : nullptr,
+                                  a.dh0 ? uint32_t(N) * srow4 : 0u);
+    const int nr0 = nr[0];
+
+    constexpr int V = L <= 16 ? 1 : L / 16;
+    uint32_t voff[V], voff4[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const bool in = lane + 64 * v < d;
+        voff[v] = in ? uint32_t(lane + 64 * v) * sizeof(IO) : kOob;
+        voff4[v] = in ? uint32_t(lane + 64 * v) * 4u : kOob;
+    }
+    struct Rows {
+        IO y[4][V], g[4][V], h[4][V], s[4][V];
+        float r[4][V];
+    };
+    auto single = [&](int ci) __attribute__((always_inline)) {  // a heavy cell, as in chain_fwd4
+        const int c = c_begin + ci;
+        const int e_beg = uniform(cptr[ci]), e_end = uniform(cptr[ci + 1]);
+        const bool staged = e_end - pc0 <= nst;
+        float A[V];
+        {  // the end cotangent, cut by a reset after the cell's last event
+            const int t_last = e_end > e_beg
+                                   ? (uniform(staged ? cev[e_end - 1 - pc0] : ev[e_end - 1]) >> 8)
+                                   : -1;
+            const bool cut = nr[t_last + 1] < T;
+            const float* dhc = a.dh_T ? a.dh_T + (int64_t(b) * N + c) * d : nullptr;
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+                A[v] = (dhc && !cut && lane + 64 * v < d) ? dhc[lane + 64 * v] : 0.0f;
+        }
+        int tnext = T;  // the later event's position
+        int t_first = T;
+        auto walk = [&](auto staged_c) __attribute__((always_inline)) {
+            constexpr bool kStaged = decltype(staged_c)::value;
+            for (int w1 = e_end; w1 > e_beg; w1 -= kEvWin) {
+                const int m = min(kEvWin, w1 - e_beg);
+                const int w0 = w1 - m;
+                int evw;
+                if constexpr (kStaged) evw = lane < m ? cev[w0 - pc0 + lane] : 0;
+                else evw = lane < m ? ev[w0 + lane] : 0;
+                // the window's positions, slot offsets, share offsets and next resets, for all
+                // its events at once (lane i: event i), read per event with readlane
+                const int tw = evw >> 8;
+                const uint32_t sow = uint32_t(tw * K + (evw & 255)) * srow;
+                const uint32_t stw = uint32_t(tw) * srow4;
+                const int nrw = lane < m ? nr[tw + 1] : T;
+                Rows ra, rb;
+                // batch j holds window indices [j - 4 + 1, j], fetched latest first
+                auto fetch = [&](int j, Rows& r) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int idx = j - i;
+                        const uint32_t so = __builtin_amdgcn_readlane(sow, max(idx, 0));
+                        const uint32_t st = __builtin_amdgcn_readlane(stw, max(idx, 0));
+                        const bool in = idx >= 0;
+#pragma unroll
+                        for (int v = 0; v < V; ++v) {
+                            const uint32_t vo = in ? voff[v] : kOob;
+                            r.y[i][v] = bload<IO>(ry, vo, so);
+                            r.g[i][v] = bload<IO>(rg, vo, so);
+                            r.h[i][v] = bload<IO>(rho, vo, so);
+                            r.s[i][v] = bload<IO>(rds, vo, so);
+                            r.r[i][v] = bload<float>(rsh, in ? voff4[v] : kOob, st);
+                        }
+                    }
+                };
+                auto step = [&](int j, const Rows& r) __attribute__((always_inline)) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int idx = j - i;
+                        if (idx >= 0) {
+                            const int t = __builtin_amdgcn_readlane(tw, idx);
+                            const int nrq = __builtin_amdgcn_readlane(nrw, idx);
+                            const uint32_t so = __builtin_amdgcn_readlane(sow, idx);
+                            const bool zero = nrq <= tnext && tnext < T;  // a reset in (t, tnext]
+#pragma unroll
+                            for (int v = 0; v < V; ++v) {
+                                const float carried = (zero ? 0.0f : A[v]) + to_f32(r.s[i][v]);
+                                const float share = r.r[i][v];
+                                const float gg = carried + share;
+                                const float bg = fast_sigmoid(to_f32(r.g[i][v]));
+                                const float cc = fast_tanh(to_f32(r.y[i][v]));
+                                const float dc = bg * gg * (1.0f - cc * cc);
+                                const float db = (cc - to_f32(r.h[i][v])) * gg * (bg * (1.0f - bg));
+                                bstore_f32<IO>(dc, rdy, voff[v], so);
+                                bstore_f32<IO>(db, rdg, voff[v], so);
+                                A[v] = (1.0f - bg) * carried - bg * share;
+                            }
+                            tnext = t;
+                        }
+                    }
+                };
+                fetch(m - 1, ra);
+                for (int j = m - 1; j >= 0; j -= 2 * 4) {
+                    fetch(j - 4, rb);
+                    step(j, ra);
+                    if (j - 4 < 0) break;
+                    fetch(j - 2 * 4, ra);
+                    step(j - 4, rb);
+                }
+            }
+        };
+        if (staged) walk(std::true_type{});
+        else walk(std::false_type{});
+        t_first = tnext;
+        if (a.dh0) {  // the start state's cotangent: cut by a reset at or before the first event
+            const bool z = nr[0] <= min(t_first, T - 1);
+            float* d0 = a.dh0 + (int64_t(b) * N + c) * d;
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+                if (lane + 64 * v < d) d0[lane + 64 * v] = z ? 0.0f : A[v];
+        }
+    };
+    const int heavy = heavy_cells(cptr, order, nc);
+
+    for (;;) {
+        int item = lane == 0 ? atomicAdd(next, 1) : 0;  // a heavy cell, or the next Q light ones
+        item = __builtin_amdgcn_readfirstlane(item);
+        if (item < heavy) {
+            single(uniform(order[item]));
+            continue;
+        }
+        const int slot = heavy + (item - heavy) * Q;
+        if (slot >= nc) break;
+        const int my = slot + gq;
+        const bool has = my < nc;
+        const int ci = has ? order[my] : 0;
+        const int c = c_begin + ci;
+        const int e0 = has ? cptr[ci] : 0;
+        const int n = has ? cptr[ci + 1] - e0 : 0;
+        const int nmax = __builtin_amdgcn_readfirstlane(n);  // heaviest first: the first group's
+        const bool staged = ballot(has && e0 + n - pc0 > nst) == 0ull;
+        const uint32_t oh = has && cin ? uint32_t(c) * srow4 + ocol4 : kOob;
+        float A[4];
+        {  // the end cotangent, cut by a reset after the cell's last event
+            const int last = n > 0 ? (staged ? cev[e0 + n - 1 - pc0] : ev[e0 + n - 1]) >> 8 : -1;
+            const bool cut = nr[last + 1] < T;
+            const RawF raw = load_raw(rdhT, cut ? kOob : oh, f32);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) A[i] = lane_of(raw, i);
+        }
+        int tnext = T;  // the later event's position
+        struct Batch {
+            Raw<IO> y[NB], g[NB], h[NB], s[NB];
+            RawF r[NB];
+            int t[NB], sl[NB], nr[NB];
+        };
+        auto walk = [&](auto staged_c) __attribute__((always_inline)) {
+            constexpr bool kStaged = decltype(staged_c)::value;
+            // step j of a cell is its event n - 1 - j: latest first
+            auto fetch = [&](int j, Batch& q) __attribute__((always_inline)) {
+                int e[NB];
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const int at = e0 + max(n - 1 - (j + i), 0);
+                    if constexpr (kStaged) e[i] = n > 0 ? cev[at - pc0] : 0;
+                    else e[i] = n > 0 ? ev[at] : 0;
+                }
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const bool in = j + i < n && cin;
+                    q.t[i] = e[i] >> 8;
+                    q.sl[i] = q.t[i] * K + (e[i] & 255);
+                    q.nr[i] = nr[q.t[i] + 1];
+                    const uint32_t vo = in ? uint32_t(q.sl[i]) * srow + ocol : kOob;
+                    q.g[i] = load_raw(rg, vo, kind);
+                    q.s[i] = load_raw(rds, vo, kind);
+                    q.r[i] = load_raw(rsh, in ? uint32_t(q.t[i]) * srow4 + ocol4 : kOob, f32);
+                    q.y[i] = load_raw(ry, vo, kind);
+                    q.h[i] = load_raw(rho, vo, kind);
+                }
+            };
+            auto step = [&](int j, const Batch& q) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    if (j + i >= nmax) break;  // uniform
+                    const bool in = j + i < n;
+                    const bool zero = q.nr[i] <= tnext && tnext < T;  // a reset in (t, tnext]
+                    const uint32_t vo = in && cin ? uint32_t(q.sl[i]) * srow + ocol : kOob;
+                    float dc[4], db[4];
+#pragma unroll
+                    for (int x = 0; x < 4; ++x) {
+                        const float carried = (zero ? 0.0f : A[x]) + lane_of(q.s[i], x);
+                        const float share = lane_of(q.r[i], x);
+                        const float gg = carried + share;
+                        const float bg = fast_sigmoid(lane_of(q.g[i], x));
+                        const float cc = fast_tanh(lane_of(q.y[i], x));
+                        dc[x] = bg * gg * (1.0f - cc * cc);
+                        db[x] = (cc - lane_of(q.h[i], x)) * gg * (bg * (1.0f - bg));
+                        const float An = (1.0f - bg) * carried - bg * share;
+                        A[x] = in ? An : A[x];
+                    }
+                    store4(dc, rdy, vo, kind);
+                    store4(db, rdg, vo, kind);
+                    tnext = in ? q.t[i] : tnext;
+                }
+            };
+            Batch qa, qb;
+            fetch(0, qa);
+            for (int j = 0; j < nmax; j += 2 * NB) {
+                fetch(j + NB, qb);
+                step(j, qa);
+                if (j + NB >= nmax) break;
+                fetch(j + 2 * NB, qa);
+                step(j + NB, qb);
+            }
+        };
+        if (nmax > 0) {
+            if (staged) walk(std::true_type{});
+            else walk(std::false_type{});
+        }
+        // the start state's cotangent: cut by a reset at or before the first event
+        const bool z = nr0 <= min(tnext, T - 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) A[i] = z ? 0.0f : A[i];
+        store4(A, rdh0, oh, f32);
+    }
+    const int n_slots = T * K, pad_begin = ptr[N];
+    if (g == 0) {  // exact zeros on the row's padded slots, a lane group a slot
+        const float zero[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int p = pad_begin + tid / L; p < n_slots; p += kQuadThreads / L) {
+            const int q = ev[p];
+            const uint32_t vo = cin ? uint32_t((q >> 8) * K + (q & 255)) * srow + ocol : kOob;
+            store4(zero, rdy, vo, kind);
+            store4(zero, rdg, vo, kind);
+        }
+    }
+}
+
 }  // namespace chain
 }  // namespace hsn

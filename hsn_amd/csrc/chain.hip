@@ -1,7 +1,10 @@
 // The cell-chain path of hsn_win_forward / hsn_win_backward (chain.cuh): the path choice, the
 // workspace layout and the launchers.
+#include <algorithm>
 #include <atomic>
+#include <initializer_list>
 #include <string>
+#include <type_traits>
 
 #include "abi_util.h"
 #include "chain.cuh"
@@ -22,6 +25,15 @@ inline size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 inline int chain_cells(int B, int N) {
     int C = 16;
     while (C < N && int64_t(B) * ((N + C - 1) / C) > 2048) C *= 2;
+    return C < N ? C : N;
+}
+
+// The same for the kernels that walk several cells a wavefront: about 512 workgroups of eight
+// wavefronts, two a CU, which the registers hold at once; at most 1024 cells (heavy_first's
+// comparisons grow with their square).
+inline int quad_cells(int B, int N) {
+    int C = 32;
+    while (C < N && C < 1024 && int64_t(B) * ((N + C - 1) / C) > 512) C *= 2;
     return C < N ? C : N;
 }
 
@@ -143,7 +155,7 @@ WorkspaceLayout workspace_layout(int op, int B, int T, int N, int d, int K, size
         if (op == HSN_OP_FORWARD) {
             L.delta = at;
             at = align_up(at + size_t(slots) * d * 4);
-            const int C = chain_cells(B, N);
+            const int C = std::min(chain_cells(B, N), quad_cells(B, N));
             L.hmax = at;
             at = align_up(at + size_t(B) * T * ((N + C - 1) / C) * 4);
         }
@@ -187,6 +199,51 @@ void launch_chain_bwd(const chain::BwdArgs& a, size_t lds, hipStream_t st) {
     HSN_HIP(hipGetLastError());
 }
 
+// The kernels that walk several cells a wavefront take d a multiple of 4 and rows aligned to four
+// elements (every access is four columns of a row).
+template <typename IO>
+bool takes_four(int d, std::initializer_list<const void*> rows) {
+    if (d % 4 != 0 || d > 256) return false;
+    for (const void* p : rows)
+        if (reinterpret_cast<uintptr_t>(p) % (4 * sizeof(IO)) != 0) return false;
+    return true;
+}
+template <class F>
+void by_lanes(int d, const F& f) {
+    if (d <= 16) f(std::integral_constant<int, 4>{});
+    else if (d <= 32) f(std::integral_constant<int, 8>{});
+    else if (d <= 64) f(std::integral_constant<int, 16>{});
+    else if (d <= 128) f(std::integral_constant<int, 32>{});
+    else f(std::integral_constant<int, 64>{});
+}
+template <typename IO>
+void launch_chain_fwd4(const chain::FwdArgs& a, hipStream_t st) {
+    const size_t lds = size_t(chain::quad_words(a.T, a.C, a.stage)) * 4;
+    by_lanes(a.d, [&](auto lanes) {
+        constexpr int L = decltype(lanes)::value;
+        auto k = a.delta ? (a.hm_groups ? chain::chain_fwd4<IO, L, true, true>
+                                        : chain::chain_fwd4<IO, L, true, false>)
+                         : (a.hm_groups ? chain::chain_fwd4<IO, L, false, true>
+                                        : chain::chain_fwd4<IO, L, false, false>);
+        HSN_HIP(allow_lds(k, lds));
+        hipLaunchKernelGGL(k, chain::chain_grid(a.B, (a.N + a.C - 1) / a.C),
+                           dim3(chain::kQuadThreads), lds, st, a);
+    });
+    HSN_HIP(hipGetLastError());
+}
+template <typename IO>
+void launch_chain_bwd4(const chain::BwdArgs& a, hipStream_t st) {
+    const size_t lds = size_t(chain::quad_words(a.T, a.C, a.stage)) * 4;
+    by_lanes(a.d, [&](auto lanes) {
+        constexpr int L = decltype(lanes)::value;
+        auto k = chain::chain_bwd4<IO, L>;
+        HSN_HIP(allow_lds(k, lds));
+        hipLaunchKernelGGL(k, chain::chain_grid(a.B, (a.N + a.C - 1) / a.C),
+                           dim3(chain::kQuadThreads), lds, st, a);
+    });
+    HSN_HIP(hipGetLastError());
+}
+
 template <typename IO, int V>
 void launch_delta(const chain::DeltaArgs& a, bool pair, hipStream_t st) {
     const dim3 grid((a.T + 3) / 4, a.B);
@@ -195,15 +252,30 @@ void launch_delta(const chain::DeltaArgs& a, bool pair, hipStream_t st) {
     HSN_HIP(hipGetLastError());
 }
 
+// Whether the several-cells kernels' LDS holds the row (T large).
+template <typename Args>
+bool quad_fits(const Args& a) {
+    const int C = quad_cells(a.B, a.N);
+    return int64_t(chain::quad_words(a.T, C, chain_stage(a.T, a.N, a.K, C))) * 4 <= kLdsMax;
+}
+
 template <typename IO>
-void forward_io(const chain::FwdArgs& fa, const chain::DeltaArgs& da, const chain::ScanArgs& sa,
-                bool pair, size_t lds, hipStream_t st) {
+void forward_io(chain::FwdArgs& fa, chain::DeltaArgs& da, const chain::ScanArgs& sa, bool pair,
+                hipStream_t st) {
+    const bool four = takes_four<IO>(fa.d, {fa.y, fa.g, fa.h_old, fa.h_sel}) &&
+                      takes_four<float>(fa.d, {fa.h0, fa.h_T, fa.delta}) &&
+                      int64_t(fa.N) * fa.d * 4 < (int64_t(1) << 31) && quad_fits(fa);
+    fa.C = four ? quad_cells(fa.B, fa.N) : chain_cells(fa.B, fa.N);
+    fa.stage = chain_stage(fa.T, fa.N, fa.K, fa.C);
+    da.G = (fa.N + fa.C - 1) / fa.C;
+    const size_t lds = size_t(chain::chain_words(fa.T, fa.C, fa.stage)) * 4;
     const int V = (fa.d + 63) / 64;
+    if (four) launch_chain_fwd4<IO>(fa, st);
     switch (V) {
-        case 1: launch_chain_fwd<IO, 1>(fa, lds, st); launch_delta<IO, 1>(da, pair, st); break;
-        case 2: launch_chain_fwd<IO, 2>(fa, lds, st); launch_delta<IO, 2>(da, pair, st); break;
-        case 3: launch_chain_fwd<IO, 3>(fa, lds, st); launch_delta<IO, 3>(da, pair, st); break;
-        default: launch_chain_fwd<IO, 4>(fa, lds, st); launch_delta<IO, 4>(da, pair, st); break;
+        case 1: if (!four) launch_chain_fwd<IO, 1>(fa, lds, st); launch_delta<IO, 1>(da, pair, st); break;
+        case 2: if (!four) launch_chain_fwd<IO, 2>(fa, lds, st); launch_delta<IO, 2>(da, pair, st); break;
+        case 3: if (!four) launch_chain_fwd<IO, 3>(fa, lds, st); launch_delta<IO, 3>(da, pair, st); break;
+        default: if (!four) launch_chain_fwd<IO, 4>(fa, lds, st); launch_delta<IO, 4>(da, pair, st); break;
     }
     hipLaunchKernelGGL((chain::summary_scan_fwd<IO>), dim3((fa.d + 63) / 64, fa.B),
                        dim3(64 * chain::kScanWaves), 0, st, sa);
@@ -211,11 +283,17 @@ void forward_io(const chain::FwdArgs& fa, const chain::DeltaArgs& da, const chai
 }
 
 template <typename IO>
-void backward_io(const chain::BwdArgs& ba, const chain::ScanArgs& sa, size_t lds,
-                 hipStream_t st) {
+void backward_io(chain::BwdArgs& ba, const chain::ScanArgs& sa, hipStream_t st) {
+    const bool four = takes_four<IO>(ba.d, {ba.y, ba.g, ba.h_old, ba.dsel, ba.dy, ba.dg}) &&
+                      takes_four<float>(ba.d, {ba.share, ba.dh_T, ba.dh0}) &&
+                      int64_t(ba.N) * ba.d * 4 < (int64_t(1) << 31) && quad_fits(ba);
+    ba.C = four ? quad_cells(ba.B, ba.N) : chain_cells(ba.B, ba.N);
+    ba.stage = chain_stage(ba.T, ba.N, ba.K, ba.C);
+    const size_t lds = size_t(chain::chain_words(ba.T, ba.C, ba.stage)) * 4;
     hipLaunchKernelGGL((chain::summary_scan_bwd<IO>), dim3((ba.d + 63) / 64, ba.B),
                        dim3(64 * chain::kScanWaves), 0, st, sa);
     HSN_HIP(hipGetLastError());
+    if (four) return launch_chain_bwd4<IO>(ba, st);
     const int V = (ba.d + 63) / 64;
     switch (V) {
         case 1: launch_chain_bwd<IO, 1>(ba, lds, st); break;
@@ -248,17 +326,15 @@ void chain_forward(const void* y, const void* gate_pre, int io_dtype, const uint
     uint32_t* hm_groups = h_max ? reinterpret_cast<uint32_t*>(ws + L.hmax) : nullptr;
     fa.hm_groups = hm_groups, fa.h_T = h_T, fa.age_T = age_T, fa.pos_T = pos_T;
     fa.B = B, fa.T = T, fa.N = N, fa.d = d, fa.K = K;
-    fa.C = chain_cells(B, N), fa.stage = chain_stage(T, N, K, fa.C);
-    const size_t lds = size_t(chain::chain_words(T, fa.C, fa.stage)) * 4;
     chain::DeltaArgs da{};
     da.h_old = h_old, da.h_sel = h_sel, da.delta = delta, da.slots = slots, da.D = D;
     da.hm_groups = hm_groups, da.h_max = h_max;
-    da.B = B, da.T = T, da.N = N, da.d = d, da.K = K, da.G = (N + fa.C - 1) / fa.C;
+    da.B = B, da.T = T, da.N = N, da.d = d, da.K = K;
     chain::ScanArgs sa{};
     sa.D = D, sa.q0 = q0, sa.q_pre = q_pre, sa.q_post = q_post, sa.q_T = q_T;
     sa.reset = reset, sa.B = B, sa.T = T, sa.d = d, sa.divn = make_divn(N);
-    if (io_dtype == HSN_DTYPE_F32) forward_io<float>(fa, da, sa, pair, lds, st);
-    else forward_io<bf16_t>(fa, da, sa, pair, lds, st);
+    if (io_dtype == HSN_DTYPE_F32) forward_io<float>(fa, da, sa, pair, st);
+    else forward_io<bf16_t>(fa, da, sa, pair, st);
 }
 
 void chain_backward(const void* y, const void* gate_pre, const void* h_old, int io_dtype,
@@ -278,10 +354,8 @@ void chain_backward(const void* y, const void* gate_pre, const void* h_old, int 
     ba.y = y, ba.g = gate_pre, ba.h_old = h_old, ba.dsel = d_h_sel, ba.ptr = ptr, ba.ev = ev;
     ba.reset = reset, ba.share = share, ba.dh_T = d_h_T, ba.dy = dy, ba.dg = dgate, ba.dh0 = d_h0;
     ba.B = B, ba.T = T, ba.N = N, ba.d = d, ba.K = K;
-    ba.C = chain_cells(B, N), ba.stage = chain_stage(T, N, K, ba.C);
-    const size_t lds = size_t(chain::chain_words(T, ba.C, ba.stage)) * 4;
-    if (io_dtype == HSN_DTYPE_F32) backward_io<float>(ba, sa, lds, st);
-    else backward_io<bf16_t>(ba, sa, lds, st);
+    if (io_dtype == HSN_DTYPE_F32) backward_io<float>(ba, sa, st);
+    else backward_io<bf16_t>(ba, sa, st);
 }
 
 }  // namespace hsn

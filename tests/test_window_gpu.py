@@ -791,3 +791,74 @@ def test_rms_candidate_at_the_edges_of_its_lanes(dev, B, T, K, d, shift, io):
                                        cand_norm=True, cand_w=w.to(dev))
     _close(dy, ref[0], tol, "dy")
     _close(d_w, ref[4], tol * max(1.0, (B * T * K) ** 0.5 / 8), "d_cand_w")
+
+
+@pytest.mark.parametrize("io", ["f32", "bf16"])
+@pytest.mark.parametrize("B,T,N,K,d,shift", [
+    (2, 9, 5, 2, 4, 0),       # 16 cells a wavefront, fewer cells than that
+    (3, 300, 40, 3, 24, 0),   # 8 lanes a cell, one idle pair; T past one block of 256 positions
+    (2, 200, 12, 5, 64, 0),   # every cell heavy (83 events of more than 64): a wavefront a cell
+    (1, 130, 700, 70, 64, 0), # more slots than lanes, cells without events
+    (2, 40, 33, 4, 100, 0),   # 32 lanes a cell, seven idle
+    (1, 30, 20, 3, 256, 0),   # one cell a wavefront, four columns a lane
+    (2, 50, 40, 3, 24, 1),    # rows off the four-element alignment: a column a lane
+])
+def test_chains_of_several_cells_a_wavefront(dev, B, T, N, K, d, shift, io):
+    """The cell chains with four columns a lane at the edges of their lanes, against the float64
+    oracle: padded slots in the row (a cut budget: cell 0 then goes alone), resets at the first and
+    last positions and twice in a row, cells that one position in two selects, row maxima over
+    intervals of every length, ages and the carried gradients."""
+    from hsn_amd import _lib, window
+
+    g = torch.Generator().manual_seed(100 * d + T)
+    dt = torch.float32 if io == "f32" else torch.bfloat16
+    rnd = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    valid = torch.rand(B, T, K, generator=g) > 0.15
+    cells = torch.argsort(torch.rand(B, T, N, generator=g) + 1.5 * (torch.arange(N) >= K) * (
+        torch.rand(B, T, 1, generator=g) < 0.5), dim=-1)[..., :K]
+    cells = torch.where(valid, cells, torch.zeros_like(cells))
+    reset = torch.rand(B, T, generator=g) < 0.02
+    reset[0, [0, T // 2, T // 2 + 1, T - 1]] = True
+    y, gate = rnd(B, T, K, d).to(dt), (1.0 + rnd(B, T, K, d)).to(dt)
+    h0, q0 = 0.3 * rnd(B, N, d), rnd(B, d)
+    age0, pos0 = torch.randint(0, 9, (B, N), generator=g), torch.zeros(B, dtype=torch.int64)
+    cot = [rnd(B, T, d).to(dt), rnd(B, T, d).to(dt), rnd(B, T, K, d).to(dt), rnd(B, N, d), rnd(B, d)]
+    # the oracle's forward position by position on the given decisions
+    h, q, age, pos = h0.double(), q0.double(), age0.clone(), pos0.clone()
+    want = {k: [] for k in ("q_pre", "q_post", "h_sel", "h_old", "h_max")}
+    for t in range(T):
+        h, q, age, pos = O.reset_state(h, q, age, pos, reset[:, t])
+        want["q_pre"].append(q)
+        h, q, age, pos, sel, hmax, old = O.cell_update(y[:, t].double(), gate[:, t].double(), h, q, age,
+                                                       pos, cells[:, t], valid[:, t])
+        for k, v in (("q_post", q), ("h_sel", sel), ("h_old", old), ("h_max", hmax)):
+            want[k].append(v)
+    want = {k: torch.stack(v, dim=1) for k, v in want.items()}
+
+    def put(t):  # `shift`: a contiguous view that many elements into a buffer
+        if not shift:
+            return t.to(dev)
+        return torch.empty(t.numel() + shift, dtype=t.dtype, device=dev)[shift:].view(t.shape).copy_(t)
+
+    slots = torch.where(valid, cells, torch.full_like(cells, -1)).to(torch.int32).to(dev)
+    tol = F32_TOL if io == "f32" else BF16_TOL
+    _lib.set_path("chain")
+    try:
+        h_max = torch.empty(B, T, device=dev)
+        got = window.forward(put(y), put(gate), reset.to(dev), slots, h0.to(dev), q0.to(dev),
+                             age0.to(dev), pos0.to(dev), N, h_max=h_max)
+        for k in ("q_pre", "q_post", "h_sel", "h_old", "h_max"):
+            _close(got[k], want[k].float(), tol, k)
+        _close(got["h"], h.float(), F32_TOL, "h")
+        assert torch.equal(got["age"].cpu(), age) and torch.equal(got["pos"].cpu(), pos)
+        h_old = want["h_old"].to(dt)
+        ref = O.window_backward(y, gate, h_old, cells, valid, reset, N, cot[0], cot[1],
+                                torch.where(valid[..., None], cot[2], torch.zeros_like(cot[2])), cot[3],
+                                cot[4])
+        grads = window.backward(put(y), put(gate), put(h_old), slots, reset.to(dev), N,
+                                *(c.to(dev) for c in cot))
+        for name, a, b in zip(("dy", "dgate", "d_h0"), grads, ref):
+            _close(a, b, tol if name != "d_h0" else max(tol, F32_TOL), name)
+        assert bool((grads[0].cpu()[~valid] == 0).all())
+    finally:
+        _lib.set_path("auto")
