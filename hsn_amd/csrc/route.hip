@@ -687,6 +687,220 @@ __global__ __launch_bounds__(256) void route_parallel(RouteArgs a) {
         decide_select<NPL, kOne, IO, IDX>(a, b, p, cand[wv], tab[wv], ord[wv]);
 }
 
+// The decision of one position without probes, one unit, contiguous bf16 logits of 16-byte rows,
+// no reserved cells: the selection of decide_select with two cells a register. Lane l holds the
+// eight consecutive cells 512 c + 8 l .. + 7 of each 16-byte load c < W (a load's 64 lanes are 1 KB
+// of the row).
+//  1. A logit's key is its bf16 order image less 0x7f: -inf is 0, +inf 0xff01, and the NaNs of
+//     either sign lie above (0xff02 up). Both halves of a register at once, as are the lane's
+//     two maxima (one of each half's cells).
+//  2. L, the largest key that at least K + 1 of the 128 maxima reach. The candidates' key >= L, a
+//     bit each (a saturating subtraction of L - 1), compacted with ballot and mbcnt a bit a lane
+//     at a time; a candidate's logit is read again by the lane that ranks it.
+//  3. The ranks in the selection's order (score descending, cell ascending). Without a cost the key
+//     orders the scores (-0 read as +0), and key and cell are one word; with one (score = logit -
+//     lambda cost, rounded) the score's own key does. There are K + 1 candidates or more, so
+//     theta's highest unselected score is a candidate's.
+// The score is a monotone image of the key that may map neighbouring keys to one score: a cell
+// below L could then tie with slot K and have the lower index. Such a position, and one with a
+// NaN, more than 64 candidates or a threshold of 0, returns false (decide_rescan).
+template <int W, typename IDX>
+__device__ bool decide_packed(const RouteArgs& a, int b, int p, uint32_t* code, uint4* tab,
+                              uint64_t* ord) {
+    typedef unsigned short U2 __attribute__((ext_vector_type(2)));
+    typedef short S2 __attribute__((ext_vector_type(2)));
+    constexpr int kW = 4 * W;  // registers: two cells each
+    const int lane = lane_id();
+    const int N = a.N, K = a.K;
+    const bf16_t* logits = static_cast<const bf16_t*>(a.logits) + b * a.l_row + p * a.l_pos;
+    const rsrc_t r = make_rsrc(logits, uint32_t(N) * 2u);
+    U2 key[kW];
+    {
+        uint32_t w[kW];
+#pragma unroll
+        for (int c = 0; c < W; ++c) {
+            const uint32_t vo = uint32_t(c * 1024 + lane * 16);  // past the row: reads 0
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, vo < uint32_t(N) * 2u ? vo : kOob, 0, 0);
+            __builtin_memcpy(&w[4 * c], &v, 16);
+        }
+#pragma unroll
+        for (int i = 0; i < kW; ++i) {
+            const S2 s = __builtin_bit_cast(S2, w[i]) >> 15;
+            const uint32_t k = w[i] ^ (__builtin_bit_cast(uint32_t, s) | 0x80008000u);
+            key[i] = __builtin_bit_cast(U2, k) - U2{0x7f, 0x7f};
+        }
+        if (N < 512 * W) {  // cells past the row: below every threshold
+#pragma unroll
+            for (int i = 0; i < kW; ++i)
+                if ((i / 4) * 512 + lane * 8 >= N) key[i] = U2{0, 0};
+        }
+    }
+    U2 top = key[0];
+#pragma unroll
+    for (int i = 1; i < kW; ++i) top = __builtin_elementwise_max(top, key[i]);
+    const uint32_t t0 = top.x, t1 = top.y;
+    if (ballot(umax(t0, t1) > 0xff01u) != 0u) return false;  // a NaN
+    uint32_t L = 0u;
+#pragma unroll
+    for (int bit = 15; bit >= 0; --bit) {
+        const uint32_t c = L | (1u << bit);
+        L = __popcll(ballot(t0 >= c)) + __popcll(ballot(t1 >= c)) > K ? c : L;
+    }
+    if (L == 0u) return false;
+    const U2 under = {static_cast<unsigned short>(L - 1u), static_cast<unsigned short>(L - 1u)};
+    int C = 0;
+#pragma unroll
+    for (int h = 0; h < (kW + 15) / 16; ++h) {
+        constexpr int kB = kW < 16 ? kW : 16;
+        uint32_t m = 0u;  // register i of the block: bit kB - 1 - i, its second cell 16 above
+#pragma unroll
+        for (int i = 0; i < kB; ++i)
+            m = (m << 1) | __builtin_bit_cast(uint32_t, __builtin_elementwise_min(
+                               __builtin_elementwise_sub_sat(key[16 * h + i], under), U2{1, 1}));
+        for (uint64_t any = ballot(m != 0u); any != 0u; any = ballot(m != 0u)) {
+            const int at = C + lanes_below(any);
+            if (m != 0u && at < kWave)
+                code[at] = uint32_t(lane) << 6 | uint32_t(h) << 5 | uint32_t(__builtin_ctz(m));
+            m &= m - 1u;
+            C += __popcll(any);
+        }
+    }
+    if (C > kWave) return false;
+    __builtin_amdgcn_wave_barrier();  // the codes' writes before their reads
+    const bool is_c = lane < C;
+    const uint32_t cd = is_c ? code[lane] : 0u;
+    constexpr uint32_t kB = kW < 16 ? kW : 16;
+    const uint32_t reg = 16u * ((cd >> 5) & 1u) + (kB - 1u - (cd & 15u));
+    const uint32_t n = (reg >> 2) * 512u + (cd >> 6) * 8u + (reg & 3u) * 2u + ((cd >> 4) & 1u);
+    const uint32_t raw = __builtin_amdgcn_raw_buffer_load_b16(r, is_c ? n * 2u : kOob, 0, 0) & 0xffffu;
+    const float v = __uint_as_float(raw << 16);
+    const bool scale_cost = a.lambda > 0.0f;
+    const float cost0 = a.cost[0];
+    const float lc = scale_cost ? mul_rn(a.lambda, cost0) : 0.0f;
+    const float score = scale_cost ? sub_rn(v, lc) : v;
+    const uint32_t sk = score_key(score);
+    int rank = 0;
+    if (scale_cost) {
+        if (ballot(is_c && score != score) != 0u) return false;  // an infinite or NaN cost
+        const uint64_t mine = (uint64_t(sk) << 32) | ~n;
+        ord[lane] = is_c ? mine : 0u;
+        __builtin_amdgcn_wave_barrier();
+        for (int j = 0; j < C; j = uniform(j + 4)) {
+            const uint64_t o0 = ord[j], o1 = ord[j + 1], o2 = ord[j + 2], o3 = ord[j + 3];
+            rank += static_cast<int>(o0 > mine) + static_cast<int>(o1 > mine) +
+                    static_cast<int>(o2 > mine) + static_cast<int>(o3 > mine);
+        }
+    } else {  // the bf16 score's key is in the upper half of its fp32 key
+        uint32_t* const o32 = reinterpret_cast<uint32_t*>(ord);
+        const uint32_t mine = (sk & 0xffff0000u) | (0xffffu ^ n);
+        o32[lane] = is_c ? mine : 0u;
+        __builtin_amdgcn_wave_barrier();
+        for (int j = 0; j < C; j = uniform(j + 4)) {
+            const uint4 o = *reinterpret_cast<const uint4*>(o32 + j);
+            rank += static_cast<int>(o.x > mine) + static_cast<int>(o.y > mine) +
+                    static_cast<int>(o.z > mine) + static_cast<int>(o.w > mine);
+        }
+    }
+    // slot K against the largest score below L (an infinite or NaN cost compares false)
+    const uint32_t ku = L - 1u + 0x7fu;
+    const uint32_t kx = (ku & 0x8000u) ? ku ^ 0x8000u : ~ku & 0xffffu;
+    const float vb = __uint_as_float(kx << 16);
+    const float sb = scale_cost ? sub_rn(vb, lc) : vb;
+    const uint64_t last = ballot(is_c && rank == K - 1);
+    const uint32_t sl = static_cast<uint32_t>(
+        __builtin_amdgcn_readlane(static_cast<int>(sk), __builtin_ctzll(last)));
+    if (sb != sb || sl <= score_key(sb)) return false;
+    if (is_c && rank < K) tab[rank] = make_uint4(sk, n, __float_as_uint(score), 0u);
+    const int32_t pool = is_c && rank >= K ? ford(score) : ford(-INFINITY);
+    finish_select<true, IDX>(a, b, p, tab, pool, false, cost0);
+    return true;
+}
+
+// The positions decide_packed leaves: K rounds of a wavefront argmax over the lanes' best cells
+// (score descending, cell ascending), the cells of the lane that won read again, one a lane, for its
+// next one. Words of (score key, ~cell) order them, 0 no cell.
+template <int W, typename IDX>
+__device__ void decide_rescan(const RouteArgs& a, int b, int p, uint4* tab) {
+    const int lane = lane_id();
+    const int N = a.N, K = a.K;
+    const bf16_t* logits = static_cast<const bf16_t*>(a.logits) + b * a.l_row + p * a.l_pos;
+    const rsrc_t r = make_rsrc(logits, uint32_t(N) * 2u);
+    const bool scale_cost = a.lambda > 0.0f;
+    const float cost0 = a.cost[0];
+    const float lc = scale_cost ? mul_rn(a.lambda, cost0) : 0.0f;
+    auto score = [&](uint32_t raw) __attribute__((always_inline)) -> float {
+        const float v = __uint_as_float(raw << 16);
+        return scale_cost ? sub_rn(v, lc) : v;
+    };
+    auto word = [&](uint32_t raw, int n) __attribute__((always_inline)) -> uint64_t {
+        return n < N ? (uint64_t(score_key(score(raw))) << 32) | ~uint32_t(n) : 0ull;
+    };
+    auto largest = [&](uint64_t w) __attribute__((always_inline)) -> uint64_t {
+        auto mx = [](uint32_t x, uint32_t y) { return x > y ? x : y; };
+        const uint32_t hi = static_cast<uint32_t>(w >> 32);
+        const uint32_t wh = wave_reduce_u32(hi, mx, 0u);
+        const uint32_t wl = wave_reduce_u32(hi == wh ? static_cast<uint32_t>(w) : 0u, mx, 0u);
+        return (uint64_t(wh) << 32) | wl;
+    };
+    // every cell of the lane, as decide_packed lays them out
+    auto each = [&](auto&& f) __attribute__((always_inline)) {
+#pragma unroll 1
+        for (int c = 0; c < W; ++c) {
+            const int n0 = c * 512 + lane * 8;
+            uint32_t w[4];
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, n0 < N ? uint32_t(n0) * 2u : kOob, 0, 0);
+            __builtin_memcpy(w, &v, 16);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) f((w[j / 2] >> (16 * (j & 1))) & 0xffffu, n0 + j);
+        }
+    };
+    uint64_t best = 0ull;
+    each([&](uint32_t raw, int n) {
+        const uint64_t w = word(raw, n);
+        best = w > best ? w : best;
+    });
+    for (int k = 0; k < K; k = uniform(k + 1)) {
+        const uint64_t win = largest(best);
+        const int src = __builtin_ctzll(ballot(best == win));
+        const int n = (lane >> 3) * 512 + src * 8 + (lane & 7);  // that lane's cells
+        const bool in = lane < 8 * W && n < N;
+        const uint32_t raw = __builtin_amdgcn_raw_buffer_load_b16(r, in ? uint32_t(n) * 2u : kOob, 0, 0) & 0xffffu;
+        const uint64_t w = in ? word(raw, n) : 0ull;
+        if (w == win) tab[k] = make_uint4(static_cast<uint32_t>(w >> 32), uint32_t(n), __float_as_uint(score(raw)), 0u);
+        const uint64_t next = largest(w < win ? w : 0ull);
+        if (lane == src) best = next;
+    }
+    // every cell still in the pool (words at or below its lane's best)
+    int32_t pool = ford(-INFINITY);
+    bool pool_nan = false;
+    each([&](uint32_t raw, int n) {
+        const bool out = n < N && word(raw, n) <= best;
+        const float s = score(raw);
+        pool = max(pool, out ? ford(s) : ford(-INFINITY));
+        pool_nan = pool_nan | (out & (s != s));
+    });
+    finish_select<true, IDX>(a, b, p, tab, pool, pool_nan, cost0);
+}
+
+// Whole window without probes in decide_packed's range: a wavefront per (row, position), four a
+// workgroup. Bound by a position's vector instructions at N = 1024 and by the logits' bytes at
+// N = 4096. Measured: B256 T1024 N4096 K32 445 us, 4.8 TB/s of the logits' 2.15 GB (a workgroup a
+// position, a cell a register: 913); B64 T512 N1024 K16 28 us (a wavefront a position, a cell a
+// register: 42).
+template <int W, typename IDX>
+__global__ __launch_bounds__(256) void route_packed(RouteArgs a) {
+    const int wv = uniform(threadIdx.x / kWave);
+    const int p = blockIdx.x * (blockDim.x / kWave) + wv;
+    const int b = blockIdx.y;
+    if (p >= a.P) return;
+    __shared__ uint32_t code[4][kWave];
+    __shared__ uint4 tab[4][kWave];
+    __shared__ __align__(16) uint64_t ord[4][kWave + 4];
+    if (decide_packed<W, IDX>(a, b, p, code[wv], tab[wv], ord[wv])) return;
+    __builtin_amdgcn_wave_barrier();
+    decide_rescan<W, IDX>(a, b, p, tab[wv]);
+}
+
 // Whole window without probes, one unit, a workgroup per (row, position) for rows too wide for a
 // wavefront's registers (N > 1024): 256 threads of CPT consecutive cells each (thread t holds
 // cells t*CPT ..), the selection of decide_select across the workgroup:
@@ -943,6 +1157,21 @@ hipError_t launch_route(const RouteArgs& a, bool sequential, hipStream_t stream)
         if (N <= 64) return launch_grouped<32, 2, 1, IO, IDX>(a, stream);
         if (N <= 128) return launch_grouped<32, 4, 2, IO, IDX>(a, stream);
         return launch_grouped<32, 8, 4, IO, IDX>(a, stream);
+    }
+    // Two cells a register: contiguous bf16 rows, and K up to 40 of the 128 maxima, so the
+    // candidates (about 49 of random logits at 40) rarely pass the 64 lanes. 32768 positions, us,
+    // against the general selection: N 2048 K 16 28 (105), K 40 35 (130); N 1024 K 16 24 (37),
+    // every logit equal 92 (209). Not up to N = 512: K 8 21.1 (21.6), every logit equal 75 (58).
+    if constexpr (sizeof(IO) == 2) {
+        if (!sequential && a.M == 1 && a.reserved == 0 && a.width == 1 && a.K <= 40 && a.N > 512 &&
+            a.N % 8 == 0 && (reinterpret_cast<uintptr_t>(a.logits) & 15) == 0) {
+            const dim3 grid((a.P + 3) / 4, a.B);
+            auto* const k = a.N <= 1024   ? route_packed<2, IDX>
+                            : a.N <= 2048 ? route_packed<4, IDX>
+                                          : route_packed<8, IDX>;
+            hipLaunchKernelGGL(k, grid, dim3(256), 0, stream, a);
+            return hipGetLastError();
+        }
     }
     if (!sequential && a.M == 1 && a.N > 1024) {  // a workgroup per position (N <= 4096)
         hipLaunchKernelGGL((route_block<16, IO, IDX>), dim3(a.P, a.B), dim3(256), 0, stream, a);

@@ -862,3 +862,59 @@ def test_chains_of_several_cells_a_wavefront(dev, B, T, N, K, d, shift, io):
         assert bool((grads[0].cpu()[~valid] == 0).all())
     finally:
         _lib.set_path("auto")
+
+
+PACKED_ROUTES = [
+    # N, K, settings, special values: bf16 rows around the two-cells-a-register rule
+    (512, 8, dict(), "plain"),                   # the general selection
+    (576, 31, dict(limit=0.3), "zipf"),          # slots past the budget
+    (520, 16, dict(lambda_cost=0.05), "ties"),   # a second load of one lane only; the score's own key
+    (1024, 40, dict(), "plain"),                 # the most slots
+    (1024, 41, dict(), "plain"),                 # one more: the general selection
+    (1032, 16, dict(), "nan"),                   # NaN of either sign, +-inf
+    (2048, 32, dict(lambda_cost=0.5), "nan"),
+    (4088, 24, dict(), "infs"),                  # a threshold of -inf
+    (4096, 32, dict(), "ties"),                  # more than 64 candidates
+    (4096, 1, dict(), "near"),
+    (4096, 32, dict(lambda_cost=64.0), "near"),  # neighbouring logits of one score
+    (2048, 8, dict(lambda_cost=64.0), "zeros"),
+    (1024, 16, dict(), "zeros"),                 # +-0 around the threshold
+    (1016, 12, dict(), "sign"),
+    (1023, 16, dict(), "ties"),                  # no multiple of 8: a lane's cells one by one
+]
+
+
+@pytest.mark.parametrize("case", range(len(PACKED_ROUTES)))
+@pytest.mark.parametrize("shift", [0, 1])
+def test_packed_route_matches_oracle(dev, case, shift):
+    """The bf16 router's two cells a register against the oracle, exactly; `shift`: rows off
+    the 16-byte alignment."""
+    from hsn_amd import window
+
+    N, K, kw, kind = PACKED_ROUTES[case]
+    B, T = 2, 5
+    g = torch.Generator().manual_seed(7000 + case)
+    x = _logits(B, T, N, 1, kind if kind in ("plain", "ties", "nan", "zipf", "zeros") else "plain", g)
+    if kind == "nan":
+        x[0, 3, N // 2, 0] = -float("nan")
+    elif kind == "infs":
+        x[:, :, 3:, 0] = -float("inf")
+    elif kind == "near":  # the steps of bf16 near 0, below half a unit of the cost's last place
+        x = x * 1e-6
+    elif kind == "sign":  # K - 1 positive cells, then +0 and -0
+        x = torch.where(torch.rand(x.shape, generator=g) < 0.5, 0.0, -0.0)
+        x[:, :, 100:100 + K - 1] = 1.0
+    logits = x.to(torch.bfloat16)
+    dl = torch.empty(logits.numel() + 8, dtype=logits.dtype, device=dev)[shift:shift + logits.numel()]
+    dl = dl.view(logits.shape).copy_(logits)
+    cost = torch.full((1,), 1.0 / 64)
+    cfg = _route_cfg(k=K, **kw)
+    got = [v.cpu() for v in window.route(dl, cost.to(dev), cfg)]
+    for t in range(T):
+        want = O.router_select(logits[:, t], None, cost, **_oracle_route_kwargs(cfg))
+        for name, gv, wv in zip(("cells", "units", "valid", "theta", "refreshed"), got, want):
+            if name == "theta":
+                same = gv[:, t] == wv  # a zero's sign is the oracle's reduction order: -0 == +0
+                assert bool((same | (torch.isnan(gv[:, t]) & torch.isnan(wv))).all()), (t, gv[:, t], wv)
+            else:
+                assert torch.equal(gv[:, t].long(), wv.long()), (name, t, gv[:, t], wv)
