@@ -9,7 +9,7 @@
 //                 the events (t << 8 | k) of each cell in time order, then the padded slots in
 //                 time order. Counts by LDS atomics (integers: any order), ranks within a block
 //                 of positions from a bit per position per cell (popcount below t):
-//                 deterministic.
+//                 deterministic. By ranges of cells (row_lists_ranges) where the row allows.
 //   chain_fwd     (row, group of cells; a wavefront per cell): h_old, h_sel, the end state, the
 //                 ages, each valid slot's delta h_sel - h_old in fp32 where the rows are bf16
 //                 or omitted; the row maximum of |h| per position from each cell's value on the
@@ -221,6 +221,169 @@ static __global__ __launch_bounds__(kListThreads) void row_lists(ListArgs a) {
         if (tid == 0) misc[0] = pad0 + wsum[PKW];
 #pragma unroll
         for (int u = 0; u < kListU; ++u) cur[u] = nxt[u];
+    }
+}
+
+// The same lists by (row, range of cells): a wavefront takes its share of the row's positions in
+// order. It counts its slots of each of the range's cells (two 16-bit counts a word), the counts'
+// prefix over the cells and the wavefronts gives every wavefront its own place in each cell's list,
+// and it places its slots position by position (a position's cells are distinct; a wavefront's LDS
+// operations complete in order) by the counts' old values. The range's part of the row's list is put
+// together in LDS and written in order; the last range's goes on with the padded slots. A row of
+// T K <= 32768 slots, so offsets are 16 bits. Bound by the instructions a slot (every range reads the
+// row's slots twice), hence ranges only as far as they fill the chip. The LDS operations of a step's
+// positions are issued without a wait between: with one, B256 T1024 N4096 K32 took 90 us instead
+// of 37, two ranges a row and sixteen wavefronts.
+constexpr int kRangeSlots = 32768;
+
+__host__ __device__ inline int range_waves(int N) { return N > 2048 ? 8 : 16; }
+__host__ __device__ inline int range_cells(int B, int N) {  // cells a range, even
+    int R = 1;
+    while (int64_t(B) * R < 256 && N / (2 * R) >= 64) R *= 2;
+    const int NR = (N + R - 1) / R;
+    return NR + (NR & 1);
+}
+__host__ __device__ inline int range_words(int W, int NR, int T, int K) {  // LDS words
+    return W * (NR / 2) + (T * K + 1) / 2 + 3 * W + 2;
+}
+
+// SUB: positions a step, at most 64 / K.
+template <int W, int SUB>
+__global__ __launch_bounds__(64 * W) void row_lists_ranges(ListArgs a, int NR) {
+    extern __shared__ uint32_t lds_u[];
+    constexpr int kThreads = 64 * W;
+    const int b = blockIdx.y, z = blockIdx.x;
+    const int tid = threadIdx.x, lane = lane_id(), w = uniform(tid / 64);
+    const int T = a.T, N = a.N, K = a.K, NW = NR / 2;
+    const uint32_t c_lo = z * NR, c_hi = min(N, int(c_lo) + NR), span = c_hi - c_lo;
+    const bool last = int(c_hi) == N;
+    uint32_t* const cnt = lds_u;  // [W][NW]
+    uint16_t* const stage = reinterpret_cast<uint16_t*>(cnt + W * NW);  // [T K]
+    int* const under = reinterpret_cast<int*>(cnt + W * NW + (T * K + 1) / 2);  // [W]: lower ranges' slots
+    int* const pads = under + W;  // [W]: padded slots
+    int* const wsum = pads + W;   // [W]: the scan's partials
+    const int per = (T + W - 1) / W;
+    const int s_lo = min(T, w * per) * K, s_n = min(T, (w + 1) * per) * K - s_lo;
+    const int32_t* const slots = a.slots + int64_t(b) * T * K + s_lo;
+    for (int i = tid; i < W * NW; i += kThreads) cnt[i] = 0u;
+    __syncthreads();
+    uint32_t* const mine = cnt + w * NW;
+    int lo = 0, pad = 0;
+    constexpr int kU = 8;  // loads in flight
+    for (int s0 = 0; s0 < s_n; s0 += 64 * kU) {
+        uint32_t cs[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) cs[u] = slots[min(s0 + 64 * u + lane, s_n - 1)];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+            if (s0 + 64 * u >= s_n) break;
+            const bool here = s0 + 64 * u + lane < s_n;
+            const uint32_t rel = cs[u] - c_lo;
+            if (z > 0) lo += here && cs[u] < c_lo ? 1 : 0;
+            if (last) pad += here && cs[u] >= uint32_t(N) ? 1 : 0;
+            if (here && rel < span) atomicAdd(&mine[rel >> 1], (rel & 1u) ? 0x10000u : 1u);
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        lo += __shfl_xor(lo, o, 64);
+        pad += __shfl_xor(pad, o, 64);
+    }
+    if (lane == 0) under[w] = lo, pads[w] = pad;
+    __syncthreads();
+    // consecutive words of two cells a thread: the wavefronts' prefix, then the cells'
+    const int each = (NW + kThreads - 1) / kThreads, i0 = tid * each, i1 = min(NW, i0 + each);
+    int own = 0;
+    for (int i = i0; i < i1; ++i) {
+        uint32_t run = 0u;
+#pragma unroll
+        for (int v = 0; v < W; ++v) run += cnt[v * NW + i];
+        own += (run & 0xffffu) + (run >> 16);
+    }
+    int incl = own;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += u;
+    }
+    if (lane == 63) wsum[w] = incl;
+    int first = 0;  // the row's events in lower ranges
+#pragma unroll
+    for (int v = 0; v < W; ++v) first += under[v];
+    __syncthreads();
+    int at = incl - own, total = 0;
+#pragma unroll
+    for (int v = 0; v < W; ++v) {
+        at += v < w ? wsum[v] : 0;
+        total += wsum[v];
+    }
+    int32_t* const ptr = a.ptr + int64_t(b) * (N + 1);
+    for (int i = i0; i < i1; ++i) {
+        uint32_t n[W], run = 0u;
+#pragma unroll
+        for (int v = 0; v < W; ++v) n[v] = cnt[v * NW + i];
+#pragma unroll
+        for (int v = 0; v < W; ++v) run += n[v];
+        const int n0 = run & 0xffffu, n1 = run >> 16;
+        uint32_t place = uint32_t(at) | (uint32_t(at + n0) << 16);
+#pragma unroll
+        for (int v = 0; v < W; ++v) {
+            cnt[v * NW + i] = place;
+            place += n[v];
+        }
+        const uint32_t c = c_lo + 2 * i;
+        if (c < c_hi) ptr[c] = first + at;
+        if (c + 1 < c_hi) ptr[c + 1] = first + at + n0;
+        at += n0 + n1;
+    }
+    if (last && tid == 0) ptr[N] = first + total;
+    int pad_at = total, n_out = total;
+    if (last) {
+#pragma unroll
+        for (int v = 0; v < W; ++v) {
+            pad_at += v < w ? pads[v] : 0;
+            n_out += pads[v];
+        }
+    }
+    __syncthreads();
+    const int step = SUB * K;  // whole positions, at most 64 slots
+    const int sub = SUB > 1 ? lane / K : 0;
+    constexpr int kV = SUB >= 8 ? 1 : 8 / SUB;  // steps in flight
+    for (int s0 = 0; s0 < s_n; s0 += step * kV) {
+        uint32_t cs[kV], old[kV][SUB];
+#pragma unroll
+        for (int u = 0; u < kV; ++u) cs[u] = slots[min(s0 + step * u + lane, s_n - 1)];
+#pragma unroll
+        for (int u = 0; u < kV; ++u) {
+            const bool here = lane < step && s0 + step * u + lane < s_n;
+            const uint32_t rel = cs[u] - c_lo;
+#pragma unroll
+            for (int j = 0; j < SUB; ++j)
+                if (here && rel < span && (SUB == 1 || sub == j))
+                    old[u][j] = atomicAdd(&mine[rel >> 1], (rel & 1u) ? 0x10000u : 1u);
+        }
+#pragma unroll
+        for (int u = 0; u < kV; ++u) {
+            const int s = s0 + step * u + lane;
+            const bool here = lane < step && s < s_n;
+            const uint32_t rel = cs[u] - c_lo;
+            uint32_t o = old[u][0];
+#pragma unroll
+            for (int j = 1; j < SUB; ++j) o = sub == j ? old[u][j] : o;
+            if (here && rel < span)
+                stage[(rel & 1u) ? o >> 16 : o & 0xffffu] = static_cast<uint16_t>(s_lo + s);
+            if (last) {
+                const bool out = here && cs[u] >= uint32_t(N);
+                const uint64_t m = ballot(out);
+                if (out) stage[pad_at + lanes_below(m)] = static_cast<uint16_t>(s_lo + s);
+                pad_at += __popcll(m);
+            }
+        }
+    }
+    __syncthreads();
+    int32_t* const ev = a.ev + int64_t(b) * T * K + first;
+    const uint32_t inv = 0xffffffffu / uint32_t(K) + 1u;  // s / K for s < 2^15: exact (K = 1: 0)
+    for (int i = tid; i < n_out; i += kThreads) {
+        const uint32_t s = stage[i], t = K > 1 ? __umulhi(s, inv) : s;
+        ev[i] = static_cast<int32_t>((t << 8) | (s - t * K));
     }
 }
 

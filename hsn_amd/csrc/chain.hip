@@ -171,6 +171,30 @@ namespace {
 void build_lists(const int32_t* slots, int32_t* ptr, int32_t* ev, int B, int T, int N, int K,
                  hipStream_t st) {
     chain::ListArgs la{slots, ptr, ev, B, T, N, K};
+    const int NR = chain::range_cells(B, N), W = chain::range_waves(NR);
+    const size_t range_lds = size_t(chain::range_words(W, NR, T, K)) * 4;
+    // By ranges of cells where a position's slots fit a wavefront (its order is what places the
+    // slots) and the row's list fits the LDS beside the counts. Measured (us) against the whole row
+    // a workgroup: B64 T512 N1024 K16 9.6 (20.2), B256 T1024 N4096 K32 37 (105), B128 T128 N512 K8
+    // 5.8 (7.7), B32 T8192 N1024 K4 43 (170), B8 T64 N64 K4 5.8 (7.0), B1024 T64 N128 K4 18 (24).
+    if (K <= 64 && int64_t(T) * K <= chain::kRangeSlots && range_lds <= size_t(kLdsMax)) {
+        auto launch = [&](auto waves, auto sub) {
+            constexpr int kW = decltype(waves)::value, kSub = decltype(sub)::value;
+            auto k = chain::row_lists_ranges<kW, kSub>;
+            HSN_HIP(allow_lds(k, range_lds));
+            hipLaunchKernelGGL(k, dim3((N + NR - 1) / NR, B), dim3(64 * kW), range_lds, st, la, NR);
+        };
+        auto by_sub = [&](auto waves) {
+            if (K > 32) launch(waves, std::integral_constant<int, 1>{});
+            else if (K > 16) launch(waves, std::integral_constant<int, 2>{});
+            else if (K > 8) launch(waves, std::integral_constant<int, 4>{});
+            else launch(waves, std::integral_constant<int, 8>{});
+        };
+        if (W == 8) by_sub(std::integral_constant<int, 8>{});
+        else by_sub(std::integral_constant<int, 16>{});
+        HSN_HIP(hipGetLastError());
+        return;
+    }
     const size_t lds = size_t(chain::list_words(N, T, K)) * 4;
     HSN_HIP(allow_lds(chain::row_lists, lds));
     hipLaunchKernelGGL(chain::row_lists, dim3(B), dim3(chain::kListThreads), lds, st, la);

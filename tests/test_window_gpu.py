@@ -802,6 +802,16 @@ def test_rms_candidate_at_the_edges_of_its_lanes(dev, B, T, K, d, shift, io):
     (2, 40, 33, 4, 100, 0),   # 32 lanes a cell, seven idle
     (1, 30, 20, 3, 256, 0),   # one cell a wavefront, four columns a lane
     (2, 50, 40, 3, 24, 1),    # rows off the four-element alignment: a column a lane
+    # the event lists: one slot, eight, four, two and one position a step, with lanes left over;
+    # eight wavefronts a row; a row a workgroup of one range; too many slots for the ranges
+    (2, 40, 20, 1, 4, 0),
+    (2, 33, 50, 7, 4, 0),
+    (1, 70, 257, 12, 4, 0),
+    (1, 40, 90, 20, 4, 0),
+    (1, 37, 65, 64, 4, 0),
+    (256, 9, 2100, 3, 4, 0),
+    (300, 6, 130, 3, 4, 0),
+    (1, 520, 80, 64, 4, 0),
 ])
 def test_chains_of_several_cells_a_wavefront(dev, B, T, N, K, d, shift, io):
     """The cell chains with four columns a lane at the edges of their lanes, against the float64
