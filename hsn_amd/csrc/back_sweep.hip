@@ -350,9 +350,33 @@ constexpr float kLog2ef = 1.44269504088896341f;
 __device__ __forceinline__ float exp_fast(float x) {
     return __builtin_amdgcn_exp2f(x * kLog2ef);
 }
-template <int ACT>
+// The exact GELU's derivative for products in 16 bits, without erff's two ranges. With a = |x| and
+// g(a) = erfcx(a / sqrt 2) / 2 it is exp(-a^2 / 2) (g(a) - a / sqrt(2 pi)) below zero and one less
+// that above. g is t p(t), t = 1 / (1 + 0.35 a), p of degree 8 fitted here by reweighted least
+// squares to 2.5e-8 of the value on [0, 9]. Over N(0, 1) the result is 3.4e-8 rms off the 64-bit
+// one, erff's form 2.7e-8; its product is rounded to 16 bits (2e-3) at once. fp32 products keep erff.
+__device__ __forceinline__ float gelu_grad_fast(float x) {
+    const float a = fabsf(x);
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(0.35f, a, 1.0f));
+    const float y = x * 0.84932180028801907f;  // y^2 = x^2 / 2 log2 e
+    const float e = __builtin_amdgcn_exp2f(-(y * y));
+    float p = -0.027885600924491882f;
+    p = __builtin_fmaf(p, t, 0.13761627674102783f);
+    p = __builtin_fmaf(p, t, -0.24204465746879578f);
+    p = __builtin_fmaf(p, t, 0.1428307741880417f);
+    p = __builtin_fmaf(p, t, -0.01125725544989109f);
+    p = __builtin_fmaf(p, t, 0.10018155723810196f);
+    p = __builtin_fmaf(p, t, 0.12127800285816193f);
+    p = __builtin_fmaf(p, t, 0.13964590430259705f);
+    p = __builtin_fmaf(p, t, 0.13963499665260315f);
+    const float q = e * __builtin_fmaf(-a, kRsqrt2Pif, p * t);
+    return x >= 0.0f ? 1.0f - q : q;
+}
+template <int ACT, typename P>
 __device__ __forceinline__ float act_grad_t(float x) {
-    if constexpr (ACT == HSN_ACT_GELU) {
+    if constexpr (ACT == HSN_ACT_GELU && sizeof(P) == 2) {
+        return gelu_grad_fast(x);
+    } else if constexpr (ACT == HSN_ACT_GELU) {
         const float cdf = 0.5f * (1.0f + erff(x * kRsqrt2f));
         return cdf + x * (exp_fast(-0.5f * x * x) * kRsqrt2Pif);
     } else if constexpr (ACT == HSN_ACT_RELU) {
@@ -684,7 +708,7 @@ __global__ __launch_bounds__(kCellThreads) void back_cell(hsn_back_sweep s, int 
                 float v = 0.0f;
                 if (okrow[i] && hin) {
                     const float hv1 = to_f32(hid_lds[(4 * lq + i) * H + h]);
-                    v = round_p<P>(acc[i]) * act_grad_t<ACT>(hv1);
+                    v = round_p<P>(acc[i]) * act_grad_t<ACT, P>(hv1);
                     part[i] += v * (hv1 - bias[u]);
                 }
                 if (hin) dh[(4 * lq + i) * L.dh_stride + h] = from_f32<P>(v);

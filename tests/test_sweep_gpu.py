@@ -111,6 +111,22 @@ def test_sweep_with_bf16_products(dev, name, fused):
     _close(out[1], want_db, BF16_TOL, f"{name} bf16 dL/db")
 
 
+@pytest.mark.parametrize("scale", [0.0, 1.0, 5.0, 40.0])
+def test_bf16_products_over_the_activation_range(dev, scale):
+    """The fused step's GELU derivative in 16 bits where it bends, at zero, and where it is 0 or 1
+    (the hidden record rounded beforehand, without the cell norm's sum, which grows with it)."""
+    p = sweep_problem(B=2, T=8, K=4, N=30, d=32, H=40, M=4, cell_norm=False, seed=13)
+    hidden = p["record"]["hidden"]
+    p["record"]["hidden"] = (scale * torch.randn(hidden.shape, generator=torch.Generator().manual_seed(3))
+                             ).bfloat16().to(hidden.dtype)
+    want_dc, want_db = sweep_oracle(p)
+    args, kw = _args(p, dev, torch.bfloat16)
+    out = _run(args, kw, True)
+    assert out is not None
+    _close(out[0], want_dc, BF16_TOL, f"hidden scale {scale} bf16 dL/dc")
+    _close(out[1], want_db, BF16_TOL, f"hidden scale {scale} bf16 dL/db")
+
+
 def test_fixed_unit_slots_take_the_same_sweep(dev, fused):
     """Leading slots with a fixed unit (``n_fast``) are swept like the others: the same values as
     without the distinction."""
