@@ -258,7 +258,7 @@ def _update_inplace_fake(h, q, age, idx, valid, c, b):
 def _functional(h, q, age, idx, valid, c, b):
     B, N, d = h.shape
     K = idx.shape[1]
-    if age.dtype not in (torch.int32, torch.int64) or N > 4194176:
+    if age.dtype not in (torch.int32, torch.int64):
         return _functional_by_copies(h, q, age, idx, valid, c, b)
     h, q, age, c, b = h.contiguous(), q.contiguous(), age.contiguous(), c.contiguous(), b.contiguous()
     hn, qn, an, old = torch.empty_like(h), torch.empty_like(q), torch.empty_like(age), torch.empty_like(c)
@@ -270,8 +270,8 @@ def _functional(h, q, age, idx, valid, c, b):
 
 
 def _functional_by_copies(h, q, age, idx, valid, c, b):
-    """The functional update where its kernel does not take the ages' dtype or the cell count: the
-    in-place update of copies."""
+    """The functional update where its kernel does not take the ages' dtype: the in-place
+    update of copies."""
     hn = h.clone(memory_format=torch.contiguous_format)
     qn = q.clone(memory_format=torch.contiguous_format)
     # the kernel zeroes the selected cells of an int32 mask of ones, and the same cells' ages are

@@ -152,7 +152,7 @@ int hsn_gated_delta_update(void* h, void* q, int32_t* age, const int32_t* cell_i
 /*
  * The gated delta update into fresh tensors (the same values as a copy updated in place): h_new
  * [B,N,d], q_new [B,d], age_new [B,N] (the ages int32_t or int64_t: `age_bits`) and h_old_saved;
- * h, q and age are only read. No output may overlap an input. N <= 4194176.
+ * h, q and age are only read. No output may overlap an input.
  */
 int hsn_gated_delta_update_copy(const void* h, const void* q, const void* age, int age_bits,
                                 const int32_t* cell_idx, const int32_t* valid, const void* c,

@@ -478,9 +478,9 @@ def test_unit_mlp_takes_operands_off_the_four_element_alignment(ops, cuda_device
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("B,N,K,d", [(1, 1, 1, 4), (3, 130, 19, 36), (2, 64, 8, 6), (2, 65, 9, 300)])
 def test_update_into_fresh_tensors_equals_the_update_in_place(ops, cuda_device, B, N, K, d, dtype):
-    """One launch that copies and updates gives the copies' in-place update bit for bit: a partial
-    last block of copied cells, d off the four-element copies and above the workgroup's threads,
-    padded slots, and cells repeated inside a batch of 8 slots and across batches."""
+    """The copies and their update in two launches give the copies' in-place update bit for bit: an
+    element count off the 16-byte copies, d above the workgroup's threads, padded slots, and cells
+    repeated inside a batch of 8 slots and across batches."""
     g = torch.Generator().manual_seed(B * 100 + N)
     dev = cuda_device
     rnd = lambda *s: torch.randn(*s, generator=g).to(dtype).to(dev)  # noqa: E731
