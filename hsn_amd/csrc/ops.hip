@@ -35,10 +35,10 @@ __global__ __launch_bounds__(256) void copy_or_zero(const F* src, F* dst, int64_
 // batch; a cell that an earlier slot of the group already updated takes that slot's stored value
 // (in-place order, as if each slot read h after the slots before it).
 // The summary is q_in's plus the row's change (q_in and q may be the same).
-template <typename F>
+template <typename F, int W>
 __global__ __launch_bounds__(256) void gated_update_fwd(F* h, const F* q_in, F* q, void* age,
-                                                        int age_wide, Idx cell_idx,
-                                                        Flags valid, const F* c,
+                                                        int age_wide, Idx<W> cell_idx,
+                                                        Flags<W> valid, const F* c,
                                                         const F* bgate, F* h_old_saved, int B,
                                                         int N, int d, int K) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -90,9 +90,9 @@ __global__ __launch_bounds__(256) void gated_update_fwd(F* h, const F* q_in, F* 
     q[qi] = from_f32<F>(to_f32(q_in[qi]) + delta / static_cast<float>(N));
 }
 
-template <typename F>
-__global__ __launch_bounds__(256) void gated_update_bwd(Idx cell_idx,
-                                                        Flags valid, const F* c,
+template <typename F, int W>
+__global__ __launch_bounds__(256) void gated_update_bwd(Idx<W> cell_idx,
+                                                        Flags<W> valid, const F* c,
                                                         const F* bgate, const F* h_old,
                                                         const F* G, const F* g, F* grad_h,
                                                         F* grad_q, F* grad_c, F* grad_b, int B,
@@ -139,9 +139,9 @@ __global__ __launch_bounds__(256) void gated_update_bwd(Idx cell_idx,
     }
 }
 
-template <typename F>
+template <typename F, int W>
 __global__ __launch_bounds__(256) void gather_fwd(const F* u, const F* eps, const F* h, const F* m,
-                                                  Idx cell_idx, F* v, int B, int N,
+                                                  Idx<W> cell_idx, F* v, int B, int N,
                                                   int d, int K) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t w = 4 * int64_t(d);
@@ -158,8 +158,8 @@ __global__ __launch_bounds__(256) void gather_fwd(const F* u, const F* eps, cons
     v[e] = out;
 }
 
-template <typename F>
-__global__ __launch_bounds__(256) void gather_bwd(const F* grad_v, Idx cell_idx,
+template <typename F, int W>
+__global__ __launch_bounds__(256) void gather_bwd(const F* grad_v, Idx<W> cell_idx,
                                                   F* grad_u, F* grad_eps, F* grad_h, F* grad_m,
                                                   int B, int N, int d, int K) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -211,8 +211,8 @@ __global__ __launch_bounds__(256) void gather_bwd(const F* grad_v, Idx cell_idx,
 // order, rounded once to F (the ABI's accumulation). A thread per (row, column) walks the slots;
 // each slot writes its cell's sum over the slots up to it (the same cells found by a scan of the
 // earlier slots), so the cell's last slot writes the whole sum.
-template <typename F>
-__global__ __launch_bounds__(256) void gather_bwd_narrow(const F* grad_v, Idx cell_idx,
+template <typename F, int W>
+__global__ __launch_bounds__(256) void gather_bwd_narrow(const F* grad_v, Idx<W> cell_idx,
                                                          F* grad_u, F* grad_eps, F* grad_h,
                                                          F* grad_m, int B, int N, int d, int K) {
     const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -302,80 +302,97 @@ void launch_copy_or_zero(const F* src, F* dst, int64_t n, hipStream_t st) {
                        dst, n, n16);
 }
 
-// The width bits of a dtype code (HSN_CELLS_I64 and so on), taken off it.
-Idx cells_of(const void* p, int dtype) { return Idx{p, (dtype & HSN_CELLS_I64) != 0}; }
-Flags flags_of(const void* p, int dtype) { return Flags{p, (dtype & HSN_VALID_U8) != 0}; }
+// A call's index and flag arrays in one instantiation's types (`bits`: the dtype code's width bits).
+template <int W>
+Idx<W> cells_of(const void* p, int bits) { return Idx<W>{p, (bits & HSN_CELLS_I64) != 0}; }
+template <int W>
+Flags<W> flags_of(const void* p, int bits) { return Flags<W>{p, (bits & HSN_VALID_U8) != 0}; }
 
 template <typename F>
 struct RunUpdateCopy {
-    static void run(const void* h, const void* q, const void* age, int age_wide, Idx cell_idx,
-                    Flags valid, const void* c, const void* b, void* h_new, void* q_new,
-                    void* age_new, void* h_old_saved, int B, int N, int d, int K, hipStream_t st) {
+    static void run(const void* h, const void* q, const void* age, int age_wide, const void* cell_idx,
+                    const void* valid, const void* c, const void* b, void* h_new, void* q_new,
+                    void* age_new, void* h_old_saved, int B, int N, int d, int K, hipStream_t st, int bits) {
         constexpr int64_t kPer = 16 / sizeof(F);
         const int64_t n = int64_t(B) * N * d, na = int64_t(B) * N;
         const int64_t n16 = aligned(h, 16) && aligned(h_new, 16) ? n / kPer : 0;
         hipLaunchKernelGGL((copy_state<F>), dim3(grid_of(n16 + (n - n16 * kPer) + na)), dim3(256), 0, st,
                            static_cast<const F*>(h), static_cast<F*>(h_new), n, n16, age, age_new, na,
                            age_wide);
-        hipLaunchKernelGGL((gated_update_fwd<F>), dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
-                           static_cast<F*>(h_new), static_cast<const F*>(q), static_cast<F*>(q_new),
-                           age_new, age_wide, cell_idx, valid, static_cast<const F*>(c),
-                           static_cast<const F*>(b), static_cast<F*>(h_old_saved), B, N, d, K);
+        by_widths(bits, kWidths, [&](auto width) {
+            constexpr int w = decltype(width)::value;
+            hipLaunchKernelGGL((gated_update_fwd<F, w>), dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
+                               static_cast<F*>(h_new), static_cast<const F*>(q), static_cast<F*>(q_new),
+                               age_new, age_wide, cells_of<w>(cell_idx, bits), flags_of<w>(valid, bits), static_cast<const F*>(c),
+                               static_cast<const F*>(b), static_cast<F*>(h_old_saved), B, N, d, K);
+        });
     }
 };
 
 template <typename F>
 struct RunUpdate {
-    static void run(void* h, void* q, int32_t* age, Idx cell_idx, Flags valid,
+    static void run(void* h, void* q, int32_t* age, const void* cell_idx, const void* valid,
                     const void* c, const void* b, void* h_old_saved, int B, int N, int d, int K,
-                    hipStream_t st) {
-        hipLaunchKernelGGL((gated_update_fwd<F>), dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
-                           static_cast<F*>(h), static_cast<const F*>(q), static_cast<F*>(q), age, 0,
-                           cell_idx, valid, static_cast<const F*>(c), static_cast<const F*>(b),
-                           static_cast<F*>(h_old_saved), B, N, d, K);
+                    hipStream_t st, int bits) {
+        by_widths(bits, kWidths, [&](auto width) {
+            constexpr int w = decltype(width)::value;
+            hipLaunchKernelGGL((gated_update_fwd<F, w>), dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
+                               static_cast<F*>(h), static_cast<const F*>(q), static_cast<F*>(q), age, 0,
+                               cells_of<w>(cell_idx, bits), flags_of<w>(valid, bits), static_cast<const F*>(c), static_cast<const F*>(b),
+                               static_cast<F*>(h_old_saved), B, N, d, K);
+        });
     }
 };
 
 template <typename F>
 struct RunUpdateBwd {
-    static void run(Idx cell_idx, Flags valid, const void* c, const void* b,
+    static void run(const void* cell_idx, const void* valid, const void* c, const void* b,
                     const void* h_old, const void* G, const void* g, void* grad_h, void* grad_q,
-                    void* grad_c, void* grad_b, int B, int N, int d, int K, hipStream_t st) {
+                    void* grad_c, void* grad_b, int B, int N, int d, int K, hipStream_t st, int bits) {
         const int64_t n = int64_t(B) * N * d;
         launch_copy_or_zero(static_cast<const F*>(G), static_cast<F*>(grad_h), n, st);
-        hipLaunchKernelGGL((gated_update_bwd<F>), dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
-                           cell_idx, valid, static_cast<const F*>(c), static_cast<const F*>(b),
-                           static_cast<const F*>(h_old), static_cast<const F*>(G),
-                           static_cast<const F*>(g), static_cast<F*>(grad_h),
-                           static_cast<F*>(grad_q), static_cast<F*>(grad_c),
-                           static_cast<F*>(grad_b), B, N, d, K);
+        by_widths(bits, kWidths, [&](auto width) {
+            constexpr int w = decltype(width)::value;
+            hipLaunchKernelGGL((gated_update_bwd<F, w>), dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
+                               cells_of<w>(cell_idx, bits), flags_of<w>(valid, bits), static_cast<const F*>(c), static_cast<const F*>(b),
+                               static_cast<const F*>(h_old), static_cast<const F*>(G),
+                               static_cast<const F*>(g), static_cast<F*>(grad_h),
+                               static_cast<F*>(grad_q), static_cast<F*>(grad_c),
+                               static_cast<F*>(grad_b), B, N, d, K);
+        });
     }
 };
 
 template <typename F>
 struct RunGather {
     static void run(const void* u, const void* eps, const void* h, const void* m,
-                    Idx cell_idx, void* v, int B, int N, int d, int K, hipStream_t st) {
-        hipLaunchKernelGGL((gather_fwd<F>), dim3(grid_of(int64_t(B) * K * 4 * d)), dim3(256), 0,
-                           st, static_cast<const F*>(u), static_cast<const F*>(eps),
-                           static_cast<const F*>(h), static_cast<const F*>(m), cell_idx,
-                           static_cast<F*>(v), B, N, d, K);
+                    const void* cell_idx, void* v, int B, int N, int d, int K, hipStream_t st, int bits) {
+        by_widths(bits, HSN_CELLS_I64, [&](auto width) {
+            constexpr int w = decltype(width)::value;
+            hipLaunchKernelGGL((gather_fwd<F, w>), dim3(grid_of(int64_t(B) * K * 4 * d)), dim3(256), 0,
+                               st, static_cast<const F*>(u), static_cast<const F*>(eps),
+                               static_cast<const F*>(h), static_cast<const F*>(m), cells_of<w>(cell_idx, bits),
+                               static_cast<F*>(v), B, N, d, K);
+        });
     }
 };
 
 template <typename F>
 struct RunGatherBwd {
-    static void run(const void* grad_v, Idx cell_idx, void* grad_u, void* grad_eps,
-                    void* grad_h, void* grad_m, int B, int N, int d, int K, hipStream_t st) {
+    static void run(const void* grad_v, const void* cell_idx, void* grad_u, void* grad_eps,
+                    void* grad_h, void* grad_m, int B, int N, int d, int K, hipStream_t st, int bits) {
         const int64_t n = int64_t(B) * N * d;
         launch_copy_or_zero(static_cast<const F*>(nullptr), static_cast<F*>(grad_h), n, st);
-        // fp32 rows: repeats forwarded in registers in slot order (exact); 16-bit rows: each
-        // cell's sum kept in fp32 and rounded once
-        auto kernel = std::is_same<F, float>::value ? gather_bwd<F> : gather_bwd_narrow<F>;
-        hipLaunchKernelGGL(kernel, dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
-                           static_cast<const F*>(grad_v), cell_idx, static_cast<F*>(grad_u),
-                           static_cast<F*>(grad_eps), static_cast<F*>(grad_h),
-                           static_cast<F*>(grad_m), B, N, d, K);
+        by_widths(bits, HSN_CELLS_I64, [&](auto width) {
+            constexpr int w = decltype(width)::value;
+            // fp32 rows: repeats forwarded in registers in slot order (exact); 16-bit rows: each
+            // cell's sum kept in fp32 and rounded once
+            auto kernel = std::is_same<F, float>::value ? gather_bwd<F, w> : gather_bwd_narrow<F, w>;
+            hipLaunchKernelGGL(kernel, dim3(grid_of(int64_t(B) * d)), dim3(256), 0, st,
+                               static_cast<const F*>(grad_v), cells_of<w>(cell_idx, bits), static_cast<F*>(grad_u),
+                               static_cast<F*>(grad_eps), static_cast<F*>(grad_h),
+                               static_cast<F*>(grad_m), B, N, d, K);
+        });
     }
 };
 
@@ -389,7 +406,7 @@ extern "C" int hsn_gather_concat(const void* u, const void* eps, const void* h, 
     check_dtype(dtype & ~kWidths, "hsn_gather_concat");
     HSN_REQUIRE(u && eps && h && m && cell_idx && v, HSN_ERR_INVALID_ARGUMENT,
                 "hsn_gather_concat: a pointer is NULL");
-    by_dtype<RunGather>(dtype & ~kWidths, u, eps, h, m, cells_of(cell_idx, dtype), v, B, N, d, K, as_stream(stream));
+    by_dtype<RunGather>(dtype & ~kWidths, u, eps, h, m, cell_idx, v, B, N, d, K, as_stream(stream), dtype);
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }
@@ -404,8 +421,8 @@ extern "C" int hsn_gather_concat_bwd(const void* grad_v, const int32_t* cell_idx
                 "hsn_gather_concat_bwd: deterministic must be 0 or 1");
     HSN_REQUIRE(grad_v && cell_idx && grad_u && grad_eps && grad_h && grad_m,
                 HSN_ERR_INVALID_ARGUMENT, "hsn_gather_concat_bwd: a pointer is NULL");
-    by_dtype<RunGatherBwd>(dtype & ~kWidths, grad_v, cells_of(cell_idx, dtype), grad_u, grad_eps, grad_h, grad_m, B, N, d, K,
-                           as_stream(stream));
+    by_dtype<RunGatherBwd>(dtype & ~kWidths, grad_v, cell_idx, grad_u, grad_eps, grad_h, grad_m, B, N, d, K,
+                           as_stream(stream), dtype);
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }
@@ -419,8 +436,8 @@ extern "C" int hsn_gated_delta_update(void* h, void* q, int32_t* age, const int3
     check_dtype(dtype & ~kWidths, "hsn_gated_delta_update");
     HSN_REQUIRE(h && q && age && cell_idx && valid && c && b && h_old_saved,
                 HSN_ERR_INVALID_ARGUMENT, "hsn_gated_delta_update: a pointer is NULL");
-    by_dtype<RunUpdate>(dtype & ~kWidths, h, q, age, cells_of(cell_idx, dtype), flags_of(valid, dtype), c, b, h_old_saved, B, N, d, K,
-                        as_stream(stream));
+    by_dtype<RunUpdate>(dtype & ~kWidths, h, q, age, cell_idx, valid, c, b, h_old_saved, B, N, d, K,
+                        as_stream(stream), dtype);
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }
@@ -438,9 +455,9 @@ extern "C" int hsn_gated_delta_update_copy(const void* h, const void* q, const v
                 HSN_ERR_INVALID_ARGUMENT, "hsn_gated_delta_update_copy: a pointer is NULL");
     HSN_REQUIRE(age_bits == 32 || age_bits == 64, HSN_ERR_INVALID_ARGUMENT,
                 "hsn_gated_delta_update_copy: age_bits must be 32 or 64");
-    by_dtype<RunUpdateCopy>(dtype & ~kWidths, h, q, age, age_bits == 64 ? 1 : 0, cells_of(cell_idx, dtype),
-                            flags_of(valid, dtype), c, b, h_new, q_new, age_new, h_old_saved, B, N, d, K,
-                            as_stream(stream));
+    by_dtype<RunUpdateCopy>(dtype & ~kWidths, h, q, age, age_bits == 64 ? 1 : 0, cell_idx,
+                            valid, c, b, h_new, q_new, age_new, h_old_saved, B, N, d, K,
+                            as_stream(stream), dtype);
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }
@@ -456,8 +473,8 @@ extern "C" int hsn_gated_delta_update_bwd(const int32_t* cell_idx, const int32_t
     HSN_REQUIRE(cell_idx && valid && c && b && h_old_saved && grad_h_out && grad_q_out &&
                     grad_h && grad_q && grad_c && grad_b,
                 HSN_ERR_INVALID_ARGUMENT, "hsn_gated_delta_update_bwd: a pointer is NULL");
-    by_dtype<RunUpdateBwd>(dtype & ~kWidths, cells_of(cell_idx, dtype), flags_of(valid, dtype), c, b, h_old_saved, grad_h_out, grad_q_out,
-                           grad_h, grad_q, grad_c, grad_b, B, N, d, K, as_stream(stream));
+    by_dtype<RunUpdateBwd>(dtype & ~kWidths, cell_idx, valid, c, b, h_old_saved, grad_h_out, grad_q_out,
+                           grad_h, grad_q, grad_c, grad_b, B, N, d, K, as_stream(stream), dtype);
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }

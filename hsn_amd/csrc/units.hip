@@ -1163,9 +1163,10 @@ __global__ __launch_bounds__(256) void mlp_dv_tiles(const int32_t* unit_idx, con
 // csr_messages
 // ------------------------------------------------------------------------------------------
 
+template <int W>
 struct Csr {
-    Idx indptr;   // [N + 1]
-    Idx indices;  // [E]
+    Idx<W> indptr;   // [N + 1]
+    Idx<W> indices;  // [E]
     int N, E;
     // the edge range of row i, clamped into [0, E] (empty for a row outside [0, N))
     __device__ __forceinline__ void range(int i, int& e0, int& e1) const {
@@ -1181,9 +1182,9 @@ struct Csr {
 // S[s][c] = sum_e a[e] h[r_s, indices[e], c] for 16 slots from s0 and columns [c0, c0 + nc),
 // into LDS (row stride `ld`); every thread of the workgroup takes (slot, column) pairs and walks
 // its slot's edges in order.
-template <typename T>
-__device__ __forceinline__ void gather_sums(const T* h, const T* a, Idx cell_idx,
-                                            const Csr& g, int s0, int BK, int K, int d, int c0,
+template <typename T, int W>
+__device__ __forceinline__ void gather_sums(const T* h, const T* a, Idx<W> cell_idx,
+                                            const Csr<W>& g, int s0, int BK, int K, int d, int c0,
                                             int nc, float* S, int ld) {
     for (int x = threadIdx.x; x < 16 * nc; x += blockDim.x) {
         const int s = x / nc, cc = x - s * nc;
@@ -1211,9 +1212,9 @@ constexpr int kListCap = 1024;
 // gather_sums_listed's static LDS (the 16 slots' edge list), which counts against the same
 // 64 KiB default limit as a caller's dynamic LDS
 constexpr size_t kListLds = (17 + 16 + 2 * size_t(kListCap)) * 4;
-template <typename T>
+template <typename T, int W>
 __device__ __forceinline__ void gather_sums_listed(const T* h, const T* a,
-                                                   Idx cell_idx, const Csr& g, int s0,
+                                                   Idx<W> cell_idx, const Csr<W>& g, int s0,
                                                    int BK, int K, int d, float* S) {
     __shared__ int lstart[17], le0[16], lsrc[kListCap];
     __shared__ float lw[kListCap];
@@ -1277,9 +1278,9 @@ __device__ __forceinline__ void gather_sums_listed(const T* h, const T* a,
 }
 
 // (BK / 16, d / 64) workgroups: m[s][o] = sum_c V[o][c] S[s][c] for 16 slots (S in LDS).
-template <typename T>
-__global__ __launch_bounds__(256) void csr_fwd(const T* h, const Csr g, const T* a, const T* V,
-                                               Idx cell_idx, T* m, int B, int K,
+template <typename T, int W>
+__global__ __launch_bounds__(256) void csr_fwd(const T* h, const Csr<W> g, const T* a, const T* V,
+                                               Idx<W> cell_idx, T* m, int B, int K,
                                                int d) {
     extern __shared__ float S[];  // [16][d]
     const int lane = lane_id(), w = threadIdx.x >> 6, lr = lane & 15, lq = lane >> 4;
@@ -1307,9 +1308,9 @@ __global__ __launch_bounds__(256) void csr_fwd(const T* h, const Csr g, const T*
 // kDhCells source cells accumulated in LDS: every slot in order adds a[e] (V^T grad_m[r, k])[c]
 // to the source cell of each of its edges, in edge order, so every sum has a fixed order.
 constexpr int kDhCells = 128;
-template <typename T>
-__global__ __launch_bounds__(64) void csr_dh(const Csr g, const T* a, const T* V,
-                                             Idx cell_idx, const T* grad_m, T* grad_h,
+template <typename T, int W>
+__global__ __launch_bounds__(64) void csr_dh(const Csr<W> g, const T* a, const T* V,
+                                             Idx<W> cell_idx, const T* grad_m, T* grad_h,
                                              int K, int d) {
     __shared__ float acc[kDhCells][64];
     const int r = blockIdx.x, lane = lane_id(), c = blockIdx.y * 64 + lane;
@@ -1345,9 +1346,9 @@ __global__ __launch_bounds__(64) void csr_dh(const Csr g, const T* a, const T* V
 
 // A wavefront per edge e (target row i, source j): grad_a[e] = sum over the slots (r, k) that
 // selected row i, in order, of grad_m[r, k] . (V h[r, j]).
-template <typename T>
-__global__ __launch_bounds__(256) void csr_da(const T* h, const Csr g, const T* V,
-                                              Idx cell_idx, const T* grad_m, T* grad_a,
+template <typename T, int W>
+__global__ __launch_bounds__(256) void csr_da(const T* h, const Csr<W> g, const T* V,
+                                              Idx<W> cell_idx, const T* grad_m, T* grad_a,
                                               int B, int K, int d) {
     const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = lane_id();
     if (e >= g.E) return;
@@ -1407,8 +1408,8 @@ __host__ __device__ inline DhLds dh_lds(int K) {
 
 // Entries [p0, p0 + cnt) of the row's edge list into LDS: an entry's source (-1 outside
 // [from, to)), weight and slot; every thread of the workgroup calls it.
-template <typename T>
-__device__ __forceinline__ void list_edges(const Csr& g, const T* a, const int* se0, const int* start,
+template <typename T, int W>
+__device__ __forceinline__ void list_edges(const Csr<W>& g, const T* a, const int* se0, const int* start,
                                            int K, int p0, int cnt, int from, int to, int* lsrc,
                                            float* lw, int* lslot) {
     for (int x = threadIdx.x; x < cnt; x += 256) {
@@ -1433,9 +1434,9 @@ __device__ __forceinline__ void list_edges(const Csr& g, const T* a, const int* 
 // than kDhList continues from the sums of the blocks before, exact in fp32 only: 16-bit storage
 // walks every cell. At B 256, N 1024, K 16, d 64 with 8 edges a cell: 31.5 + 11.8 us (the zeroing), 54
 // by cells (every wavefront walking the whole list, u computed once per 128 cells).
-template <typename T, bool TOUCHED>
-__global__ __launch_bounds__(256) void csr_dh_rows(const Csr g, const T* a, const T* V,
-                                                   Idx cell_idx, const T* grad_m,
+template <typename T, bool TOUCHED, int W>
+__global__ __launch_bounds__(256) void csr_dh_rows(const Csr<W> g, const T* a, const T* V,
+                                                   Idx<W> cell_idx, const T* grad_m,
                                                    T* grad_h, int K, int d) {
     extern __shared__ __align__(16) unsigned char lds[];
     const DhLds L = dh_lds(K);
@@ -1569,9 +1570,9 @@ __global__ __launch_bounds__(256) void csr_dh_rows(const Csr g, const T* a, cons
 // LDS, then grad_m[s]^T S[s] on MFMA, wavefront w taking rows o0 + 16 w .. + 16. With one group
 // the sum goes straight to grad_V; with more, each group's [d][d] fp32 sum goes to part[group]
 // and csr_dV_sum adds the groups in order.
-template <typename T>
-__global__ __launch_bounds__(256) void csr_dV_groups(const T* h, const Csr g, const T* a,
-                                                     Idx cell_idx, const T* grad_m,
+template <typename T, int W>
+__global__ __launch_bounds__(256) void csr_dV_groups(const T* h, const Csr<W> g, const T* a,
+                                                     Idx<W> cell_idx, const T* grad_m,
                                                      T* grad_V, float* part, int B, int K, int d,
                                                      int group_slots) {
     __shared__ float S[16 * 16];
@@ -1647,9 +1648,9 @@ __global__ __launch_bounds__(256) void csr_u(const T* V, const T* grad_m, float*
 // order from its set bits. At E 8192 and 4096 slots: 22.6 us (an edge a wavefront, every workgroup
 // of four staging and searching all slots: 27).
 constexpr int kDaEdges = 8;
-template <typename T>
-__global__ __launch_bounds__(256) void csr_da_u(const T* h, const Csr g, const float* U,
-                                                Idx cell_idx, T* grad_a, int B, int K, int d) {
+template <typename T, int W>
+__global__ __launch_bounds__(256) void csr_da_u(const T* h, const Csr<W> g, const float* U,
+                                                Idx<W> cell_idx, T* grad_a, int B, int K, int d) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int BK = B * K;
     int* cells = reinterpret_cast<int*>(lds);
@@ -1735,9 +1736,9 @@ static __global__ __launch_bounds__(256) void zero_floats(float* p, int64_t n, i
 // grad_a with the slots' cells staged in LDS (B K <= 16384): a wavefront per edge e (target row
 // i, source j) finds the slots that selected row i in the LDS copy, in order, and adds
 // (V^T grad_m[r, k]) . h[r, j] for each, lane c taking column c (then a wavefront sum).
-template <typename T>
-__global__ __launch_bounds__(256) void csr_da_rows(const T* h, const Csr g, const T* V,
-                                                   Idx cell_idx, const T* grad_m,
+template <typename T, int W>
+__global__ __launch_bounds__(256) void csr_da_rows(const T* h, const Csr<W> g, const T* V,
+                                                   Idx<W> cell_idx, const T* grad_m,
                                                    T* grad_a, int B, int K, int d) {
     extern __shared__ __align__(16) unsigned char lds[];
     int* cells = reinterpret_cast<int*>(lds);
@@ -1792,10 +1793,14 @@ void check_dtype(int dtype, const char* who) {
                 HSN_ERR_UNSUPPORTED_DTYPE, std::string(who) + ": unknown dtype code");
 }
 
-// The width bits of the messages' dtype code, taken off it.
+// A call's index arrays in one instantiation's types (`bits`: the dtype code's width bits).
 constexpr int kWidths = HSN_CELLS_I64 | HSN_GRAPH_I64;
-Idx cells_of(const void* p, int dtype) { return Idx{p, (dtype & HSN_CELLS_I64) != 0}; }
-Idx graph_of(const void* p, int dtype) { return Idx{p, (dtype & HSN_GRAPH_I64) != 0}; }
+template <int W>
+Idx<W> index_of(const void* p, int bits, int bit) { return Idx<W>{p, (bits & bit) != 0}; }
+template <int W>
+units::Csr<W> csr_of(const void* indptr, const void* indices, int N, int E, int bits) {
+    return {index_of<W>(indptr, bits, HSN_GRAPH_I64), index_of<W>(indices, bits, HSN_GRAPH_I64), N, E};
+}
 
 void check_units(int P, int M, int d, int H, const char* who) {
     HSN_REQUIRE(P >= 1 && M >= 1 && d >= 1 && H >= 1, HSN_ERR_INVALID_ARGUMENT,
@@ -1931,16 +1936,25 @@ struct RunMlpBwd {
 
 template <typename T>
 struct RunCsr {
-    static void run(const void* h, Idx indptr, Idx indices, const void* a,
-                    const void* V, Idx idx, void* m, int B, int N, int d, int K, int E,
-                    hipStream_t st) {
-        const units::Csr g{indptr, indices, N, E};
+    static void run(const void* h, const void* indptr, const void* indices, const void* a,
+                    const void* V, const void* cell_idx, void* m, int B, int N, int d, int K, int E,
+                    hipStream_t st, int bits) {
+        by_widths(bits, kWidths, [&](auto width) {
+            launch<decltype(width)::value>(h, indptr, indices, a, V, cell_idx, m, B, N, d, K, E, st, bits);
+        });
+    }
+    template <int W>
+    static void launch(const void* h, const void* indptr, const void* indices, const void* a,
+                       const void* V, const void* cell_idx, void* m, int B, int N, int d, int K, int E,
+                       hipStream_t st, int bits) {
+        const units::Csr<W> g = csr_of<W>(indptr, indices, N, E, bits);
+        const Idx<W> idx = index_of<W>(cell_idx, bits, HSN_CELLS_I64);
         // S [16][d] in dynamic LDS beside the static edge list: above the default 64 KiB from
         // d = 894 on (d <= 1024: at most 72.3 KiB of the CU's 160)
         const size_t lds = size_t(16) * d * 4;
         if (lds + units::kListLds > 64 * 1024)
-            HSN_HIP(allow_lds_raw(reinterpret_cast<const void*>(units::csr_fwd<T>), lds));
-        hipLaunchKernelGGL((units::csr_fwd<T>), dim3((B * K + 15) / 16, (d + 63) / 64),
+            HSN_HIP(allow_lds_raw(reinterpret_cast<const void*>(units::csr_fwd<T, W>), lds));
+        hipLaunchKernelGGL((units::csr_fwd<T, W>), dim3((B * K + 15) / 16, (d + 63) / 64),
                            dim3(256), lds, st, static_cast<const T*>(h), g,
                            static_cast<const T*>(a), static_cast<const T*>(V), idx,
                            static_cast<T*>(m), B, K, d);
@@ -1949,10 +1963,19 @@ struct RunCsr {
 
 template <typename T>
 struct RunCsrBwd {
-    static void run(const void* h, Idx indptr, Idx indices, const void* a,
-                    const void* V, Idx idx, const void* dm, void* dh, void* da,
-                    void* dV, int B, int N, int d, int K, int E, hipStream_t st) {
-        const units::Csr g{indptr, indices, N, E};
+    static void run(const void* h, const void* indptr, const void* indices, const void* a,
+                    const void* V, const void* cell_idx, const void* dm, void* dh, void* da,
+                    void* dV, int B, int N, int d, int K, int E, hipStream_t st, int bits) {
+        by_widths(bits, kWidths, [&](auto width) {
+            launch<decltype(width)::value>(h, indptr, indices, a, V, cell_idx, dm, dh, da, dV, B, N, d, K, E, st, bits);
+        });
+    }
+    template <int W>
+    static void launch(const void* h, const void* indptr, const void* indices, const void* a,
+                       const void* V, const void* cell_idx, const void* dm, void* dh, void* da,
+                       void* dV, int B, int N, int d, int K, int E, hipStream_t st, int bits) {
+        const units::Csr<W> g = csr_of<W>(indptr, indices, N, E, bits);
+        const Idx<W> idx = index_of<W>(cell_idx, bits, HSN_CELLS_I64);
         // grad_V first: with more than one group of slots its fp32 partial sums live in grad_h's
         // memory (4-byte aligned and large enough), which the grad_h kernel then overwrites
         const int BK = B * K, chunks = (BK + 15) / 16;
@@ -1966,7 +1989,7 @@ struct RunCsrBwd {
             groups = (BK + group_slots - 1) / group_slots;
         }
         float* part = groups > 1 ? static_cast<float*>(dh) : nullptr;
-        hipLaunchKernelGGL((units::csr_dV_groups<T>), dim3(groups, (d + 15) / 16, (d + 63) / 64),
+        hipLaunchKernelGGL((units::csr_dV_groups<T, W>), dim3(groups, (d + 15) / 16, (d + 63) / 64),
                            dim3(256), 0, st, static_cast<const T*>(h), g,
                            static_cast<const T*>(a), idx, static_cast<const T*>(dm),
                            static_cast<T*>(dV), part, B, K, d, group_slots);
@@ -1980,18 +2003,18 @@ struct RunCsrBwd {
             float* U = static_cast<float*>(dh);
             hipLaunchKernelGGL((units::csr_u<T>), dim3(chunks, (d + 63) / 64), dim3(256), 0, st,
                                static_cast<const T*>(V), static_cast<const T*>(dm), U, BK, d);
-            hipLaunchKernelGGL((units::csr_da_u<T>),
+            hipLaunchKernelGGL((units::csr_da_u<T, W>),
                                dim3((E + 4 * units::kDaEdges - 1) / (4 * units::kDaEdges)), dim3(256),
                                size_t(4) * (BK + N + 1),
                                st, static_cast<const T*>(h), g, U, idx, static_cast<T*>(da), B,
                                K, d);
         } else if (E > 0 && BK <= 16384) {
-            hipLaunchKernelGGL((units::csr_da_rows<T>), dim3((E + 3) / 4), dim3(256),
+            hipLaunchKernelGGL((units::csr_da_rows<T, W>), dim3((E + 3) / 4), dim3(256),
                                size_t(4) * BK, st, static_cast<const T*>(h), g,
                                static_cast<const T*>(V), idx, static_cast<const T*>(dm),
                                static_cast<T*>(da), B, K, d);
         } else if (E > 0) {
-            hipLaunchKernelGGL((units::csr_da<T>), dim3((E + 3) / 4), dim3(256), 0, st,
+            hipLaunchKernelGGL((units::csr_da<T, W>), dim3((E + 3) / 4), dim3(256), 0, st,
                                static_cast<const T*>(h), g, static_cast<const T*>(V), idx,
                                static_cast<const T*>(dm), static_cast<T*>(da), B, K, d);
         }
@@ -2000,17 +2023,17 @@ struct RunCsrBwd {
             const int64_t n16 = reinterpret_cast<uintptr_t>(dh) % 16 == 0 ? n / 4 : 0;
             hipLaunchKernelGGL(units::zero_floats, dim3(static_cast<unsigned>((n - 3 * n16 + 255) / 256)),
                                dim3(256), 0, st, static_cast<float*>(dh), n, n16);
-            hipLaunchKernelGGL((units::csr_dh_rows<T, true>), dim3(B, (d + 63) / 64), dim3(256),
+            hipLaunchKernelGGL((units::csr_dh_rows<T, true, W>), dim3(B, (d + 63) / 64), dim3(256),
                                units::dh_lds(K).bytes, st, g, static_cast<const T*>(a),
                                static_cast<const T*>(V), idx, static_cast<const T*>(dm),
                                static_cast<T*>(dh), K, d);
         } else if (K <= 64)
-            hipLaunchKernelGGL((units::csr_dh_rows<T, false>), dim3(B, (d + 63) / 64, (N + 127) / 128),
+            hipLaunchKernelGGL((units::csr_dh_rows<T, false, W>), dim3(B, (d + 63) / 64, (N + 127) / 128),
                                dim3(256), units::dh_lds(K).bytes, st, g, static_cast<const T*>(a),
                                static_cast<const T*>(V), idx, static_cast<const T*>(dm),
                                static_cast<T*>(dh), K, d);
         else
-            hipLaunchKernelGGL((units::csr_dh<T>), dim3(B, (d + 63) / 64), dim3(64), 0, st, g,
+            hipLaunchKernelGGL((units::csr_dh<T, W>), dim3(B, (d + 63) / 64), dim3(64), 0, st, g,
                                static_cast<const T*>(a), static_cast<const T*>(V), idx,
                                static_cast<const T*>(dm), static_cast<T*>(dh), K, d);
     }
@@ -2062,8 +2085,8 @@ extern "C" int hsn_csr_messages(const void* h, const int32_t* indptr, const int3
     check_dtype(dtype & ~kWidths, "hsn_csr_messages");
     HSN_REQUIRE(h && indptr && V && cell_idx && m && (E == 0 || (indices && a)),
                 HSN_ERR_INVALID_ARGUMENT, "hsn_csr_messages: a pointer is NULL");
-    by_dtype<RunCsr>(dtype & ~kWidths, h, graph_of(indptr, dtype), graph_of(indices, dtype), a, V, cells_of(cell_idx, dtype), m, B, N, d, K, E,
-                     as_stream(stream));
+    by_dtype<RunCsr>(dtype & ~kWidths, h, indptr, indices, a, V, cell_idx, m, B, N, d, K, E,
+                     as_stream(stream), dtype);
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }
@@ -2081,8 +2104,8 @@ extern "C" int hsn_csr_messages_bwd(const void* h, const int32_t* indptr, const 
     HSN_REQUIRE(h && indptr && V && cell_idx && grad_m && grad_h && grad_V &&
                     (E == 0 || (indices && a && grad_a)),
                 HSN_ERR_INVALID_ARGUMENT, "hsn_csr_messages_bwd: a pointer is NULL");
-    by_dtype<RunCsrBwd>(dtype & ~kWidths, h, graph_of(indptr, dtype), graph_of(indices, dtype), a, V, cells_of(cell_idx, dtype), grad_m, grad_h, grad_a, grad_V,
-                        B, N, d, K, E, as_stream(stream));
+    by_dtype<RunCsrBwd>(dtype & ~kWidths, h, indptr, indices, a, V, cell_idx, grad_m, grad_h, grad_a, grad_V,
+                        B, N, d, K, E, as_stream(stream), dtype);
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }
