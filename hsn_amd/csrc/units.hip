@@ -1641,15 +1641,53 @@ __global__ __launch_bounds__(256) void csr_u(const T* V, const T* grad_m, float*
     }
 }
 
-// grad_a from U: a wavefront takes eight consecutive edges (mostly one target row's), each with
-// target row i and source j, and adds U[r, k] . h[r, j] over the slots that selected row i, in
-// order. The slots' cells and indptr are staged in LDS ((B K + N + 1) ints within 64 KiB); the
-// slots of a row are found once for its edges, 64 at a time by a ballot, and taken in ascending
-// order from its set bits. At E 8192 and 4096 slots: 22.6 us (an edge a wavefront, every workgroup
-// of four staging and searching all slots: 27).
-constexpr int kDaEdges = 8;
+// grad_a from U: a wavefront per edge e (target row i, source j) adds U[r, k] . h[r, j] over the
+// slots that selected row i, in order. The slots' cells and indptr are staged in LDS
+// ((B K + N + 1) ints within 64 KiB); the slots are found 64 at a time by a ballot and taken in
+// ascending order from its set bits.
 template <typename T, int W>
 __global__ __launch_bounds__(256) void csr_da_u(const T* h, const Csr<W> g, const float* U,
+                                                Idx<W> cell_idx, T* grad_a, int B, int K,
+                                                int d) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const int BK = B * K;
+    int* cells = reinterpret_cast<int*>(lds);
+    int* ptr = cells + BK;
+    for (int x = threadIdx.x; x < BK; x += 256) cells[x] = cell_idx[x];
+    for (int x = threadIdx.x; x <= g.N; x += 256) ptr[x] = g.indptr[x];
+    __syncthreads();
+    const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = lane_id();
+    if (e >= g.E) return;
+    int lo = 0, hi = g.N;  // the target row: the last i with indptr[i] <= e
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (ptr[mid] <= e) lo = mid;
+        else hi = mid;
+    }
+    const int e0 = min(max(ptr[lo], 0), g.E), e1 = min(max(ptr[lo + 1], e0), g.E);
+    const int src = g.indices[e];
+    float acc = 0.0f;
+    if (e >= e0 && e < e1 && src >= 0 && src < g.N) {
+        for (int f0 = 0; f0 < BK; f0 += 64) {
+            uint64_t hits = ballot(f0 + lane < BK && cells[f0 + lane] == lo);
+            while (hits) {  // uniform
+                const int flat = f0 + __builtin_ctzll(hits);
+                hits &= hits - 1;
+                const T* hr = h + (int64_t(flat / K) * g.N + src) * d;
+                const float* u = U + int64_t(flat) * d;
+                for (int c = lane; c < d; c += 64) acc += u[c] * load_f32(hr, c);
+            }
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, kWave);
+    if (lane == 0) store_f32(grad_a, e, acc);
+}
+
+// The same for kDaEdges consecutive edges a wavefront (mostly one target row's): the slots of a row
+// are found once for its edges, and a workgroup's staging serves eight times the edges.
+constexpr int kDaEdges = 8;
+template <typename T, int W>
+__global__ __launch_bounds__(256) void csr_da_u8(const T* h, const Csr<W> g, const float* U,
                                                 Idx<W> cell_idx, T* grad_a, int B, int K, int d) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int BK = B * K;
@@ -1961,6 +1999,13 @@ struct RunCsr {
     }
 };
 
+// Whether a wavefront of grad_a takes eight edges: where an edge a wavefront would be 4096 workgroups or more,
+// each staging and searching all slots, and the cells have some four edges or more. Measured, one
+// edge a wavefront against eight (us; B, K, N, edges a cell): 128, 16, 1024: 1 edge 11.7 and 43.6,
+// 8 edges 13.4 and 14.9, 16 edges 22.0 and 16.0; 32, 8, 4096: 1 edge 8.7 and 14.8, 4 edges 14.6 and
+// 12.9, 32 edges 74.3 and 27.7; 256, 16, 256: 32 edges 29.1 and 33.3; 256, 16, 64: 1 edge 34.8 and 324.
+bool da_eight(int N, int E) { return E >= 16384 && E / 4 >= N; }
+
 template <typename T>
 struct RunCsrBwd {
     static void run(const void* h, const void* indptr, const void* indices, const void* a,
@@ -2003,8 +2048,9 @@ struct RunCsrBwd {
             float* U = static_cast<float*>(dh);
             hipLaunchKernelGGL((units::csr_u<T>), dim3(chunks, (d + 63) / 64), dim3(256), 0, st,
                                static_cast<const T*>(V), static_cast<const T*>(dm), U, BK, d);
-            hipLaunchKernelGGL((units::csr_da_u<T, W>),
-                               dim3((E + 4 * units::kDaEdges - 1) / (4 * units::kDaEdges)), dim3(256),
+            const int edges = da_eight(N, E) ? units::kDaEdges : 1;
+            auto kernel = edges > 1 ? units::csr_da_u8<T, W> : units::csr_da_u<T, W>;
+            hipLaunchKernelGGL(kernel, dim3((E + 4 * edges - 1) / (4 * edges)), dim3(256),
                                size_t(4) * (BK + N + 1),
                                st, static_cast<const T*>(h), g, U, idx, static_cast<T*>(da), B,
                                K, d);
