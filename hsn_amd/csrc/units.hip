@@ -1432,8 +1432,7 @@ __device__ __forceinline__ void list_edges(const Csr<W>& g, const T* a, const in
 // its wavefronts share the list's entries, and the first entry of a source sums all of the
 // source's in list order, so a cell no entry names costs nothing but the zeroing. A list longer
 // than kDhList continues from the sums of the blocks before, exact in fp32 only: 16-bit storage
-// walks every cell. At B 256, N 1024, K 16, d 64 with 8 edges a cell: 31.5 + 11.8 us (the zeroing), 54
-// by cells (every wavefront walking the whole list, u computed once per 128 cells).
+// walks every cell. dh_touched says where it is taken.
 template <typename T, bool TOUCHED, int W>
 __global__ __launch_bounds__(256) void csr_dh_rows(const Csr<W> g, const T* a, const T* V,
                                                    Idx<W> cell_idx, const T* grad_m,
@@ -2006,6 +2005,19 @@ struct RunCsr {
 // 12.9, 32 edges 74.3 and 27.7; 256, 16, 256: 32 edges 29.1 and 33.3; 256, 16, 64: 1 edge 34.8 and 324.
 bool da_eight(int N, int E) { return E >= 16384 && E / 4 >= N; }
 
+// Whether grad_h is zeroed and then summed by touched sources (fp32): where the workgroups by cells
+// would be 1024 or more, and a row's list is short against their number: the search for a source's
+// first entry grows with the list's square. Measured, by cells against the zeroing and the touched
+// sources (us; B, K, N, d, edges a cell): 256, 16, 1024, 64 (2048 workgroups): 1 edge 35.1 and 20.8,
+// 8 edges 54.4 and 40.2, 12 edges 65.7 and 55.4, 64 edges 214 and 449; 128, 16, 1024, 64 (1024): 4
+// edges 28.7 and 22.8, 16 edges 51.4 and 68.7; 32, 8, 4096, 64 (1024): 8 edges 24.6 and 20.8, 16 edges
+// 31.8 and 32.8; 128, 8, 512, 64 (512): 1 edge 10.6 and 12.4, 32 edges 26.2 and 62.8; 1, 16, 512, 64 (4):
+// 512 edges 525 and 2645.
+bool dh_touched(int B, int N, int d, int K, int E) {
+    const int64_t groups = int64_t(B) * ((d + 63) / 64) * ((N + 127) / 128);
+    return groups >= 1024 && int64_t(K) * E <= int64_t(N) * std::min<int64_t>(256, groups / 10);
+}
+
 template <typename T>
 struct RunCsrBwd {
     static void run(const void* h, const void* indptr, const void* indices, const void* a,
@@ -2064,7 +2076,7 @@ struct RunCsrBwd {
                                static_cast<const T*>(h), g, static_cast<const T*>(V), idx,
                                static_cast<const T*>(dm), static_cast<T*>(da), B, K, d);
         }
-        if (K <= 64 && sizeof(T) == 4) {
+        if (K <= 64 && sizeof(T) == 4 && dh_touched(B, N, d, K, E)) {
             const int64_t n = int64_t(B) * N * d;
             const int64_t n16 = reinterpret_cast<uintptr_t>(dh) % 16 == 0 ? n / 4 : 0;
             hipLaunchKernelGGL(units::zero_floats, dim3(static_cast<unsigned>((n - 3 * n16 + 255) / 256)),
