@@ -22,6 +22,7 @@
 // backward together, M 8, d 64, H 512 (us): P 8192 bf16 971 -> 250, P 256 fp32 76.7 -> 55 (of
 // both, 19 and 11 are the launches that narrowed the indices: unit_order reads either width).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.cuh"
 
@@ -571,6 +572,18 @@ bool takes(int P, int M, int d, int H) {
     return P >= 1 && M >= 1 && M <= kMaxUnits && d >= 4 && d % 4 == 0 && d <= 256 && H >= 4 &&
            H % 4 == 0 && (H + 63) / 64 <= 65535 && P / block_rows(P, M, d, H) + M <= 65535;
 }
+// Forwards that the kernels without a workspace are faster at: they have no pairs to order first and a
+// quarter of the reduction a wavefront. Measured (us, without and with a workspace), fp32: P 256, M 8: d
+// 64, H 512 21 and 28; d 64, H 64 17 and 20; P 64, M 32, d 128, H 512 29 and 37; but P 1024, M 8, d 64,
+// H 512 32 and 31, P 16, M 32, d 16, H 64 17 and 13, and from 128 units on up to 2 to 3 times. 16-bit
+// storage, where they go through a row's hidden tiles in turn: P 256, M 8: d 64, H 64 13 and 23, H 128 21
+// and 24, d 128, H 64 21 and 30; P 2048, M 8, d 16, H 64 15 and 18; but d 16, H 512 40 and 28, and P 8192,
+// M 16, d 16, H 64 51 and 29.
+bool few_pairs(int P, int M, int d, int H, int dtype) {
+    if (M > 32) return false;
+    if (dtype == HSN_DTYPE_F32) return P <= 512 && int64_t(d) * H >= std::max(1024, 256 * M);
+    return P <= 2048 && (H <= 64 || (H <= 128 && d <= 64));
+}
 bool aligned4(std::initializer_list<const void*> ptrs, size_t elem) {
     for (const void* p : ptrs)
         if (reinterpret_cast<uintptr_t>(p) % (4 * elem) != 0) return false;
@@ -687,8 +700,7 @@ extern "C" int hsn_grouped_unit_mlp_workspace(int P, int M, int d, int H, int dt
                                               int64_t* bytes) {
     HSN_ABI_BEGIN
     HSN_REQUIRE(bytes != nullptr, HSN_ERR_INVALID_ARGUMENT, "hsn_grouped_unit_mlp_workspace: bytes is NULL");
-    (void)dtype;
-    const bool fits = ugemm::takes(P, M, d, H) && int64_t(M) * 4 * d * H <= INT32_MAX &&
+    const bool fits = ugemm::takes(P, M, d, H) && (backward || !ugemm::few_pairs(P, M, d, H, dtype)) && int64_t(M) * 4 * d * H <= INT32_MAX &&
                       int64_t(P) * H <= INT32_MAX && int64_t(P) * 4 * d <= INT32_MAX;
     *bytes = fits ? static_cast<int64_t>(ugemm::layout(P, M, d, H, backward != 0).bytes) : 0;
     HSN_ABI_END

@@ -41,7 +41,8 @@ struct Chunk {
     int n;
     int row;  // lane's pair (lane < n), else -1
 };
-__device__ __forceinline__ Chunk next_pairs(const int32_t* unit_idx, int P, int j, int& cur) {
+template <int W>
+__device__ __forceinline__ Chunk next_pairs(Idx<W> unit_idx, int P, int j, int& cur) {
     const int lane = lane_id();
     int n = 0, row = -1;
     while (n < 16 && cur < P) {
@@ -110,8 +111,8 @@ __device__ __forceinline__ void dz_tile(const T* grad_out, const T* W2j, const T
 // to the storage dtype), gelu(z1) in fp32 into LDS, and out += gelu(z1) W2[j][tile] accumulated
 // in registers over the tiles; out = that + b2[j]. Layer 2 reads the fp32 activation, not the
 // rounded copy, as the reference's two kernels do through an fp32 buffer.
-template <typename T>
-__global__ __launch_bounds__(256) void mlp_fwd(const T* v, const int32_t* unit_idx, const T* W1,
+template <typename T, int W>
+__global__ __launch_bounds__(256) void mlp_fwd(const T* v, Idx<W> unit_idx, const T* W1,
                                                const T* b1, const T* W2, const T* b2, T* hidden,
                                                T* out, int P, int d, int H) {
     __shared__ float act[16][64];
@@ -245,7 +246,8 @@ __device__ __forceinline__ float4 row4w(const T* w, int c, int cols, bool aligne
 // The workgroup's row tile (blockIdx.x over every unit's tiles of 16 pairs, laid end to end unit
 // after unit): returns its unit, or -1 past the last tile, with its pairs in rows[16] (-1 past
 // the unit's pairs), from LDS counts of each unit's pairs. Every thread of the workgroup calls it.
-__device__ __forceinline__ int find_row_tile(const int32_t* unit_idx, int P, int M,
+template <int W>
+__device__ __forceinline__ int find_row_tile(Idx<W> unit_idx, int P, int M,
                                              uint16_t* ucache, int* count, int* rows, int* meta) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     for (int j = tid; j < M; j += 256) count[j] = 0;
@@ -292,9 +294,9 @@ __device__ __forceinline__ int find_row_tile(const int32_t* unit_idx, int P, int
     return meta[0];
 }
 
-template <typename T, bool ALIGNED, bool SPLIT = false>  // ALIGNED: H % 4 == 0, rows of W1 in
+template <typename T, int W, bool ALIGNED, bool SPLIT = false>  // ALIGNED: H % 4 == 0, rows of W1 in
 // 16-byte pieces; SPLIT: one hidden tile a workgroup (blockIdx.y), z1 stored, no second layer
-__global__ __launch_bounds__(256) void mlp_fwd_tiles(const T* v, const int32_t* unit_idx,
+__global__ __launch_bounds__(256) void mlp_fwd_tiles(const T* v, Idx<W> unit_idx,
                                                      const T* W1, const T* b1, const T* W2,
                                                      const T* b2, T* hidden, T* out, int P, int M,
                                                      int d, int H) {
@@ -359,7 +361,7 @@ __global__ __launch_bounds__(256) void mlp_fwd_tiles(const T* v, const int32_t* 
     for (int c = tid; c < H; c += 256) b1c[c] = load_f32(b1, int64_t(j) * H + c);
     __syncthreads();  // the inputs and the bias are in LDS
 
-    v4f acc[4];
+    v4f acc[4];  // the tile's sums, a block's added at its end (shorter running sums)
     const float* arow = vs + lr * L.sv + k1;
     const int total = SPLIT ? blocks : tiles_h * blocks;
     auto load_w2 = [&](float (&w)[16], int h0, int t) {
@@ -385,13 +387,16 @@ __global__ __launch_bounds__(256) void mlp_fwd_tiles(const T* v, const int32_t* 
             const int s = bi * kTileBlock + k;
             av[k] = s < q1 ? arow[s] : 0.0f;
         }
+        v4f part[4] = {};
 #pragma unroll
         for (int k = 0; k < kTileBlock; ++k) {
-            acc[0] = mfma(av[k], cur[k].x, acc[0]);
-            acc[1] = mfma(av[k], cur[k].y, acc[1]);
-            acc[2] = mfma(av[k], cur[k].z, acc[2]);
-            acc[3] = mfma(av[k], cur[k].w, acc[3]);
+            part[0] = mfma(av[k], cur[k].x, part[0]);
+            part[1] = mfma(av[k], cur[k].y, part[1]);
+            part[2] = mfma(av[k], cur[k].z, part[2]);
+            part[3] = mfma(av[k], cur[k].w, part[3]);
         }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[t] += part[t];
         if (bi + 1 < blocks) return;
         // the tile's tail; its second-layer weights (the wavefront's first output tile; d <= 64:
         // all of them) are in flight during the shares' sum
@@ -474,8 +479,8 @@ __host__ __device__ inline OutLds out_lds(int P, int M, int H) {
     return L;
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void mlp_out_tiles(const int32_t* unit_idx, const T* W2,
+template <typename T, int W>
+__global__ __launch_bounds__(256) void mlp_out_tiles(Idx<W> unit_idx, const T* W2,
                                                      const T* b2, const T* hidden, T* out, int P,
                                                      int M, int d, int H) {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -533,8 +538,10 @@ __global__ __launch_bounds__(256) void mlp_out_tiles(const int32_t* unit_idx, co
                 float av[16];
 #pragma unroll
                 for (int s = 0; s < 16; ++s) av[s] = h0 + g * 16 + s < H ? ar[s] : 0.0f;
+                v4f part[4] = {};  // four runs of 16, added pairwise: shorter running sums
 #pragma unroll
-                for (int s = 0; s < 16; ++s) acc = mfma(av[s], wv[x][s], acc);
+                for (int s = 0; s < 16; ++s) part[s % 4] = mfma(av[s], wv[x][s], part[s % 4]);
+                acc += (part[0] + part[1]) + (part[2] + part[3]);
             }
         }
     }
@@ -573,7 +580,7 @@ __host__ __device__ inline DzLds dz_lds(int P, int M, int d) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void mlp_dz_tiles(const int32_t* unit_idx, const T* W2,
+__global__ __launch_bounds__(256) void mlp_dz_tiles(Idx<kNarrow> unit_idx, const T* W2,
                                                     const T* hidden, const T* grad_out, float* dz,
                                                     int P, int M, int d, int H) {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -649,7 +656,7 @@ __host__ __device__ inline GvLds gv_lds(int P, int M, int H) {
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void mlp_gv_tiles(const int32_t* unit_idx, const T* W1,
+__global__ __launch_bounds__(256) void mlp_gv_tiles(Idx<kNarrow> unit_idx, const T* W1,
                                                     const float* dz, T* grad_v, int P, int M,
                                                     int d, int H) {
     extern __shared__ __align__(16) unsigned char lds[];
@@ -738,7 +745,7 @@ __global__ __launch_bounds__(256) void mlp_gv_tiles(const int32_t* unit_idx, con
 // grad_W2[j][h0.., :] = sum_p gelu(z1[p])^T grad_out[p] and grad_b1[j][h0..]; the first of all
 // grad_b2[j]. A unit without pairs gets zeros.
 template <typename T>
-__global__ __launch_bounds__(256) void mlp_dw(const T* v, const int32_t* unit_idx, const T* W2,
+__global__ __launch_bounds__(256) void mlp_dw(const T* v, Idx<kNarrow> unit_idx, const T* W2,
                                               const T* hidden, const T* grad_out, T* grad_W1,
                                               T* grad_b1, T* grad_W2, T* grad_b2, int P, int d,
                                               int H) {
@@ -939,7 +946,7 @@ __global__ __launch_bounds__(256) void mlp_dw(const T* v, const int32_t* unit_id
 // (4d / 64, M) workgroups: grad_v[p][i0..] = sum_h dz1[p][h] W1[j][i][h], dz1 recomputed per
 // hidden tile of 64.
 template <typename T>
-__global__ __launch_bounds__(256) void mlp_dv(const int32_t* unit_idx, const T* W1, const T* W2,
+__global__ __launch_bounds__(256) void mlp_dv(Idx<kNarrow> unit_idx, const T* W1, const T* W2,
                                               const T* hidden, const T* grad_out, T* grad_v,
                                               int P, int d, int H) {
     __shared__ float dz[16][64];
@@ -999,7 +1006,7 @@ __host__ __device__ inline DvLds dv_lds(int P, int M, int d) {
 }
 
 template <typename T, bool ALIGNED>  // ALIGNED: rows of W1 and W2 in 16-byte pieces
-__global__ __launch_bounds__(256) void mlp_dv_tiles(const int32_t* unit_idx, const T* W1,
+__global__ __launch_bounds__(256) void mlp_dv_tiles(Idx<kNarrow> unit_idx, const T* W1,
                                                     const T* W2, const T* hidden,
                                                     const T* grad_out, T* grad_v, int P, int M,
                                                     int d, int H) {
@@ -1861,13 +1868,22 @@ inline dim3 tiles(int n, int per) { return dim3((n + per - 1) / per); }
 
 template <typename T>
 struct RunMlp {
-    static void run(const void* v, const int32_t* idx, const void* W1, const void* b1,
+    static void run(const void* v, const void* unit_idx, const void* W1, const void* b1,
                     const void* W2, const void* b2, void* hidden, void* out, int P, int M, int d,
-                    int H, hipStream_t st) {
+                    int H, hipStream_t st, int bits) {
+        by_widths(bits, HSN_CELLS_I64, [&](auto width) {
+            launch<decltype(width)::value>(v, unit_idx, W1, b1, W2, b2, hidden, out, P, M, d, H, st, bits);
+        });
+    }
+    template <int W>
+    static void launch(const void* v, const void* unit_idx, const void* W1, const void* b1,
+                       const void* W2, const void* b2, void* hidden, void* out, int P, int M, int d,
+                       int H, hipStream_t st, int bits) {
+        const Idx<W> idx = index_of<W>(unit_idx, bits, HSN_CELLS_I64);
         if (d % 4 == 0 && P <= units::kTileMaxSlots && M <= units::kTileMaxUnits &&
             units::tile_lds(P, M, d, H).bytes <= 160 * 1024) {
             const int lds = units::tile_lds(P, M, d, H).bytes;
-            auto launch = [&](auto kernel) {
+            auto one = [&](auto kernel) {
                 if (lds > 64 * 1024)
                     HSN_HIP(allow_lds_raw(reinterpret_cast<const void*>(kernel), lds));
                 hipLaunchKernelGGL(kernel, dim3((P + 15) / 16 + M), dim3(256), lds, st,
@@ -1880,8 +1896,8 @@ struct RunMlp {
             if (sizeof(T) == 4 && olds <= 160 * 1024) {
                 // fp32 storage: the hidden layer over (row tile, hidden tile) workgroups, then
                 // the second layer from the stored z1
-                auto kernel = H % 4 == 0 ? &units::mlp_fwd_tiles<T, true, true>
-                                         : &units::mlp_fwd_tiles<T, false, true>;
+                auto kernel = H % 4 == 0 ? &units::mlp_fwd_tiles<T, W, true, true>
+                                         : &units::mlp_fwd_tiles<T, W, false, true>;
                 if (lds > 64 * 1024)
                     HSN_HIP(allow_lds_raw(reinterpret_cast<const void*>(kernel), lds));
                 hipLaunchKernelGGL(kernel, dim3((P + 15) / 16 + M, (H + 63) / 64), dim3(256), lds,
@@ -1889,7 +1905,7 @@ struct RunMlp {
                                    static_cast<const T*>(b1), static_cast<const T*>(W2),
                                    static_cast<const T*>(b2), static_cast<T*>(hidden),
                                    static_cast<T*>(out), P, M, d, H);
-                auto second = &units::mlp_out_tiles<T>;
+                auto second = &units::mlp_out_tiles<T, W>;
                 if (olds > 64 * 1024)
                     HSN_HIP(allow_lds_raw(reinterpret_cast<const void*>(second), olds));
                 hipLaunchKernelGGL(second, dim3((P + 15) / 16 + M, (d + 15) / 16), dim3(256), olds,
@@ -1899,12 +1915,12 @@ struct RunMlp {
                                    H);
                 return;
             }
-            if (H % 4 == 0) launch(&units::mlp_fwd_tiles<T, true>);
-            else launch(&units::mlp_fwd_tiles<T, false>);
+            if (H % 4 == 0) one(&units::mlp_fwd_tiles<T, W, true>);
+            else one(&units::mlp_fwd_tiles<T, W, false>);
             return;
         }
         const int S = std::min((P + 15) / 16, 64);  // chunk slots per unit
-        hipLaunchKernelGGL((units::mlp_fwd<T>), dim3(M, S), dim3(256), 0, st,
+        hipLaunchKernelGGL((units::mlp_fwd<T, W>), dim3(M, S), dim3(256), 0, st,
                            static_cast<const T*>(v), idx, static_cast<const T*>(W1),
                            static_cast<const T*>(b1), static_cast<const T*>(W2),
                            static_cast<const T*>(b2), static_cast<T*>(hidden),
@@ -1914,9 +1930,10 @@ struct RunMlp {
 
 template <typename T>
 struct RunMlpBwd {
-    static void run(const void* v, const int32_t* idx, const void* W1, const void* W2,
+    static void run(const void* v, const int32_t* unit_idx, const void* W1, const void* W2,
                     const void* hidden, const void* dout, void* dv, void* dW1, void* db1,
                     void* dW2, void* db2, int P, int M, int d, int H, hipStream_t st) {
+        const Idx<kNarrow> idx{unit_idx, 0};
         // grad_v through dz1 in fp32 in grad_W2's memory (4-byte aligned, P H floats of room),
         // before the weight-gradient kernel writes grad_W2
         const int dzl = units::dz_lds(P, M, d).bytes, gvl = units::gv_lds(P, M, H).bytes;
@@ -2105,11 +2122,11 @@ extern "C" int hsn_grouped_unit_mlp_fwd(const void* v, const int32_t* unit_idx, 
                                         int dtype, void* stream) {
     HSN_ABI_BEGIN
     check_units(P, M, d, H, "hsn_grouped_unit_mlp_fwd");
-    check_dtype(dtype, "hsn_grouped_unit_mlp_fwd");
+    check_dtype(dtype & ~HSN_CELLS_I64, "hsn_grouped_unit_mlp_fwd");
     HSN_REQUIRE(v && unit_idx && W1 && b1 && W2 && b2 && hidden_saved && out,
                 HSN_ERR_INVALID_ARGUMENT, "hsn_grouped_unit_mlp_fwd: a pointer is NULL");
-    by_dtype<RunMlp>(dtype, v, unit_idx, W1, b1, W2, b2, hidden_saved, out, P, M, d, H,
-                     as_stream(stream));
+    by_dtype<RunMlp>(dtype & ~HSN_CELLS_I64, v, unit_idx, W1, b1, W2, b2, hidden_saved, out, P, M, d, H,
+                     as_stream(stream), dtype);
     HSN_HIP(hipGetLastError());
     HSN_ABI_END
 }

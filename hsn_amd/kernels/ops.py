@@ -367,8 +367,8 @@ def _mlp_workspace_bytes(P: int, M: int, d: int, H: int, code: int, backward: in
 def _mlp_space(P: int, M: int, d: int, H: int, backward: int, idx: Tensor, v: Tensor,
                *operands: Tensor) -> Optional[tuple[Tensor, int, Tensor, int]]:
     """``(idx, its bits, workspace, bytes)`` of a call of the products in unit order, or ``None``
-    where the kernels without a workspace take it: another shape, operands off four-element
-    alignment (a view into a buffer), or indices neither int32 nor int64."""
+    where the kernels without a workspace take it: another shape, a forward of few pairs, operands
+    off four-element alignment (a view into a buffer), or indices neither int32 nor int64."""
     if idx.dtype not in (torch.int32, torch.int64):
         return None
     nbytes = _mlp_workspace_bytes(P, M, d, H, _code(v), backward)
@@ -392,9 +392,9 @@ def _mlp_body(v: Tensor, idx: Tensor, w1: Tensor, b1: Tensor, w2: Tensor,
              ptr(b2), ptr(hidden), ptr(out), P, M, d, H, _code(v), ptr(ws), nbytes,
              stream_of(v.device))
         return out, hidden
-    idx = _i32(idx)
+    idx, wide = _cells(idx)
     call("hsn_grouped_unit_mlp_fwd", ptr(v), ptr(idx), ptr(w1), ptr(b1), ptr(w2), ptr(b2),
-         ptr(hidden), ptr(out), P, M, d, H, _code(v), stream_of(v.device))
+         ptr(hidden), ptr(out), P, M, d, H, _code(v) | wide, stream_of(v.device))
     return out, hidden
 
 

@@ -26,9 +26,9 @@ extern "C" {
 #define HSN_DTYPE_BF16 2
 
 /*
- * Or'ed into the dtype code of the gather, the messages and the gated update: the widths of the
- * call's index and flag arrays where they are not int32_t. cell_idx int64_t; indptr and indices
- * int64_t; valid one byte a flag. An int64_t index is clamped into [-1, 2^31 - 1] as it is read.
+ * Or'ed into the dtype code of the gather, the messages, the gated update and the unit MLP's forward
+ * (its unit_idx): the widths of the call's index and flag arrays where they are not int32_t. cell_idx
+ * (or unit_idx) int64_t; indptr and indices int64_t; valid one byte a flag. An int64_t index is clamped into [-1, 2^31 - 1] as it is read.
  */
 #define HSN_CELLS_I64 0x100
 #define HSN_GRAPH_I64 0x200
@@ -92,11 +92,11 @@ int hsn_grouped_unit_mlp_bwd(const void* v, const int32_t* unit_idx, const void*
 /*
  * The grouped unit MLP and its backward on a workspace: the same contract and results as
  * hsn_grouped_unit_mlp_{fwd,bwd} up to the order of the fp32 sums, as matrix products over the
- * pairs in unit order (64-column tiles, each unit's weights read once a tile of 32 or 64 pairs).
+ * pairs in unit order (64-column tiles, each unit's weights read once a tile of 32 pairs).
  * unit_idx [P] is int32_t or int64_t (`index_bits`); a pair whose unit lies outside [0,M) takes
- * part in nothing and gets no output. hsn_grouped_unit_mlp_workspace gives the bytes (`backward`
- * 0 or 1), or 0 for a shape these do not take: M <= 1024, d a multiple of 4 up to 256, H a
- * multiple of 4. The operands must be aligned to four elements, the workspace to 256 bytes. The
+ * part in nothing and gets no output. They take M <= 1024, d a multiple of 4 up to 256 and H a
+ * multiple of 4. hsn_grouped_unit_mlp_workspace gives the bytes (`backward` 0 or 1), or 0 for a
+ * shape they do not take and for a forward of so few pairs that hsn_grouped_unit_mlp_fwd is faster. The operands must be aligned to four elements, the workspace to 256 bytes. The
  * workspace's contents before the call do not matter, and nothing is kept in it after it. Every
  * sum has a fixed order.
  */

@@ -544,3 +544,65 @@ def test_ops_read_either_index_width(ops, cuda_device, dtype, E_extra):
     mixed = ops.messages_op(D["h"], indptr.to(dev), indices.to(torch.int32).to(dev), D["a"], D["V"],
                             cells.to(dev))
     assert torch.equal(mixed, wide[0])
+
+
+def _through(monkeypatch, ops, path):
+    """Sends the unit MLP through one kind of kernels whatever the dispatch would take: ``unit order``
+    (a workspace) or ``by rows`` (none)."""
+    real = ops._mlp_space
+
+    def space(P, M, d, H, backward, idx, v, *operands):
+        if path == "by rows":
+            return None
+        if backward:
+            return real(P, M, d, H, backward, idx, v, *operands)
+        nbytes = 4 * P * (H + 3) + 16 * M + 8192  # a forward's rows, pairs and units
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=v.device)
+        return idx.contiguous(), 64 if idx.dtype == torch.int64 else 32, ws, nbytes
+
+    monkeypatch.setattr(ops, "_mlp_space", space)
+
+
+def _mlp_problem(P, M, d, H, dtype, seed, dev, index=torch.int32):
+    g = torch.Generator().manual_seed(seed)
+    rnd = lambda *s, scale=0.5: (torch.randn(*s, generator=g) * scale).to(dtype).to(dev)  # noqa: E731
+    return dict(v=rnd(P, 4 * d), idx=torch.randint(0, M, (P,), generator=g).to(index).to(dev),
+                W1=rnd(M, 4 * d, H, scale=(4 * d) ** -0.5), b1=rnd(M, H),
+                W2=rnd(M, H, d, scale=H ** -0.5), b2=rnd(M, d), dout=rnd(P, d))
+
+
+def _mlp_run(ops, x):
+    out, hidden = ops.mlp_op(x["v"], x["idx"], x["W1"], x["b1"], x["W2"], x["b2"])
+    return out, hidden, ops.mlp_backward(x["v"], x["idx"], x["W1"], x["W2"], hidden, x["dout"])
+
+
+@pytest.mark.parametrize("index", [torch.int32, torch.int64])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("path", ["unit order", "by rows"])
+@pytest.mark.parametrize("P,M,d,H", [
+    (130, 3, 16, 68),     # several row tiles a unit, a hidden tail; the forward of few pairs
+    (700, 6, 64, 512),    # the model's widths, more pairs than the forward of few takes in fp32
+    (17000, 2, 4, 8),     # more pairs than the row tiles' slot table: the scanning kernels
+    (2000, 2, 8, 64),     # grad_W2 too small to hold dz1: grad_v in one launch by rows
+])
+def test_unit_mlp_by_either_kernels_matches_oracle(ops, cuda_device, monkeypatch, P, M, d, H, path, dtype,
+                                                   index):
+    """The kernels over the pairs in unit order and those over rows, each at both sides of the sizes
+    at which the dispatch changes from one to the other, forward and backward against the float64
+    oracle on the same rounded inputs; the weight gradients' bar grows with the square root of a
+    unit's pairs."""
+    from oracle import hsn_oracle as O
+
+    x = _mlp_problem(P, M, d, H, dtype, P + d, cuda_device, index)
+    _through(monkeypatch, ops, path)
+    out, hidden, got = _mlp_run(ops, x)
+    c = {k: t.cpu().double() if t.is_floating_point() else t.cpu() for k, t in x.items()}
+    want_out, want_h = O.grouped_unit_mlp(c["v"], c["idx"], c["W1"], c["b1"], c["W2"], c["b2"])
+    _close(hidden, want_h, dtype, "hidden")
+    _close(out, want_out, dtype, "out")
+    want = O.grouped_unit_mlp_bwd(c["v"], c["idx"], c["W1"], c["W2"], hidden.cpu().double(), c["dout"])
+    _close(got[0], want[0], dtype, "grad_v")
+    bar = TOL[dtype] * max(1.0, (P / M / 64) ** 0.5)
+    for name, g_, w_ in zip(("dW1", "db1", "dW2", "db2"), got[1:], want[1:]):
+        err = (g_.double().cpu() - w_).abs() / w_.abs().clamp(min=1.0)
+        assert float(err.max()) <= bar, f"{name}: worst {float(err.max()):.3e} (bar {bar:.1e})"
