@@ -172,8 +172,8 @@ __global__ __launch_bounds__(64 * kSortWaves) void unit_order(const I* unit_idx,
 // acc += A [X x K] B [K x 64] by four wavefronts, each its X/2 x 32 quarter, the reduction in
 // steps of KC through LDS with the next step's rows in registers while a step multiplies; a step's
 // sum is added to the total at its end (one running sum over all of K was twice as far from the
-// 64-bit result at K = 512). An
-// operand whose memory runs along the reduction (along() true) is kept [x][KC + 4] and read as
+// 64-bit result at K = 512), and with PARTS 4 a step keeps four sums, an index of every four each, so
+// that K = 64 is four runs of 16 (by_reduction). An operand whose memory runs along the reduction (along() true) is kept [x][KC + 4] and read as
 // 16 bytes, one that runs along the columns [KC][X + 4] and read as words: lane group g of a
 // wavefront takes the reduction's indices 4 g .. 4 g + 3 of each 16, the same on both sides.
 // The loaders give four consecutive elements, zero outside the operand: (x, k .. k + 3), or
@@ -208,10 +208,11 @@ __device__ __forceinline__ void fragment(const float* t, int x0, int s, int lr, 
     }
 }
 
-template <int RT, int KC, bool AALONG, bool BALONG, class LA, class LB, class Step>
+template <int RT, int KC, bool AALONG, bool BALONG, int PARTS = 1, class LA, class LB, class Step>
 __device__ __forceinline__ void tile_product(const LA& la, const LB& lb, int K, float* As, float* Bs,
                                              v4f (&acc)[RT / 32][2], const Step& each) {
     constexpr int NA = RT * KC / 4 / 256, NB = kNT * KC / 4 / 256, TM = RT / 32;
+    static_assert(PARTS == 1 || PARTS == 4, "the step's sums are added pairwise");
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, g = lane >> 4;
     const int xm = (w >> 1) * (RT / 2), xn = (w & 1) * 32;
     struct Rows {
@@ -242,7 +243,7 @@ __device__ __forceinline__ void tile_product(const LA& la, const LB& lb, int K, 
         }
         __syncthreads();
         fetch(k0 + KC, q);
-        v4f part[TM][2] = {};
+        v4f part[PARTS][TM][2] = {};
 #pragma unroll
         for (int s = 0; s < KC / 16; ++s) {
             float fa[TM][4], fb[2][4];
@@ -254,13 +255,17 @@ __device__ __forceinline__ void tile_product(const LA& la, const LB& lb, int K, 
                 for (int m = 0; m < TM; ++m)
 #pragma unroll
                     for (int n = 0; n < 2; ++n)
-                        part[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[m][i], fb[n][i],
-                                                                          part[m][n], 0, 0, 0);
+                        part[i % PARTS][m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            fa[m][i], fb[n][i], part[i % PARTS][m][n], 0, 0, 0);
         }
 #pragma unroll
         for (int m = 0; m < TM; ++m)
 #pragma unroll
-            for (int n = 0; n < 2; ++n) acc[m][n] += part[m][n];
+            for (int n = 0; n < 2; ++n) {
+                if constexpr (PARTS == 4)
+                    part[0][m][n] = (part[0][m][n] + part[1][m][n]) + (part[2][m][n] + part[3][m][n]);
+                acc[m][n] += part[0][m][n];
+            }
     };
     Rows next;
     fetch(0, next);
@@ -312,7 +317,7 @@ __device__ __forceinline__ int row_tile(const RowArgs& a, int* rows, int& r0, in
     return j;
 }
 
-template <typename T>
+template <typename T, int PARTS>
 __global__ __launch_bounds__(256) void gm_hidden(RowArgs a, const T* v, const T* W1, const T* b1,
                                                  T* hidden, float* act) {
     __shared__ __align__(16) float As[tile_words<kRT, kKC, true>()];
@@ -324,7 +329,7 @@ __global__ __launch_bounds__(256) void gm_hidden(RowArgs a, const T* v, const T*
     const int in = 4 * a.d, H = a.H, h0 = blockIdx.y * kNT;
     const T* W = W1 + int64_t(j) * in * H;
     v4f acc[kRT / 32][2] = {};
-    tile_product<kRT, kKC, true, false>(
+    tile_product<kRT, kKC, true, false, PARTS>(
         [&](int x, int k) { return x < n && k < in ? load4(v + int64_t(rows[x]) * in + k) : zero4(); },
         [&](int x, int k) { return k < in && h0 + x < H ? load4(W + int64_t(k) * H + h0 + x) : zero4(); },
         in, As, Bs, acc, NoStep{});
@@ -337,7 +342,7 @@ __global__ __launch_bounds__(256) void gm_hidden(RowArgs a, const T* v, const T*
     });
 }
 
-template <typename T>
+template <typename T, int PARTS>
 __global__ __launch_bounds__(256) void gm_out(RowArgs a, const float* act, const T* W2, const T* b2,
                                               T* out) {
     __shared__ __align__(16) float As[tile_words<kRT, kKC, true>()];
@@ -350,7 +355,7 @@ __global__ __launch_bounds__(256) void gm_out(RowArgs a, const float* act, const
     const T* W = W2 + int64_t(j) * H * d;
     const float* A = act + int64_t(r0) * H;
     v4f acc[kRT / 32][2] = {};
-    tile_product<kRT, kKC, true, false>(
+    tile_product<kRT, kKC, true, false, PARTS>(
         [&](int x, int k) { return x < n && k < H ? load4(A + int64_t(x) * H + k) : zero4(); },
         [&](int x, int k) { return k < H && o0 + x < d ? load4(W + int64_t(k) * d + o0 + x) : zero4(); },
         H, As, Bs, acc, NoStep{});
@@ -360,7 +365,7 @@ __global__ __launch_bounds__(256) void gm_out(RowArgs a, const float* act, const
     });
 }
 
-template <typename T>
+template <typename T, int PARTS>
 __global__ __launch_bounds__(256) void gm_dz(RowArgs a, const T* dout, const T* W2, const T* hidden,
                                              float* dz, float* act) {
     __shared__ __align__(16) float As[tile_words<kRT, kKC, true>()];
@@ -385,7 +390,7 @@ __global__ __launch_bounds__(256) void gm_dz(RowArgs a, const T* dout, const T* 
                 }
     }
     v4f acc[kRT / 32][2] = {};
-    tile_product<kRT, kKC, true, true>(
+    tile_product<kRT, kKC, true, true, PARTS>(
         [&](int x, int k) { return x < n && k < d ? load4(dout + int64_t(rows[x]) * d + k) : zero4(); },
         [&](int x, int k) { return h0 + x < H && k < d ? load4(W + int64_t(x) * d + k) : zero4(); },
         d, As, Bs, acc, NoStep{});
@@ -410,7 +415,7 @@ __global__ __launch_bounds__(256) void gm_dz(RowArgs a, const T* dout, const T* 
             }
 }
 
-template <typename T>
+template <typename T, int PARTS>
 __global__ __launch_bounds__(256) void gm_dv(RowArgs a, const float* dz, const T* W1, T* dv) {
     __shared__ __align__(16) float As[tile_words<kRT, kKC, true>()];
     __shared__ __align__(16) float Bs[tile_words<kNT, kKC, true>()];
@@ -422,7 +427,7 @@ __global__ __launch_bounds__(256) void gm_dv(RowArgs a, const float* dz, const T
     const T* W = W1 + (int64_t(j) * in + c0) * H;
     const float* A = dz + int64_t(r0) * H;
     v4f acc[kRT / 32][2] = {};
-    tile_product<kRT, kKC, true, true>(
+    tile_product<kRT, kKC, true, true, PARTS>(
         [&](int x, int k) { return x < n && k < H ? load4(A + int64_t(x) * H + k) : zero4(); },
         [&](int x, int k) { return c0 + x < in && k < H ? load4(W + int64_t(x) * H + k) : zero4(); },
         H, As, Bs, acc, NoStep{});
@@ -611,6 +616,17 @@ RowArgs row_args(const Layout& L, char* ws, int d, int H) {
                    reinterpret_cast<int32_t*>(ws + L.tile), reinterpret_cast<int32_t*>(ws + L.row0), d, H};
 }
 
+// The row tiles' sums a step (tile_product) by the reduction's length. Errors against 64 bits in
+// fp32, the kernels without a workspace, one sum, four (P 2000): z1 at d 16 (K 64) 0.88e-7, 1.46e-7,
+// 0.87e-7, at d 32 (K 128) 1.13e-7, 1.49e-7, 0.91e-7; out at H 64 1.75e-7, 2.20e-7, 1.32e-7. Beyond
+// K = 128 one sum a step is no further off than those kernels (z1 at d 64 1.51e-7 both), and four
+// cost registers: P 8192, d 64, H 512 in bf16 hidden 45.7 -> 52.1 us, dv 39.4 -> 47.7.
+template <class F>
+void by_reduction(int K, const F& f) {
+    if (K <= 128) f(std::integral_constant<int, 4>{});
+    else f(std::integral_constant<int, 1>{});
+}
+
 template <typename T>
 struct Forward {
     static void run(const void* v, const void* unit_idx, int index_bits, const void* W1, const void* b1,
@@ -620,12 +636,16 @@ struct Forward {
         order_pairs(unit_idx, index_bits, L, ws, P, M, st);
         const RowArgs a = row_args(L, ws, d, H);
         float* act = reinterpret_cast<float*>(ws + L.act);
-        hipLaunchKernelGGL((gm_hidden<T>), dim3(L.tiles, (H + 63) / 64), dim3(256), 0, st, a,
-                           static_cast<const T*>(v), static_cast<const T*>(W1),
-                           static_cast<const T*>(b1), static_cast<T*>(hidden), act);
+        by_reduction(4 * d, [&](auto parts) {
+            hipLaunchKernelGGL((gm_hidden<T, decltype(parts)::value>), dim3(L.tiles, (H + 63) / 64), dim3(256), 0, st, a,
+                               static_cast<const T*>(v), static_cast<const T*>(W1),
+                               static_cast<const T*>(b1), static_cast<T*>(hidden), act);
+        });
         HSN_HIP(hipGetLastError());
-        hipLaunchKernelGGL((gm_out<T>), dim3(L.tiles, (d + 63) / 64), dim3(256), 0, st, a, act,
-                           static_cast<const T*>(W2), static_cast<const T*>(b2), static_cast<T*>(out));
+        by_reduction(H, [&](auto parts) {
+            hipLaunchKernelGGL((gm_out<T, decltype(parts)::value>), dim3(L.tiles, (d + 63) / 64), dim3(256), 0, st, a, act,
+                               static_cast<const T*>(W2), static_cast<const T*>(b2), static_cast<T*>(out));
+        });
         HSN_HIP(hipGetLastError());
     }
 };
@@ -639,12 +659,16 @@ struct Backward {
         order_pairs(unit_idx, index_bits, L, ws, P, M, st);
         const RowArgs ra = row_args(L, ws, d, H);
         float *act = reinterpret_cast<float*>(ws + L.act), *dz = reinterpret_cast<float*>(ws + L.dz);
-        hipLaunchKernelGGL((gm_dz<T>), dim3(L.tiles, (H + 63) / 64), dim3(256), 0, st, ra,
-                           static_cast<const T*>(dout), static_cast<const T*>(W2),
-                           static_cast<const T*>(hidden), dz, act);
+        by_reduction(d, [&](auto parts) {
+            hipLaunchKernelGGL((gm_dz<T, decltype(parts)::value>), dim3(L.tiles, (H + 63) / 64), dim3(256), 0, st, ra,
+                               static_cast<const T*>(dout), static_cast<const T*>(W2),
+                               static_cast<const T*>(hidden), dz, act);
+        });
         HSN_HIP(hipGetLastError());
-        hipLaunchKernelGGL((gm_dv<T>), dim3(L.tiles, (4 * d + 63) / 64), dim3(256), 0, st, ra, dz,
-                           static_cast<const T*>(W1), static_cast<T*>(dv));
+        by_reduction(H, [&](auto parts) {
+            hipLaunchKernelGGL((gm_dv<T, decltype(parts)::value>), dim3(L.tiles, (4 * d + 63) / 64), dim3(256), 0, st, ra, dz,
+                               static_cast<const T*>(W1), static_cast<T*>(dv));
+        });
         HSN_HIP(hipGetLastError());
         const DwArgs a{reinterpret_cast<int32_t*>(ws + L.perm), reinterpret_cast<int32_t*>(ws + L.first),
                        reinterpret_cast<int32_t*>(ws + L.block), reinterpret_cast<int32_t*>(ws + L.bfirst),

@@ -606,3 +606,34 @@ def test_unit_mlp_by_either_kernels_matches_oracle(ops, cuda_device, monkeypatch
     for name, g_, w_ in zip(("dW1", "db1", "dW2", "db2"), got[1:], want[1:]):
         err = (g_.double().cpu() - w_).abs() / w_.abs().clamp(min=1.0)
         assert float(err.max()) <= bar, f"{name}: worst {float(err.max()):.3e} (bar {bar:.1e})"
+
+
+def _four_shares(x, W, b):
+    """``x @ W + b`` as four running fp32 sums of a quarter of the reduction each, added in order."""
+    K, total = x.shape[1], None
+    for s in range(4):
+        acc = torch.zeros(x.shape[0], W.shape[1], device=x.device)
+        for k in range(s * K // 4, (s + 1) * K // 4):
+            acc = (acc.double() + x[:, k:k + 1].double() * W[k].double()).float()
+        total = acc if total is None else total + acc
+    return total + b
+
+
+@pytest.mark.parametrize("path", ["unit order", "by rows"])
+@pytest.mark.parametrize("d,H", [(4, 64), (16, 64), (16, 512), (32, 64), (64, 64), (64, 512)])
+def test_unit_mlp_sums_are_no_further_off_than_four_running_sums(ops, cuda_device, monkeypatch, d, H, path):
+    """In fp32 both layers' results are no further from 64 bits than four running sums of a quarter of
+    the reduction each leave them on the same inputs; the errors are norms over 2000 pairs, whose
+    chance leaves 5%."""
+    x = _mlp_problem(2000, 1, d, H, torch.float32, d + H, cuda_device)
+    _through(monkeypatch, ops, path)
+    out, hidden = ops.mlp_op(x["v"], x["idx"], x["W1"], x["b1"], x["W2"], x["b2"])
+    gelu = lambda z: 0.5 * z * (1 + torch.erf(z * 0.5 ** 0.5))  # noqa: E731
+    c = {k: x[k].double() if x[k].dim() < 3 else x[k][0].double() for k in ("v", "W1", "b1", "W2", "b2")}
+    want_z = c["v"] @ c["W1"] + c["b1"]
+    want = gelu(want_z) @ c["W2"] + c["b2"]
+    z = _four_shares(x["v"], x["W1"][0], x["b1"])
+    y = _four_shares(gelu(z.double()).float(), x["W2"][0], x["b2"])
+    off = lambda a, b: float((a.double() - b).norm() / b.norm())  # noqa: E731
+    assert off(hidden, want_z) <= 1.05 * off(z, want_z)
+    assert off(out, want) <= 1.05 * off(y, want)
