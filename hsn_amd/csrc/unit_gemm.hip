@@ -72,6 +72,7 @@ struct Order {
     int32_t* row0;   // [tiles]: its first row
     int32_t* block;  // [blocks]: a weight-gradient block's unit, or -1 past the last
     int32_t* bfirst; // [M + 1]: a unit's first block (every unit has one, also without pairs)
+    int32_t* pfirst; // [M]: the first partial sum of a unit of more than one block
     int P, M, tiles, RB, blocks;
 };
 
@@ -79,7 +80,7 @@ template <typename I>
 __global__ __launch_bounds__(64 * kSortWaves) void unit_order(const I* unit_idx, Order o) {
     extern __shared__ int lds_i[];
     int* cnt = lds_i;                      // [kSortWaves][M]: counts, then the next row
-    int* part = cnt + kSortWaves * o.M;    // [3][kSortWaves]
+    int* part = cnt + kSortWaves * o.M;    // [4][kSortWaves]
     const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
     const int P = o.P, M = o.M;
     for (int i = tid; i < kSortWaves * M; i += 64 * kSortWaves) cnt[i] = 0;
@@ -110,16 +111,21 @@ __global__ __launch_bounds__(64 * kSortWaves) void unit_order(const I* unit_idx,
         for (int q = 0; q < kSortWaves; ++q) n += cnt[q * M + tid];
     const int nt = (n + kRT - 1) / kRT;
     const int nb = tid < M ? max(1, (n + o.RB - 1) / o.RB) : 0;
-    int in = n, it = nt, ib = nb;
+    const int np = nb > 1 ? nb : 0;  // partial sums
+    int in = n, it = nt, ib = nb, ip = np;
     for (int s = 1; s < 64; s <<= 1) {
-        const int a = __shfl_up(in, s, 64), b = __shfl_up(it, s, 64), c = __shfl_up(ib, s, 64);
-        if (lane >= s) in += a, it += b, ib += c;
+        const int a = __shfl_up(in, s, 64), b = __shfl_up(it, s, 64), c = __shfl_up(ib, s, 64),
+                  e = __shfl_up(ip, s, 64);
+        if (lane >= s) in += a, it += b, ib += c, ip += e;
     }
-    if (lane == 63) part[w] = in, part[kSortWaves + w] = it, part[2 * kSortWaves + w] = ib;
+    if (lane == 63)
+        part[w] = in, part[kSortWaves + w] = it, part[2 * kSortWaves + w] = ib, part[3 * kSortWaves + w] = ip;
     __syncthreads();
-    int before = 0, tbefore = 0, bbefore = 0, all = 0, ball = 0;
+    int before = 0, tbefore = 0, bbefore = 0, pbefore = 0, all = 0, ball = 0;
     for (int q = 0; q < kSortWaves; ++q) {
-        if (q < w) before += part[q], tbefore += part[kSortWaves + q], bbefore += part[2 * kSortWaves + q];
+        if (q < w)
+            before += part[q], tbefore += part[kSortWaves + q], bbefore += part[2 * kSortWaves + q],
+                pbefore += part[3 * kSortWaves + q];
         all += part[kSortWaves + q];
         ball += part[2 * kSortWaves + q];
     }
@@ -127,6 +133,7 @@ __global__ __launch_bounds__(64 * kSortWaves) void unit_order(const I* unit_idx,
         const int f = before + in - n, t = tbefore + it - nt, bl = bbefore + ib - nb;
         o.first[tid] = f;
         o.bfirst[tid] = bl;
+        o.pfirst[tid] = pbefore + ip - np;
         if (tid == M - 1) o.first[M] = f + n, o.bfirst[M] = bl + nb;
         int at = f;
         for (int q = 0; q < kSortWaves; ++q) {
@@ -441,8 +448,8 @@ __global__ __launch_bounds__(256) void gm_dv(RowArgs a, const float* dz, const T
 // ------------------------------------------------------------------------------------------
 
 struct DwArgs {
-    const int32_t *perm, *first, *block, *bfirst;
-    float* part;  // [blocks][unit_floats]: the partial sums (W1, b1, W2, b2) of a split unit's blocks
+    const int32_t *perm, *first, *block, *bfirst, *pfirst;
+    float* part;  // [2 (P / RB)][unit_floats]: the partial sums (W1, b1, W2, b2) of the split units' blocks
     int d, H, RB;
     __host__ __device__ int64_t unit_floats() const {
         return int64_t(4) * d * H + H + int64_t(H) * d + d;
@@ -488,7 +495,8 @@ __global__ __launch_bounds__(256) void gm_dw(DwArgs a, const T* v, const float* 
             [&](int x, int k) { return k < n && x0 + x < nr ? load4(v + int64_t(rows[k]) * in + x0 + x) : zero4(); },
             [&](int x, int k) { return k < n && c0 + x < nc ? load4(dz + int64_t(r0 + k) * H + c0 + x) : zero4(); },
             n, As, Bs, acc, add);
-    float* part = a.part + int64_t(bl) * a.unit_floats() + (second ? int64_t(in) * H + H : 0);
+    float* part = a.part + int64_t(a.pfirst[j] + (bl - a.bfirst[j])) * a.unit_floats() +
+                  (second ? int64_t(in) * H + H : 0);
     T* dW = second ? dW2 + int64_t(j) * H * d : dW1 + int64_t(j) * in * H;
     each_result<64>(acc, [&](int x, int c, float q) {
         if (x0 + x >= nr || c0 + c >= nc) return;
@@ -514,12 +522,12 @@ __global__ __launch_bounds__(256) void gm_dw(DwArgs a, const T* v, const float* 
 template <typename T>
 __global__ __launch_bounds__(256) void gm_dw_sum(DwArgs a, T* dW1, T* db1, T* dW2, T* db2) {
     const int j = blockIdx.y;
-    const int b0 = a.bfirst[j], blocks = a.bfirst[j + 1] - b0;
+    const int p0 = a.pfirst[j], blocks = a.bfirst[j + 1] - a.bfirst[j];
     if (blocks <= 1) return;
     const int64_t u = a.unit_floats(), n1 = int64_t(4) * a.d * a.H, n2 = int64_t(a.H) * a.d;
     for (int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x; i < u; i += int64_t(gridDim.x) * 256) {
         float q = 0.0f;
-        for (int s = 0; s < blocks; ++s) q += a.part[int64_t(b0 + s) * u + i];
+        for (int s = 0; s < blocks; ++s) q += a.part[int64_t(p0 + s) * u + i];
         if (i < n1) store_f32(dW1, j * n1 + i, q);
         else if (i < n1 + a.H) store_f32(db1, int64_t(j) * a.H + (i - n1), q);
         else if (i < n1 + a.H + n2) store_f32(dW2, j * n2 + (i - n1 - a.H), q);
@@ -537,7 +545,7 @@ __global__ __launch_bounds__(256) void gm_dw_sum(DwArgs a, T* dW1, T* db1, T* dW
 // workgroups a CU measured 57.5 + 14.4 us (the partial sums' pass) against 68 + 4.6 at P 8192,
 // M 8, d 64, H 512 in bf16, and 30.0 + 12.5 against 31.2 at P 4096 in fp32.
 int block_rows(int P, int M, int d, int H) {
-    const DwArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, d, H, 0};
+    const DwArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, d, H, 0};
     const int64_t tiles = a.tiles1() + a.tiles2();
     const int64_t want = M * tiles >= 256 ? 2 * int64_t(P) / M : P * tiles / 512;
     return static_cast<int>(std::min<int64_t>(4096, std::max<int64_t>(256, (want + 63) / 64 * 64)));
@@ -546,7 +554,7 @@ int block_rows(int P, int M, int d, int H) {
 inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 struct Layout {
-    size_t perm, first, tile, row0, block, bfirst, act, dz, part, bytes;
+    size_t perm, first, tile, row0, block, bfirst, pfirst, act, dz, part, bytes;
     int tiles, RB, blocks;
 };
 Layout layout(int P, int M, int d, int H, bool backward) {
@@ -562,11 +570,13 @@ Layout layout(int P, int M, int d, int H, bool backward) {
     L.row0 = take(size_t(L.tiles) * 4);
     L.block = take(size_t(L.blocks) * 4);
     L.bfirst = take(size_t(M + 1) * 4);
+    L.pfirst = take(size_t(M) * 4);
     L.act = take(size_t(P) * H * 4);
     if (backward) {
         L.dz = take(size_t(P) * H * 4);
-        const DwArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, d, H, L.RB};
-        L.part = take(P > L.RB ? size_t(L.blocks) * a.unit_floats() * 4 : 0);
+        const DwArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, d, H, L.RB};
+        // a unit of n > RB pairs has at most 2 (n / RB) blocks; the others write their gradients
+        L.part = take(size_t(2) * (P / L.RB) * a.unit_floats() * 4);
     }
     L.bytes = at;
     return L;
@@ -600,8 +610,8 @@ void order_pairs(const void* unit_idx, int index_bits, const Layout& L, char* ws
     const Order o{reinterpret_cast<int32_t*>(ws + L.perm), reinterpret_cast<int32_t*>(ws + L.first),
                   reinterpret_cast<int32_t*>(ws + L.tile), reinterpret_cast<int32_t*>(ws + L.row0),
                   reinterpret_cast<int32_t*>(ws + L.block), reinterpret_cast<int32_t*>(ws + L.bfirst),
-                  P, M, L.tiles, L.RB, L.blocks};
-    const size_t lds = (size_t(kSortWaves) * M + 3 * kSortWaves) * 4;
+                  reinterpret_cast<int32_t*>(ws + L.pfirst), P, M, L.tiles, L.RB, L.blocks};
+    const size_t lds = (size_t(kSortWaves) * M + 4 * kSortWaves) * 4;
     auto launch = [&](auto kernel, auto* idx) {
         if (lds > 64 * 1024) HSN_HIP(allow_lds_raw(reinterpret_cast<const void*>(kernel), lds));
         hipLaunchKernelGGL(kernel, dim3(1), dim3(64 * kSortWaves), lds, st, idx, o);
@@ -672,7 +682,8 @@ struct Backward {
         HSN_HIP(hipGetLastError());
         const DwArgs a{reinterpret_cast<int32_t*>(ws + L.perm), reinterpret_cast<int32_t*>(ws + L.first),
                        reinterpret_cast<int32_t*>(ws + L.block), reinterpret_cast<int32_t*>(ws + L.bfirst),
-                       reinterpret_cast<float*>(ws + L.part), d, H, L.RB};
+                       reinterpret_cast<int32_t*>(ws + L.pfirst), reinterpret_cast<float*>(ws + L.part),
+                       d, H, L.RB};
         const size_t lds = (tile_words<64, kKC, false>() + tile_words<kNT, kKC, false>() + L.RB) * 4;
         auto kernel = &gm_dw<T>;
         if (lds > 64 * 1024) HSN_HIP(allow_lds_raw(reinterpret_cast<const void*>(kernel), lds));

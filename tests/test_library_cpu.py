@@ -417,3 +417,24 @@ def test_device_pointers_refuse_host_tensors():
     assert _lib.ptr(None) is None
     with pytest.raises(ValueError, match="ROCm device"):
         _lib.ptr(torch.zeros(3))
+
+
+def test_unit_mlp_workspace_holds_partial_sums_of_split_units_only():
+    """The backward's workspace is the pairs' rows (two of H floats each) and partial sums for units
+    of more pairs than a block, of which there can be at most 2 (P / block): a large bank with few
+    pairs a unit takes no more than its pairs."""
+    import ctypes
+
+    from hsn_amd import _lib
+
+    def space(P, M, d, H, backward=1):
+        out = ctypes.c_int64(0)
+        _lib.call("hsn_grouped_unit_mlp_workspace", P, M, d, H, 0, backward, ctypes.byref(out))
+        return out.value
+
+    unit = 4 * (4 * 64 * 512 + 512 + 512 * 64 + 64)  # one unit's weight gradients in fp32
+    lists = lambda P, M: 4 * (4 * P + 8 * M) + 8192  # noqa: E731
+    for P, M in ((300, 1024), (255, 1024), (2000, 1024), (8192, 8)):
+        blocks = P // 256  # a block holds 256 pairs or more
+        assert space(P, M, 64, 512) <= 2 * 4 * P * 512 + 2 * blocks * unit + lists(P, M), (P, M)
+    assert space(300, 1024, 64, 512) < 4 << 20
