@@ -368,14 +368,18 @@ def _mlp_space(P: int, M: int, d: int, H: int, backward: int, idx: Tensor, v: Te
                *operands: Tensor) -> Optional[tuple[Tensor, int, Tensor, int]]:
     """``(idx, its bits, workspace, bytes)`` of a call of the products in unit order, or ``None``
     where the kernels without a workspace take it: another shape, a forward of few pairs, operands
-    off four-element alignment (a view into a buffer), or indices neither int32 nor int64."""
+    off four-element alignment (a view into a buffer), indices neither int32 nor int64, or no
+    memory left for a workspace."""
     if idx.dtype not in (torch.int32, torch.int64):
         return None
     nbytes = _mlp_workspace_bytes(P, M, d, H, _code(v), backward)
     step = 4 * v.element_size()
     if nbytes == 0 or any(t.data_ptr() % step for t in (v, *operands)):
         return None
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=v.device)
+    try:
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=v.device)
+    except torch.OutOfMemoryError:
+        return None
     return idx.contiguous(), 64 if idx.dtype == torch.int64 else 32, ws, nbytes
 
 

@@ -637,3 +637,21 @@ def test_unit_mlp_sums_are_no_further_off_than_four_running_sums(ops, cuda_devic
     off = lambda a, b: float((a.double() - b).norm() / b.norm())  # noqa: E731
     assert off(hidden, want_z) <= 1.05 * off(z, want_z)
     assert off(out, want) <= 1.05 * off(y, want)
+
+
+def test_unit_mlp_without_memory_for_a_workspace(ops, cuda_device, monkeypatch):
+    """Where no workspace can be had the kernels over rows take the call: a bank that fits the memory
+    runs, with the same results up to the order of the fp32 sums."""
+    x = _mlp_problem(600, 4, 16, 64, torch.float32, 9, cuda_device)
+    out, hidden, got = _mlp_run(ops, x)
+    real = torch.empty
+
+    def full(*size, **kw):
+        if kw.get("dtype") == torch.uint8:
+            raise torch.OutOfMemoryError("no memory")
+        return real(*size, **kw)
+
+    monkeypatch.setattr(ops.torch, "empty", full)
+    out2, hidden2, got2 = _mlp_run(ops, x)
+    for a, b in zip((out, hidden, *got), (out2, hidden2, *got2)):
+        torch.testing.assert_close(a, b, atol=2e-5, rtol=2e-5)
