@@ -41,7 +41,6 @@ using units::gelu_grad;
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int kMaxUnits = 1024;  // LDS counts of a unit per wavefront of unit_order: 64 KiB
-constexpr int kSortWaves = 16;
 constexpr int kRT = 32;  // rows of a row tile
 constexpr int kNT = 64;  // columns of a tile
 constexpr int kKC = 64;  // reduction indices a step
@@ -76,7 +75,7 @@ struct Order {
     int P, M, tiles, RB, blocks;
 };
 
-template <typename I>
+template <typename I, int kSortWaves>
 __global__ __launch_bounds__(64 * kSortWaves) void unit_order(const I* unit_idx, Order o) {
     extern __shared__ int lds_i[];
     int* cnt = lds_i;                      // [kSortWaves][M]: counts, then the next row
@@ -611,14 +610,23 @@ void order_pairs(const void* unit_idx, int index_bits, const Layout& L, char* ws
                   reinterpret_cast<int32_t*>(ws + L.tile), reinterpret_cast<int32_t*>(ws + L.row0),
                   reinterpret_cast<int32_t*>(ws + L.block), reinterpret_cast<int32_t*>(ws + L.bfirst),
                   reinterpret_cast<int32_t*>(ws + L.pfirst), P, M, L.tiles, L.RB, L.blocks};
-    const size_t lds = (size_t(kSortWaves) * M + 4 * kSortWaves) * 4;
+    // One wavefront for up to 128 pairs and 64 units: 2.8 us against sixteen wavefronts' 4.7 (P 64, M 8);
+    // a step of 64 pairs goes through its units in turn, so more pairs than two steps do not gain
+    // (P 512, M 32: the forward 41 us against 33).
+    const int waves = P <= 128 && M <= 64 ? 1 : 16;
+    const size_t lds = (size_t(waves) * M + 4 * waves) * 4;
     auto launch = [&](auto kernel, auto* idx) {
         if (lds > 64 * 1024) HSN_HIP(allow_lds_raw(reinterpret_cast<const void*>(kernel), lds));
-        hipLaunchKernelGGL(kernel, dim3(1), dim3(64 * kSortWaves), lds, st, idx, o);
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(64 * waves), lds, st, idx, o);
         HSN_HIP(hipGetLastError());
     };
-    if (index_bits == 64) launch(&unit_order<int64_t>, static_cast<const int64_t*>(unit_idx));
-    else launch(&unit_order<int32_t>, static_cast<const int32_t*>(unit_idx));
+    auto by_waves = [&](auto* idx) {
+        using I = std::remove_const_t<std::remove_pointer_t<decltype(idx)>>;
+        if (waves == 1) launch(&unit_order<I, 1>, idx);
+        else launch(&unit_order<I, 16>, idx);
+    };
+    if (index_bits == 64) by_waves(static_cast<const int64_t*>(unit_idx));
+    else by_waves(static_cast<const int32_t*>(unit_idx));
 }
 
 RowArgs row_args(const Layout& L, char* ws, int d, int H) {
@@ -684,9 +692,8 @@ struct Backward {
                        reinterpret_cast<int32_t*>(ws + L.block), reinterpret_cast<int32_t*>(ws + L.bfirst),
                        reinterpret_cast<int32_t*>(ws + L.pfirst), reinterpret_cast<float*>(ws + L.part),
                        d, H, L.RB};
-        const size_t lds = (tile_words<64, kKC, false>() + tile_words<kNT, kKC, false>() + L.RB) * 4;
+        const size_t lds = (tile_words<64, kKC, false>() + tile_words<kNT, kKC, false>() + L.RB) * 4;  // <= 50 KiB
         auto kernel = &gm_dw<T>;
-        if (lds > 64 * 1024) HSN_HIP(allow_lds_raw(reinterpret_cast<const void*>(kernel), lds));
         hipLaunchKernelGGL(kernel, dim3(a.tiles1() + a.tiles2(), L.blocks), dim3(256), lds, st, a,
                            static_cast<const T*>(v), dz, act, static_cast<const T*>(dout),
                            static_cast<T*>(dW1), static_cast<T*>(db1), static_cast<T*>(dW2),
