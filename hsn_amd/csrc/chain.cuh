@@ -1221,10 +1221,51 @@ __device__ __forceinline__ void store4(const float (&x)[4], rsrc_t r, uint32_t v
     __builtin_amdgcn_raw_buffer_store_b64(v, r, vo, 0u, 0);
 }
 
-// LDS words of a quad workgroup: chain_words, and the maxima's two coarse scales.
+// LDS words of a quad workgroup: chain_words, the maxima's two coarse scales and the order's bins.
+constexpr int kLightBins = 65, kHeavyBins = 72, kOrderBins = kHeavyBins + kLightBins;
 __host__ __device__ inline int coarse_words(int T) { return (T + 15) / 16 + (T + 255) / 256; }
 __host__ __device__ inline int quad_words(int T, int C, int stage) {
-    return chain_words(T, C, stage) + coarse_words(T);
+    return chain_words(T, C, stage) + coarse_words(T) + kOrderBins;
+}
+
+// The group's cells by events, most first, into order[0 .. nc): exactly by their number up to kHeavy of
+// them, by a quarter of a power of two above; within a bin in any order, on which nothing depends (a
+// cell's chain is its own, the maxima are integers'). A counting sort: heavy_first compares every
+// pair of cells, 10 us of a workgroup of 1024. cptr must be visible to every thread; ends with a barrier.
+__device__ __forceinline__ void order_cells(const int* cptr, int nc, int* order, int* bins, int tid) {
+    auto bin = [&](int i) __attribute__((always_inline)) {
+        const int n = cptr[i + 1] - cptr[i];
+        if (n <= kHeavy) return kHeavyBins + kHeavy - n;
+        const int e = 31 - __builtin_clz(n);  // 6 .. 23 (T < 2^23)
+        return kHeavyBins - 1 - (4 * (e - 6) + ((n >> (e - 2)) & 3));
+    };
+    for (int i = tid; i < kOrderBins; i += kQuadThreads) bins[i] = 0;
+    __syncthreads();
+    for (int i = tid; i < nc; i += kQuadThreads) atomicAdd(&bins[bin(i)], 1);
+    __syncthreads();
+    if (tid < kWave) {  // the bins' first places
+        constexpr int kPer = (kOrderBins + kWave - 1) / kWave;
+        int n[kPer], own = 0;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            n[i] = kPer * tid + i < kOrderBins ? bins[kPer * tid + i] : 0;
+            own += n[i];
+        }
+        int at = own;
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int u = __shfl_up(at, o, kWave);
+            if (tid >= o) at += u;
+        }
+        at -= own;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            if (kPer * tid + i < kOrderBins) bins[kPer * tid + i] = at;
+            at += n[i];
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < nc; i += kQuadThreads) order[atomicAdd(&bins[bin(i)], 1)] = i;
+    __syncthreads();
 }
 
 // val into the maxima of positions [p0, p1), by the L lanes of a group.
@@ -1249,7 +1290,7 @@ __device__ __forceinline__ void mark(uint32_t* hm, uint32_t* hc, uint32_t* hs, i
     mark_run<L>(hs, ca / 16, cb / 16, val, l);
 }
 
-// The cells of more than kHeavy events: the first of the order (heaviest first).
+// The cells of more than kHeavy events: the first of the order.
 __device__ __forceinline__ int heavy_cells(const int* cptr, const int* order, int nc) {
     int lo = 0, hi = nc;
     while (lo < hi) {
@@ -1279,6 +1320,7 @@ __global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
     int* order = cev + a.stage;                               // [C]
     uint32_t* hc = reinterpret_cast<uint32_t*>(order + a.C);  // [(T + 15) / 16]
     uint32_t* hs = hc + (T + 15) / 16;                        // [(T + 255) / 256]
+    int* bins = reinterpret_cast<int*>(hs + (T + 255) / 256);  // [kOrderBins]
     const int c_begin = g * a.C, c_end = min(N, c_begin + a.C);
     const int nc = c_end - c_begin;
     const int32_t* ptr = a.ptr + int64_t(b) * (N + 1);
@@ -1295,7 +1337,7 @@ __global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
     if (tid == 0) next[0] = 0;
     const int lrT = reset_table(a.reset ? a.reset + int64_t(b) * T : nullptr, T, nr, rbits, nx,
                                 tid, kQuadThreads);
-    heavy_first(cptr, nc, order, tid, kQuadThreads);
+    order_cells(cptr, nc, order, bins, tid);
     const int64_t slot0 = int64_t(b) * T * K;
     const uint32_t row_bytes = uint32_t(T) * K * d * sizeof(IO);
     const IO* kind = nullptr;
@@ -1628,6 +1670,7 @@ __global__ __launch_bounds__(kQuadThreads, sizeof(IO) == 4 ? 4 : 5) void chain_b
     int* cptr = next + 1;
     int* cev = cptr + a.C + 1;
     int* order = cev + a.stage;
+    int* bins = order + a.C + coarse_words(T);
     const int c_begin = g * a.C, c_end = min(N, c_begin + a.C);
     const int nc = c_end - c_begin;
     const int32_t* ptr = a.ptr + int64_t(b) * (N + 1);
@@ -1638,7 +1681,7 @@ __global__ __launch_bounds__(kQuadThreads, sizeof(IO) == 4 ? 4 : 5) void chain_b
     for (int i = tid; i < nst; i += kQuadThreads) cev[i] = ev[pc0 + i];
     if (tid == 0) next[0] = 0;
     reset_table(a.reset ? a.reset + int64_t(b) * T : nullptr, T, nr, rbits, nx, tid, kQuadThreads);
-    heavy_first(cptr, nc, order, tid, kQuadThreads);
+    order_cells(cptr, nc, order, bins, tid);
     const int64_t slot0 = int64_t(b) * T * K;
     const uint32_t row_bytes = uint32_t(T) * K * d * sizeof(IO);
     const IO* kind = nullptr;

@@ -29,8 +29,7 @@ inline int chain_cells(int B, int N) {
 }
 
 // The same for the kernels that walk several cells a wavefront: about 512 workgroups of eight
-// wavefronts, two a CU, which the registers hold at once; at most 1024 cells (heavy_first's
-// comparisons grow with their square).
+// wavefronts, two a CU, which the registers hold at once; at most 1024 cells.
 inline int quad_cells(int B, int N) {
     int C = 32;
     while (C < N && C < 1024 && int64_t(B) * ((N + C - 1) / C) > 512) C *= 2;
