@@ -1165,7 +1165,7 @@ __global__ __launch_bounds__(kChainThreads) void chain_bwd(BwdArgs a) {
 // The chains, several cells a wavefront (chain_fwd4, chain_bwd4)
 // ------------------------------------------------------------------------------------------
 //
-// For d a multiple of 4 up to 256 and rows aligned to four elements, a cell's columns lie in L
+// For d a multiple of 4 up to 128 and rows aligned to four elements, a cell's columns lie in L
 // lanes, four a lane (16-byte accesses of fp32 rows, 8-byte ones of bf16), and a wavefront walks
 // 64 / L cells side by side, so one instruction serves an event of each. The cells are taken
 // heaviest first, so neighbours hold about as many events; a lane whose cell has no event left
@@ -1370,7 +1370,7 @@ __global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
     // one cell by the whole wavefront, a column a lane and register (lane + 64 v): the cells of more
     // than kHeavy events, whose chain a wavefront of several cells would walk more slowly, and cell
     // 0 where the row has padded slots
-    constexpr int V = L <= 16 ? 1 : L / 16;
+    constexpr int V = L <= 16 ? 1 : 2;
     constexpr bool want_max = HMAX;
     uint32_t voff[V], voff4[V];
 #pragma unroll
@@ -1703,7 +1703,7 @@ __global__ __launch_bounds__(kQuadThreads, sizeof(IO) == 4 ? 4 : 5) void chain_b
                                   a.dh0 ? uint32_t(N) * srow4 : 0u);
     const int nr0 = nr[0];
 
-    constexpr int V = L <= 16 ? 1 : L / 16;
+    constexpr int V = L <= 16 ? 1 : 2;
     uint32_t voff[V], voff4[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
