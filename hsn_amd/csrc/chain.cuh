@@ -1511,6 +1511,7 @@ __global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
     };
 
     const int heavy = heavy_cells(cptr, order, nc);
+    if (pads && g == 0 && tid < kWave) single(std::true_type{}, 0);  // first: it has the padded slots too
     uint32_t idle = 0u;  // the largest |h| of the cells without an event (this lane's columns)
     for (;;) {
         int item = lane == 0 ? atomicAdd(next, 1) : 0;  // a heavy cell, or the next Q light ones
@@ -1643,7 +1644,6 @@ __global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
         const uint32_t v = wave_max_from_groups<1>(idle);
         if (lane < L) mark<L>(hm, hc, hs, 0, min(T, nr0), v, l);
     }
-    if (pads && g == 0 && tid < kWave) single(std::true_type{}, 0);
     if (a.pos_T && g == 0 && tid == 0) a.pos_T[b] = lrT >= 0 ? int64_t(T - lrT) : a.pos0[b] + T;
     if constexpr (HMAX) {  // the group's maxima, reduced over the groups by summary_delta
         __syncthreads();
