@@ -519,6 +519,7 @@ struct FwdArgs {
     int64_t* pos_T;        // [B] (optional)
     int B, T, N, d, K;
     int C, stage;  // cells per workgroup, staged events per workgroup
+    int heavy;     // chain_fwd4: cells of more events are walked alone
 };
 
 template <typename IO, int V>
@@ -983,7 +984,7 @@ struct BwdArgs {
     void* dg;
     float* dh0;  // optional
     int B, T, N, d, K;
-    int C, stage;
+    int C, stage, heavy;
 };
 
 // Per cell, latest event first (python/hsn/train/split.py:154-173): with the cotangent A of the
@@ -1188,7 +1189,7 @@ __global__ __launch_bounds__(kChainThreads) void chain_bwd(BwdArgs a) {
 
 constexpr int kQuadWaves = 8;
 constexpr int kQuadThreads = 64 * kQuadWaves;
-constexpr int kHeavy = 64;
+constexpr int kHeavy = 64;  // and the limit of FwdArgs / BwdArgs::heavy
 constexpr int NB = 2;  // events of a cell in a batch, two batches in flight
 
 struct RawB { uint32_t v[2]; };  // four bf16
@@ -1290,12 +1291,12 @@ __device__ __forceinline__ void mark(uint32_t* hm, uint32_t* hc, uint32_t* hs, i
     mark_run<L>(hs, ca / 16, cb / 16, val, l);
 }
 
-// The cells of more than kHeavy events: the first of the order.
-__device__ __forceinline__ int heavy_cells(const int* cptr, const int* order, int nc) {
+// The cells of more than `heavy` events (at most kHeavy): the first of the order.
+__device__ __forceinline__ int heavy_cells(const int* cptr, const int* order, int nc, int heavy) {
     int lo = 0, hi = nc;
     while (lo < hi) {
         const int mid = (lo + hi) >> 1, ci = order[mid];
-        if (cptr[ci + 1] - cptr[ci] > kHeavy) lo = mid + 1;
+        if (cptr[ci + 1] - cptr[ci] > heavy) lo = mid + 1;
         else hi = mid;
     }
     return uniform(lo);
@@ -1510,7 +1511,7 @@ __global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
         if (a.age_T && lane == 0) end_age(c, tprev);
     };
 
-    const int heavy = heavy_cells(cptr, order, nc);
+    const int heavy = heavy_cells(cptr, order, nc, a.heavy);
     if (pads && g == 0 && tid < kWave) single(std::true_type{}, 0);  // first: it has the padded slots too
     uint32_t idle = 0u;  // the largest |h| of the cells without an event (this lane's columns)
     for (;;) {
@@ -1813,7 +1814,7 @@ __global__ __launch_bounds__(kQuadThreads, sizeof(IO) == 4 ? 4 : 5) void chain_b
                 if (lane + 64 * v < d) d0[lane + 64 * v] = z ? 0.0f : A[v];
         }
     };
-    const int heavy = heavy_cells(cptr, order, nc);
+    const int heavy = heavy_cells(cptr, order, nc, a.heavy);
 
     for (;;) {
         int item = lane == 0 ? atomicAdd(next, 1) : 0;  // a heavy cell, or the next Q light ones

@@ -28,12 +28,40 @@ inline int chain_cells(int B, int N) {
     return C < N ? C : N;
 }
 
-// The same for the kernels that walk several cells a wavefront: about 512 workgroups of eight
-// wavefronts, two a CU, which the registers hold at once; at most 1024 cells.
-inline int quad_cells(int B, int N) {
-    int C = 32;
-    while (C < N && C < 1024 && int64_t(B) * ((N + C - 1) / C) > 512) C *= 2;
+// The same for the kernels that walk several cells a wavefront. Eight cells, a wavefront each, while
+// their workgroups are no more than two a CU (one where a cell has eight events or more on average);
+// else 32 and more, so that most wavefronts have cells side by side, up to 1024; 16 where 32 would leave
+// the chip idle. One workgroup a CU for cells of many events: a heavy cell's chain waits for the CU's
+// other wavefronts (not above d = 64, where only two cells walk side by side: B32 T512 N1024 K16 d128
+// bf16 evenly 146 + 164 us, two a CU 146 + 139). Measured (us, forward and backward of a window: the
+// kernel of one cell a wavefront, 32 cells or more and two workgroups a CU whatever the shape, this):
+//   B1 T1024 N64 K8 d64 bf16 123 + 121, 184 + 181, 82 + 77; B8 T512 N128 K8 d128 71 + 70, 87 + 92, 54 + 49;
+//   B16 T512 N512 K8 d64 58 + 47, 54 + 37, 54 + 37; with Zipf popularity B64 T512 N1024 K16 d64 355 + 241,
+//   259 + 222, 231 + 186, and evenly 212 + 148, 164 + 125, 162 + 122 (two a CU 160 + 122); evenly
+//   B64 T512 N64 K8 d64 99 + 75, 139 + 103, 95 + 70 (eight cells, two a CU 91 + 65, but Zipf 185 + 143
+//   against 166 + 129).
+inline int quad_cells(int B, int T, int N, int d, int K) {
+    const bool many = int64_t(T) * K >= int64_t(8) * N;
+    auto groups = [&](int C) { return int64_t(B) * ((N + C - 1) / C); };
+    int C = 8;
+    if (groups(8) > (many ? 256 : 512)) {
+        C = groups(32) >= 160 ? 32 : 16;
+        while (C < N && C < 1024 && groups(C) > (many && d <= 64 ? 256 : 512)) C *= 2;
+    }
     return C < N ? C : N;
+}
+
+// Events up to which a cell is walked beside others: none where every cell has a wavefront; 64 where
+// the cells have 8 to 32 on average and a workgroup more than 16 of them, else 24. A longer chain, alone, takes each event at half the time,
+// but the wavefront's other lanes are lost. Measured, 24 against 64 (us): mean 1 to 4, Zipf: B256 T64
+// N128 K8 d64 67 + 44 and 85 + 60, B11 T66 N1655 K3 d16 49 + 28 and 60 + 38; mean 8, normal: B64 T512
+// N1024 K16 d64 184 + 141 and 168 + 128; mean 32, evenly: B64 T512 N128 K8 d64 106 + 75 and 94 + 63; mean 64
+// (half of the cells on either side of 64): B64 T512 N64 K8 d64 95 + 70 and 124 + 79; 16 cells, Zipf: B64
+// T64 N64 K16 d128 58 + 46 and 69 + 62.
+inline int quad_heavy(int T, int N, int K, int C) {
+    const int64_t events = int64_t(T) * K;
+    if (C <= 8) return 0;
+    return C > 16 && events >= int64_t(8) * N && events <= int64_t(32) * N ? chain::kHeavy : 24;
 }
 
 // Events staged in LDS per workgroup: twice the group's expected count, 256..8192.
@@ -154,7 +182,7 @@ WorkspaceLayout workspace_layout(int op, int B, int T, int N, int d, int K, size
         if (op == HSN_OP_FORWARD) {
             L.delta = at;
             at = align_up(at + size_t(slots) * d * 4);
-            const int C = std::min(chain_cells(B, N), quad_cells(B, N));
+            const int C = std::min(chain_cells(B, N), quad_cells(B, T, N, d, K));
             L.hmax = at;
             at = align_up(at + size_t(B) * T * ((N + C - 1) / C) * 4);
         }
@@ -279,7 +307,7 @@ void launch_delta(const chain::DeltaArgs& a, bool pair, hipStream_t st) {
 // Whether the several-cells kernels' LDS holds the row (T large).
 template <typename Args>
 bool quad_fits(const Args& a) {
-    const int C = quad_cells(a.B, a.N);
+    const int C = quad_cells(a.B, a.T, a.N, a.d, a.K);
     return int64_t(chain::quad_words(a.T, C, chain_stage(a.T, a.N, a.K, C))) * 4 <= kLdsMax;
 }
 
@@ -289,8 +317,9 @@ void forward_io(chain::FwdArgs& fa, chain::DeltaArgs& da, const chain::ScanArgs&
     const bool four = takes_four<IO>(fa.d, {fa.y, fa.g, fa.h_old, fa.h_sel}) &&
                       takes_four<float>(fa.d, {fa.h0, fa.h_T, fa.delta}) &&
                       int64_t(fa.N) * fa.d * 4 < (int64_t(1) << 31) && quad_fits(fa);
-    fa.C = four ? quad_cells(fa.B, fa.N) : chain_cells(fa.B, fa.N);
+    fa.C = four ? quad_cells(fa.B, fa.T, fa.N, fa.d, fa.K) : chain_cells(fa.B, fa.N);
     fa.stage = chain_stage(fa.T, fa.N, fa.K, fa.C);
+    fa.heavy = quad_heavy(fa.T, fa.N, fa.K, fa.C);
     da.G = (fa.N + fa.C - 1) / fa.C;
     const size_t lds = size_t(chain::chain_words(fa.T, fa.C, fa.stage)) * 4;
     const int V = (fa.d + 63) / 64;
@@ -311,8 +340,9 @@ void backward_io(chain::BwdArgs& ba, const chain::ScanArgs& sa, hipStream_t st) 
     const bool four = takes_four<IO>(ba.d, {ba.y, ba.g, ba.h_old, ba.dsel, ba.dy, ba.dg}) &&
                       takes_four<float>(ba.d, {ba.share, ba.dh_T, ba.dh0}) &&
                       int64_t(ba.N) * ba.d * 4 < (int64_t(1) << 31) && quad_fits(ba);
-    ba.C = four ? quad_cells(ba.B, ba.N) : chain_cells(ba.B, ba.N);
+    ba.C = four ? quad_cells(ba.B, ba.T, ba.N, ba.d, ba.K) : chain_cells(ba.B, ba.N);
     ba.stage = chain_stage(ba.T, ba.N, ba.K, ba.C);
+    ba.heavy = quad_heavy(ba.T, ba.N, ba.K, ba.C);
     const size_t lds = size_t(chain::chain_words(ba.T, ba.C, ba.stage)) * 4;
     hipLaunchKernelGGL((chain::summary_scan_bwd<IO>), dim3((ba.d + 63) / 64, ba.B),
                        dim3(64 * chain::kScanWaves), 0, st, sa);

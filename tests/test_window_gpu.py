@@ -874,6 +874,21 @@ def test_chains_of_several_cells_a_wavefront(dev, B, T, N, K, d, shift, io):
         _lib.set_path("auto")
 
 
+@pytest.mark.parametrize("io", ["f32", "bf16"])
+@pytest.mark.parametrize("B,T,N,K,d", [
+    (64, 70, 80, 3, 24),     # three groups a row, the last of 16 cells; the first cells above 24 events
+    (40, 40, 330, 5, 100),   # eleven groups of 32, two cells side by side
+    (40, 40, 330, 5, 4),     # the same, sixteen cells side by side
+    (64, 70, 40, 8, 64),     # groups of 16 cells: eight events or more a cell on average
+    (300, 20, 50, 2, 128),   # 64 cells a group would do: the row's 50
+    (520, 12, 40, 4, 20),    # a group a row
+])
+def test_chains_side_by_side_in_several_groups(dev, B, T, N, K, d, io):
+    """The same where the grid is full and cells are walked side by side: several groups of cells a row,
+    the last one short, with heavy cells beside light ones and cells without events."""
+    test_chains_of_several_cells_a_wavefront(dev, B, T, N, K, d, 0, io)
+
+
 PACKED_ROUTES = [
     # N, K, settings, special values: bf16 rows around the two-cells-a-register rule
     (512, 8, dict(), "plain"),                   # the general selection
