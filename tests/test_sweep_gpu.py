@@ -180,3 +180,58 @@ def test_runner_declines_what_it_does_not_take(dev):
     wargs, wkw = _args(wide, dev)
     assert runner(*wargs, **wkw) is None  # d above 256
     assert runner.calls == 0
+
+
+def _activation_grad(dev, x, products):
+    """The fused step's activation derivative at ``x`` [B, K] as sigma carries it, in fp32: one hidden
+    unit of cotangent 1 and nothing else but the cell norm's sum, so that the first of two positions'
+    dL/dc is -sigma / in_dim = -act'(x) x / in_dim (a power of two)."""
+    from hsn_amd.state_sweep import CellConstants, SweepRunner
+
+    (B, K), T, d, H, N = x.shape, 2, 16, 64, 16
+    zeros = lambda *s: torch.zeros(*s, device=dev)  # noqa: E731
+    ones = lambda *s: torch.ones(*s, device=dev)  # noqa: E731
+    w2 = zeros(1, H, d)
+    w2[0, 0, 0] = 1.0
+    consts = CellConstants(w_out=torch.eye(d, device=dev), cand_gain=None, cand_eps=1e-6, w2=w2,
+                           w1_state=zeros(1, 2 * d, H), b1=zeros(1, H), gate_state=zeros(d, 2 * d),
+                           gate_bias=zeros(d), norm_gain_state=ones(2 * d), in_dim=4 * d, v=zeros(d, d),
+                           edge_weights=zeros(N, 1), pad_src=torch.zeros(N, 1, dtype=torch.int64, device=dev),
+                           activation="gelu", pad_mask=torch.ones(N, 1, dtype=torch.bool, device=dev))
+    hidden, d_h_sel = zeros(B, T, K, H), zeros(B, T, K, d)
+    hidden[:, 1, :, 0], d_h_sel[:, 1, :, 0] = x, 1.0
+    record = {"y": zeros(B, T, K, d), "alpha": ones(B, T, K), "hidden": hidden.to(products),
+              "gate_pre": zeros(B, T, K, d), "m": zeros(B, T, K, d), "rms": ones(B, T, K)}
+    cells = torch.arange(K, device=dev).expand(B, T, K).contiguous()
+    out = SweepRunner(graph=False, fused=True)(
+        zeros(B, T, K, d), ones(B, T, K, d), ones(B, T, K, d), cells, torch.zeros_like(cells),
+        torch.ones(B, T, K, dtype=torch.bool, device=dev), torch.zeros(B, T, dtype=torch.bool, device=dev),
+        N, zeros(B, T, d), zeros(B, T, d), d_h_sel, None, record, consts, n_read=0)
+    assert out is not None
+    return out[0][:, 0, :, 0] * (-4 * d)
+
+
+@pytest.mark.parametrize("scale", [1 / 3, 1.0, 3.0])
+def test_bf16_products_take_the_activation_no_further_off(dev, scale):
+    """With products in 16 bits sigma still sums the GELU's derivative in fp32: over 4096 hidden values
+    it is as close to 64 bits as the fp32 products' (erff), within the norms' chance."""
+    x = (scale * torch.randn(512, 8, generator=torch.Generator().manual_seed(5))).bfloat16().float()
+    x64 = x.double()
+    want = x64 * (0.5 * (1 + torch.erf(x64 * 0.5 ** 0.5)) + x64 * torch.exp(-0.5 * x64 * x64) * (2 * torch.pi) ** -0.5)
+    keep = x != 0
+    off = {}
+    for products in (torch.float32, torch.bfloat16):
+        got = _activation_grad(dev, x.to(dev), products).double().cpu()
+        off[products] = float((((got - want) / x64)[keep] ** 2).mean().sqrt())
+    print(f"hidden scale {scale:.2f}: fp32 {off[torch.float32]:.2e}, bf16 {off[torch.bfloat16]:.2e}")
+    assert off[torch.bfloat16] <= 1.03 * off[torch.float32]
+
+
+def test_activation_of_infinite_and_nan_hidden_values(dev):
+    """An infinite or NaN hidden value gives NaN with either products (inf 0 in x phi(x), as the plain
+    formula has it), and the largest finite ones 0 or 1."""
+    x = torch.tensor([[float("inf"), -float("inf"), float("nan"), 3e38, -3e38, 1e20, -1e20, 1.0]]).bfloat16().float()
+    for products in (torch.float32, torch.bfloat16):
+        got = _activation_grad(dev, x.to(dev), products).cpu()
+        assert bool(torch.isnan(got[0, :3]).all()), (products, got)
+        assert got[0, 4] == 0 and got[0, 6] == 0 and got[0, 5] == x[0, 5], (products, got)
