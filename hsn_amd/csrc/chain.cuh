@@ -533,6 +533,175 @@ __device__ __forceinline__ void fetch_rows(IO (&yv)[V], IO (&gv)[V], rsrc_t ry, 
     }
 }
 
+// The age of cell c at the window's end: its last event's position (-1: none) and the row's last reset.
+__device__ __forceinline__ void end_age(const FwdArgs& a, int b, int c, int tprev, int lrT) {
+    int64_t age;
+    if (tprev >= 0 && tprev >= lrT) age = (a.T - 1) - tprev;
+    else if (lrT >= 0) age = a.T - lrT;
+    else age = a.age0[int64_t(b) * a.N + c] + a.T;
+    a.age_T[int64_t(b) * a.N + c] = age;
+}
+
+// What a wavefront that walks one cell at a time holds of its row and its columns (lane + 64 v).
+template <int V>
+struct FwdRow {
+    int b, pc0, nst, lrT, pad_begin;  // staged events: cev[0 .. nst) is ev[pc0 ..)
+    const int32_t* ev;
+    const int *cev, *nr;
+    uint32_t* hm;
+    rsrc_t ry, rg, rho, rhs, rdl;
+    uint32_t srow, srow4, voff[V], voff4[V];
+};
+template <typename IO, int V>
+__device__ __forceinline__ void column_offsets(int d, uint32_t (&voff)[V], uint32_t (&voff4)[V]) {
+    const int lane = lane_id();
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        const bool in = lane + 64 * v < d;
+        voff[v] = in ? uint32_t(lane + 64 * v) * sizeof(IO) : kOob;
+        voff4[v] = in ? uint32_t(lane + 64 * v) * 4u : kOob;
+    }
+}
+
+// Cell c, whose events are the row's list from e_beg to e_end, by the whole wavefront; cell 0 takes the
+// row's padded slots too (PADS: the caller has none, this is it, or look).
+enum Pads { kNoPads, kPadCell, kPadsMaybe };
+template <typename IO, int V, int NB, bool DELTA, bool HMAX, Pads PADS>
+__device__ __forceinline__ void walk_cell(const FwdArgs& a, const FwdRow<V>& r, int c, int e_beg, int e_end) {
+    const int lane = lane_id();
+    const int T = a.T, N = a.N, d = a.d, K = a.K, n_slots = T * K;
+    float h[V];
+    const float* h0c = a.h0 + (int64_t(r.b) * N + c) * d;
+#pragma unroll
+    for (int v = 0; v < V; ++v) h[v] = lane + 64 * v < d ? h0c[lane + 64 * v] : 0.0f;
+    float hold_last[V];  // the state before the latest event (cell 0's padded slots)
+#pragma unroll
+    for (int v = 0; v < V; ++v) hold_last[v] = 0.0f;
+    uint32_t vprev = HMAX ? cell_abs_max<V>(h, lane, d) : 0u;
+    int tprev = -1, s = 0;
+    int nrprev = r.nr[0];  // the first reset after the latest event
+    // cell 0's padded slots at positions below `limit`, in time order (a window of 64 of
+    // them in the lanes)
+    int pp = r.pad_begin, pwb = -1, pwv = 0;
+    auto flush = [&](int limit) __attribute__((always_inline)) {
+        while (pp < n_slots) {
+            if (pwb < 0 || pp >= pwb + kEvWin) {
+                pwb = pp;
+                pwv = lane < n_slots - pp ? r.ev[pp + lane] : 0x7fffffff;
+            }
+            const int off = pp - pwb;
+            const uint64_t below = ballot(lane >= off && (pwv >> 8) < limit);
+            const int n = __popcll(below);
+            for (int i = 0; i < n; ++i) {
+                const int q = __builtin_amdgcn_readlane(pwv, off + i);
+                const int t = q >> 8;
+                const uint32_t so = uint32_t(t * K + (q & 255)) * r.srow;
+                const bool same = t == tprev;
+                const bool zero = nrprev <= t;
+#pragma unroll
+                for (int v = 0; v < V; ++v) {
+                    const float now = zero ? 0.0f : h[v];
+                    bstore_f32<IO>(same ? hold_last[v] : now, r.rho, r.voff[v], so);
+                    bstore_f32<IO>(same ? h[v] : now, r.rhs, r.voff[v], so);
+                }
+            }
+            pp += n;
+            if (off + n < kEvWin) break;  // the next one is at or after `limit`
+        }
+    };
+    const bool pad_here = PADS == kPadCell || (PADS == kPadsMaybe && c == 0 && r.pad_begin < n_slots);
+    // one event: position t, its slot's byte offsets (so: storage rows, so4: fp32 rows) and
+    // the first reset after t
+    auto update = [&](auto pad_c, int t, uint32_t so, uint32_t so4, int nrq, const IO (&yv)[V],
+                      const IO (&gv)[V]) __attribute__((always_inline)) {
+        constexpr bool kPad = decltype(pad_c)::value;
+        const bool zero = nrprev <= t;  // a reset since the cell's last event
+        if constexpr (HMAX) max_interval(r.hm, s, min(t, nrprev), vprev, lane);
+        if constexpr (kPad) flush(t);
+#pragma unroll
+        for (int v = 0; v < V; ++v) {
+            const float hold = zero ? 0.0f : h[v];
+            const float bg = fast_sigmoid(to_f32(gv[v]));
+            const float cand = fast_tanh(to_f32(yv[v]));
+            const float hn = (1.0f - bg) * hold + bg * cand;
+            bstore_f32<IO>(hold, r.rho, r.voff[v], so);
+            bstore_f32<IO>(hn, r.rhs, r.voff[v], so);
+            if constexpr (DELTA) bstore(hn - hold, r.rdl, r.voff4[v], so4);
+            if constexpr (kPad) hold_last[v] = hold;
+            h[v] = hn;
+        }
+        if constexpr (HMAX) vprev = cell_abs_max<V>(h, lane, d);
+        s = t;
+        tprev = t;
+        nrprev = nrq;
+        if constexpr (kPad) flush(t + 1);
+    };
+    // windows of 64 events (one per lane), in batches of NB with two batches in flight; a
+    // window's positions, slot offsets and next resets are computed for all its events at
+    // once (lane i: event i) and read per event with readlane
+    auto walk = [&](auto staged_c, auto pad_c) __attribute__((always_inline)) {
+        constexpr bool kStaged = decltype(staged_c)::value;
+        for (int w0 = e_beg; w0 < e_end; w0 += kEvWin) {
+            const int m = min(kEvWin, e_end - w0);
+            int evw;
+            if constexpr (kStaged) evw = lane < m ? r.cev[w0 - r.pc0 + lane] : 0;
+            else evw = lane < m ? r.ev[w0 + lane] : 0;
+            const int tw = evw >> 8;
+            const int slw = tw * K + (evw & 255);
+            const uint32_t sow = uint32_t(slw) * r.srow;
+            const uint32_t so4w = uint32_t(slw) * r.srow4;
+            const int nrw = lane < m ? r.nr[tw + 1] : T;
+            IO ya[NB][V], ga[NB][V], yb[NB][V], gb[NB][V];
+            auto fetch = [&](int j, IO (&yv)[NB][V], IO (&gv)[NB][V])
+                             __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const uint32_t so = __builtin_amdgcn_readlane(sow, min(j + i, kEvWin - 1));
+                    fetch_rows<IO, V>(yv[i], gv[i], r.ry, r.rg, r.voff, so, j + i < m);
+                }
+            };
+            auto step = [&](int j, const IO (&yv)[NB][V], const IO (&gv)[NB][V])
+                            __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    if (j + i < m) {
+                        const int idx = j + i;
+                        update(pad_c, __builtin_amdgcn_readlane(tw, idx),
+                               __builtin_amdgcn_readlane(sow, idx),
+                               DELTA ? __builtin_amdgcn_readlane(so4w, idx) : 0u,
+                               __builtin_amdgcn_readlane(nrw, idx), yv[i], gv[i]);
+                    }
+                }
+            };
+            fetch(0, ya, ga);
+            for (int j = 0; j < m; j += 2 * NB) {
+                fetch(j + NB, yb, gb);
+                step(j, ya, ga);
+                if (j + NB >= m) break;
+                fetch(j + 2 * NB, ya, ga);
+                step(j + NB, yb, gb);
+            }
+        }
+    };
+    if constexpr (PADS == kPadCell) {
+        walk(std::false_type{}, std::true_type{});
+    } else {
+        if (PADS == kPadsMaybe && pad_here) walk(std::false_type{}, std::true_type{});
+        else if (e_end - r.pc0 <= r.nst) walk(std::true_type{}, std::false_type{});
+        else walk(std::false_type{}, std::false_type{});
+    }
+    if (PADS != kNoPads && pad_here) flush(T);
+    if constexpr (HMAX) max_interval(r.hm, s, min(T, nrprev), vprev, lane);
+    const bool cleared = nrprev < T;  // a reset after the cell's last event
+    if (a.h_T) {
+        float* hTc = a.h_T + (int64_t(r.b) * N + c) * d;
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (lane + 64 * v < d) hTc[lane + 64 * v] = cleared ? 0.0f : h[v];
+    }
+    if (a.age_T && lane == 0) end_age(a, r.b, c, tprev, r.lrT);
+}
+
 template <typename IO, int V, int NB, bool DELTA, bool HMAX>
 __global__ __launch_bounds__(kChainThreads) void chain_fwd(FwdArgs a) {
     extern __shared__ uint32_t lds_u[];
@@ -549,7 +718,6 @@ __global__ __launch_bounds__(kChainThreads) void chain_fwd(FwdArgs a) {
     int* cptr = next + 1;                                // [C + 1]
     int* cev = cptr + a.C + 1;                           // [stage]
     int* order = cev + a.stage;                          // [C]
-    constexpr bool want_max = HMAX;
     const int c_begin = g * a.C, c_end = min(N, c_begin + a.C);
     const int nc = c_end - c_begin;
     const int32_t* ptr = a.ptr + int64_t(b) * (N + 1);
@@ -566,24 +734,16 @@ __global__ __launch_bounds__(kChainThreads) void chain_fwd(FwdArgs a) {
     heavy_first(cptr, nc, order, tid, kChainThreads);
     const int64_t slot0 = int64_t(b) * T * K;
     const uint32_t row_bytes = uint32_t(T) * K * d * sizeof(IO);
-    const rsrc_t ry = make_rsrc(static_cast<const IO*>(a.y) + slot0 * d, row_bytes);
-    const rsrc_t rg = make_rsrc(static_cast<const IO*>(a.g) + slot0 * d, row_bytes);
-    const rsrc_t rho = make_rsrc(a.h_old ? static_cast<IO*>(a.h_old) + slot0 * d : nullptr,
-                                 a.h_old ? row_bytes : 0u);
-    const rsrc_t rhs = make_rsrc(a.h_sel ? static_cast<IO*>(a.h_sel) + slot0 * d : nullptr,
-                                 a.h_sel ? row_bytes : 0u);
-    const rsrc_t rdl = make_rsrc(a.delta ? a.delta + slot0 * d : nullptr,
-                                 a.delta ? uint32_t(T) * K * d * 4u : 0u);
-    uint32_t voff[V], voff4[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-        const bool in = lane + 64 * v < d;
-        voff[v] = in ? uint32_t(lane + 64 * v) * sizeof(IO) : kOob;
-        voff4[v] = in ? uint32_t(lane + 64 * v) * 4u : kOob;
-    }
-    const uint32_t srow = uint32_t(d) * sizeof(IO), srow4 = uint32_t(d) * 4u;
-    const int n_slots = T * K;
-    const int pad_begin = ptr[N];
+    FwdRow<V> r;
+    r.b = b, r.pc0 = pc0, r.nst = nst, r.lrT = lrT, r.pad_begin = ptr[N];
+    r.ev = ev, r.cev = cev, r.nr = nr, r.hm = hm;
+    r.ry = make_rsrc(static_cast<const IO*>(a.y) + slot0 * d, row_bytes);
+    r.rg = make_rsrc(static_cast<const IO*>(a.g) + slot0 * d, row_bytes);
+    r.rho = make_rsrc(a.h_old ? static_cast<IO*>(a.h_old) + slot0 * d : nullptr, a.h_old ? row_bytes : 0u);
+    r.rhs = make_rsrc(a.h_sel ? static_cast<IO*>(a.h_sel) + slot0 * d : nullptr, a.h_sel ? row_bytes : 0u);
+    r.rdl = make_rsrc(a.delta ? a.delta + slot0 * d : nullptr, a.delta ? uint32_t(T) * K * d * 4u : 0u);
+    r.srow = uint32_t(d) * sizeof(IO), r.srow4 = uint32_t(d) * 4u;
+    column_offsets<IO, V>(d, r.voff, r.voff4);
 
     for (;;) {
         int slot = lane == 0 ? atomicAdd(next, 1) : 0;
@@ -592,141 +752,10 @@ __global__ __launch_bounds__(kChainThreads) void chain_fwd(FwdArgs a) {
         const int ci = uniform(order[slot]);
         const int c = c_begin + ci;
         const int e_beg = uniform(cptr[ci]), e_end = uniform(cptr[ci + 1]);
-        float h[V];
-        const float* h0c = a.h0 + (int64_t(b) * N + c) * d;
-#pragma unroll
-        for (int v = 0; v < V; ++v) h[v] = lane + 64 * v < d ? h0c[lane + 64 * v] : 0.0f;
-        float hold_last[V];  // the state before the latest event (cell 0's padded slots)
-#pragma unroll
-        for (int v = 0; v < V; ++v) hold_last[v] = 0.0f;
-        uint32_t vprev = want_max ? cell_abs_max<V>(h, lane, d) : 0u;
-        int tprev = -1, s = 0;
-        int nrprev = nr[0];  // the first reset after the latest event
-        // cell 0's padded slots at positions below `limit`, in time order (a window of 64 of
-        // them in the lanes)
-        int pp = pad_begin, pwb = -1, pwv = 0;
-        auto flush = [&](int limit) __attribute__((always_inline)) {
-            while (pp < n_slots) {
-                if (pwb < 0 || pp >= pwb + kEvWin) {
-                    pwb = pp;
-                    pwv = lane < n_slots - pp ? ev[pp + lane] : 0x7fffffff;
-                }
-                const int off = pp - pwb;
-                const uint64_t below = ballot(lane >= off && (pwv >> 8) < limit);
-                const int n = __popcll(below);
-                for (int i = 0; i < n; ++i) {
-                    const int q = __builtin_amdgcn_readlane(pwv, off + i);
-                    const int t = q >> 8;
-                    const uint32_t so = uint32_t(t * K + (q & 255)) * srow;
-                    const bool same = t == tprev;
-                    const bool zero = nrprev <= t;
-#pragma unroll
-                    for (int v = 0; v < V; ++v) {
-                        const float now = zero ? 0.0f : h[v];
-                        bstore_f32<IO>(same ? hold_last[v] : now, rho, voff[v], so);
-                        bstore_f32<IO>(same ? h[v] : now, rhs, voff[v], so);
-                    }
-                }
-                pp += n;
-                if (off + n < kEvWin) break;  // the next one is at or after `limit`
-            }
-        };
-        const bool pad_here = c == 0 && pad_begin < n_slots;
-        // one event: position t, its slot's byte offsets (so: storage rows, so4: fp32 rows) and
-        // the first reset after t
-        auto update = [&](auto pad_c, int t, uint32_t so, uint32_t so4, int nrq, const IO (&yv)[V],
-                          const IO (&gv)[V]) __attribute__((always_inline)) {
-            constexpr bool kPad = decltype(pad_c)::value;
-            const bool zero = nrprev <= t;  // a reset since the cell's last event
-            if constexpr (want_max) max_interval(hm, s, min(t, nrprev), vprev, lane);
-            if constexpr (kPad) flush(t);
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                const float hold = zero ? 0.0f : h[v];
-                const float bg = fast_sigmoid(to_f32(gv[v]));
-                const float cand = fast_tanh(to_f32(yv[v]));
-                const float hn = (1.0f - bg) * hold + bg * cand;
-                bstore_f32<IO>(hold, rho, voff[v], so);
-                bstore_f32<IO>(hn, rhs, voff[v], so);
-                if constexpr (DELTA) bstore(hn - hold, rdl, voff4[v], so4);
-                if constexpr (kPad) hold_last[v] = hold;
-                h[v] = hn;
-            }
-            if constexpr (want_max) vprev = cell_abs_max<V>(h, lane, d);
-            s = t;
-            tprev = t;
-            nrprev = nrq;
-            if constexpr (kPad) flush(t + 1);
-        };
-        // windows of 64 events (one per lane), in batches of NB with two batches in flight; a
-        // window's positions, slot offsets and next resets are computed for all its events at
-        // once (lane i: event i) and read per event with readlane
-        auto walk = [&](auto staged_c, auto pad_c) __attribute__((always_inline)) {
-            constexpr bool kStaged = decltype(staged_c)::value;
-            for (int w0 = e_beg; w0 < e_end; w0 += kEvWin) {
-                const int m = min(kEvWin, e_end - w0);
-                int evw;
-                if constexpr (kStaged) evw = lane < m ? cev[w0 - pc0 + lane] : 0;
-                else evw = lane < m ? ev[w0 + lane] : 0;
-                const int tw = evw >> 8;
-                const int slw = tw * K + (evw & 255);
-                const uint32_t sow = uint32_t(slw) * srow;
-                const uint32_t so4w = uint32_t(slw) * srow4;
-                const int nrw = lane < m ? nr[tw + 1] : T;
-                IO ya[NB][V], ga[NB][V], yb[NB][V], gb[NB][V];
-                auto fetch = [&](int j, IO (&yv)[NB][V], IO (&gv)[NB][V])
-                                 __attribute__((always_inline)) {
-#pragma unroll
-                    for (int i = 0; i < NB; ++i) {
-                        const uint32_t so = __builtin_amdgcn_readlane(sow, min(j + i, kEvWin - 1));
-                        fetch_rows<IO, V>(yv[i], gv[i], ry, rg, voff, so, j + i < m);
-                    }
-                };
-                auto step = [&](int j, const IO (&yv)[NB][V], const IO (&gv)[NB][V])
-                                __attribute__((always_inline)) {
-#pragma unroll
-                    for (int i = 0; i < NB; ++i) {
-                        if (j + i < m) {
-                            const int idx = j + i;
-                            update(pad_c, __builtin_amdgcn_readlane(tw, idx),
-                                   __builtin_amdgcn_readlane(sow, idx),
-                                   DELTA ? __builtin_amdgcn_readlane(so4w, idx) : 0u,
-                                   __builtin_amdgcn_readlane(nrw, idx), yv[i], gv[i]);
-                        }
-                    }
-                };
-                fetch(0, ya, ga);
-                for (int j = 0; j < m; j += 2 * NB) {
-                    fetch(j + NB, yb, gb);
-                    step(j, ya, ga);
-                    if (j + NB >= m) break;
-                    fetch(j + 2 * NB, ya, ga);
-                    step(j + NB, yb, gb);
-                }
-            }
-        };
-        if (pad_here) walk(std::false_type{}, std::true_type{});
-        else if (e_end - pc0 <= nst) walk(std::true_type{}, std::false_type{});
-        else walk(std::false_type{}, std::false_type{});
-        if (pad_here) flush(T);
-        if (want_max) max_interval(hm, s, min(T, nrprev), vprev, lane);
-        const bool cleared = nrprev < T;  // a reset after the cell's last event
-        if (a.h_T) {
-            float* hTc = a.h_T + (int64_t(b) * N + c) * d;
-#pragma unroll
-            for (int v = 0; v < V; ++v)
-                if (lane + 64 * v < d) hTc[lane + 64 * v] = cleared ? 0.0f : h[v];
-        }
-        if (a.age_T && lane == 0) {
-            int64_t age;
-            if (tprev >= 0 && tprev >= lrT) age = (T - 1) - tprev;
-            else if (lrT >= 0) age = T - lrT;
-            else age = a.age0[int64_t(b) * N + c] + T;
-            a.age_T[int64_t(b) * N + c] = age;
-        }
+        walk_cell<IO, V, NB, DELTA, HMAX, kPadsMaybe>(a, r, c, e_beg, e_end);
     }
     if (a.pos_T && g == 0 && tid == 0) a.pos_T[b] = lrT >= 0 ? int64_t(T - lrT) : a.pos0[b] + T;
-    if (want_max) {  // the group's maxima, reduced over the groups by summary_delta
+    if (HMAX) {  // the group's maxima, reduced over the groups by summary_delta
         __syncthreads();
         const int G = gridDim.y;
         uint32_t* hg = a.hm_groups + int64_t(b) * T * G + g;
@@ -987,10 +1016,124 @@ struct BwdArgs {
     int C, stage, heavy;
 };
 
+// The backward's FwdRow.
+template <int V>
+struct BwdRow {
+    int b, pc0, nst;
+    const int32_t* ev;
+    const int *cev, *nr;
+    rsrc_t ry, rg, rho, rds, rdy, rdg, rsh;
+    uint32_t srow, srow4, voff[V], voff4[V];
+};
+
 // Per cell, latest event first (python/hsn/train/split.py:154-173): with the cotangent A of the
 // cell's state after the event and the share R / N of its position, g = A + d_h_sel + R / N;
 // dc = b g, db = (c - h_old) g, then through c = tanh(y) and b = sigmoid(gate); the state before
 // the event gets (1 - b)(A + d_h_sel) - b R / N (h_old enters the summary's delta with -1 / N).
+template <typename IO, int V, int NB>
+__device__ __forceinline__ void walk_cell(const BwdArgs& a, const BwdRow<V>& r, int c, int e_beg, int e_end) {
+    const int lane = lane_id();
+    const int T = a.T, N = a.N, d = a.d, K = a.K;
+    struct Rows {
+        IO y[NB][V], g[NB][V], h[NB][V], s[NB][V];
+        float r[NB][V];
+    };
+    const bool staged = e_end - r.pc0 <= r.nst;
+    float A[V];
+    {  // the end cotangent, cut by a reset after the cell's last event
+        const int t_last = e_end > e_beg
+                               ? (uniform(staged ? r.cev[e_end - 1 - r.pc0] : r.ev[e_end - 1]) >> 8)
+                               : -1;
+        const bool cut = r.nr[t_last + 1] < T;
+        const float* dhc = a.dh_T ? a.dh_T + (int64_t(r.b) * N + c) * d : nullptr;
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            A[v] = (dhc && !cut && lane + 64 * v < d) ? dhc[lane + 64 * v] : 0.0f;
+    }
+    int tnext = T;  // the later event's position
+    int t_first = T;
+    auto walk = [&](auto staged_c) __attribute__((always_inline)) {
+        constexpr bool kStaged = decltype(staged_c)::value;
+        for (int w1 = e_end; w1 > e_beg; w1 -= kEvWin) {
+            const int m = min(kEvWin, w1 - e_beg);
+            const int w0 = w1 - m;
+            int evw;
+            if constexpr (kStaged) evw = lane < m ? r.cev[w0 - r.pc0 + lane] : 0;
+            else evw = lane < m ? r.ev[w0 + lane] : 0;
+            // the window's positions, slot offsets, share offsets and next resets, for all
+            // its events at once (lane i: event i), read per event with readlane
+            const int tw = evw >> 8;
+            const uint32_t sow = uint32_t(tw * K + (evw & 255)) * r.srow;
+            const uint32_t stw = uint32_t(tw) * r.srow4;
+            const int nrw = lane < m ? r.nr[tw + 1] : T;
+            Rows qa, qb;
+            // batch j holds window indices [j - NB + 1, j], fetched latest first
+            auto fetch = [&](int j, Rows& q) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const int idx = j - i;
+                    const uint32_t so = __builtin_amdgcn_readlane(sow, max(idx, 0));
+                    const uint32_t st = __builtin_amdgcn_readlane(stw, max(idx, 0));
+                    const bool in = idx >= 0;
+#pragma unroll
+                    for (int v = 0; v < V; ++v) {
+                        const uint32_t vo = in ? r.voff[v] : kOob;
+                        q.y[i][v] = bload<IO>(r.ry, vo, so);
+                        q.g[i][v] = bload<IO>(r.rg, vo, so);
+                        q.h[i][v] = bload<IO>(r.rho, vo, so);
+                        q.s[i][v] = bload<IO>(r.rds, vo, so);
+                        q.r[i][v] = bload<float>(r.rsh, in ? r.voff4[v] : kOob, st);
+                    }
+                }
+            };
+            auto step = [&](int j, const Rows& q) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < NB; ++i) {
+                    const int idx = j - i;
+                    if (idx >= 0) {
+                        const int t = __builtin_amdgcn_readlane(tw, idx);
+                        const int nrq = __builtin_amdgcn_readlane(nrw, idx);
+                        const uint32_t so = __builtin_amdgcn_readlane(sow, idx);
+                        const bool zero = nrq <= tnext && tnext < T;  // a reset in (t, tnext]
+#pragma unroll
+                        for (int v = 0; v < V; ++v) {
+                            const float carried = (zero ? 0.0f : A[v]) + to_f32(q.s[i][v]);
+                            const float share = q.r[i][v];
+                            const float gg = carried + share;
+                            const float bg = fast_sigmoid(to_f32(q.g[i][v]));
+                            const float cc = fast_tanh(to_f32(q.y[i][v]));
+                            const float dc = bg * gg * (1.0f - cc * cc);
+                            const float db = (cc - to_f32(q.h[i][v])) * gg * (bg * (1.0f - bg));
+                            bstore_f32<IO>(dc, r.rdy, r.voff[v], so);
+                            bstore_f32<IO>(db, r.rdg, r.voff[v], so);
+                            A[v] = (1.0f - bg) * carried - bg * share;
+                        }
+                        tnext = t;
+                    }
+                }
+            };
+            fetch(m - 1, qa);
+            for (int j = m - 1; j >= 0; j -= 2 * NB) {
+                fetch(j - NB, qb);
+                step(j, qa);
+                if (j - NB < 0) break;
+                fetch(j - 2 * NB, qa);
+                step(j - NB, qb);
+            }
+        }
+    };
+    if (staged) walk(std::true_type{});
+    else walk(std::false_type{});
+    t_first = tnext;
+    if (a.dh0) {  // the start state's cotangent: cut by a reset at or before the first event
+        const bool z = r.nr[0] <= min(t_first, T - 1);
+        float* d0 = a.dh0 + (int64_t(r.b) * N + c) * d;
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            if (lane + 64 * v < d) d0[lane + 64 * v] = z ? 0.0f : A[v];
+    }
+}
+
 template <typename IO, int V, int NB>
 __global__ __launch_bounds__(kChainThreads) void chain_bwd(BwdArgs a) {
     extern __shared__ uint32_t lds_u[];
@@ -1019,29 +1162,20 @@ __global__ __launch_bounds__(kChainThreads) void chain_bwd(BwdArgs a) {
     heavy_first(cptr, nc, order, tid, kChainThreads);
     const int64_t slot0 = int64_t(b) * T * K;
     const uint32_t row_bytes = uint32_t(T) * K * d * sizeof(IO);
-    const rsrc_t ry = make_rsrc(static_cast<const IO*>(a.y) + slot0 * d, row_bytes);
-    const rsrc_t rg = make_rsrc(static_cast<const IO*>(a.g) + slot0 * d, row_bytes);
-    const rsrc_t rho = make_rsrc(static_cast<const IO*>(a.h_old) + slot0 * d, row_bytes);
-    const rsrc_t rds = make_rsrc(a.dsel ? static_cast<const IO*>(a.dsel) + slot0 * d : nullptr,
-                                 a.dsel ? row_bytes : 0u);
-    const rsrc_t rdy = make_rsrc(static_cast<IO*>(a.dy) + slot0 * d, row_bytes);
-    const rsrc_t rdg = make_rsrc(static_cast<IO*>(a.dg) + slot0 * d, row_bytes);
-    const rsrc_t rsh = make_rsrc(a.share + int64_t(b) * T * d, uint32_t(T) * d * 4u);
-    uint32_t voff[V], voff4[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-        const bool in = lane + 64 * v < d;
-        voff[v] = in ? uint32_t(lane + 64 * v) * sizeof(IO) : kOob;
-        voff4[v] = in ? uint32_t(lane + 64 * v) * 4u : kOob;
-    }
-    const uint32_t srow = uint32_t(d) * sizeof(IO), srow4 = uint32_t(d) * 4u;
+    BwdRow<V> r;
+    r.b = b, r.pc0 = pc0, r.nst = nst, r.ev = ev, r.cev = cev, r.nr = nr;
+    r.ry = make_rsrc(static_cast<const IO*>(a.y) + slot0 * d, row_bytes);
+    r.rg = make_rsrc(static_cast<const IO*>(a.g) + slot0 * d, row_bytes);
+    r.rho = make_rsrc(static_cast<const IO*>(a.h_old) + slot0 * d, row_bytes);
+    r.rds = make_rsrc(a.dsel ? static_cast<const IO*>(a.dsel) + slot0 * d : nullptr, a.dsel ? row_bytes : 0u);
+    r.rdy = make_rsrc(static_cast<IO*>(a.dy) + slot0 * d, row_bytes);
+    r.rdg = make_rsrc(static_cast<IO*>(a.dg) + slot0 * d, row_bytes);
+    r.rsh = make_rsrc(a.share + int64_t(b) * T * d, uint32_t(T) * d * 4u);
+    r.srow = uint32_t(d) * sizeof(IO), r.srow4 = uint32_t(d) * 4u;
+    column_offsets<IO, V>(d, r.voff, r.voff4);
     const int n_slots = T * K;
     const int pad_begin = ptr[N];
 
-    struct Rows {
-        IO y[NB][V], g[NB][V], h[NB][V], s[NB][V];
-        float r[NB][V];
-    };
     for (;;) {
         int slot = lane == 0 ? atomicAdd(next, 1) : 0;
         slot = __builtin_amdgcn_readfirstlane(slot);
@@ -1049,100 +1183,7 @@ __global__ __launch_bounds__(kChainThreads) void chain_bwd(BwdArgs a) {
         const int ci = uniform(order[slot]);
         const int c = c_begin + ci;
         const int e_beg = uniform(cptr[ci]), e_end = uniform(cptr[ci + 1]);
-        const bool staged = e_end - pc0 <= nst;
-        float A[V];
-        {  // the end cotangent, cut by a reset after the cell's last event
-            const int t_last = e_end > e_beg
-                                   ? (uniform(staged ? cev[e_end - 1 - pc0] : ev[e_end - 1]) >> 8)
-                                   : -1;
-            const bool cut = nr[t_last + 1] < T;
-            const float* dhc = a.dh_T ? a.dh_T + (int64_t(b) * N + c) * d : nullptr;
-#pragma unroll
-            for (int v = 0; v < V; ++v)
-                A[v] = (dhc && !cut && lane + 64 * v < d) ? dhc[lane + 64 * v] : 0.0f;
-        }
-        int tnext = T;  // the later event's position
-        int t_first = T;
-        auto walk = [&](auto staged_c) __attribute__((always_inline)) {
-            constexpr bool kStaged = decltype(staged_c)::value;
-            for (int w1 = e_end; w1 > e_beg; w1 -= kEvWin) {
-                const int m = min(kEvWin, w1 - e_beg);
-                const int w0 = w1 - m;
-                int evw;
-                if constexpr (kStaged) evw = lane < m ? cev[w0 - pc0 + lane] : 0;
-                else evw = lane < m ? ev[w0 + lane] : 0;
-                // the window's positions, slot offsets, share offsets and next resets, for all
-                // its events at once (lane i: event i), read per event with readlane
-                const int tw = evw >> 8;
-                const uint32_t sow = uint32_t(tw * K + (evw & 255)) * srow;
-                const uint32_t stw = uint32_t(tw) * srow4;
-                const int nrw = lane < m ? nr[tw + 1] : T;
-                Rows ra, rb;
-                // batch j holds window indices [j - NB + 1, j], fetched latest first
-                auto fetch = [&](int j, Rows& r) __attribute__((always_inline)) {
-#pragma unroll
-                    for (int i = 0; i < NB; ++i) {
-                        const int idx = j - i;
-                        const uint32_t so = __builtin_amdgcn_readlane(sow, max(idx, 0));
-                        const uint32_t st = __builtin_amdgcn_readlane(stw, max(idx, 0));
-                        const bool in = idx >= 0;
-#pragma unroll
-                        for (int v = 0; v < V; ++v) {
-                            const uint32_t vo = in ? voff[v] : kOob;
-                            r.y[i][v] = bload<IO>(ry, vo, so);
-                            r.g[i][v] = bload<IO>(rg, vo, so);
-                            r.h[i][v] = bload<IO>(rho, vo, so);
-                            r.s[i][v] = bload<IO>(rds, vo, so);
-                            r.r[i][v] = bload<float>(rsh, in ? voff4[v] : kOob, st);
-                        }
-                    }
-                };
-                auto step = [&](int j, const Rows& r) __attribute__((always_inline)) {
-#pragma unroll
-                    for (int i = 0; i < NB; ++i) {
-                        const int idx = j - i;
-                        if (idx >= 0) {
-                            const int t = __builtin_amdgcn_readlane(tw, idx);
-                            const int nrq = __builtin_amdgcn_readlane(nrw, idx);
-                            const uint32_t so = __builtin_amdgcn_readlane(sow, idx);
-                            const bool zero = nrq <= tnext && tnext < T;  // a reset in (t, tnext]
-#pragma unroll
-                            for (int v = 0; v < V; ++v) {
-                                const float carried = (zero ? 0.0f : A[v]) + to_f32(r.s[i][v]);
-                                const float share = r.r[i][v];
-                                const float gg = carried + share;
-                                const float bg = fast_sigmoid(to_f32(r.g[i][v]));
-                                const float cc = fast_tanh(to_f32(r.y[i][v]));
-                                const float dc = bg * gg * (1.0f - cc * cc);
-                                const float db = (cc - to_f32(r.h[i][v])) * gg * (bg * (1.0f - bg));
-                                bstore_f32<IO>(dc, rdy, voff[v], so);
-                                bstore_f32<IO>(db, rdg, voff[v], so);
-                                A[v] = (1.0f - bg) * carried - bg * share;
-                            }
-                            tnext = t;
-                        }
-                    }
-                };
-                fetch(m - 1, ra);
-                for (int j = m - 1; j >= 0; j -= 2 * NB) {
-                    fetch(j - NB, rb);
-                    step(j, ra);
-                    if (j - NB < 0) break;
-                    fetch(j - 2 * NB, ra);
-                    step(j - NB, rb);
-                }
-            }
-        };
-        if (staged) walk(std::true_type{});
-        else walk(std::false_type{});
-        t_first = tnext;
-        if (a.dh0) {  // the start state's cotangent: cut by a reset at or before the first event
-            const bool z = nr[0] <= min(t_first, T - 1);
-            float* d0 = a.dh0 + (int64_t(b) * N + c) * d;
-#pragma unroll
-            for (int v = 0; v < V; ++v)
-                if (lane + 64 * v < d) d0[lane + 64 * v] = z ? 0.0f : A[v];
-        }
+        walk_cell<IO, V, NB>(a, r, c, e_beg, e_end);
     }
     if (g == 0) {  // exact zeros on the row's padded slots, every wavefront a share
         const int wv = tid >> 6;
@@ -1151,11 +1192,11 @@ __global__ __launch_bounds__(kChainThreads) void chain_bwd(BwdArgs a) {
             const int pe = lane < m ? ev[pw + lane] : 0;
             for (int i = 0; i < m; ++i) {
                 const int q = __builtin_amdgcn_readlane(pe, i);
-                const uint32_t so = uint32_t((q >> 8) * K + (q & 255)) * srow;
+                const uint32_t so = uint32_t((q >> 8) * K + (q & 255)) * r.srow;
 #pragma unroll
                 for (int v = 0; v < V; ++v) {
-                    bstore_f32<IO>(0.0f, rdy, voff[v], so);
-                    bstore_f32<IO>(0.0f, rdg, voff[v], so);
+                    bstore_f32<IO>(0.0f, r.rdy, r.voff[v], so);
+                    bstore_f32<IO>(0.0f, r.rdg, r.voff[v], so);
                 }
             }
         }
@@ -1360,155 +1401,18 @@ __global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
                                  a.h_T ? uint32_t(N) * srow4 : 0u);
     const int nr0 = nr[0];
 
-    auto end_age = [&](int c, int tprev) __attribute__((always_inline)) {
-        int64_t age;
-        if (tprev >= 0 && tprev >= lrT) age = (T - 1) - tprev;
-        else if (lrT >= 0) age = T - lrT;
-        else age = a.age0[int64_t(b) * N + c] + T;
-        a.age_T[int64_t(b) * N + c] = age;
-    };
-
-    // one cell by the whole wavefront, a column a lane and register (lane + 64 v): the cells of more
-    // than kHeavy events, whose chain a wavefront of several cells would walk more slowly, and cell
-    // 0 where the row has padded slots
+    // one cell by the whole wavefront (walk_cell): the cells of more than a.heavy events, whose chain a
+    // wavefront of several cells would walk more slowly, and cell 0 where the row has padded slots
     constexpr int V = L <= 16 ? 1 : 2;
-    constexpr bool want_max = HMAX;
-    uint32_t voff[V], voff4[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-        const bool in = lane + 64 * v < d;
-        voff[v] = in ? uint32_t(lane + 64 * v) * sizeof(IO) : kOob;
-        voff4[v] = in ? uint32_t(lane + 64 * v) * 4u : kOob;
-    }
+    FwdRow<V> r;
+    r.b = b, r.pc0 = pc0, r.nst = nst, r.lrT = lrT, r.pad_begin = pad_begin;
+    r.ev = ev, r.cev = cev, r.nr = nr, r.hm = hm;
+    r.ry = ry, r.rg = rg, r.rho = rho, r.rhs = rhs, r.rdl = rdl;
+    r.srow = srow, r.srow4 = srow4;
+    column_offsets<IO, V>(d, r.voff, r.voff4);
     auto single = [&](auto pad_cell, int ci) __attribute__((always_inline)) {
-        constexpr bool kPadCell = decltype(pad_cell)::value;
-        const int c = c_begin + ci;
-        const int e_beg = uniform(cptr[ci]), e_end = uniform(cptr[ci + 1]);
-        float h[V];
-        const float* h0c = a.h0 + (int64_t(b) * N + c) * d;
-#pragma unroll
-        for (int v = 0; v < V; ++v) h[v] = lane + 64 * v < d ? h0c[lane + 64 * v] : 0.0f;
-        float hold_last[V];  // the state before the latest event (cell 0's padded slots)
-#pragma unroll
-        for (int v = 0; v < V; ++v) hold_last[v] = 0.0f;
-        uint32_t vprev = want_max ? cell_abs_max<V>(h, lane, d) : 0u;
-        int tprev = -1, s = 0;
-        int nrprev = nr[0];  // the first reset after the latest event
-        // cell 0's padded slots at positions below `limit`, in time order (a window of 64 of
-        // them in the lanes)
-        int pp = pad_begin, pwb = -1, pwv = 0;
-        auto flush = [&](int limit) __attribute__((always_inline)) {
-            while (pp < n_slots) {
-                if (pwb < 0 || pp >= pwb + kEvWin) {
-                    pwb = pp;
-                    pwv = lane < n_slots - pp ? ev[pp + lane] : 0x7fffffff;
-                }
-                const int off = pp - pwb;
-                const uint64_t below = ballot(lane >= off && (pwv >> 8) < limit);
-                const int n = __popcll(below);
-                for (int i = 0; i < n; ++i) {
-                    const int q = __builtin_amdgcn_readlane(pwv, off + i);
-                    const int t = q >> 8;
-                    const uint32_t so = uint32_t(t * K + (q & 255)) * srow;
-                    const bool same = t == tprev;
-                    const bool zero = nrprev <= t;
-#pragma unroll
-                    for (int v = 0; v < V; ++v) {
-                        const float now = zero ? 0.0f : h[v];
-                        bstore_f32<IO>(same ? hold_last[v] : now, rho, voff[v], so);
-                        bstore_f32<IO>(same ? h[v] : now, rhs, voff[v], so);
-                    }
-                }
-                pp += n;
-                if (off + n < kEvWin) break;  // the next one is at or after `limit`
-            }
-        };
-        // one event: position t, its slot's byte offsets (so: storage rows, so4: fp32 rows) and
-        // the first reset after t
-        auto update = [&](auto pad_c, int t, uint32_t so, uint32_t so4, int nrq, const IO (&yv)[V],
-                          const IO (&gv)[V]) __attribute__((always_inline)) {
-            constexpr bool kPad = decltype(pad_c)::value;
-            const bool zero = nrprev <= t;  // a reset since the cell's last event
-            if constexpr (want_max) max_interval(hm, s, min(t, nrprev), vprev, lane);
-            if constexpr (kPad) flush(t);
-#pragma unroll
-            for (int v = 0; v < V; ++v) {
-                const float hold = zero ? 0.0f : h[v];
-                const float bg = fast_sigmoid(to_f32(gv[v]));
-                const float cand = fast_tanh(to_f32(yv[v]));
-                const float hn = (1.0f - bg) * hold + bg * cand;
-                bstore_f32<IO>(hold, rho, voff[v], so);
-                bstore_f32<IO>(hn, rhs, voff[v], so);
-                if constexpr (DELTA) bstore(hn - hold, rdl, voff4[v], so4);
-                if constexpr (kPad) hold_last[v] = hold;
-                h[v] = hn;
-            }
-            if constexpr (want_max) vprev = cell_abs_max<V>(h, lane, d);
-            s = t;
-            tprev = t;
-            nrprev = nrq;
-            if constexpr (kPad) flush(t + 1);
-        };
-        // windows of 64 events (one per lane), in batches of 4 with two batches in flight; a
-        // window's positions, slot offsets and next resets are computed for all its events at
-        // once (lane i: event i) and read per event with readlane
-        auto walk = [&](auto staged_c, auto pad_c) __attribute__((always_inline)) {
-            constexpr bool kStaged = decltype(staged_c)::value;
-            for (int w0 = e_beg; w0 < e_end; w0 += kEvWin) {
-                const int m = min(kEvWin, e_end - w0);
-                int evw;
-                if constexpr (kStaged) evw = lane < m ? cev[w0 - pc0 + lane] : 0;
-                else evw = lane < m ? ev[w0 + lane] : 0;
-                const int tw = evw >> 8;
-                const int slw = tw * K + (evw & 255);
-                const uint32_t sow = uint32_t(slw) * srow;
-                const uint32_t so4w = uint32_t(slw) * srow4;
-                const int nrw = lane < m ? nr[tw + 1] : T;
-                IO ya[4][V], ga[4][V], yb[4][V], gb[4][V];
-                auto fetch = [&](int j, IO (&yv)[4][V], IO (&gv)[4][V])
-                                 __attribute__((always_inline)) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const uint32_t so = __builtin_amdgcn_readlane(sow, min(j + i, kEvWin - 1));
-                        fetch_rows<IO, V>(yv[i], gv[i], ry, rg, voff, so, j + i < m);
-                    }
-                };
-                auto step = [&](int j, const IO (&yv)[4][V], const IO (&gv)[4][V])
-                                __attribute__((always_inline)) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        if (j + i < m) {
-                            const int idx = j + i;
-                            update(pad_c, __builtin_amdgcn_readlane(tw, idx),
-                                   __builtin_amdgcn_readlane(sow, idx),
-                                   DELTA ? __builtin_amdgcn_readlane(so4w, idx) : 0u,
-                                   __builtin_amdgcn_readlane(nrw, idx), yv[i], gv[i]);
-                        }
-                    }
-                };
-                fetch(0, ya, ga);
-                for (int j = 0; j < m; j += 2 * 4) {
-                    fetch(j + 4, yb, gb);
-                    step(j, ya, ga);
-                    if (j + 4 >= m) break;
-                    fetch(j + 2 * 4, ya, ga);
-                    step(j + 4, yb, gb);
-                }
-            }
-        };
-        if constexpr (kPadCell) walk(std::false_type{}, std::true_type{});
-        else if (e_end - pc0 <= nst) walk(std::true_type{}, std::false_type{});
-        else walk(std::false_type{}, std::false_type{});
-        if constexpr (kPadCell) flush(T);
-        if (want_max) max_interval(hm, s, min(T, nrprev), vprev, lane);
-        const bool cleared = nrprev < T;  // a reset after the cell's last event
-        if (a.h_T) {
-            float* hTc = a.h_T + (int64_t(b) * N + c) * d;
-#pragma unroll
-            for (int v = 0; v < V; ++v)
-                if (lane + 64 * v < d) hTc[lane + 64 * v] = cleared ? 0.0f : h[v];
-        }
-        if (a.age_T && lane == 0) end_age(c, tprev);
+        constexpr Pads kPads = decltype(pad_cell)::value ? kPadCell : kNoPads;
+        walk_cell<IO, V, 4, DELTA, HMAX, kPads>(a, r, c_begin + ci, uniform(cptr[ci]), uniform(cptr[ci + 1]));
     };
 
     const int heavy = heavy_cells(cptr, order, nc, a.heavy);
@@ -1549,7 +1453,7 @@ __global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) h[i] = cleared ? 0.0f : h[i];
             store4(h, rhT, oh, static_cast<const float*>(nullptr));
-            if (a.age_T && l == 0 && has) end_age(c, -1);
+            if (a.age_T && l == 0 && has) end_age(a, b, c, -1, lrT);
             continue;
         }
         auto abs_max = [&]() __attribute__((always_inline)) {
@@ -1639,7 +1543,7 @@ __global__ __launch_bounds__(kQuadThreads, 5) void chain_fwd4(FwdArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) h[i] = cleared ? 0.0f : h[i];
         store4(h, rhT, oh, static_cast<const float*>(nullptr));
-        if (a.age_T && l == 0 && has) end_age(c, tprev);
+        if (a.age_T && l == 0 && has) end_age(a, b, c, tprev, lrT);
     }
     if constexpr (HMAX) {
         const uint32_t v = wave_max_from_groups<1>(idle);
@@ -1705,114 +1609,13 @@ __global__ __launch_bounds__(kQuadThreads, sizeof(IO) == 4 ? 4 : 5) void chain_b
     const int nr0 = nr[0];
 
     constexpr int V = L <= 16 ? 1 : 2;
-    uint32_t voff[V], voff4[V];
-#pragma unroll
-    for (int v = 0; v < V; ++v) {
-        const bool in = lane + 64 * v < d;
-        voff[v] = in ? uint32_t(lane + 64 * v) * sizeof(IO) : kOob;
-        voff4[v] = in ? uint32_t(lane + 64 * v) * 4u : kOob;
-    }
-    struct Rows {
-        IO y[4][V], g[4][V], h[4][V], s[4][V];
-        float r[4][V];
-    };
+    BwdRow<V> r;
+    r.b = b, r.pc0 = pc0, r.nst = nst, r.ev = ev, r.cev = cev, r.nr = nr;
+    r.ry = ry, r.rg = rg, r.rho = rho, r.rds = rds, r.rdy = rdy, r.rdg = rdg, r.rsh = rsh;
+    r.srow = srow, r.srow4 = srow4;
+    column_offsets<IO, V>(d, r.voff, r.voff4);
     auto single = [&](int ci) __attribute__((always_inline)) {  // a heavy cell, as in chain_fwd4
-        const int c = c_begin + ci;
-        const int e_beg = uniform(cptr[ci]), e_end = uniform(cptr[ci + 1]);
-        const bool staged = e_end - pc0 <= nst;
-        float A[V];
-        {  // the end cotangent, cut by a reset after the cell's last event
-            const int t_last = e_end > e_beg
-                                   ? (uniform(staged ? cev[e_end - 1 - pc0] : ev[e_end - 1]) >> 8)
-                                   : -1;
-            const bool cut = nr[t_last + 1] < T;
-            const float* dhc = a.dh_T ? a.dh_T + (int64_t(b) * N + c) * d : nullptr;
-#pragma unroll
-            for (int v = 0; v < V; ++v)
-                A[v] = (dhc && !cut && lane + 64 * v < d) ? dhc[lane + 64 * v] : 0.0f;
-        }
-        int tnext = T;  // the later event's position
-        int t_first = T;
-        auto walk = [&](auto staged_c) __attribute__((always_inline)) {
-            constexpr bool kStaged = decltype(staged_c)::value;
-            for (int w1 = e_end; w1 > e_beg; w1 -= kEvWin) {
-                const int m = min(kEvWin, w1 - e_beg);
-                const int w0 = w1 - m;
-                int evw;
-                if constexpr (kStaged) evw = lane < m ? cev[w0 - pc0 + lane] : 0;
-                else evw = lane < m ? ev[w0 + lane] : 0;
-                // the window's positions, slot offsets, share offsets and next resets, for all
-                // its events at once (lane i: event i), read per event with readlane
-                const int tw = evw >> 8;
-                const uint32_t sow = uint32_t(tw * K + (evw & 255)) * srow;
-                const uint32_t stw = uint32_t(tw) * srow4;
-                const int nrw = lane < m ? nr[tw + 1] : T;
-                Rows ra, rb;
-                // batch j holds window indices [j - 4 + 1, j], fetched latest first
-                auto fetch = [&](int j, Rows& r) __attribute__((always_inline)) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int idx = j - i;
-                        const uint32_t so = __builtin_amdgcn_readlane(sow, max(idx, 0));
-                        const uint32_t st = __builtin_amdgcn_readlane(stw, max(idx, 0));
-                        const bool in = idx >= 0;
-#pragma unroll
-                        for (int v = 0; v < V; ++v) {
-                            const uint32_t vo = in ? voff[v] : kOob;
-                            r.y[i][v] = bload<IO>(ry, vo, so);
-                            r.g[i][v] = bload<IO>(rg, vo, so);
-                            r.h[i][v] = bload<IO>(rho, vo, so);
-                            r.s[i][v] = bload<IO>(rds, vo, so);
-                            r.r[i][v] = bload<float>(rsh, in ? voff4[v] : kOob, st);
-                        }
-                    }
-                };
-                auto step = [&](int j, const Rows& r) __attribute__((always_inline)) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int idx = j - i;
-                        if (idx >= 0) {
-                            const int t = __builtin_amdgcn_readlane(tw, idx);
-                            const int nrq = __builtin_amdgcn_readlane(nrw, idx);
-                            const uint32_t so = __builtin_amdgcn_readlane(sow, idx);
-                            const bool zero = nrq <= tnext && tnext < T;  // a reset in (t, tnext]
-#pragma unroll
-                            for (int v = 0; v < V; ++v) {
-                                const float carried = (zero ? 0.0f : A[v]) + to_f32(r.s[i][v]);
-                                const float share = r.r[i][v];
-                                const float gg = carried + share;
-                                const float bg = fast_sigmoid(to_f32(r.g[i][v]));
-                                const float cc = fast_tanh(to_f32(r.y[i][v]));
-                                const float dc = bg * gg * (1.0f - cc * cc);
-                                const float db = (cc - to_f32(r.h[i][v])) * gg * (bg * (1.0f - bg));
-                                bstore_f32<IO>(dc, rdy, voff[v], so);
-                                bstore_f32<IO>(db, rdg, voff[v], so);
-                                A[v] = (1.0f - bg) * carried - bg * share;
-                            }
-                            tnext = t;
-                        }
-                    }
-                };
-                fetch(m - 1, ra);
-                for (int j = m - 1; j >= 0; j -= 2 * 4) {
-                    fetch(j - 4, rb);
-                    step(j, ra);
-                    if (j - 4 < 0) break;
-                    fetch(j - 2 * 4, ra);
-                    step(j - 4, rb);
-                }
-            }
-        };
-        if (staged) walk(std::true_type{});
-        else walk(std::false_type{});
-        t_first = tnext;
-        if (a.dh0) {  // the start state's cotangent: cut by a reset at or before the first event
-            const bool z = nr[0] <= min(t_first, T - 1);
-            float* d0 = a.dh0 + (int64_t(b) * N + c) * d;
-#pragma unroll
-            for (int v = 0; v < V; ++v)
-                if (lane + 64 * v < d) d0[lane + 64 * v] = z ? 0.0f : A[v];
-        }
+        walk_cell<IO, V, 4>(a, r, c_begin + ci, uniform(cptr[ci]), uniform(cptr[ci + 1]));
     };
     const int heavy = heavy_cells(cptr, order, nc, a.heavy);
 
