@@ -128,9 +128,18 @@ def _flags(t: Tensor) -> Tensor:
     return t.to(torch.int32).contiguous()
 
 
-def _index(t: Tensor) -> Tensor:
-    """An index tensor an op takes as it is (int32 or int64), contiguous."""
-    return t.contiguous() if t.dtype == torch.int64 else _i32(t)
+def _own(t: Tensor, *inputs: Optional[Tensor]) -> Tensor:
+    """``t``, contiguous; a copy where a gradient can reach one of ``inputs``: the op saves it for its
+    backward, and the caller may reuse its buffer before that (the next position's selection)."""
+    if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in inputs):
+        return t.clone(memory_format=torch.contiguous_format)
+    return t.contiguous()
+
+
+def _index(t: Tensor, *inputs: Optional[Tensor]) -> Tensor:
+    """An index tensor for an op: int64 as :func:`_own` has it, int32 as it is (an int32 buffer has
+    to stay until the backward)."""
+    return _own(t, *inputs) if t.dtype == torch.int64 else _i32(t)
 
 
 #: The dtype code's width bits (include/hsn_ops.h): the kernels read these arrays as they are.
@@ -588,7 +597,7 @@ def gather_concat(u: Optional[Tensor], eps: Tensor, h: Tensor, m: Tensor, cell_i
     if u.dtype != h.dtype or eps.dtype != h.dtype:
         raise ValueError("u, eps and h must have the same state dtype")
     return _eager(gather_op, _gather_body, u.contiguous(), eps.contiguous(), h.contiguous(),
-                  m.to(h.dtype).contiguous(), _index(cell_idx))
+                  m.to(h.dtype).contiguous(), _index(cell_idx, u, eps, h, m))
 
 
 def grouped_unit_mlp(v: Tensor, unit_idx: Tensor, bank: Any, *, static: bool = False,
@@ -622,7 +631,8 @@ def grouped_unit_mlp(v: Tensor, unit_idx: Tensor, bank: Any, *, static: bool = F
     # reach the masters through the cast
     w1 = bank.W1 if w1_flat is None else \
         w1_flat.reshape(bank.in_dim, bank.n_units, bank.hidden).permute(1, 0, 2)
-    out, _ = _eager(mlp_op, _mlp_body, v.to(dtype).contiguous(), _index(unit_idx),
+    out, _ = _eager(mlp_op, _mlp_body, v.to(dtype).contiguous(),
+                    _index(unit_idx, v, w1, bank.b1, bank.W2, bank.b2),
                     w1.to(dtype).contiguous(), bank.b1.to(dtype).contiguous(),
                     bank.W2.to(dtype).contiguous(), bank.b2.to(dtype).contiguous())
     return out
@@ -646,9 +656,10 @@ def csr_messages(h: Tensor, graph: Any, V: Any, cell_idx: Tensor, *,
         raise ValueError("CSR messages need a projection without bias")
     a = graph.edge_weights() if weights is None else weights.reshape(-1)[graph._edge_pos]
     dtype = _dtype_for(h)
-    return _eager(messages_op, _messages_body, h.to(dtype).contiguous(), _index(graph.indptr),
-                  _index(graph.indices), a.to(dtype).contiguous(), V.weight.to(dtype).contiguous(),
-                  _index(cell_idx))
+    flow = (h, a, V.weight)
+    return _eager(messages_op, _messages_body, h.to(dtype).contiguous(), _index(graph.indptr, *flow),
+                  _index(graph.indices, *flow), a.to(dtype).contiguous(),
+                  V.weight.to(dtype).contiguous(), _index(cell_idx, *flow))
 
 
 def _check_valid(valid: Any, shape: tuple, device: torch.device) -> None:
@@ -707,7 +718,8 @@ def gated_delta_update(state: Any, cell_idx: Tensor, c: Tensor, b: Tensor, valid
     _check_valid(valid, tuple(cell_idx.shape), h.device)
     if validate:
         _check_selection(cell_idx, valid, int(h.shape[1]))
+    flow = (h, state.q, c, b)
     hn, qn, age, _ = _eager(state_update_op, _functional, h.contiguous(), state.q.contiguous(),
-                            state.age.contiguous(), _index(cell_idx), valid.contiguous(), c.contiguous(),
-                            b.contiguous())
+                            state.age.contiguous(), _index(cell_idx, *flow), _own(valid, *flow),
+                            c.contiguous(), b.contiguous())
     return _with_state(state, hn, qn, age, state.pos)

@@ -181,6 +181,57 @@ def test_update_adapter_checks_the_selection(ops, cuda_device):
     assert torch.equal((nxt.h.cpu() != 0).any(-1), touched)
 
 
+def _adapter_calls(ops, dev):
+    """Each adapter on int64 indices (and bool flags): ``{name: (its index and flag buffers, call)}``,
+    the call giving a loss to go backward from and the inputs to take gradients of."""
+    g = torch.Generator().manual_seed(3)
+    rnd = lambda *s: (torch.randn(*s, generator=g) * 0.5).to(dev).requires_grad_(True)  # noqa: E731
+    B, K, N, d, M, H, D = 3, 4, 12, 8, 3, 20, 2
+    cells = torch.stack([torch.randperm(N, generator=g)[:K] for _ in range(B)]).to(dev)
+    valid = (torch.rand(B, K, generator=g) < 0.7).to(dev)
+    units = torch.randint(0, M, (B * K,), generator=g).to(dev)
+    graph = _Graph(torch.arange(N + 1, device=dev) * D, torch.randint(0, N, (N * D,), generator=g).to(dev),
+                   rnd(N * D), D)
+    h, m, v, c = rnd(B, N, d), rnd(B, K, d), rnd(B * K, 4 * d), rnd(B, K, d)
+    b = torch.rand(B, K, d, generator=g).to(dev).requires_grad_(True)
+    u, eps, q = rnd(B, d), rnd(B, d), rnd(B, d)
+    bank = types.SimpleNamespace(W1=rnd(M, 4 * d, H), b1=rnd(M, H), W2=rnd(M, H, d), b2=rnd(M, d), d=d,
+                                 in_dim=4 * d, hidden=H, n_units=M, activation_name="gelu")
+    V = nn.Linear(d, d, bias=False).to(dev)
+    from hsn_amd.state import CellGraphState
+
+    state = CellGraphState(h, q, torch.zeros(B, N, dtype=torch.int64, device=dev),
+                           torch.zeros(B, dtype=torch.int64, device=dev))
+
+    def update():
+        nxt = ops.gated_delta_update(state, cells, c, b, valid)
+        return nxt.h.square().sum() + nxt.q.square().sum()
+
+    return {
+        "gather_concat": ([cells], lambda: ops.gather_concat(u, eps, h, m, cells).square().sum(),
+                          (u, eps, h, m)),
+        "grouped_unit_mlp": ([units], lambda: ops.grouped_unit_mlp(v, units, bank).square().sum(),
+                             (v, bank.W1, bank.b1, bank.W2, bank.b2)),
+        "csr_messages": ([graph.indptr, graph.indices, cells],
+                         lambda: ops.csr_messages(h, graph, V, cells).square().sum(),
+                         (h, V.weight, graph._a)),
+        "gated_delta_update": ([cells, valid], update, (h, q, c, b)),
+    }
+
+
+@pytest.mark.parametrize("name", OPS)
+def test_adapters_leave_the_selection_s_buffers_to_the_caller(ops, cuda_device, name):
+    """A training loop may reuse the buffers of a position's int64 selection and bool flags before the
+    backward: the gradients are those of the forward's own values."""
+    buffers, call, inputs = _adapter_calls(ops, cuda_device)[name]
+    want = torch.autograd.grad(call(), inputs)
+    loss = call()
+    for t in buffers:
+        t.copy_(t.flip(0)) if t.dtype != torch.bool else t.logical_not_()
+    for a, w in zip(torch.autograd.grad(loss, inputs), want):
+        assert torch.equal(a, w), name
+
+
 # ---- the raw ops ----------------------------------------------------------------------------
 
 
