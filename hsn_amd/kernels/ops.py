@@ -67,27 +67,31 @@ def available() -> bool:
 
 def prepare_cuda(device: int = 0) -> None:
     """Make the library ready on ``device`` before warm-up or graph capture (the reference's
-    ``prepare_cuda``): load it, then run every raw op and its backward once on tiny inputs there,
-    so no kernel is loaded for the first time inside a capture."""
+    ``prepare_cuda``): load it, then run every raw op and its backward on tiny inputs there, in each
+    storage dtype and with either width of the indices and flags, so no kernel is loaded for the first
+    time inside a capture. The unit MLP runs by rows and in unit order."""
     from .. import _lib
 
     _lib.library()
     dev = torch.device("cuda", device)
     with torch.cuda.device(dev):
-        f = lambda *shape: torch.full(shape, 0.5, device=dev)  # noqa: E731
-        idx = torch.zeros(1, 1, dtype=torch.int32, device=dev)
-        one = torch.ones(1, 1, dtype=torch.int32, device=dev)
-        gather_backward(gather_op(f(1, 4), f(1, 4), f(1, 2, 4), f(1, 1, 4), idx), idx, 2)
-        unit = torch.zeros(1, dtype=torch.int32, device=dev)
-        out, hidden = mlp_op(f(1, 16), unit, f(1, 16, 4), f(1, 4), f(1, 4, 4), f(1, 4))
-        mlp_backward(f(1, 16), unit, f(1, 16, 4), f(1, 4, 4), hidden, out)
-        indptr = torch.tensor([0, 1, 1], dtype=torch.int32, device=dev)
-        edges = torch.zeros(1, dtype=torch.int32, device=dev)
-        m = messages_op(f(1, 2, 4), indptr, edges, f(1), f(4, 4), idx)
-        messages_backward(f(1, 2, 4), indptr, edges, f(1), f(4, 4), idx, m)
-        age = torch.zeros(1, 2, dtype=torch.int32, device=dev)
-        _, _, _, old = update_op(f(1, 2, 4), f(1, 4), age, idx, one, f(1, 1, 4), f(1, 1, 4))
-        update_backward(idx, one, f(1, 1, 4), f(1, 1, 4), old, f(1, 2, 4), f(1, 4))
+        for dtype in _DTYPE:
+            f = lambda *shape: torch.full(shape, 0.5, dtype=dtype, device=dev)  # noqa: E731
+            for wide in (False, True):
+                itype, vtype = (torch.int64, torch.bool) if wide else (torch.int32, torch.int32)
+                i = lambda *shape: torch.zeros(*shape, dtype=itype, device=dev)  # noqa: E731
+                idx, one = i(1, 1), torch.ones(1, 1, dtype=vtype, device=dev)
+                gather_backward(gather_op(f(1, 4), f(1, 4), f(1, 2, 4), f(1, 1, 4), idx), idx, 2)
+                # in unit order: the first in fp32, the last in 16 bits; the others by rows
+                for d, H in ((4, 4), (4, 6), (68, 132)):
+                    out, hidden = mlp_op(f(1, 4 * d), i(1), f(1, 4 * d, H), f(1, H), f(1, H, d), f(1, d))
+                    mlp_backward(f(1, 4 * d), i(1), f(1, 4 * d, H), f(1, H, d), hidden, out)
+                indptr = torch.tensor([0, 1, 1], dtype=itype, device=dev)
+                m = messages_op(f(1, 2, 4), indptr, i(1), f(1), f(4, 4), idx)
+                messages_backward(f(1, 2, 4), indptr, i(1), f(1), f(4, 4), idx, m)
+                age = torch.zeros(1, 2, dtype=itype, device=dev)
+                _, _, _, old = update_op(f(1, 2, 4), f(1, 4), age, idx, one, f(1, 1, 4), f(1, 1, 4))
+                update_backward(idx, one, f(1, 1, 4), f(1, 1, 4), old, f(1, 2, 4), f(1, 4))
         torch.cuda.synchronize(dev)
 
 

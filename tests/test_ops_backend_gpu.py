@@ -232,6 +232,34 @@ def test_adapters_leave_the_selection_s_buffers_to_the_caller(ops, cuda_device, 
         assert torch.equal(a, w), name
 
 
+def test_prepare_cuda_loads_every_form(ops, cuda_device, monkeypatch):
+    """prepare_cuda launches the int64 and bool forms beside the int32 ones, in every storage dtype,
+    and the unit MLP both with and without a workspace."""
+    seen = set()
+    real = ops.call
+
+    def spy(name, *args):
+        if name.startswith("hsn_grouped_unit_mlp_") and name.endswith("_ws"):
+            seen.add((name, args[2], args[-4]))
+        elif name != "hsn_grouped_unit_mlp_workspace":
+            at = {"hsn_grouped_unit_mlp_bwd": -3, "hsn_gather_concat_bwd": -3, "hsn_csr_messages_bwd": -3}
+            seen.add((name, args[at.get(name, -2)]))
+        return real(name, *args)
+
+    monkeypatch.setattr(ops, "call", spy)
+    ops.prepare_cuda(cuda_device.index or 0)
+    for code in range(3):
+        for wide in (0, 1):
+            for name, bits in (("hsn_gather_concat", 0x100), ("hsn_gather_concat_bwd", 0x100),
+                               ("hsn_csr_messages", 0x300), ("hsn_csr_messages_bwd", 0x300),
+                               ("hsn_gated_delta_update_copy", 0x500), ("hsn_gated_delta_update_bwd", 0x500),
+                               ("hsn_grouped_unit_mlp_fwd", 0x100)):
+                assert (name, code | bits * wide) in seen, (name, code, wide)
+            for way in ("fwd", "bwd"):
+                assert (f"hsn_grouped_unit_mlp_{way}_ws", 32 << wide, code) in seen, (way, code, wide)
+        assert ("hsn_grouped_unit_mlp_bwd", code) in seen, code
+
+
 # ---- the raw ops ----------------------------------------------------------------------------
 
 
