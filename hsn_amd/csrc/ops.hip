@@ -304,9 +304,9 @@ void launch_copy_or_zero(const F* src, F* dst, int64_t n, hipStream_t st) {
 
 // A call's index and flag arrays in one instantiation's types (`bits`: the dtype code's width bits).
 template <int W>
-Idx<W> cells_of(const void* p, int bits) { return Idx<W>{p, (bits & HSN_CELLS_I64) != 0}; }
+Idx<W> cells_of(const void* p, int bits) { return index_array<W>(p, (bits & HSN_CELLS_I64) != 0); }
 template <int W>
-Flags<W> flags_of(const void* p, int bits) { return Flags<W>{p, (bits & HSN_VALID_U8) != 0}; }
+Flags<W> flags_of(const void* p, int bits) { return flag_array<W>(p, (bits & HSN_VALID_U8) != 0); }
 
 template <typename F>
 struct RunUpdateCopy {

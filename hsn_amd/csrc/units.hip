@@ -1840,7 +1840,7 @@ void check_dtype(int dtype, const char* who) {
 // A call's index arrays in one instantiation's types (`bits`: the dtype code's width bits).
 constexpr int kWidths = HSN_CELLS_I64 | HSN_GRAPH_I64;
 template <int W>
-Idx<W> index_of(const void* p, int bits, int bit) { return Idx<W>{p, (bits & bit) != 0}; }
+Idx<W> index_of(const void* p, int bits, int bit) { return index_array<W>(p, (bits & bit) != 0); }
 template <int W>
 units::Csr<W> csr_of(const void* indptr, const void* indices, int N, int E, int bits) {
     return {index_of<W>(indptr, bits, HSN_GRAPH_I64), index_of<W>(indices, bits, HSN_GRAPH_I64), N, E};
@@ -1933,7 +1933,7 @@ struct RunMlpBwd {
     static void run(const void* v, const int32_t* unit_idx, const void* W1, const void* W2,
                     const void* hidden, const void* dout, void* dv, void* dW1, void* db1,
                     void* dW2, void* db2, int P, int M, int d, int H, hipStream_t st) {
-        const Idx<kNarrow> idx{unit_idx, 0};
+        const Idx<kNarrow> idx{unit_idx};
         // grad_v through dz1 in fp32 in grad_W2's memory (4-byte aligned, P H floats of room),
         // before the weight-gradient kernel writes grad_W2
         const int dzl = units::dz_lds(P, M, d).bytes, gvl = units::gv_lds(P, M, H).bytes;
