@@ -379,15 +379,16 @@ def test_unit_mlp_and_messages_are_reproducible(ops, cuda_device):
 
 
 @pytest.mark.parametrize("P,M,d,H", [
-    (40, 3, 6, 50),      # d not a multiple of 4: the scanning kernel
-    (64, 4, 16, 77),     # H not a multiple of 4: the row-tile kernel's unaligned loads
-    (20000, 2, 4, 8),    # more pairs than the row-tile kernel's slot table: the scanning kernel
-    (300, 6, 64, 512),   # the reference model's widths, several tiles a unit
-    (2000, 2, 8, 64),    # grad_W2 too small to hold dz1: grad_v in one launch
+    (40, 3, 6, 50),      # d not a multiple of 4: the scanning kernels
+    (64, 4, 16, 77),     # H not a multiple of 4: the row tiles' unaligned loads
+    (20000, 2, 4, 8),    # many pairs of a narrow bank: in unit order
+    (300, 6, 64, 512),   # the reference model's widths: forward by row tiles, backward in unit order
+    (2000, 2, 8, 64),    # both in unit order, units of several blocks
 ])
 def test_unit_mlp_forward_paths_match_oracle(ops, cuda_device, P, M, d, H):
-    """Both forward kernels and both grad_v kernels (by row tiles, and the pair-scanning ones for
-    shapes the first do not take) against the oracle in float64 on fp32 inputs."""
+    """The kernels that the dispatch takes for these shapes, forward and backward, against the oracle in
+    float64 on fp32 inputs (each kind of kernels over all of its shapes:
+    ``test_unit_mlp_by_either_kernels_matches_oracle``)."""
     from oracle import hsn_oracle as O
 
     g = torch.Generator().manual_seed(P + d)
@@ -584,6 +585,7 @@ def _mlp_run(ops, x):
     (700, 6, 64, 512),    # the model's widths, more pairs than the forward of few takes in fp32
     (17000, 2, 4, 8),     # more pairs than the row tiles' slot table: the scanning kernels
     (2000, 2, 8, 64),     # grad_W2 too small to hold dz1: grad_v in one launch by rows
+    (2000, 2, 8, 66),     # the same, W1's rows off the four-element loads (by rows only)
 ])
 def test_unit_mlp_by_either_kernels_matches_oracle(ops, cuda_device, monkeypatch, P, M, d, H, path, dtype,
                                                    index):
@@ -593,6 +595,8 @@ def test_unit_mlp_by_either_kernels_matches_oracle(ops, cuda_device, monkeypatch
     unit's pairs."""
     from oracle import hsn_oracle as O
 
+    if H % 4:
+        path = "by rows"
     x = _mlp_problem(P, M, d, H, dtype, P + d, cuda_device, index)
     _through(monkeypatch, ops, path)
     out, hidden, got = _mlp_run(ops, x)

@@ -438,3 +438,47 @@ def test_a_list_of_more_chunks_than_a_packed_launch_takes(dev):
     dsts = [torch.empty_like(s) for s in srcs]
     assert trainer.copy(dsts, srcs)
     assert all(torch.equal(d, s) for d, s in zip(dsts, srcs))
+
+
+def _adamw_equals_short_lists(trainer, rows, what):
+    """One AdamW, a lerp and a scaling over the lists ``rows`` (parameters, gradients, both moments)
+    bit for bit the same passes over lists of 40 tensors."""
+    c = torch.tensor([0.7], dtype=torch.float64, device=rows[0][0].device)
+    hyper = dict(lr=1e-3, beta1=0.9, beta2=0.999, eps=1e-8, weight_decay=0.01, step=3)
+    want = [[t.clone() for t in row] for row in rows]
+    assert trainer.scale64(rows[1], c) and trainer.adamw(*rows, **hyper) and trainer.lerp(rows[1], rows[0], 0.3)
+    for i in range(0, len(rows[0]), 40):
+        p, g, m, v = (row[i:i + 40] for row in want)
+        assert trainer.scale64(g, c) and trainer.adamw(p, g, m, v, **hyper) and trainer.lerp(g, p, 0.3)
+    for name, got, ref in zip(("params", "grads", "exp_avgs", "exp_avg_sqs"), rows, want):
+        for j, (x, y) in enumerate(zip(got, ref)):
+            assert torch.equal(x, y), f"{what}: {name}[{j}]"
+
+
+def test_wide_descriptors_of_a_long_list(dev):
+    """More than 65535 chunks and more than 88 tensors: the wide descriptors in several launches, of
+    four operands, two and one."""
+    from hsn_amd import trainer
+
+    g = torch.Generator(device=dev).manual_seed(11)
+    sizes = [(1, 1025, 7, 1024, 2000)[i % 5] for i in range(99)] + [67_200_000, 3]
+    rows = [[torch.randn(k, device=dev, generator=g) for k in sizes] for _ in range(4)]
+    rows[3] = [t.square_() for t in rows[3]]
+    _adamw_equals_short_lists(trainer, rows, "a long list")
+
+
+def test_wide_descriptors_of_tensors_far_apart(dev):
+    """Tensors more than 2^32 elements from the row's lowest address: the wide descriptors too."""
+    from hsn_amd import trainer
+
+    g = torch.Generator(device=dev).manual_seed(12)
+    far = torch.empty(2**32 + 4096, device=dev)
+    rows = [[torch.randn(k, device=dev, generator=g) for k in (5, 1030, 300)] for _ in range(4)]
+    for row in rows[:2]:  # parameters and gradients: the first and last tensor at the buffer's ends
+        at = 0 if row is rows[0] else 64
+        row[0] = far[at:at + 5].copy_(row[0])
+        row[2] = far[2**32 + 1024 * (at > 0):][:300].copy_(row[2])
+    rows[3] = [t.square_() for t in rows[3]]
+    _adamw_equals_short_lists(trainer, rows, "far apart")
+    del far, rows
+    torch.cuda.empty_cache()
