@@ -1161,9 +1161,16 @@ hipError_t launch_route(const RouteArgs& a, bool sequential, hipStream_t stream)
     // Two cells a register: contiguous bf16 rows, and K up to 40 of the 128 maxima, so the
     // candidates (about 49 of random logits at 40) rarely pass the 64 lanes. 32768 positions, us,
     // against the general selection: N 2048 K 16 28 (105), K 40 35 (130); N 1024 K 16 24 (37),
-    // every logit equal 92 (209). Not up to N = 512: K 8 21.1 (21.6), every logit equal 75 (58).
+    // every logit equal 92 (209). Not up to N = 512: K 8 21.1 (21.6), every logit equal 75 (58). Above
+    // N = 1024 not under 1024 positions, where the general selection has a workgroup each on the chip: 256
+    // positions N 4096 K 8 5.0 (5.4), every logit equal 19.7 (10.8); 1024 K 8 5.2 (7.4), equal 19.9 (17.5),
+    // K 1 equal 17.4 (9.8). Nor above N = 2048 and K = 32 under 16384: one position of more than 64
+    // candidates then takes as long as all the others (2048 positions K 40 26 (12); 16384: 50 (58)).
     if constexpr (sizeof(IO) == 2) {
-        if (!sequential && a.M == 1 && a.reserved == 0 && a.width == 1 && a.K <= 40 && a.N > 512 &&
+        const int64_t positions = int64_t(a.B) * a.P;
+        const bool enough = a.N <= 1024 ||
+                            (positions >= 1024 && (a.K <= 32 || a.N <= 2048 || positions >= 16384));
+        if (!sequential && a.M == 1 && a.reserved == 0 && a.width == 1 && a.K <= 40 && a.N > 512 && enough &&
             a.N % 8 == 0 && (reinterpret_cast<uintptr_t>(a.logits) & 15) == 0) {
             const dim3 grid((a.P + 3) / 4, a.B);
             auto* const k = a.N <= 1024   ? route_packed<2, IDX>

@@ -909,11 +909,9 @@ PACKED_ROUTES = [
 ]
 
 
-@pytest.mark.parametrize("case", range(len(PACKED_ROUTES)))
-@pytest.mark.parametrize("shift", [0, 1])
-def test_packed_route_matches_oracle(dev, case, shift):
-    """The bf16 router's two cells a register against the oracle, exactly; `shift`: rows off
-    the 16-byte alignment."""
+def _packed_route(dev, case, shift, rows=1, times=1):
+    """The bf16 router on case ``case``'s logits, their rows and positions repeated, against the
+    oracle's decisions on them, exactly."""
     from hsn_amd import window
 
     N, K, kw, kind = PACKED_ROUTES[case]
@@ -930,11 +928,20 @@ def test_packed_route_matches_oracle(dev, case, shift):
         x = torch.where(torch.rand(x.shape, generator=g) < 0.5, 0.0, -0.0)
         x[:, :, 100:100 + K - 1] = 1.0
     logits = x.to(torch.bfloat16)
-    dl = torch.empty(logits.numel() + 8, dtype=logits.dtype, device=dev)[shift:shift + logits.numel()]
-    dl = dl.view(logits.shape).copy_(logits)
+    many = logits.repeat(rows, times, 1, 1)
+    dl = torch.empty(many.numel() + 8, dtype=many.dtype, device=dev)[shift:shift + many.numel()]
+    dl = dl.view(many.shape).copy_(many)
     cost = torch.full((1,), 1.0 / 64)
     cfg = _route_cfg(k=K, **kw)
-    got = [v.cpu() for v in window.route(dl, cost.to(dev), cfg)]
+    got = []
+    for v in window.route(dl, cost.to(dev), cfg):
+        tiles = v.cpu().view(rows, B, times, T, *v.shape[2:])
+        same = tiles[:1, :, :1]
+        if tiles.is_floating_point():
+            assert bool(((tiles == same) | (torch.isnan(tiles) & torch.isnan(same))).all())
+        else:
+            assert torch.equal(tiles, same.expand_as(tiles))
+        got.append(tiles[0, :, 0])
     for t in range(T):
         want = O.router_select(logits[:, t], None, cost, **_oracle_route_kwargs(cfg))
         for name, gv, wv in zip(("cells", "units", "valid", "theta", "refreshed"), got, want):
@@ -943,3 +950,28 @@ def test_packed_route_matches_oracle(dev, case, shift):
                 assert bool((same | (torch.isnan(gv[:, t]) & torch.isnan(wv))).all()), (t, gv[:, t], wv)
             else:
                 assert torch.equal(gv[:, t].long(), wv.long()), (name, t, gv[:, t], wv)
+
+
+@pytest.mark.parametrize("case", range(len(PACKED_ROUTES)))
+@pytest.mark.parametrize("shift", [0, 1])
+def test_packed_route_matches_oracle(dev, case, shift):
+    """The bf16 router's two cells a register against the oracle, exactly (above N = 1024 the general
+    selection: these are ten positions); `shift`: rows off the 16-byte alignment."""
+    _packed_route(dev, case, shift)
+
+
+@pytest.mark.parametrize("case", [i for i, c in enumerate(PACKED_ROUTES) if c[0] > 1024])
+def test_packed_route_of_many_positions_matches_oracle(dev, case):
+    """The same above N = 1024 from 1024 positions on, where two cells go a register; with more than 32
+    slots of more than 2048 cells from 16384."""
+    _packed_route(dev, case, 0, rows=11, times=10)
+
+
+def test_packed_route_of_the_most_cells_and_slots(dev):
+    """40 slots of 4096 cells: 16384 positions take two cells a register, 1100 the general selection."""
+    PACKED_ROUTES.append((4096, 40, dict(), "plain"))
+    try:
+        _packed_route(dev, len(PACKED_ROUTES) - 1, 0, rows=11, times=10)
+        _packed_route(dev, len(PACKED_ROUTES) - 1, 0, rows=52, times=32)
+    finally:
+        PACKED_ROUTES.pop()
