@@ -253,8 +253,11 @@ def _trainer_main(args) -> int:
     kernel_ms = sum(a.elapsed_time(b) for a, b in events) / args.steps
     achieved = elements * TRAINER_BYTES_PER_ELEMENT / (kernel_ms * 1e-3) / 1e9
     # tensors a launch of the AdamW pass: 200 in a packed launch (lists of up to 65535 chunks of
-    # 1024 elements), else 88
-    per_launch = 200 if sum(-(-n // 1024) for n in sizes) <= 65535 else 88
+    # 1024 elements, each operand's tensors within 2^32 elements of its lowest address), else 88
+    starts = [[t.data_ptr() for t in row] for row in (params, grads, exp_avgs, exp_avg_sqs)]
+    packed = (sum(-(-n // 1024) for n in sizes) <= 65535
+              and all((max(row) - min(row)) // 4 < 1 << 32 for row in starts))
+    per_launch = 200 if packed else 88
     launches = -(-len([n for n in sizes if n]) // per_launch)
     result = {
         "metric": f"trainer AdamW pass elements/sec ({args.trainer} parameter list, 1 GPU)",
