@@ -1217,12 +1217,13 @@ __global__ __launch_bounds__(kChainThreads) void chain_bwd(BwdArgs a) {
 // cells side by side, 1.64 with the heavy ones alone).
 //
 // What bounds it is a cell's chain of loads, with 64 / L cells' rows in flight a wavefront. Measured
-// (us, forward and backward; one cell a wavefront in brackets): B64 T512 N1024 d64 K16 bf16 97 and
-// 115 (120 and 128); B128 T128 N512 d128 K8 fp32 75 and 104 (80 and 123), 67 and 93 being their
-// bytes at a copy's 5.03 TB/s; B256 T1024 N4096 d64 K32 bf16 Zipf 1639 and 1695 (1734 and 1654). Eight
-// wavefronts a workgroup and about two workgroups a CU: four wavefronts 109 and 120 at the first
-// shape, 2048 workgroups 149 and 131. Batches of four events 97 and 116, all cells' 200 events side
-// by side (kHeavy 200) 111 and 122.
+// (us, forward and backward; one cell a wavefront in brackets): B64 T512 N1024 d64 K16 bf16 96 and
+// 106 (128 and 133); B128 T128 N512 d128 K8 fp32 70 and 101 (80 and 123), 67 and 93 being their
+// bytes at a copy's 5.03 TB/s; B256 T1024 N4096 d64 K32 bf16 Zipf 1681 and 1717 (1734 forward; the backward
+// on one card 1804 against 1786: a few cells' serial chains, which nothing beside them shortens, but 1472
+// against 1661 for evenly popular cells). Four wavefronts a workgroup instead of eight 109 and 120 at the
+// first shape, batches of four events 97 and 116. The cells a workgroup and the events up to which a
+// cell is walked beside others follow from the shape (quad_cells, quad_heavy in chain.hip).
 //
 // The row maxima are marked per interval between a cell's events on three scales (positions, 16
 // and 256 of them), at most five LDS atomics an interval instead of one a position and wavefront;

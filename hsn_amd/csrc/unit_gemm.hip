@@ -14,13 +14,15 @@
 //               gelu(z1)^T dout with the column sums (the bias gradients); a unit of more than
 //               one block leaves fp32 partial sums, which gm_dw_sum adds in block order.
 //
-// What bounds it: the fp32 matrix rate. Every product is v_mfma_f32_16x16x4_f32 on operands
-// widened to fp32 (16-bit inputs multiply exactly, dz1 and gelu(z1) stay fp32), 2 P (4d H + H d)
-// FLOP a pass against about 150 TFLOP/s. A tile of 32 rows reuses a unit's weights 32 times; the
-// kernels over 16 pairs a workgroup (units.hip) read them once a 16 pairs, and their weight
-// gradients walk all of a unit's pairs in one workgroup a tile, 16 pairs a step. Forward and
-// backward together, M 8, d 64, H 512 (us): P 8192 bf16 971 -> 250, P 256 fp32 76.7 -> 55 (of
-// both, 19 and 11 are the launches that narrowed the indices: unit_order reads either width).
+// Every product is v_mfma_f32_16x16x4_f32 on operands widened to fp32 (16-bit inputs multiply
+// exactly, dz1 and gelu(z1) stay fp32), 2 P (4d H + H d) FLOP a pass against some 150 TFLOP/s. What
+// bounds it at P 8192: the loads between a step's products (matrix busy 0.39 in gm_hidden, 0.49 in
+// gm_dv, 0.30 in gm_dw, 0.15 to 0.17 in the others); at P 256: each launch's serial steps on few
+// workgroups. A tile of 32 rows reuses a unit's weights 32 times; the kernels over 16 pairs a workgroup
+// (units.hip) read them once a 16 pairs, and their weight gradients walk all of a unit's pairs in one
+// workgroup a tile, 16 pairs a step. Forward and backward together, M 8, d 64, H 512 (us): P 8192 bf16
+// 971 -> 229; P 256 fp32 77 -> 52, the forward of few pairs by units.hip (few_pairs below). Of the 971 and
+// 77, 19 and 11 are launches that narrowed the indices: unit_order reads either width.
 #include <algorithm>
 #include <type_traits>
 
