@@ -68,8 +68,9 @@ def available() -> bool:
 def prepare_cuda(device: int = 0) -> None:
     """Make the library ready on ``device`` before warm-up or graph capture (the reference's
     ``prepare_cuda``): load it, then run every raw op and its backward on tiny inputs there, in each
-    storage dtype and with either width of the indices and flags, so no kernel is loaded for the first
-    time inside a capture. The unit MLP runs by rows and in unit order."""
+    storage dtype and with either width of the indices and flags, so no code object is loaded for the
+    first time inside a capture. The unit MLP runs by rows and in unit order; kernels that only larger
+    calls take (more pairs, more edges) are in the same code objects."""
     from .. import _lib
 
     _lib.library()
